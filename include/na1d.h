@@ -223,6 +223,27 @@ int na1d_fused_backward_strided_dropout(void *dq, void *dk, void *dv, float *drp
                                         void *stream);
 
 /*
+ * Dilated windows in one launch: slot j of row t meets row t + (j - left) * dilation (the reference computes this on
+ * the CPU only, models/PCF_NATransformer.py:101-116,158-170).  The rows of one residue class t mod dilation only ever
+ * meet each other; the kernels work on all classes of all sequences side by side, each in place.  p_drop, seed:
+ * attention dropout as in na1d_fused_forward_dropout (0 switches it off), rows named by their place in the whole
+ * sequence.  lse is [N*H, T] as in the undilated calls.  dilation >= 1; 1 is na1d_fused_forward_strided /
+ * na1d_fused_backward_strided, whose other arguments and limits apply (head_dim > 128: NA1D_ERR_UNSUPPORTED).
+ * The workspace of the backward has na1d_fused_backward_dilated_workspace_bytes() bytes.
+ */
+int na1d_fused_forward_dilated(void *out, float *lse, const void *q, const void *k, const void *v, const float *rpb,
+                               const int32_t *t_valid, int64_t N, int64_t H, int64_t T, int64_t C, int64_t W,
+                               int64_t left, int64_t dilation, float scale, int dtype, const int64_t *qkv_strides,
+                               const int64_t *out_strides, float p_drop, uint64_t seed, void *stream);
+int na1d_fused_backward_dilated(void *dq, void *dk, void *dv, float *drpb, const void *q, const void *k, const void *v,
+                                const void *dout, const float *lse, const float *rpb, const int32_t *t_valid, int64_t N,
+                                int64_t H, int64_t T, int64_t C, int64_t W, int64_t left, int64_t dilation, float scale,
+                                int dtype, const int64_t *qkv_strides, const int64_t *out_strides, float p_drop,
+                                uint64_t seed, void *workspace, int64_t workspace_bytes, void *stream);
+int64_t na1d_fused_backward_dilated_workspace_bytes(int64_t N, int64_t H, int64_t T, int64_t C, int64_t W, int64_t left,
+                                                    int64_t dilation, int dtype);
+
+/*
  * Dense ("global") attention over whole sequences, forward and backward: replaces the body of the reference's
  * GlobalAttention.forward between the head split and the head merge (models/PCF_NATransformer.py:199-221),
  *     attn = softmax((q * scale) @ k^T + mask);  out = attn @ v

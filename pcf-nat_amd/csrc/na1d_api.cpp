@@ -62,6 +62,13 @@ int check_layout(const int64_t *strides, const Geom &g, na1d::Layout &l) {
     return NA1D_OK;
 }
 
+// Geometry and layouts of a dilated window's residue classes.
+void dilate(Geom &g, na1d::Layout &in, na1d::Layout &outl, int64_t dilation) {
+    na1d::set_dilation(g, dilation);
+    in.row *= g.dilation;
+    outl.row *= g.dilation;
+}
+
 #define NA1D_CHECK(...)                     \
     Geom g;                                 \
     {                                       \
@@ -333,6 +340,59 @@ int na1d_fused_backward_strided_dropout(void *dq, void *dk, void *dv, float *drp
     if (!mfma_allowed()) return NA1D_ERR_UNSUPPORTED;
     return mfma_fused_bwd(dq, dk, dv, drpb, q, k, v, nullptr, dout, lse, rpb, t_valid, g, in, outl, scale, dtype,
                           (float *)workspace, workspace ? workspace_bytes : 0, (hipStream_t)stream);
+}
+
+int na1d_fused_forward_dilated(void *out, float *lse, const void *q, const void *k, const void *v, const float *rpb,
+                               const int32_t *t_valid, int64_t N, int64_t H, int64_t T, int64_t C, int64_t W,
+                               int64_t left, int64_t dilation, float scale, int dtype, const int64_t *qkv_strides,
+                               const int64_t *out_strides, float p_drop, uint64_t seed, void *stream) {
+    if (N < 0 || H < 1 || N > INT64_MAX / H || dilation < 1) return NA1D_ERR_SHAPE;
+    NA1D_CHECK(out, q, k, N * H, T, C, W, left, H, dtype, g);
+    if (bad_scale(scale)) return NA1D_ERR_SCALE;
+    if (!v) return NA1D_ERR_NULL;
+    if (misaligned(v)) return NA1D_ERR_ALIGN;
+    if (!(p_drop >= 0.f && p_drop < 1.f) || T > 0x7fffffffLL) return NA1D_ERR_SHAPE;
+    na1d::Layout in, outl;
+    const int ls = check_layout(qkv_strides, g, in), lo = check_layout(out_strides, g, outl);
+    if (ls != NA1D_OK || lo != NA1D_OK) return ls != NA1D_OK ? ls : lo;
+    if (!mfma_allowed()) return NA1D_ERR_UNSUPPORTED;
+    dilate(g, in, outl, dilation);
+    g.drop = na1d::make_dropout(p_drop, seed, (uint32_t)g.dilation, 0, (uint32_t)g.seq_rows);
+    return mfma_fused_fwd(out, lse, q, k, v, rpb, t_valid, g, in, outl, scale, dtype, (hipStream_t)stream);
+}
+
+int na1d_fused_backward_dilated(void *dq, void *dk, void *dv, float *drpb, const void *q, const void *k, const void *v,
+                                const void *dout, const float *lse, const float *rpb, const int32_t *t_valid, int64_t N,
+                                int64_t H, int64_t T, int64_t C, int64_t W, int64_t left, int64_t dilation, float scale,
+                                int dtype, const int64_t *qkv_strides, const int64_t *out_strides, float p_drop,
+                                uint64_t seed, void *workspace, int64_t workspace_bytes, void *stream) {
+    if (N < 0 || H < 1 || N > INT64_MAX / H || dilation < 1) return NA1D_ERR_SHAPE;
+    NA1D_CHECK(dq, q, k, N * H, T, C, W, left, H, dtype, g);
+    if (bad_scale(scale)) return NA1D_ERR_SCALE;
+    if (!dk || !dv || !v || !dout || !lse) return NA1D_ERR_NULL;
+    if (misaligned(dk) || misaligned(dv) || misaligned(v) || misaligned(dout)) return NA1D_ERR_ALIGN;
+    if (workspace && misaligned(workspace)) return NA1D_ERR_ALIGN;
+    if (!(p_drop >= 0.f && p_drop < 1.f) || T > 0x7fffffffLL) return NA1D_ERR_SHAPE;
+    na1d::Layout in, outl;
+    const int ls = check_layout(qkv_strides, g, in), lo = check_layout(out_strides, g, outl);
+    if (ls != NA1D_OK || lo != NA1D_OK) return ls != NA1D_OK ? ls : lo;
+    if (!mfma_allowed()) return NA1D_ERR_UNSUPPORTED;
+    dilate(g, in, outl, dilation);
+    g.drop = na1d::make_dropout(p_drop, seed, (uint32_t)g.dilation, 0, (uint32_t)g.seq_rows);
+    return mfma_fused_bwd(dq, dk, dv, drpb, q, k, v, nullptr, dout, lse, rpb, t_valid, g, in, outl, scale, dtype,
+                          (float *)workspace, workspace ? workspace_bytes : 0, (hipStream_t)stream);
+}
+
+int64_t na1d_fused_backward_dilated_workspace_bytes(int64_t N, int64_t H, int64_t T, int64_t C, int64_t W, int64_t left,
+                                                    int64_t dilation, int dtype) {
+    if (N < 0 || H < 1 || N > INT64_MAX / H || dilation < 1) return NA1D_ERR_SHAPE;
+    Geom g;
+    const int st = check_shape(N * H, T, C, W, left, H, dtype, g);
+    if (st < 0) return st;
+    if (st > 0 || !mfma_allowed()) return 0;
+    if (T > 0x7fffffffLL) return NA1D_ERR_SHAPE;
+    na1d::set_dilation(g, dilation);
+    return na1d::mfma::fused_bwd_workspace_bytes(g, dtype);
 }
 
 int na1d_global_forward(void *out, float *lse, const void *q, const void *k, const void *v, const int32_t *t_valid,

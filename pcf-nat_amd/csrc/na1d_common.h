@@ -117,7 +117,21 @@ struct Geom {
     int C, W, L;      // head_dim, window, left
     int H;            // heads (B % H == 0); 1 for the un-fused entry points
     Dropout drop;     // fused operator only; off by default
+    // Dilated windows (fused matrix-core kernels only).  Slot j of row t is row t + (j - L) * dilation, so the rows of
+    // one residue class t mod dilation only ever meet each other: `classes` independent sequences interleaved in every
+    // one of the B, T rows long at most (classes >= short_from have one row less), of seq_rows rows in all.  The
+    // layouts that go with it hold the row stride of a class.
+    int dilation = 1, classes = 1, short_from = 1;
+    int64_t seq_rows = 0;          // 0: T
 };
+inline void set_dilation(Geom &g, int64_t dilation) {
+    const int64_t rows = g.T;
+    if (dilation > rows) dilation = rows;      // every row meets itself alone either way
+    g.dilation = g.classes = (int)dilation;
+    g.short_from = rows % dilation ? (int)(rows % dilation) : g.classes;
+    g.seq_rows = rows;
+    g.T = (rows + dilation - 1) / dilation;
+}
 
 // Element strides of a [samples, heads, T, C] view of a tensor whose channels are contiguous.  The packed
 // [B = samples * heads, T, C] tensor of the reference is {H*T*C, T*C, C}; a head-interleaved projection

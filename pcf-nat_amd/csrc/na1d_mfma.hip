@@ -30,7 +30,7 @@ fused_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__
                  const char *__restrict__ k, const char *__restrict__ v, const float *__restrict__ rpb,
                  const int32_t *__restrict__ t_valid, uint32_t items, int T, int W, int L, int H, int tiles, int nt,
                  int strips, float scale, uint32_t strips_magic, uint32_t heads_magic, Strides in, Strides outl,
-                 int shift_arg, Dropout drop) {
+                 int shift_arg, Dropout drop, Classes cls) {
     const int shift = NBV == 3 ? 16 : shift_arg;     // three key blocks always start one tile before the query tile
     constexpr int CS = C * HG;                       // channels of a staged row
     constexpr int NW = HG > 1 ? kGroupWaves : kWaves; // waves of the workgroup
@@ -42,6 +42,7 @@ fused_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__
     constexpr bool PK = ONE == 2;
     fetch_args_now(out, lse, q, k, v, rpb, t_valid, items, T, W, L, H, tiles, nt, strips, scale, strips_magic, heads_magic,
                    in.sample, in.head, in.pitch, in.width, outl.sample, outl.head, outl.pitch, outl.width, shift_arg);
+    if constexpr (!PK) fetch_args_now(cls.count);
     if constexpr (DROP) fetch_args_now(drop.threshold, drop.seed_lo, drop.seed_hi, drop.inv_keep, drop.row_stride, drop.row_offset, drop.seq_rows);
     // dynamic LDS (launch_fwd): K and V regions of nt+2 tiles starting one tile before the strip (row 16*i0 - 16:
     // copies that start on a tile boundary measured faster here than ones that start at the first key, and the
@@ -79,6 +80,11 @@ fused_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__
         i0 = wi.strip * nt;
         i1 = min(i0 + nt, tiles);
     }
+    int cr = 0;                                      // residue class of a dilated window
+    if (!PK && cls.count > 1) {
+        cr = split_class(sample, T, cls);
+        if constexpr (DROP) drop.row_offset = (uint32_t)cr;
+    }
     const uint32_t head = head0 + hw, b = sample * H + head;
     const int g = lane >> 4, n = lane & 15;
 
@@ -86,7 +92,7 @@ fused_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__
     // fetches nothing beyond what this strip needs
     // first what the strip copies need, and nothing else: a workgroup's life starts with the time to its first copy
     const int in_pitch = PK ? 2 * C : in.pitch;
-    const int64_t in_off = PK ? (int64_t)((uint64_t)lin_pk * (uint32_t)(T * 2 * C)) : sample * in.sample + head0 * in.head;
+    const int64_t in_off = PK ? (int64_t)((uint64_t)lin_pk * (uint32_t)(T * 2 * C)) : sample * in.sample + head0 * in.head + (int64_t)(cr * cls.in_row);
     const int key_bytes = (ONE ? T : min(T, 16 * (i1 + 1))) * in_pitch, qry_bytes = (ONE ? T : min(T, 16 * i1)) * in_pitch;
     const Rsrc qs = make_rsrc(q + in_off, qry_bytes), ks = make_rsrc(k + in_off, key_bytes);
     const Rsrc vs = make_rsrc(v + in_off, key_bytes);
@@ -120,14 +126,19 @@ fused_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__
     BiasTable bias_raw;                      // (the wait for the copies covers this load too, wherever it is issued)
     load_bias_table(bias_raw, rpb ? rpb + head * W : nullptr, W, lane);
     const int out_pitch = PK ? 2 * C : outl.pitch, out_width = PK ? 2 * C : outl.width;
-    const int64_t out_off = PK ? in_off : sample * outl.sample + head * outl.head;
+    const int64_t out_off = PK ? in_off : sample * outl.sample + head * outl.head + (int64_t)(cr * cls.out_row);
     const Rsrc os = make_rsrc(out + out_off, T * out_pitch);
-    const Rsrc ls = make_rsrc(lse ? lse + (int64_t)b * T : nullptr, lse ? T * 4 : 0);
+    const int lse_pitch = PK ? 4 : 4 * cls.d;
+    const Rsrc ls = make_rsrc(lse ? lse + ((int64_t)b * (PK ? T : cls.rows) + cr) : nullptr, lse ? T * lse_pitch : 0);
     const bool out_whole_lines = stores_whole_lines(out_pitch, C, 0);
     const bool out_grouped = HG > 1 && outl.head == 2 * C && outl.width == 2 * C && outl.pitch >= HG * 2 * C;
 
     int tv = T;
-    if (t_valid) tv = max(0, min(T, load_uniform_i32(t_valid, sample)));
+    if (t_valid) {
+        tv = load_uniform_i32(t_valid, sample);
+        if (!PK && cls.count > 1) tv = class_valid(tv, cr, cls);
+        tv = max(0, min(T, tv));
+    }
     // The matrix core adds the bias for nothing: accumulators start at rpb / scale (-inf outside the window), so
     // x = q.k + rpb / scale comes out of the instruction, z = x * scale * log2(e) is the logit in the log2 domain,
     // and exp2(z - max z) is one multiply-add per slot on the way into the exponential (scale > 0).
@@ -267,7 +278,7 @@ fused_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__
         } else {
             store_tile<C>(os, qrow * out_pitch, ow, g, out_whole_lines, out_width);
         }
-        if (lse && g == 0) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(lse_row), ls, qrow * 4, 0, 0);
+        if (lse && g == 0) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(lse_row), ls, qrow * lse_pitch, 0, 0);
     }
     if (HG > 1 && out_grouped) {
         // The heads of a group lie side by side in the output too: the strip's output rows, collected in the Q
@@ -276,7 +287,7 @@ fused_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__
         barrier_lds();
         constexpr int kRounds = (region_bytes<CS>(MT) / kChunk + NW - 1) / NW;
         constexpr int kChunkRows = kChunk / LL::kRowBytes;
-        const Rsrc gs = make_rsrc(out + sample * outl.sample + head0 * outl.head, min(T, 16 * i1) * outl.pitch);
+        const Rsrc gs = make_rsrc(out + sample * outl.sample + head0 * outl.head + (int64_t)(cr * cls.out_row), min(T, 16 * i1) * outl.pitch);
         const int lane_off = direct_lane_offset<CS>(wave, lane, outl.pitch, HG * outl.width);
         const int chunks = region_bytes<CS>(i1 - i0) / kChunk;
 #pragma unroll
@@ -302,7 +313,7 @@ template <class DT, int C, int HG>
 int launch_fwd_hg(void *out, float *lse, const void *q, const void *k, const void *v, const float *rpb,
                   const int32_t *t_valid, const Geom &g, const Layout &in, const Layout &outl, float scale,
                   hipStream_t s) {
-    const Split sp = make_split(g.B / HG, g.T, HG > 1 ? kGroupTiles : Strip<C>::kMaxTiles);
+    const Split sp = make_split(g.B / HG * g.classes, g.T, HG > 1 ? kGroupTiles : Strip<C>::kMaxTiles);
     if (!items_ok(sp, g) || !strides_ok(in, g) || !strides_ok(outl, g)) return NA1D_ERR_UNSUPPORTED;
     const bool two = window_blocks(g) == 2;
     // the kernel's form: 0 strips of longer sequences or grouped heads, 1 whole sequences, 2 whole sequences of packed
@@ -332,7 +343,7 @@ int launch_fwd_hg(void *out, float *lse, const void *q, const void *k, const voi
                   (const char *)q, (const char *)k, (const char *)v,
                   rpb, t_valid, (uint32_t)sp.items, (int)g.T, g.W, g.L, g.H, sp.tiles, sp.nt, sp.strips, scale,
                   div_magic(sp.strips), div_magic(g.H / HG), byte_strides(in, g), byte_strides(outl, g), window_shift(g),
-                  g.drop);
+                  g.drop, classes_of(g, in, outl));
     return launch_status();
 }
 
@@ -402,7 +413,7 @@ fused_bwd_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__restrict_
                  const char *__restrict__ dout, const float *__restrict__ lse, const float *__restrict__ rpb,
                  const int32_t *__restrict__ t_valid, uint32_t items, int T, int W, int L, int H, int tiles, int nt,
                  int strips, float scale, float *__restrict__ drpb_partial, int kv_bytes, uint32_t strips_magic,
-                 uint32_t heads_magic, Strides in, Strides outl, int shift_arg, Dropout drop) {
+                 uint32_t heads_magic, Strides in, Strides outl, int shift_arg, Dropout drop, Classes cls) {
     const int shift = NBV == 3 ? 16 : shift_arg;     // three key blocks always start one tile before the query tile
     using LL = Lds<C>;
     constexpr int CT = C / 16;
@@ -412,6 +423,7 @@ fused_bwd_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__restrict_
                    outl.sample, outl.head, outl.pitch, outl.width, shift_arg);
     if constexpr (DROP) fetch_args_now(drop.threshold, drop.seed_lo, drop.seed_hi, drop.inv_keep, drop.row_stride, drop.row_offset, drop.seq_rows);
     constexpr bool PK = ONE == 2;
+    if constexpr (!PK) fetch_args_now(cls.count);
     constexpr int HALO = ONE ? 0 : 1;                      // query tiles either side of the strip whose scores pass 2 needs
     constexpr int kRowsQ = (MT + 2 * HALO) * 16;
     constexpr int TPW = (MT + 2 * HALO + kWaves - 1) / kWaves;    // query tiles per wave, at most
@@ -456,23 +468,29 @@ fused_bwd_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__restrict_
         i0 = wi.strip * nt;
         i1 = min(i0 + nt, tiles);
     }
-    const uint32_t b = ONE ? item : sample * H + head;       // one strip per sequence: the item is the sequence
+    int cr = 0;                                              // residue class of a dilated window
+    if (!PK && cls.count > 1) {
+        cr = split_class(sample, T, cls);
+        if constexpr (DROP) drop.row_offset = (uint32_t)cr;
+    }
+    const uint32_t b = PK ? item : sample * H + head;        // packed whole sequences: the item is the sequence
     const int g = lane >> 4, n = lane & 15;
 
     const int in_pitch = PK ? 2 * C : in.pitch, out_pitch = PK ? 2 * C : outl.pitch;
     const int in_width = PK ? 2 * C : in.width;
-    const int64_t in_off = PK ? (int64_t)((uint64_t)item * (uint32_t)(T * 2 * C)) : sample * in.sample + head * in.head;
-    const int64_t out_off = PK ? in_off : sample * outl.sample + head * outl.head;
+    const int64_t in_off = PK ? (int64_t)((uint64_t)item * (uint32_t)(T * 2 * C)) : sample * in.sample + head * in.head + (int64_t)(cr * cls.in_row);
+    const int64_t out_off = PK ? in_off : sample * outl.sample + head * outl.head + (int64_t)(cr * cls.out_row);
     {
         const int key_bytes = (ONE ? T : min(T, 16 * (i1 + 2))) * in_pitch;
         const int qry_rows = ONE ? T : min(T, 16 * (i1 + HALO));
         const Rsrc ks = make_rsrc(k + in_off, key_bytes), vs = make_rsrc(v + in_off, key_bytes);
         const Rsrc qs = make_rsrc(q + in_off, qry_rows * in_pitch), gs = make_rsrc(dout + out_off, qry_rows * out_pitch);
-        const Rsrc ls = make_rsrc(lse + (int64_t)b * T, T * 4);
+        const int lse_pitch = PK ? 4 : 4 * cls.d;
+        const Rsrc ls = make_rsrc(lse + ((int64_t)b * (PK ? T : cls.rows) + cr), T * lse_pitch);
         const int lane_off = PK ? direct_lane_offset<C>(wave, lane) : direct_lane_offset<C>(wave, lane, in.pitch, in.width);
         const int lane_off_g = PK ? lane_off : direct_lane_offset<C>(wave, lane, outl.pitch, outl.width);
         // lse of the query-side rows, one per lane (natural log; rows past the region's end are never read)
-        if (64 * wave < kRowsQ) load_to_lds<4, 0>(ls, (LDS_PTR(char))(lse_lds + 64 * wave), (16 * (i0 - HALO) + tid) * 4);
+        if (64 * wave < kRowsQ) load_to_lds<4, 0>(ls, (LDS_PTR(char))(lse_lds + 64 * wave), (16 * (i0 - HALO) + tid) * lse_pitch);
         if constexpr (PK) {           // the pitch is the default argument, a constant
             stage_direct<C, MT + 1 + NBV, kReadOnceBwd>(ks, -16 - shift, k_lds, nt + 1 + NBV, wave, lane_off);
             stage_direct<C, MT, kReadOnceBwd>(qs, 0, q_lds, nt, wave, lane_off);
@@ -499,7 +517,11 @@ fused_bwd_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__restrict_
     load_bias_table(bias_raw, rpb ? rpb + head * W : nullptr, W, lane);
 
     int tv = T;
-    if (t_valid) tv = max(0, min(T, load_uniform_i32(t_valid, sample)));
+    if (t_valid) {
+        tv = load_uniform_i32(t_valid, sample);
+        if (!PK && cls.count > 1) tv = class_valid(tv, cr, cls);
+        tv = max(0, min(T, tv));
+    }
     // as in the forward: the accumulators start at rpb / scale, z = x * scale * log2(e) - lse is one multiply-add
     const float scale2 = scale * kLog2e;
     const float inv_scale = __builtin_amdgcn_rcpf(scale);
@@ -764,7 +786,7 @@ int launch_bwd(void *dq, void *dk, void *dv, float *drpb, const void *q, const v
                const void *dout, const float *lse, const float *rpb, const int32_t *t_valid, const Geom &g,
                const Layout &in, const Layout &outl, float scale, float *workspace, int64_t workspace_bytes,
                hipStream_t s) {
-    const Split sp = make_split(g.B, g.T, StripBwd<C>::kMaxTiles, kBwdMinItems);
+    const Split sp = make_split(g.B * g.classes, g.T, StripBwd<C>::kMaxTiles, kBwdMinItems);
     if (!items_ok(sp, g) || !strides_ok(in, g) || !strides_ok(outl, g)) return NA1D_ERR_UNSUPPORTED;
     // a workspace that is passed is used or refused: falling back to atomics would silently give up the fixed order
     // the caller asked for
@@ -802,16 +824,16 @@ int launch_bwd(void *dq, void *dk, void *dv, float *drpb, const void *q, const v
     launch_kernel(kern, (unsigned)sp.items, lds, s, (char *)dq, (char *)dk, (char *)dv, drpb, (const char *)q,
                   (const char *)k, (const char *)v, (const char *)dout, lse, rpb, t_valid, (uint32_t)sp.items, (int)g.T,
                   g.W, g.L, g.H, sp.tiles, sp.nt, sp.strips, scale, partial, kv_bytes, div_magic(sp.strips),
-                  div_magic(g.H), ib, ob, window_shift(g), g.drop);
+                  div_magic(g.H), ib, ob, window_shift(g), g.drop, classes_of(g, in, outl));
     // not behind a launch that was refused (events set on a capturing stream): the sums it would fold do not exist
     if (partial && drpb && !launch_events().refused)
-        drpb_reduce_kernel<kPartialStride><<<(unsigned)(g.H * g.W), 128, 0, s>>>(drpb, partial, (int)(g.B / g.H), g.H, sp.strips, g.W);
+        drpb_reduce_kernel<kPartialStride><<<(unsigned)(g.H * g.W), 128, 0, s>>>(drpb, partial, (int)(g.B / g.H * g.classes), g.H, sp.strips, g.W);
     return launch_status();
 }
 
 template <class DT, int C>
 int64_t bwd_workspace(const Geom &g) {
-    return make_split(g.B, g.T, StripBwd<C>::kMaxTiles, kBwdMinItems).items * kPartialStride * (int64_t)sizeof(float);
+    return make_split(g.B * g.classes, g.T, StripBwd<C>::kMaxTiles, kBwdMinItems).items * kPartialStride * (int64_t)sizeof(float);
 }
 
 int fused_bwd(void *dq, void *dk, void *dv, float *drpb, const void *q, const void *k, const void *v,

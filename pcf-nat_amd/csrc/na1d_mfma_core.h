@@ -515,11 +515,34 @@ struct Strides {
 inline Strides byte_strides(const Layout &l, const Geom &g) {
     return Strides{2 * l.sample, 2 * l.head, (int)(2 * l.row), 2 * g.C};
 }
+// Dilated windows as the kernels take them (see Geom): a launch has `classes` sequences to every one of the tensors',
+// class r starting r rows behind it with every dilation-th row its own (the pitches are those of the class).
+struct Classes {
+    int d, count, short_from, rows;      // dilation, classes, first class that is one row shorter, rows of a whole sequence
+    int in_row, out_row;                 // bytes from one row of a whole sequence to the next
+    uint32_t magic;                      // div_magic(count)
+};
+// The launch's sample number -> sample of the tensors (in place) and residue class, whose length T becomes.
+__device__ inline int split_class(uint32_t &sample, int &T, const Classes &c) {
+    const uint32_t all = sample;
+    sample = (uint32_t)(((uint64_t)all * c.magic) >> 32);
+    const int r = (int)(all - sample * (uint32_t)c.count);
+    if (r >= c.short_from) --T;
+    return r;
+}
+// Valid rows of class r in a sequence of `tv` valid rows.
+__device__ inline int class_valid(int tv, int r, const Classes &c) { return tv > r ? (tv - r + c.d - 1) / c.d : 0; }
+
 // Offsets inside one sequence are 32-bit: the rows of a sequence, plus the halo rows the copies ask for
 // beyond its end, must span less than 2^30 bytes.
 inline bool strides_ok(const Layout &l, const Geom &g) { return l.row >= g.C && g.T + 96 <= (1 << 29) / l.row; }
 inline bool items_ok(const Split &sp, const Geom &g) {
-    return sp.items <= 0x7fffff00LL && div_magic_ok(sp.items, g.H) && div_magic_ok(sp.items, sp.strips);
+    return sp.items <= 0x7fffff00LL && div_magic_ok(sp.items, g.H) && div_magic_ok(sp.items, sp.strips) &&
+           div_magic_ok(sp.items, g.classes);
+}
+inline Classes classes_of(const Geom &g, const Layout &in, const Layout &out) {
+    return Classes{g.dilation, g.classes, g.short_from, (int)(g.seq_rows ? g.seq_rows : g.T), (int)(2 * in.row / g.dilation),
+                   (int)(2 * out.row / g.dilation), div_magic(g.classes)};
 }
 
 // Workgroup id -> (sample, head, strip).  Heads vary fastest, then strips: workgroups that run side by side

@@ -45,7 +45,7 @@ wide_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__r
                 const char *__restrict__ k, const char *__restrict__ v, const float *__restrict__ rpb,
                 const int32_t *__restrict__ t_valid, uint32_t items, int T, int W, int L, int H, int tiles, int nt,
                 int strips, float scale, uint32_t strips_magic, uint32_t heads_magic, Strides in, Strides outl,
-                int shift, Dropout drop) {
+                int shift, Dropout drop, Classes cls) {
     using LL = Lds<C>;
     constexpr int CT = C / 16;
     constexpr int MT = Strip<C>::kMaxTiles;
@@ -66,15 +66,24 @@ wide_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__r
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const WorkItem wi = work_item(blockIdx.x, items, strips, strips_magic, H, heads_magic);
-    const uint32_t b = wi.sample * H + wi.head, sample = wi.sample, head = wi.head;
+    uint32_t sample = wi.sample;
+    const uint32_t head = wi.head;
+    int cr = 0;                                              // residue class of a dilated window
+    if (cls.count > 1) {
+        cr = split_class(sample, T, cls);
+        if constexpr (DROP) drop.row_offset = (uint32_t)cr;
+    }
+    const uint32_t b = sample * H + head;
     const int i0 = wi.strip * nt, i1 = min(i0 + nt, tiles);
     const int g = lane >> 4, n = lane & 15;
 
-    const int64_t in_off = sample * in.sample + head * in.head, out_off = sample * outl.sample + head * outl.head;
+    const int64_t in_off = sample * in.sample + head * in.head + (int64_t)(cr * cls.in_row);
+    const int64_t out_off = sample * outl.sample + head * outl.head + (int64_t)(cr * cls.out_row);
+    const int lse_pitch = 4 * cls.d;
     const int key_rows = max(0, min(T, 16 * (i0 - sb + kt)));
     const Rsrc qs = make_rsrc(q + in_off, min(T, 16 * i1) * in.pitch), ks = make_rsrc(k + in_off, key_rows * in.pitch);
     const Rsrc vs = make_rsrc(v + in_off, key_rows * in.pitch), os = make_rsrc(out + out_off, T * outl.pitch);
-    const Rsrc ls = make_rsrc(lse ? lse + (int64_t)b * T : nullptr, lse ? T * 4 : 0);
+    const Rsrc ls = make_rsrc(lse ? lse + ((int64_t)b * cls.rows + cr) : nullptr, lse ? T * lse_pitch : 0);
     const bool out_whole_lines = stores_whole_lines(outl.pitch, C, 0);
     {
         const int lane_off = direct_lane_offset<C>(wave, lane, in.pitch, in.width);
@@ -85,7 +94,7 @@ wide_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__r
     }
 
     int tv = T;
-    if (t_valid) tv = max(0, min(T, t_valid[sample]));
+    if (t_valid) tv = max(0, min(T, cls.count > 1 ? class_valid(t_valid[sample], cr, cls) : t_valid[sample]));
     const float scale2 = scale * kLog2e;
 
     RowLane<C> k_lane, q_lane;
@@ -164,7 +173,7 @@ wide_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__r
         store_tile<C>(os, qrow * outl.pitch, ow, g, out_whole_lines, outl.width);   // rows past T are dropped by the store
         if (g == 0)
             __builtin_amdgcn_raw_buffer_store_b32(
-                __float_as_uint((m + __builtin_amdgcn_logf(sum)) * kLn2), ls, qrow * 4, 0, 0);
+                __float_as_uint((m + __builtin_amdgcn_logf(sum)) * kLn2), ls, qrow * lse_pitch, 0, 0);
     }
 }
 
@@ -172,7 +181,7 @@ template <class DT, int C, int NBV>
 int launch_wide_fwd_n(void *out, float *lse, const void *q, const void *k, const void *v, const float *rpb,
                       const int32_t *t_valid, const Geom &g, const Layout &in, const Layout &outl, float scale,
                       int shift, hipStream_t s) {
-    const Split sp = make_split(g.B, g.T, Strip<C>::kMaxTiles);
+    const Split sp = make_split(g.B * g.classes, g.T, Strip<C>::kMaxTiles);
     if (!items_ok(sp, g) || !strides_ok(in, g) || !strides_ok(outl, g)) return NA1D_ERR_UNSUPPORTED;
     auto kern = g.drop.threshold ? wide_fwd_kernel<DT, C, NBV, true> : wide_fwd_kernel<DT, C, NBV, false>;
     const int kt = sp.nt - 1 + NBV + ((shift & 15) ? 1 : 0);
@@ -181,7 +190,8 @@ int launch_wide_fwd_n(void *out, float *lse, const void *q, const void *k, const
     note_kernel("wide_fwd_kernel", DT::tag, C, NBV, g.drop.threshold != 0);
     launch_kernel(kern, (unsigned)sp.items, lds, s, (char *)out, lse, (const char *)q, (const char *)k, (const char *)v,
                   rpb, t_valid, (uint32_t)sp.items, (int)g.T, g.W, g.L, g.H, sp.tiles, sp.nt, sp.strips, scale,
-                  div_magic(sp.strips), div_magic(g.H), byte_strides(in, g), byte_strides(outl, g), shift, g.drop);
+                  div_magic(sp.strips), div_magic(g.H), byte_strides(in, g), byte_strides(outl, g), shift, g.drop,
+                  classes_of(g, in, outl));
     return launch_status();
 }
 
@@ -239,7 +249,7 @@ wide_bwd_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__restrict__
                 const char *__restrict__ dout, const float *__restrict__ lse, const float *__restrict__ rpb,
                 const int32_t *__restrict__ t_valid, uint32_t items, int T, int W, int L, int H, int tiles, int nt,
                 int strips, float scale, float *__restrict__ drpb_partial, int kv_bytes, uint32_t strips_magic,
-                uint32_t heads_magic, Strides in, Strides outl, int shift, Dropout drop) {
+                uint32_t heads_magic, Strides in, Strides outl, int shift, Dropout drop, Classes cls) {
     using LL = Lds<C>;
     constexpr int CT = C / 16;
     constexpr int kScoreTile = 16 * 16 * 2;                // one 16x16 tile of 16-bit scores
@@ -267,21 +277,30 @@ wide_bwd_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__restrict__
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const WorkItem wi = work_item(blockIdx.x, items, strips, strips_magic, H, heads_magic);
-    const uint32_t item = wi.item, b = wi.sample * H + wi.head, sample = wi.sample, head = wi.head;
+    uint32_t sample = wi.sample;
+    const uint32_t item = wi.item, head = wi.head;
+    int cr = 0;                                              // residue class of a dilated window
+    if (cls.count > 1) {
+        cr = split_class(sample, T, cls);
+        if constexpr (DROP) drop.row_offset = (uint32_t)cr;
+    }
+    const uint32_t b = sample * H + head;
     const int i0 = wi.strip * nt, i1 = min(i0 + nt, tiles);
     const int g = lane >> 4, n = lane & 15;
     const int q0 = i0 - hb;                                 // first query-side tile
 
-    const int64_t in_off = sample * in.sample + head * in.head, out_off = sample * outl.sample + head * outl.head;
+    const int64_t in_off = sample * in.sample + head * in.head + (int64_t)(cr * cls.in_row);
+    const int64_t out_off = sample * outl.sample + head * outl.head + (int64_t)(cr * cls.out_row);
+    const int lse_pitch = 4 * cls.d;
     {
         const int key_rows = max(0, min(T, 16 * (q0 + ktiles) - shift));
         const int qry_rows = max(0, min(T, 16 * (q0 + qtiles)));
         const Rsrc ks = make_rsrc(k + in_off, key_rows * in.pitch), vs = make_rsrc(v + in_off, key_rows * in.pitch);
         const Rsrc qs = make_rsrc(q + in_off, qry_rows * in.pitch), gs = make_rsrc(dout + out_off, qry_rows * outl.pitch);
-        const Rsrc ls = make_rsrc(lse + (int64_t)b * T, T * 4);
+        const Rsrc ls = make_rsrc(lse + ((int64_t)b * cls.rows + cr), T * lse_pitch);
         const int lane_off = direct_lane_offset<C>(wave, lane, in.pitch, in.width);
         const int lane_off_g = direct_lane_offset<C>(wave, lane, outl.pitch, outl.width);
-        load_to_lds<4, 0>(ls, (LDS_PTR(char))(lse_lds + 64 * wave), (16 * q0 + tid) * 4);
+        load_to_lds<4, 0>(ls, (LDS_PTR(char))(lse_lds + 64 * wave), (16 * q0 + tid) * lse_pitch);
         constexpr int KT = kWideQueryTiles + NBV - 1;
         stage_direct<C, KT, kReadShared>(ks, 16 * q0 - shift, k_lds, ktiles, wave, lane_off, in.pitch);
         stage_direct<C, kWideQueryTiles, kReadShared>(qs, 16 * q0, q_lds, qtiles, wave, lane_off, in.pitch);
@@ -291,7 +310,7 @@ wide_bwd_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__restrict__
     }
 
     int tv = T;
-    if (t_valid) tv = max(0, min(T, t_valid[sample]));
+    if (t_valid) tv = max(0, min(T, cls.count > 1 ? class_valid(t_valid[sample], cr, cls) : t_valid[sample]));
     const float scale2 = scale * kLog2e;
     const float mask2 = kMaskValue * kLog2e;
 
@@ -497,7 +516,7 @@ inline bool wide_bwd_split(const Geom &g, const WideCover &c, Split &sp, int &kv
     int mt = w.mt;
     while (mt >= 1 && wide_bwd_lds<C>(mt, c.nbv, w, kv_bytes) > 160 * 1024) --mt;   // LDS of one CU
     if (mt < 1) return false;
-    sp = make_split(g.B, g.T, mt);
+    sp = make_split(g.B * g.classes, g.T, mt);
     lds = wide_bwd_lds<C>(sp.nt, c.nbv, w, kv_bytes);
     return true;
 }
@@ -523,9 +542,9 @@ int launch_wide_bwd_n(void *dq, void *dk, void *dv, float *drpb, const void *q, 
     launch_kernel(kern, (unsigned)sp.items, lds, s, (char *)dq, (char *)dk, (char *)dv, drpb, (const char *)q,
                   (const char *)k, (const char *)v, (const char *)dout, lse, rpb, t_valid, (uint32_t)sp.items, (int)g.T,
                   g.W, g.L, g.H, sp.tiles, sp.nt, sp.strips, scale, partial, kv_bytes, div_magic(sp.strips), div_magic(g.H),
-                  byte_strides(in, g), byte_strides(outl, g), c.shift, g.drop);
+                  byte_strides(in, g), byte_strides(outl, g), c.shift, g.drop, classes_of(g, in, outl));
     if (partial && drpb && !launch_events().refused)
-        drpb_reduce_kernel<kWidePartialStride><<<(unsigned)(g.H * g.W), 128, 0, s>>>(drpb, partial, (int)(g.B / g.H), g.H,
+        drpb_reduce_kernel<kWidePartialStride><<<(unsigned)(g.H * g.W), 128, 0, s>>>(drpb, partial, (int)(g.B / g.H * g.classes), g.H,
                                                                                      sp.strips, g.W);
     return launch_status();
 }

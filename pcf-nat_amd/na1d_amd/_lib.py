@@ -26,7 +26,8 @@ SYMBOLS = _UNFUSED + ("na1d_fused_forward", "na1d_fused_backward", "na1d_fused_b
                       "na1d_fused_forward_dropout", "na1d_fused_backward_dropout",
                       "na1d_fused_backward_noalloc", "na1d_force_generic", "na1d_profile_last_kernel",
                       "na1d_fused_forward_strided_dropout", "na1d_fused_backward_strided_dropout",
-                      "na1d_version", "na1d_status_string")
+                      "na1d_fused_forward_dilated", "na1d_fused_backward_dilated",
+                      "na1d_fused_backward_dilated_workspace_bytes", "na1d_version", "na1d_status_string")
 UNSUPPORTED = -8
 
 _lib = None
@@ -80,6 +81,13 @@ def load():
     lib.na1d_fused_backward_strided_dropout.restype = _int
     lib.na1d_fused_backward_strided_dropout.argtypes = [_ptr] * 11 + [_i64] * 6 + [_f32, _int, _ptr, _ptr, _f32, _u64,
                                                                                 _i64, _i64, _i64, _ptr, _i64, _ptr]
+    lib.na1d_fused_forward_dilated.restype = _int
+    lib.na1d_fused_forward_dilated.argtypes = [_ptr] * 7 + [_i64] * 7 + [_f32, _int, _ptr, _ptr, _f32, _u64, _ptr]
+    lib.na1d_fused_backward_dilated.restype = _int
+    lib.na1d_fused_backward_dilated.argtypes = [_ptr] * 11 + [_i64] * 7 + [_f32, _int, _ptr, _ptr, _f32, _u64, _ptr, _i64,
+                                                                          _ptr]
+    lib.na1d_fused_backward_dilated_workspace_bytes.restype = _i64
+    lib.na1d_fused_backward_dilated_workspace_bytes.argtypes = [_i64] * 7 + [_int]
     lib.na1d_fused_backward_noalloc.restype = _int
     lib.na1d_fused_backward_noalloc.argtypes = [_ptr] * 12 + [_i64] * 6 + [_f32, _int, _ptr]
     lib.na1d_force_generic.restype = _int
@@ -213,6 +221,42 @@ def call_fused_backward_strided(dq, dk, dv, drpb, q, k, v, dout, lse, rpb, t_val
     if st != UNSUPPORTED:
         check(st, "na1d_fused_backward_strided")
     return st
+
+
+def call_fused_forward_dilated(out, lse, q, k, v, rpb, t_valid, W, left, dilation, scale, dropout=None):
+    """All residue classes of a dilated window in one launch, on ``[N, H, T, C]`` views as in
+    :func:`call_fused_forward_strided`.  ``dropout``: ``None`` or ``(p, seed)``."""
+    lib = load()
+    N, H, T, C = q.shape
+    assert q.stride() == k.stride() == v.stride()
+    with torch.cuda.device(out.device):
+        st = lib.na1d_fused_forward_dilated(_p(out), _p(lse), _p(q), _p(k), _p(v), _p(rpb), _p(t_valid), N, H, T, C, W,
+                                            left, dilation, scale, dtype_tag(q.dtype), _strides3(q), _strides3(out),
+                                            *(dropout or (0.0, 0)), _stream(out))
+    if st != UNSUPPORTED:
+        check(st, "na1d_fused_forward_dilated")
+    return st
+
+
+def call_fused_backward_dilated(dq, dk, dv, drpb, q, k, v, dout, lse, rpb, t_valid, W, left, dilation, scale,
+                                workspace=None, dropout=None):
+    lib = load()
+    N, H, T, C = q.shape
+    assert q.stride() == k.stride() == v.stride() == dq.stride() == dk.stride() == dv.stride()
+    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    with torch.cuda.device(dq.device):
+        st = lib.na1d_fused_backward_dilated(_p(dq), _p(dk), _p(dv), _p(drpb), _p(q), _p(k), _p(v), _p(dout), _p(lse),
+                                             _p(rpb), _p(t_valid), N, H, T, C, W, left, dilation, scale,
+                                             dtype_tag(q.dtype), _strides3(q), _strides3(dout), *(dropout or (0.0, 0)),
+                                             _p(workspace), ws_bytes, _stream(dq))
+    check(st, "na1d_fused_backward_dilated")
+
+
+def fused_backward_dilated_workspace_bytes(N, H, T, C, W, left, dilation, dtype) -> int:
+    n = load().na1d_fused_backward_dilated_workspace_bytes(N, H, T, C, W, left, dilation, dtype_tag(dtype))
+    if n < 0:
+        check(int(n), "na1d_fused_backward_dilated_workspace_bytes")
+    return int(n)
 
 
 def call_global_forward(out, lse, q, k, v, t_valid, B, H, T, C, scale, dropout=None):

@@ -22,38 +22,44 @@ def _residue_lengths(t_valid, r, d):
     return None if t_valid is None else ((t_valid - r + d - 1) // d).clamp_(min=0).to(torch.int32)
 
 
-def _strided_or_packed_forward(out4, lse, q4, k4, v4, rpb, t_valid, W, left, scale, dropout=None):
-    """Forward on ``[N, H, T, C]`` views through the strided entry point, or - for shapes it does not cover -
-    on packed copies through the packed one.  Returns the packed output when it had to be made.  ``dropout``:
-    ``None`` or ``(p, seed, row_stride, row_offset, seq_rows)``."""
-    if _lib.call_fused_forward_strided(out4, lse, q4, k4, v4, rpb, t_valid, W, left, scale, dropout=dropout) == 0:
-        return None
-    if dropout is not None and len(dropout) > 2 and tuple(dropout[2:4]) != (1, 0):
+def _forward_views(out4, q4, k4, v4, rpb, t_valid, W, left, scale, dilation, dropout):
+    """Forward on ``[N, H, T, C]`` views.  One launch where a matrix-core kernel covers the shape; otherwise (head_dim
+    above 128) the residue classes of the dilated window one after the other on packed copies.  Returns
+    ``(lses, packed_outs)``, the latter ``None`` for the one launch."""
+    N, H, T, C = q4.shape
+    lse = torch.empty((N * H, T), dtype=torch.float32, device=q4.device)
+    if _lib.call_fused_forward_dilated(out4, lse, q4, k4, v4, rpb, t_valid, W, left, dilation, scale, dropout=dropout) == 0:
+        return [lse], None
+    if dropout is not None and dilation > 1:
         raise _lib.NA1DError("attention dropout with dilated windows needs head_dim <= 128 (the packed entry points "
                              "name rows by their place in the tensor they are given)")
-    N, H, T, C = q4.shape
-    qp, kp, vp = (z.contiguous().view(N * H, T, C) for z in (q4, k4, v4))
-    op = torch.empty_like(qp)
-    _lib.call_fused_forward(op, lse, qp, kp, vp, rpb, t_valid, N * H, H, T, C, W, left, scale,
-                            dropout=None if dropout is None else dropout[:2])
-    out4.copy_(op.view(N, H, T, C))
-    return op
+    lses, packed_outs = [], []
+    for r in range(min(dilation, T)):
+        qp, kp, vp = (_residue(z, r, dilation).contiguous() for z in (q4, k4, v4))
+        t = qp.shape[2]
+        op, lse = torch.empty_like(qp), torch.empty((N * H, t), dtype=torch.float32, device=q4.device)
+        _lib.call_fused_forward(op, lse, qp, kp, vp, rpb, _residue_lengths(t_valid, r, dilation), N * H, H, t, C, W, left,
+                                scale, dropout=dropout)
+        _residue(out4, r, dilation).copy_(op)
+        lses.append(lse)
+        packed_outs.append(op)
+    return lses, packed_outs
 
 
-def _strided_or_packed_backward(dq4, dk4, dv4, drpb, q4, k4, v4, packed_out, dout4, lse, rpb, t_valid, W, left, scale, ws,
-                                dropout=None):
-    if packed_out is None:
-        st = _lib.call_fused_backward_strided(dq4, dk4, dv4, drpb, q4, k4, v4, dout4, lse, rpb, t_valid, W, left, scale,
-                                              workspace=ws, dropout=dropout)
-        assert st == 0
+def _backward_views(dq4, dk4, dv4, drpb, q4, k4, v4, packed_outs, dout4, lses, rpb, t_valid, W, left, scale, dilation, ws,
+                    dropout):
+    if packed_outs is None:
+        _lib.call_fused_backward_dilated(dq4, dk4, dv4, drpb, q4, k4, v4, dout4, lses[0], rpb, t_valid, W, left, dilation,
+                                         scale, workspace=ws, dropout=dropout)
         return
-    N, H, T, C = q4.shape
-    qp, kp, vp, gp = (z.contiguous().view(N * H, T, C) for z in (q4, k4, v4, dout4))
-    dqp, dkp, dvp = torch.empty_like(qp), torch.empty_like(kp), torch.empty_like(vp)
-    _lib.call_fused_backward(dqp, dkp, dvp, drpb, qp, kp, vp, packed_out, gp, lse, rpb, t_valid, N * H, H, T, C, W, left,
-                             scale, workspace=ws, dropout=None if dropout is None else dropout[:2])
-    for dst, src in ((dq4, dqp), (dk4, dkp), (dv4, dvp)):
-        dst.copy_(src.view(N, H, T, C))
+    N, H, _, C = q4.shape
+    for r, (lse, op) in enumerate(zip(lses, packed_outs)):
+        qp, kp, vp, gp = (_residue(z, r, dilation).contiguous() for z in (q4, k4, v4, dout4))
+        dqp, dkp, dvp = torch.empty_like(qp), torch.empty_like(kp), torch.empty_like(vp)
+        _lib.call_fused_backward(dqp, dkp, dvp, drpb, qp, kp, vp, op, gp, lse, rpb, _residue_lengths(t_valid, r, dilation),
+                                 N * H, H, qp.shape[2], C, W, left, scale, workspace=ws, dropout=dropout)
+        for dst, src in ((dq4, dqp), (dk4, dkp), (dv4, dvp)):
+            _residue(dst, r, dilation).copy_(src)
 
 
 def _deterministic_workspace_bytes(B, H, T, C, win_size, left, dilation, dtype):
@@ -73,6 +79,8 @@ def _deterministic_workspace(B, H, T, C, win_size, left, like, dilation=1):
     if nbytes <= 0:
         raise _lib.NA1DError("deterministic=True: no fixed-order reduction of the bias gradient for head_dim %d "
                              "(it covers head_dim <= 128)" % C)
+    if dilation > 1:          # one launch over all classes
+        nbytes = _lib.fused_backward_dilated_workspace_bytes(B // H, H, T, C, win_size, left, dilation, like.dtype)
     return torch.empty(nbytes, dtype=torch.uint8, device=like.device)
 
 
@@ -99,19 +107,9 @@ class _FusedNA1D(torch.autograd.Function):
                                     dropout=dropout)
             ctx.save_for_backward(q, k, v, out, rpb, t_valid, lse)
             return out
-        # Dilation d: slot j of row t is row t + (j - left) * d, so the rows of one residue class t mod d only
-        # ever meet each other - d independent, undilated problems on every d-th row, read and written in place.
         shape4 = (B // num_heads, num_heads, T, C)
-        q4, k4, v4, o4 = (z.view(shape4) for z in (q, k, v, out))
-        lses, ctx.packed_outs = [], []
-        for r in range(min(dilation, T)):
-            qr = _residue(q4, r, dilation)
-            lse = torch.empty((B, qr.shape[2]), dtype=torch.float32, device=q.device)
-            ctx.packed_outs.append(_strided_or_packed_forward(
-                _residue(o4, r, dilation), lse, qr, _residue(k4, r, dilation), _residue(v4, r, dilation), rpb,
-                _residue_lengths(t_valid, r, dilation), win_size, left, scale,
-                dropout=None if dropout is None else (*dropout, dilation, r, T)))     # rows named by their place in T
-            lses.append(lse)
+        lses, ctx.packed_outs = _forward_views(*(z.view(shape4) for z in (out, q, k, v)), rpb, t_valid, win_size, left,
+                                               scale, dilation, dropout)
         ctx.save_for_backward(q, k, v, out, rpb, t_valid, *lses)
         return out
 
@@ -132,12 +130,9 @@ class _FusedNA1D(torch.autograd.Function):
                                      B, num_heads, T, C, win_size, left, scale, workspace=ws, dropout=ctx.dropout)
         else:
             shape4 = (B // num_heads, num_heads, T, C)
-            views = [z.view(shape4) for z in (dq, dk, dv, q, k, v, dout)]
-            for r, lse in enumerate(lses):
-                a = [_residue(z, r, dilation) for z in views]
-                _strided_or_packed_backward(a[0], a[1], a[2], drpb, a[3], a[4], a[5], ctx.packed_outs[r], a[6], lse, rpb,
-                                            _residue_lengths(t_valid, r, dilation), win_size, left, scale, ws,
-                                            dropout=None if ctx.dropout is None else (*ctx.dropout, dilation, r, T))
+            dq4, dk4, dv4, q4, k4, v4, g4 = (z.view(shape4) for z in (dq, dk, dv, q, k, v, dout))
+            _backward_views(dq4, dk4, dv4, drpb, q4, k4, v4, ctx.packed_outs, g4, lses, rpb, t_valid, win_size, left, scale,
+                            dilation, ws, ctx.dropout)
         if drpb is not None:
             drpb = drpb.view(ctx.rpb_shape)
         return dq, dk, dv, drpb, None, None, None, None, None, None, None, None
@@ -206,15 +201,7 @@ class _FusedNA1DQKV(torch.autograd.Function):
         q4, k4, v4 = (qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3))       # [N, H, T, C] views
         out = torch.empty((N, T, H, C), dtype=qkv.dtype, device=qkv.device)
         o4 = out.permute(0, 2, 1, 3)
-        lses, ctx.packed_outs = [], []
-        for r in range(min(dilation, T)):                                         # see _FusedNA1D.forward
-            qr = _residue(q4, r, dilation)
-            lse = torch.empty((N * H, qr.shape[2]), dtype=torch.float32, device=qkv.device)
-            ctx.packed_outs.append(_strided_or_packed_forward(
-                _residue(o4, r, dilation), lse, qr, _residue(k4, r, dilation), _residue(v4, r, dilation), rpb,
-                _residue_lengths(t_valid, r, dilation), win_size, left, scale,
-                dropout=None if dropout is None else (*dropout, dilation, r, T)))
-            lses.append(lse)
+        lses, ctx.packed_outs = _forward_views(o4, q4, k4, v4, rpb, t_valid, win_size, left, scale, dilation, dropout)
         ctx.save_for_backward(qkv, rpb, t_valid, *lses)
         ctx.geom = (win_size, left, scale, deterministic, dilation)
         return out.view(N, T, H * C)
@@ -231,13 +218,9 @@ class _FusedNA1DQKV(torch.autograd.Function):
             drpb = torch.zeros((H, win_size), dtype=torch.float32, device=qkv.device)
             if deterministic:
                 ws = _deterministic_workspace(N * H, H, T, C, win_size, left, qkv, dilation)
-        views = [dqkv[:, :, i].permute(0, 2, 1, 3) for i in range(3)] + [qkv[:, :, i].permute(0, 2, 1, 3) for i in range(3)]
-        for r, lse in enumerate(lses):
-            a = [_residue(z, r, dilation) for z in views]
-            _strided_or_packed_backward(a[0], a[1], a[2], drpb, a[3], a[4], a[5], ctx.packed_outs[r],
-                                        _residue(g4, r, dilation), lse, rpb, _residue_lengths(t_valid, r, dilation),
-                                        win_size, left, scale, ws,
-                                        dropout=None if ctx.dropout is None else (*ctx.dropout, dilation, r, T))
+        dq4, dk4, dv4, q4, k4, v4 = (z[:, :, i].permute(0, 2, 1, 3) for z in (dqkv, qkv) for i in range(3))
+        _backward_views(dq4, dk4, dv4, drpb, q4, k4, v4, ctx.packed_outs, g4, lses, rpb, t_valid, win_size, left, scale,
+                        dilation, ws, ctx.dropout)
         if drpb is not None:
             drpb = drpb.view(ctx.rpb_shape)
         return dqkv, drpb, None, None, None, None, None, None, None

@@ -1000,3 +1000,36 @@ def test_no_entry_point_writes_outside_its_outputs(geom):
     for name, (buf, view, pad) in {**outs, **f32}.items():
         assert (buf[:pad] == 3.0).all() and (buf[pad + view.numel():] == 3.0).all(), name
         assert torch.isfinite(view.float()).all(), name
+
+
+# classes of 17 and 16 rows (the last tile of the shorter one is empty), fewer rows than classes, a class boundary at
+# every strip, 48 channels, a wide window, one class of a single row
+@pytest.mark.parametrize("geom,D", [((2, 4, 33, 16, 27, 13), 2), ((2, 2, 5, 32, 15, 7), 9), ((2, 4, 259, 32, 15, 7), 2),
+                                    ((2, 3, 130, 48, 20, 9), 3), ((2, 2, 97, 32, 65, 32), 3), ((1, 2, 34, 16, 5, 2), 33)])
+@pytest.mark.parametrize("p_drop", [0.0, 0.25])
+def test_dilated_window_in_one_launch_at_class_edges(geom, D, p_drop):
+    """Every residue class of every sequence in one launch, packed and in the projection layout, against the oracle at
+    the tolerance of the other parity tests; the two layouts agree bit for bit."""
+    N, H, T, C, W, L = geom
+    dtype, seed = torch.float16, 99
+    q, k, v, do = make_inputs(N * H, T, C, W, 31, dtype, n=4, scale=C ** -0.5)
+    rpb = torch.randn(H, W, generator=torch.Generator().manual_seed(8)) * 0.3
+    pad = torch.tensor([0, min(T - 1, T // 3 + 1)])[:N]
+    keep = O.dropout_keep(N * H, T, W, p_drop, seed) if p_drop else None
+    qf, kf, vf = q.float(), k.float(), v.float()
+    want, _, _ = O.na1d_forward(qf, kf, vf, W, L, rpb, pad, H, D, keep=keep, p_drop=p_drop)
+    grads = O.na1d_backward(qf, kf, vf, do.float(), W, L, rpb, pad, H, D, keep=keep, p_drop=p_drop)
+    tv = (T - pad).to(torch.int32).cuda()
+    qd, kd, vd = (t.cuda().requires_grad_(True) for t in (q, k, v))
+    rd = rpb.cuda().requires_grad_(True)
+    out = na1d_fused(qd, kd, vd, W, L, rpb=rd, t_valid=tv, num_heads=H, dilation=D, dropout_p=p_drop, seed=seed)
+    out.backward(do.cuda())
+    for got, ref in zip((out, qd.grad, kd.grad, vd.grad, rd.grad), (want, *grads)):
+        assert O.rel_l2(got.float(), ref) < TOL[dtype]
+    split = lambda t: t.view(N, H, T, C).permute(0, 2, 1, 3)
+    qkv = torch.stack([split(t) for t in (q, k, v)], 2).contiguous().cuda().requires_grad_(True)
+    out2 = na1d_fused_qkv(qkv, W, L, rpb=rpb.cuda(), t_valid=tv, dilation=D, dropout_p=p_drop, seed=seed)
+    out2.backward(split(do).reshape(N, T, H * C).cuda())
+    assert torch.equal(out2.view(N, T, H, C), split(out.detach()))
+    for i, t in enumerate((qd, kd, vd)):
+        assert torch.equal(qkv.grad[:, :, i], split(t.grad))
