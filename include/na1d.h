@@ -268,6 +268,51 @@ int na1d_global_backward(void *dq, void *dk, void *dv, const void *q, const void
 int64_t na1d_global_backward_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t C, int dtype);
 
 /*
+ * A whole speaker-embedding model in inference (models/PCF_NATransformer.py:402-462, models/MFA_NATransformer.py:
+ * 400-466): patch embeddings, encoder layers, the projection of all blocks' outputs, attentive statistics pooling
+ * (models/Pooling.py:16-59) and the final linear layer, launched back to back on `stream` without a host decision or an
+ * allocation in between.  Batch norms are given folded: into the projection behind them, or as an affine map per channel.
+ *
+ * Weights are 16-bit (`dtype`) matrices [outputs, inputs] in fragment order: element (o, i) lies at
+ *     ((o / 16 * (inputs / 32) + i / 32) * 64 + i % 32 / 8 * 16 + o % 16) * 8 + i % 8
+ * so that the 16 x 32 block a matrix instruction reads is one contiguous kilobyte.  Biases and affine maps are fp32.
+ * Tokens have 256 channels, the MLP 1024, the attention of the pooling 128; `wide` (channels of the projection) is a
+ * multiple of 256, in_chans * patch a multiple of 32 and at most 256, `emb` a multiple of 16.
+ */
+typedef struct na1d_encoder_layer {
+    int32_t heads, window, left, dilation;      /* window 0: dense attention */
+    int32_t groups;                             /* 2, 4, 8: the projections' weights are block-diagonal; else 1 */
+    int32_t embeds, block_end;                  /* adds the patch embedding w_embed to its input; last layer of a block */
+    float scale;
+    const void *w_qkv, *w_proj, *w_fc1, *w_fc2; /* w_qkv: output rows in the order (which, head, channel) */
+    const float *b_qkv, *b_proj, *b_fc1, *b_fc2;
+    const float *rpb;                           /* [heads, window] */
+    const void *w_embed;                        /* [256, in_chans * patch] */
+    const float *b_embed;
+    const void *w_pos;                          /* dense: [256, 256] on the positions' rows; the layer's */
+    const float *gain, *shift;                  /* qkv projection reads x * gain + shift + w_pos . pos[t] */
+} na1d_encoder_layer;
+typedef struct na1d_encoder {
+    int32_t dtype, layers, blocks, in_chans, patch, wide, emb;
+    const na1d_encoder_layer *layer;
+    const void *pos;                            /* 16-bit [pos_rows, 256]: NULL without dense layers */
+    int64_t pos_rows;
+    const void *w_wide;                         /* [wide, 256 * blocks]: relu(. + b_wide) * a_wide + c_wide */
+    const float *b_wide, *a_wide, *c_wide;
+    const void *w_att, *w_ctx, *w_logit;        /* pooling: [128, wide] on tokens, [128, 2 * wide] on (mean, std), [wide, 128] */
+    const float *b_att, *a_att, *c_att;         /* tanh(relu(. + b_att) * a_att + c_att); the logits need no bias: softmax */
+    const float *a_pool, *c_pool;               /* affine map of the pooled (mean, std) [2 * wide] */
+    const void *w_fc;                           /* [emb, 2 * wide] */
+    const float *b_fc;
+} na1d_encoder;
+
+/* x: fp32 [N, in_chans, frames]; lens: fp32 [N] relative lengths in (0, 1] or NULL; out: 16-bit [N, emb].  The workspace
+ * has na1d_encode_workspace_bytes() bytes, 16-byte aligned.  NA1D_ERR_UNSUPPORTED: sizes outside the above. */
+int64_t na1d_encode_workspace_bytes(const na1d_encoder *e, int64_t N, int64_t frames);
+int na1d_encode(const na1d_encoder *e, void *out, const float *x, const float *lens, int64_t N, int64_t frames,
+                void *workspace, int64_t workspace_bytes, void *stream);
+
+/*
  * Profiling hook; no counterpart in the reference.  From this call on, the matrix-core fused kernels that the
  * CALLING THREAD launches record `start` just before and `stop` just after the kernel itself (hipEvent_t handles,
  * recorded by hipExtLaunchKernel: the dispatch's own begin and end, i.e. what a profiler's kernel trace reports,

@@ -404,7 +404,8 @@ int na1d_global_forward(void *out, float *lse, const void *q, const void *k, con
     if (misaligned(v)) return NA1D_ERR_ALIGN;
     if (!(p_drop >= 0.f && p_drop < 1.f)) return NA1D_ERR_SHAPE;
     g.drop = na1d::make_dropout(p_drop, seed);
-    return na1d::mfma::global_fwd(out, lse, q, k, v, t_valid, g, scale, dtype, (hipStream_t)stream);
+    const na1d::Layout packed = na1d::packed_layout(g);
+    return na1d::mfma::global_fwd(out, lse, q, k, v, t_valid, g, packed, packed, scale, dtype, (hipStream_t)stream);
 }
 
 int na1d_global_backward(void *dq, void *dk, void *dv, const void *q, const void *k, const void *v, const void *out,
@@ -421,6 +422,27 @@ int na1d_global_backward(void *dq, void *dk, void *dv, const void *q, const void
     g.drop = na1d::make_dropout(p_drop, seed);
     return na1d::mfma::global_bwd(dq, dk, dv, (float *)workspace, q, k, v, out, dout, lse, t_valid, g, scale, dtype,
                                   (hipStream_t)stream);
+}
+
+int64_t na1d_encode_workspace_bytes(const na1d_encoder *e, int64_t N, int64_t frames) {
+    if (!e || !e->layer) return NA1D_ERR_NULL;
+    if (e->dtype != NA1D_BF16 && e->dtype != NA1D_FP16) return NA1D_ERR_DTYPE;
+    if (N < 0) return NA1D_ERR_SHAPE;
+    if (!mfma_allowed() || !na1d::enc::encoder_ok(*e, N, frames)) return NA1D_ERR_UNSUPPORTED;
+    return na1d::enc::workspace_bytes(*e, N, frames);
+}
+
+int na1d_encode(const na1d_encoder *e, void *out, const float *x, const float *lens, int64_t N, int64_t frames,
+                void *workspace, int64_t workspace_bytes, void *stream) {
+    const int64_t need = na1d_encode_workspace_bytes(e, N, frames);
+    if (need < 0) return (int)need;
+    if (N == 0) return NA1D_OK;
+    if (!out || !x || !workspace) return NA1D_ERR_NULL;
+    if (misaligned(out) || misaligned(workspace)) return NA1D_ERR_ALIGN;
+    if (workspace_bytes < need) return NA1D_ERR_WORKSPACE;
+    for (int i = 0; i < e->layers; ++i)
+        if (bad_scale(e->layer[i].scale)) return NA1D_ERR_SCALE;
+    return na1d::enc::run(*e, out, x, lens, N, frames, workspace, (hipStream_t)stream);
 }
 
 int na1d_fused_backward_noalloc(void *dq, void *dk, void *dv, float *drpb, const void *q, const void *k, const void *v,

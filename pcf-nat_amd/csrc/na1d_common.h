@@ -200,10 +200,18 @@ int wide_bwd(void *dq, void *dk, void *dv, float *drpb, const void *q, const voi
 int64_t wide_bwd_workspace_bytes(const Geom &g);               // 0 when the shape is not covered
 // Dense attention over whole sequences (the models' global layers); g.W and g.L are not used.
 int global_fwd(void *out, float *lse, const void *q, const void *k, const void *v, const int32_t *t_valid,
-               const Geom &g, float scale, int dtype, hipStream_t s);
+               const Geom &g, const Layout &in, const Layout &out_layout, float scale, int dtype, hipStream_t s);
 int global_bwd(void *dq, void *dk, void *dv, float *delta, const void *q, const void *k, const void *v, const void *out,
                const void *dout, const float *lse, const int32_t *t_valid, const Geom &g, float scale, int dtype,
                hipStream_t s);
 }  // namespace mfma
+
+// ---- the speaker-embedding models in inference: na1d_encoder.hip ------------------
+namespace enc {
+bool encoder_ok(const na1d_encoder &e, int64_t N, int64_t frames);
+int64_t workspace_bytes(const na1d_encoder &e, int64_t N, int64_t frames);
+int run(const na1d_encoder &e, void *out, const float *x, const float *lens, int64_t N, int64_t frames, void *ws,
+        hipStream_t s);
+}  // namespace enc
 
 }  // namespace na1d

@@ -1,0 +1,139 @@
+// What the token-local kernels of the speaker-embedding models share: everything of an encoder layer that is not
+// attention works on one token at a time, so a workgroup that holds a few tokens in LDS can run a layer's output
+// projection, its MLP and the next layer's qkv projection without touching memory in between.
+#pragma once
+
+#include "na1d_mfma_core.h"
+
+namespace na1d {
+namespace enc {
+
+using namespace mfma;
+
+constexpr int kDim = 256;            // channels of a token
+constexpr int kHidden = 1024;        // channels of the MLP's hidden layer
+constexpr int kRow = 2 * kDim;       // bytes of a token's row in LDS: the staged tiles are all this wide
+constexpr int kFrag = 1024;          // bytes of a weight fragment: 16 outputs x 32 inputs, in the order of the lanes
+
+// A tile of token rows in LDS: 512 bytes a row, its 16-byte units XOR-swizzled with the row's place in a 16-row tile
+// (the rows an operand read touches land in distinct banks, and the swizzle is the same for every tile).
+__device__ inline int tile_addr(int row, int unit) { return row * kRow + ((unit ^ (row & 15)) << 4); }
+
+// Copy `rows` (a multiple of 16) token rows of `width` bytes, `pitch` bytes apart, into such a tile with loads that write
+// LDS directly; the resource ends behind the last row there is, and bytes past a row's width arrive as zeros.
+template <int ROWS, int NW, int AUX>
+__device__ inline void stage_tokens(Rsrc src, LDS_PTR(char) tile, int pitch, int width, int wave, int lane) {
+    constexpr int kChunks = ROWS * kRow / kChunk;          // two rows each
+#pragma unroll
+    for (int j = 0; j < (kChunks + NW - 1) / NW; ++j) {
+        const int c = j * NW + wave, row = 2 * c + (lane >> 5);
+        const int at = ((lane & 31) ^ (row & 15)) * 16;
+        if (kChunks % NW == 0 || c < kChunks) load_to_lds<16, AUX>(src, tile + c * kChunk, at < width ? row * pitch + at : kNowhere);
+    }
+}
+
+// Where a product's operands are: step s of output tile j of this wave multiplies weight fragment
+// first + j * stride + skip(j) + s by the tokens' 32 channels number x0 + skip(j) + s.  `skip` is there for grouped
+// projections (block-diagonal weights), whose output tiles start at inputs of their own: SKIP = 0: all at the same,
+// 1: two steps later from tile to tile, 2: odd tiles four steps later.
+template <int TILES, int STEPS, int SKIP = 0> struct Product {
+    static constexpr int kTiles = TILES, kSteps = STEPS, kSkip = SKIP;
+    Rsrc w;
+    int first, stride, x0;               // wave-uniform, in fragments / steps
+    static __device__ constexpr int skip(int j) { return SKIP == 1 ? 2 * j : SKIP == 2 ? 4 * (j & 1) : 0; }
+    __device__ inline u32x4 load(int j, int s, int lane16) const {
+        return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w, lane16, (first + j * stride + skip(j) + s) * kFrag, 0));
+    }
+};
+__device__ inline Rsrc weight_rsrc(const char *w, int outputs, int inputs) { return make_rsrc(w, outputs * inputs * 2); }
+
+// The weight fragments on their way: they come straight from memory into registers (packed so that a fragment is one
+// contiguous kilobyte; every workgroup reads the same ones, so they sit in the L2s), PF steps ahead of their use, also
+// across the border of two products: while one runs out its slots fill with the next one's first steps.
+template <int NTW, int PF> struct Ring {
+    u32x4 w[PF][NTW];
+    template <class P> __device__ inline void fill(const P &p, int slot, int s, int lane16) {
+#pragma unroll
+        for (int j = 0; j < P::kTiles; ++j) w[slot][j] = p.load(j, s, lane16);
+    }
+    template <class P> __device__ inline void begin(const P &p, int lane16) {
+#pragma unroll
+        for (int s = 0; s < PF; ++s)
+            if (s < P::kSteps) fill(p, s, s, lane16);
+    }
+};
+struct Nothing {
+    static constexpr int kTiles = 0, kSteps = 0;
+    __device__ inline u32x4 load(int, int, int) const { return u32x4{}; }
+};
+
+// acc[j][i] += W[tile j of this wave] . X[token tile i]^T; lane (n, g) ends up with outputs 4g .. 4g+3 of each tile for
+// token n of each token tile.  The ring holds this product's first PF steps on entry and `next`'s on exit.
+template <class DT, int MT, int NTW, int PF, int NA, class P, class Q>
+__device__ inline void multiply(f32x4 (&acc)[NA][MT], int a0, Ring<NTW, PF> &ring, const P &p, const Q &next, LDS_PTR(char) tile,
+                                int n, int g, int lane16) {
+    static_assert(P::kSteps % PF == 0 || P::kSteps < PF, "slots of a product");
+    if constexpr (P::kSteps < PF) {
+#pragma unroll
+        for (int s = P::kSteps; s < PF; ++s)
+            if (s < Q::kSteps) ring.fill(next, s, s, lane16);
+    }
+    const int xr = n * kRow, xs = 4 * p.x0 + g;
+#pragma unroll
+    for (int s = 0; s < P::kSteps; ++s) {
+        u32x4 x[MT];
+#pragma unroll
+        for (int j = 0; j < P::kTiles; ++j) {
+            if (j == 0 || P::kSkip) {
+                LDS_PTR(char) at = tile + xr + (((xs + 4 * (P::skip(j) + s)) ^ n) << 4);
+#pragma unroll
+                for (int i = 0; i < MT; ++i) x[i] = *reinterpret_cast<LDS_PTR(u32x4)>(at + i * 16 * kRow);
+            }
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[a0 + j][i] = Mma<DT>::k32(ring.w[s % PF][j], x[i], acc[a0 + j][i]);
+        }
+        if (s + PF < P::kSteps) {
+            ring.fill(p, s % PF, s + PF, lane16);
+        } else {
+            const int t = P::kSteps < PF ? s : s + PF - P::kSteps;
+            if (t < Q::kSteps) ring.fill(next, s % PF, t, lane16);
+        }
+    }
+}
+template <int NTW, int MT> __device__ inline void clear(f32x4 (&acc)[NTW][MT]) {
+#pragma unroll
+    for (int j = 0; j < NTW; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+// Two 16-bit values of a register as floats.
+template <class DT> __device__ inline f32x2 widen(uint32_t w);
+template <> __device__ inline f32x2 widen<BF16>(uint32_t w) {
+    return f32x2{__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u)};
+}
+template <> __device__ inline f32x2 widen<FP16>(uint32_t w) {
+    return __builtin_convertvector(__builtin_bit_cast(f16x2, w), f32x2);
+}
+template <class DT> __device__ inline f32x4 widen4(u32x2 w) {
+    const f32x2 a = widen<DT>(w.x), b = widen<DT>(w.y);
+    return f32x4{a.x, a.y, b.x, b.y};
+}
+template <class DT> __device__ inline u32x2 narrow4(f32x4 v) { return u32x2{Mma<DT>::pack(v[0], v[1]), Mma<DT>::pack(v[2], v[3])}; }
+
+// x * Phi(x), the exact (erf) GELU, by formula 7.1.26 of Abramowitz and Stegun's handbook (error of erf below 1.5e-7):
+// with t = 1 / (1 + p z), z = |x| / sqrt 2, erfc(z) = t (a1 + t (a2 + ...)) exp(-z^2), and
+// gelu(x) = max(x, 0) - |x| erfc(z) / 2 for either sign.
+__device__ inline float gelu(float x) {
+    const float ax = __builtin_fabsf(x);
+    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(ax, 0.3275911f * 0.70710678f, 1.f));
+    float e = __builtin_fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
+    e = __builtin_fmaf(t, e, 0.5f * 1.421413741f);
+    e = __builtin_fmaf(t, e, 0.5f * -0.284496736f);
+    e = __builtin_fmaf(t, e, 0.5f * 0.254829592f);
+    const float ex = __builtin_amdgcn_exp2f(x * x * -0.72134752f);
+    return __builtin_fmaf(-ax * t, e * ex, __builtin_fmaxf(x, 0.f));
+}
+
+}  // namespace enc
+}  // namespace na1d

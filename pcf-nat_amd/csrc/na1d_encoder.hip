@@ -1,0 +1,865 @@
+// The token-local part of the speaker-embedding models (models/PCF_NATransformer.py, models/MFA_NATransformer.py) in
+// inference on the matrix cores: projections, MLPs, residuals, patch embeddings.
+#include "na1d_encoder.h"
+
+namespace na1d {
+namespace enc {
+
+// =============================================================================
+// Between two attentions
+// =============================================================================
+// One workgroup takes 16 * MT tokens through everything between the attention of one layer and that of the next:
+//   x1 = x + proj(attention),  x2 = x1 + fc2(gelu(fc1(x1)))          the rest of the layer before   (`attn` != null)
+//   x2 += embed(patches)                                             where a block takes its own embedding
+//   qkv = x2 . Wqkv^T + b                                            the head of the next layer     (`qkv` != null)
+// with batch norms folded into the projections behind them.  Tokens sit in two LDS tiles; the hidden layer passes
+// through one of them 256 channels at a time and never exists in memory; the weights of a layer (1.6 MB) stream from L2.
+struct LayerArgs {
+    const char *attn, *x_in;
+    const char *w_proj, *w_fc1, *w_fc2;
+    const float *b_proj, *b_fc1, *b_fc2;
+    char *block_out;                  // the layer's output where a block ends
+    const char *patches, *w_embed;
+    const float *b_embed;
+    char *x_out;                      // the residual stream the next layer reads
+    const char *w_qkv;
+    const float *b_qkv;
+    char *qkv;
+    const float *gain, *posb;         // dense layers: qkv of x * gain + posb[token's place]
+    int x_in_pitch, block_pitch, patch_width, M, T;
+    uint32_t T_magic;
+    int tail_groups, head_groups;     // block-diagonal weights: 8, 4, 2; otherwise 1
+};
+
+// Grouped projections (PCF-NAT: blocks of 8, 4, 2 and 1 groups) have block-diagonal weights; which 32-input steps of an
+// output tile are not zero follows from the number of groups G alone:
+//   output projection, fc1   outputs of a group see the 256 / G inputs of the same group
+//   fc2                      256 hidden channels (chunk c) reach kOut outputs, from kOut * (c * kOut / 256 ...) on
+//   qkv                      output f (head-major order, see _qkv_channel_order) sees group (f mod 256/G) / (256/G^2)
+template <int G, int NW> struct Groups {
+    static constexpr int kSize = kDim / G;                             // channels of a group
+    static constexpr int NTW = 16 / NW, CW = 16 * NTW;                 // output tiles / channels a wave has of 256
+    static constexpr int kProj = (kSize > CW ? kSize : CW) / 32;       // steps of the output projection (CW channels may touch several groups)
+    static constexpr int kFc1 = kSize / 32;
+    static constexpr int kOutTiles = G == 1 ? 16 : G == 2 ? 8 : 4;     // output tiles a chunk of 256 hidden channels reaches
+    static constexpr int kSets = 16 / kOutTiles;                       // different ones
+    static constexpr int kPer = kOutTiles >= NW ? kOutTiles / NW : 1;  // of them to a wave
+    static constexpr int kActive = kOutTiles < NW ? kOutTiles : NW;    // waves that have any
+    static constexpr int kFc2 = G == 8 ? 4 : 8;
+    static constexpr int kAcc = kSets * kPer;                          // output tiles of a wave over all chunks
+    static constexpr int kQkv = G == 1 ? 8 : G == 4 ? 2 : 4;
+    static constexpr int kQkvSkip = G == 4 ? 1 : G == 8 ? 2 : 0;
+    using Proj = Product<NTW, kProj>;
+    using Fc1 = Product<NTW, kFc1>;
+    using Fc2 = Product<kPer, kFc2>;
+    using Qkv = Product<NTW, kQkv, kQkvSkip>;
+    static __device__ inline Proj proj(Rsrc w, int wave) {
+        const int k0 = wave * CW / (32 * kProj) * kProj;
+        return Proj{w, wave * NTW * 8 + k0, 8, k0};
+    }
+    static __device__ inline Fc1 fc1(Rsrc w, int c, int wave) {
+        const int k0 = (256 * c + wave * CW) / (kHidden / G) * kFc1;
+        return Fc1{w, (16 * c + wave * NTW) * 8 + k0, 8, k0};
+    }
+    static __device__ inline Fc2 fc2(Rsrc w, int c, int wave) {
+        const int set = c * kSets / 4, tile = set * kOutTiles + wave * kPer;
+        const int k0 = G == 8 ? wave / 2 * 4 : 0;
+        return Fc2{w, tile * (kHidden / 32) + 8 * c + k0, kHidden / 32, k0};
+    }
+    static __device__ inline Qkv qkv(Rsrc w, int which, int wave) {
+        const int k0 = G == 2 ? wave * CW % 128 / 64 * 4 : G == 4 ? wave * NTW % 4 * 2 : 0;
+        return Qkv{w, (16 * which + wave * NTW) * 8 + k0, 8, k0};
+    }
+};
+
+template <class DT, int MT, int NW, int PF> struct LayerWave {
+    static constexpr int NTW = 16 / NW, CW = 16 * NTW;
+    const LayerArgs &a;
+    LDS_PTR(char) p_lds;
+    LDS_PTR(char) q_lds;
+    int wave, lane, n, g, lane16;
+    Ring<NTW, PF> ring;
+
+    // LDS place of channels c + 4g .. + 3 of token n (c: a multiple of 16, wave-uniform)
+    __device__ inline int piece(int c) const { return n * kRow + (((c / 8 + (g >> 1)) ^ n) << 4) + (g & 1) * 8; }
+    __device__ inline LDS_PTR(u32x2) at(LDS_PTR(char) tile, int c, int i) const {
+        return reinterpret_cast<LDS_PTR(u32x2)>(tile + piece(c) + i * 16 * kRow);
+    }
+    __device__ inline f32x4 bias(const float *b, int c) const { return *reinterpret_cast<const f32x4 *>(b + c + 4 * g); }
+
+    // attention rows in p_lds, x in q_lds (on their way) -> x2 in q_lds
+    template <int G> __device__ inline void tail() {
+        using S = Groups<G, NW>;
+        const Rsrc w1 = weight_rsrc(a.w_fc1, kHidden, kDim), w2 = weight_rsrc(a.w_fc2, kDim, kHidden);
+        const auto proj = S::proj(weight_rsrc(a.w_proj, kDim, kDim), wave);
+        ring.begin(proj, lane16);
+        f32x4 hid[NTW][MT];
+        clear(hid);
+        wait_direct();
+        barrier_lds();
+        multiply<DT, MT>(hid, 0, ring, proj, S::fc1(w1, 0, wave), p_lds, n, g, lane16);
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) {
+            const int c = CW * wave + 16 * j;
+            const f32x4 b = bias(a.b_proj, c);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) *at(q_lds, c, i) = narrow4<DT>(hid[j][i] + b + widen4<DT>(*at(q_lds, c, i)));
+        }
+        f32x4 acc[S::kAcc][MT];
+        clear(acc);
+        const bool active = wave < S::kActive;
+        auto chunk = [&](int c, int a0, bool last) {      // a0: the chunk's output tiles in acc, a constant
+            clear(hid);
+            barrier_lds();                           // x1 is whole (first round); every wave is done with the hidden channels before
+            multiply<DT, MT>(hid, 0, ring, S::fc1(w1, c, wave), S::fc2(w2, c, wave), q_lds, n, g, lane16);
+#pragma unroll
+            for (int j = 0; j < NTW; ++j) {
+                const int ch = CW * wave + 16 * j;
+                const f32x4 b = bias(a.b_fc1, 256 * c + ch);
+#pragma unroll
+                for (int i = 0; i < MT; ++i) {
+                    f32x4 h = hid[j][i] + b;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) h[r] = gelu(h[r]);
+                    *at(p_lds, ch, i) = narrow4<DT>(h);
+                }
+            }
+            barrier_lds();
+            if (active)
+                multiply<DT, MT>(acc, a0, ring, S::fc2(w2, c, wave), S::fc1(w1, last ? 0 : c + 1, wave), p_lds, n, g, lane16);
+            else
+                ring.begin(S::fc1(w1, last ? 0 : c + 1, wave), lane16);
+        };
+        if constexpr (S::kSets == 1) {
+#pragma unroll 1
+            for (int c = 0; c < 4; ++c) chunk(c, 0, c == 3);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) chunk(c, c * S::kSets / 4 * S::kPer, c == 3);
+        }
+        if (active) {
+#pragma unroll
+            for (int t = 0; t < S::kAcc; ++t) {
+                const int c = 16 * (t / S::kPer * S::kOutTiles + wave * S::kPer + t % S::kPer);
+                const f32x4 b = bias(a.b_fc2, c);
+#pragma unroll
+                for (int i = 0; i < MT; ++i) *at(q_lds, c, i) = narrow4<DT>(acc[t][i] + b + widen4<DT>(*at(q_lds, c, i)));
+            }
+        }
+    }
+
+    template <int G> __device__ inline void head(int64_t m0, int rows) {
+        using S = Groups<G, NW>;
+        const Rsrc w = weight_rsrc(a.w_qkv, 3 * kDim, kDim);
+        ring.begin(S::qkv(w, 0, wave), lane16);
+        barrier_lds();
+        const Rsrc qs = make_rsrc(a.qkv + m0 * (3 * kRow), rows * (3 * kRow));
+#pragma unroll 1
+        for (int which = 0; which < 3; ++which) {
+            f32x4 acc[NTW][MT];
+            clear(acc);
+            multiply<DT, MT>(acc, 0, ring, S::qkv(w, which, wave), S::qkv(w, min(which + 1, 2), wave), q_lds, n, g, lane16);
+            u32x2 o[MT][NTW];
+#pragma unroll
+            for (int j = 0; j < NTW; ++j) {
+                const f32x4 b = bias(a.b_qkv, which * kDim + CW * wave + 16 * j);
+#pragma unroll
+                for (int i = 0; i < MT; ++i) o[i][j] = narrow4<DT>(acc[j][i] + b);
+            }
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+                store_tile<CW, 0>(qs, (16 * i + n) * (3 * kRow) + which * kRow + 2 * CW * wave, o[i], g, 2 * CW);
+        }
+    }
+
+    // rows of q_lds to memory, whole
+    __device__ inline void write_rows(char *dst, int64_t m0, int rows, int pitch) const {
+        const Rsrc d = make_rsrc(dst + m0 * pitch, rows * pitch);
+#pragma unroll
+        for (int r = 0; r < 16 * MT * 32 / (64 * NW); ++r) {
+            const int u = r * 64 * NW + wave * 64 + lane, row = u >> 5, unit = u & 31;
+            const u32x4 v = *reinterpret_cast<LDS_PTR(u32x4)>(q_lds + tile_addr(row, unit));
+            __builtin_amdgcn_raw_buffer_store_b128(v, d, row * pitch + unit * 16, 0, 0);
+        }
+    }
+};
+
+template <class DT, int MT, int NW, int PF>
+__global__ void __launch_bounds__(64 * NW, MT == 2 ? 3 : 2)
+layer_kernel(LayerArgs a) {
+    using W = LayerWave<DT, MT, NW, PF>;
+    constexpr int NTW = W::NTW, CW = W::CW;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // p_lds: attention rows, then 256 hidden channels at a time, then patches; q_lds: x, then x1, then x2
+    W w{a, (LDS_PTR(char))smem, (LDS_PTR(char))smem + 16 * MT * kRow, wave, lane, lane & 15, lane >> 4, lane * 16};
+    const int64_t m0 = (int64_t)blockIdx.x * (16 * MT);
+    const int rows = (int)min((int64_t)(16 * MT), a.M - m0);
+    if (a.attn) {
+        const Rsrc as = make_rsrc(a.attn + m0 * kRow, rows * kRow), xs = make_rsrc(a.x_in + m0 * a.x_in_pitch, rows * a.x_in_pitch);
+        stage_tokens<16 * MT, NW, kReadOnce>(as, w.p_lds, kRow, kRow, wave, lane);
+        stage_tokens<16 * MT, NW, kReadOnce>(xs, w.q_lds, a.x_in_pitch, kRow, wave, lane);
+        switch (a.tail_groups) {
+            case 8: w.template tail<8>(); break;
+            case 4: w.template tail<4>(); break;
+            case 2: w.template tail<2>(); break;
+            default: w.template tail<1>();
+        }
+        if (a.block_out) {
+            barrier_lds();
+            w.write_rows(a.block_out, m0, rows, a.block_pitch);
+        }
+    }
+    if (!a.qkv) return;
+    if (a.patches) {
+        if (a.attn) barrier_lds();                   // every wave is done with the hidden channels
+        const Rsrc es = make_rsrc(a.patches + m0 * a.patch_width, rows * a.patch_width);
+        stage_tokens<16 * MT, NW, kReadShared>(es, w.p_lds, a.patch_width, a.patch_width, wave, lane);
+        const int ks_all = a.patch_width / 64;       // steps of 32 inputs
+        const Rsrc we = weight_rsrc(a.w_embed, kDim, a.patch_width / 2);
+        f32x4 acc[NTW][MT];
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) {
+            const int c = CW * wave + 16 * j;
+            const f32x4 b = w.bias(a.b_embed, c);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[j][i] = a.attn ? widen4<DT>(*w.at(w.q_lds, c, i)) + b : b;
+        }
+        wait_direct();
+        barrier_lds();
+#pragma unroll 1
+        for (int s = 0; s < ks_all; ++s) {
+            const Product<NTW, 1> p{we, wave * NTW * ks_all + s, ks_all, s};
+            w.ring.fill(p, 0, 0, w.lane16);
+            multiply<DT, MT>(acc, 0, w.ring, p, Nothing{}, w.p_lds, w.n, w.g, w.lane16);
+        }
+#pragma unroll
+        for (int j = 0; j < NTW; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) *w.at(w.q_lds, CW * wave + 16 * j, i) = narrow4<DT>(acc[j][i]);
+    }
+    if (a.x_out) {
+        barrier_lds();
+        w.write_rows(a.x_out, m0, rows, kRow);
+    }
+    if (a.gain) {
+        barrier_lds();
+        const uint32_t first = (uint32_t)m0 % (uint32_t)a.T;     // place of the tile's first token in its utterance
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            const uint32_t m = first + 16 * i + w.n;             // below T + 64
+            const uint32_t t = m - div_by(m, a.T, a.T_magic) * a.T;
+            const float *pos = a.posb + (int64_t)t * kDim;
+#pragma unroll
+            for (int j = 0; j < NTW; ++j) {
+                const int c = CW * wave + 16 * j;
+                *w.at(w.q_lds, c, i) = narrow4<DT>(widen4<DT>(*w.at(w.q_lds, c, i)) * w.bias(a.gain, c) + w.bias(pos, c));
+            }
+        }
+    }
+    switch (a.head_groups) {
+        case 8: w.template head<8>(m0, rows); break;
+        case 4: w.template head<4>(m0, rows); break;
+        case 2: w.template head<2>(m0, rows); break;
+        default: w.template head<1>(m0, rows);
+    }
+}
+
+// tanh(x) = 1 - 2 / (1 + exp(2x)); its series where that would cancel
+__device__ inline float tanh_of(float x) {
+    const float t = 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * (2.f * kLog2e)));
+    const float u = x * x;
+    return __builtin_fabsf(x) < 0.0625f ? x * __builtin_fmaf(u, __builtin_fmaf(u, 2.f / 15.f, -1.f / 3.f), 1.f) : t;
+}
+
+// =============================================================================
+// Plain projections: out[m, o] = f(X[m, :] . W[o, :])
+// =============================================================================
+enum LinearEnd {
+    kAffine,          // + bias, as fp32
+    kEmbedding,       // + bias, 16-bit
+    kReluNorm,        // relu(. + bias) * scale + offset, 16-bit
+    kTanhNorm,        // tanh(relu(. + add[m / T]) * scale + offset), 16-bit
+};
+struct LinearArgs {
+    const char *x, *w;
+    char *out;
+    const float *bias, *scale, *offset;
+    int x_pitch, out_pitch, inputs, outputs, M, T;      // T: rows that share a row of `bias` (kTanhNorm)
+};
+template <class DT, LinearEnd END>
+__device__ inline void finish(const LinearArgs &a, Rsrc out, int64_t m0, int row, int c, f32x4 v) {
+    if constexpr (END == kTanhNorm) {
+        const uint32_t u = (uint32_t)(m0 + row) / (uint32_t)a.T;
+        v += *reinterpret_cast<const f32x4 *>(a.bias + (int64_t)u * a.outputs + c);
+    } else {
+        v += *reinterpret_cast<const f32x4 *>(a.bias + c);
+    }
+    if constexpr (END == kReluNorm || END == kTanhNorm) {
+        const f32x4 sc = *reinterpret_cast<const f32x4 *>(a.scale + c), of = *reinterpret_cast<const f32x4 *>(a.offset + c);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            v[r] = __builtin_fmaf(__builtin_fmaxf(v[r], 0.f), sc[r], of[r]);
+            if constexpr (END == kTanhNorm) v[r] = tanh_of(v[r]);
+        }
+    }
+    if constexpr (END == kAffine)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), out, row * a.out_pitch + 4 * c, 0, 0);
+    else
+        __builtin_amdgcn_raw_buffer_store_b64(narrow4<DT>(v), out, row * a.out_pitch + 2 * c, 0, 0);
+}
+
+// Many rows: a workgroup of four waves computes 16 * MT rows x 64 * NTW outputs.  The rows come through LDS 256 inputs at
+// a time, the next piece on its way while this one is multiplied; the weights stream from L2 into registers as above.
+template <class DT, int MT, int NTW, LinearEnd END>
+__global__ void __launch_bounds__(kThreads, 2)
+linear_kernel(LinearArgs a, int col_blocks) {
+    constexpr int PF = 4, NW = kWaves;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    LDS_PTR(char) lds = (LDS_PTR(char))smem;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
+    const uint32_t item = xcd_item(blockIdx.x, gridDim.x);           // neighbours share their rows' lines
+    const uint32_t row_block = item / (uint32_t)col_blocks;
+    const int64_t m0 = (int64_t)row_block * (16 * MT);
+    const int rows = (int)min((int64_t)(16 * MT), a.M - m0);
+    const int tile0 = ((int)(item - row_block * col_blocks) * NW + wave) * NTW;
+    const Rsrc xs = make_rsrc(a.x + m0 * a.x_pitch, rows * a.x_pitch), ws = weight_rsrc(a.w, a.outputs, a.inputs);
+    const int steps = a.inputs / 32, pieces = a.inputs / 256;
+    auto stage = [&](int piece) {
+        constexpr int kChunks = 16 * MT * kRow / kChunk;
+#pragma unroll
+        for (int j = 0; j < kChunks / NW; ++j) {
+            const int c = j * NW + wave, row = 2 * c + (lane >> 5);
+            load_to_lds<16, kReadShared>(xs, lds + (piece & 1) * (16 * MT * kRow) + c * kChunk, row * a.x_pitch + piece * kRow + ((lane & 31) ^ (row & 15)) * 16);
+        }
+    };
+    stage(0);
+    f32x4 acc[NTW][MT];
+    clear(acc);
+    Ring<NTW, PF> ring;
+    using P = Product<NTW, 8>;
+    const int lane16 = lane * 16;
+    ring.begin(P{ws, tile0 * steps, steps, 0}, lane16);
+#pragma unroll 1
+    for (int p = 0; p < pieces; ++p) {
+        wait_direct();
+        barrier_lds();
+        if (p + 1 < pieces) stage(p + 1);
+        const P now{ws, tile0 * steps + 8 * p, steps, 0}, next{ws, tile0 * steps + 8 * min(p + 1, pieces - 1), steps, 0};
+        multiply<DT, MT>(acc, 0, ring, now, next, lds + (p & 1) * (16 * MT * kRow), n, g, lane16);
+    }
+    const Rsrc os = make_rsrc(a.out + m0 * a.out_pitch, rows * a.out_pitch);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) finish<DT, END>(a, os, m0, 16 * i + n, 16 * (tile0 + j) + 4 * g, acc[j][i]);
+}
+
+// Few rows: the inputs are split over the eight waves of a workgroup that computes 16 rows x 16 * NT outputs; rows and
+// weights go from memory straight into the operands' registers and the waves' sums meet in LDS.
+template <class DT, int NT, LinearEnd END>
+__global__ void __launch_bounds__(512)
+linear_small_kernel(LinearArgs a, int col_blocks) {
+    constexpr int NW = 8, U = 4;
+    __shared__ __attribute__((aligned(16))) f32x4 sums[NW][NT][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
+    const int row_block = (int)(blockIdx.x / (uint32_t)col_blocks), tile0 = ((int)blockIdx.x - row_block * col_blocks) * NT;
+    const int64_t m0 = (int64_t)row_block * 16;
+    const int rows = (int)min((int64_t)16, a.M - m0);
+    const Rsrc xs = make_rsrc(a.x + m0 * a.x_pitch, rows * a.x_pitch), ws = weight_rsrc(a.w, a.outputs, a.inputs);
+    const int steps = a.inputs / 32;
+    f32x4 acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = wave; s0 < steps; s0 += NW * U) {
+        u32x4 x[U], w[U][NT];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {                // steps past the end: zero rows (no resource reaches kNowhere)
+            const int s = s0 + u * NW, at = s < steps ? n * a.x_pitch + 64 * s + 16 * g : kNowhere;
+            x[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xs, at, 0, 0));
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                w[u][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ws, lane * 16, ((tile0 + j) * steps + min(s, steps - 1)) * kFrag, 0));
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[j] = Mma<DT>::k32(w[u][j], x[u], acc[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) sums[wave][j][lane] = acc[j];
+    __syncthreads();
+    if (wave < NT) {
+        f32x4 v = sums[0][wave][lane];
+#pragma unroll
+        for (int k = 1; k < NW; ++k) v += sums[k][wave][lane];
+        const Rsrc os = make_rsrc(a.out + m0 * a.out_pitch, rows * a.out_pitch);
+        finish<DT, END>(a, os, m0, n, 16 * (tile0 + wave) + 4 * g, v);
+    }
+}
+
+// =============================================================================
+// Around the encoder
+// =============================================================================
+// Valid tokens and frames-as-tokens counts from relative lengths (models/PCF_NATransformer.py:406-414, Pooling.py:30-35).
+__global__ void lengths_kernel(int32_t *t_valid, float *count, const float *lens, int N, int frames, int patch, int T) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= N) return;
+    const float len = lens[i], pad = floorf(((float)frames - rintf(len * (float)frames)) / (float)patch);
+    t_valid[i] = T - (int)pad;
+    count[i] = rintf(len * (float)T);
+}
+
+// [N, in_chans, frames] fp32 -> patch rows [N * T, in_chans * patch] of 16 bit, element (c, j) of token t = x[c][t * patch + j].
+// 64 tokens to a workgroup through LDS: reads run along the frames, writes along the rows.
+template <class DT>
+__global__ void __launch_bounds__(256)
+patch_kernel(uint32_t *__restrict__ out, const float *__restrict__ x, int in_chans, int frames, int patch, int T) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    float *tile = reinterpret_cast<float *>(smem);               // [in_chans][64 * patch + 1]
+    const int span = 64 * patch, pitch = span + 1, t0 = blockIdx.x * 64, nt = min(64, T - t0), width = in_chans * patch;
+    const float *src = x + (int64_t)blockIdx.y * in_chans * frames + (int64_t)t0 * patch;
+    for (int i = threadIdx.x; i < in_chans * span; i += 256) {
+        const int c = i / span, f = i - c * span;
+        tile[c * pitch + f] = f < nt * patch ? src[(int64_t)c * frames + f] : 0.f;
+    }
+    __syncthreads();
+    uint32_t *dst = out + ((int64_t)blockIdx.y * T + t0) * (width / 2);
+    for (int i = threadIdx.x; i < nt * (width / 2); i += 256) {
+        const int t = i / (width / 2), e = 2 * (i - t * (width / 2));
+        const int c0 = e / patch, j0 = e - c0 * patch, c1 = (e + 1) / patch, j1 = e + 1 - c1 * patch;
+        dst[i] = Mma<DT>::pack(tile[c0 * pitch + t * patch + j0], tile[c1 * pitch + t * patch + j1]);
+    }
+}
+
+// Mean and standard deviation over an utterance's tokens of 64 channels: one pass over the rows, sums of the differences
+// to the first row (fp32; the first row is a sample, so nothing cancels).  Written as fp32 for the pooling's sums and in
+// 16 bit for the product with the context's weights.
+template <class DT>
+__global__ void __launch_bounds__(256)
+stats_kernel(float *__restrict__ mean_std, char *__restrict__ rounded, const char *__restrict__ h, const float *__restrict__ count,
+             int T, int wide) {
+    __shared__ float part[2][32][64 + 1];
+    const int c = threadIdx.x & 7, r = threadIdx.x >> 3, n = blockIdx.y, c0 = blockIdx.x * 64 + c * 8;
+    const int pitch = 2 * wide, valid = count ? max(0, min(T, (int)count[n])) : T;
+    const char *src = h + (int64_t)n * T * pitch + 2 * c0;
+    float first[8], s1[8], s2[8];
+    auto row = [&](int t, float (&v)[8]) {
+        const u32x4 w = *reinterpret_cast<const u32x4 *>(src + (int64_t)t * pitch);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const f32x2 p = widen<DT>(w[i]);
+            v[2 * i] = p.x;
+            v[2 * i + 1] = p.y;
+        }
+    };
+    row(0, first);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s1[i] = s2[i] = 0.f;
+#pragma unroll 4
+    for (int t = r; t < valid; t += 32) {
+        float v[8];
+        row(t, v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float d = v[i] - first[i];
+            s1[i] += d;
+            s2[i] = __builtin_fmaf(d, d, s2[i]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        part[0][r][c * 8 + i] = s1[i];
+        part[1][r][c * 8 + i] = s2[i];
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int ch = threadIdx.x;
+    float a = 0.f, b = 0.f;
+#pragma unroll 8
+    for (int k = 0; k < 32; ++k) {
+        a += part[0][k][ch];
+        b += part[1][k][ch];
+    }
+    const float x0 = (float)widen<DT>((uint32_t)*reinterpret_cast<const uint16_t *>(h + (int64_t)n * T * pitch + 2 * (blockIdx.x * 64 + ch))).x;
+    const float cnt = count ? count[n] : (float)T, m = a / cnt;
+    float var = (b - a * m) / (count ? cnt : cnt - 1.f);
+    var = var < 1e-12f ? 1e-12f : var;                          // NaN stays
+    const float mean = x0 + m, std = sqrtf(var);
+    const int64_t at = (int64_t)n * 2 * wide + blockIdx.x * 64 + ch;
+    mean_std[at] = mean;
+    mean_std[at + wide] = std;
+    reinterpret_cast<uint16_t *>(rounded)[at] = (uint16_t)Mma<DT>::pack(mean, 0.f);
+    reinterpret_cast<uint16_t *>(rounded)[at + wide] = (uint16_t)Mma<DT>::pack(std, 0.f);
+}
+
+// Attentive statistics pooling of 64 channels of an utterance: logits = W . hidden[t] on the matrix core, softmax over the
+// tokens and the weighted mean and deviation in one pass over the rows, the logits never written.  Lane (n, g) sees
+// channels 4g .. 4g+3 of each 16-channel tile for every 16th token, keeps its own running maximum (moved only when
+// outgrown by 2^8) and sums of p, p d, p d^2 (d = difference to the plain mean), and the lanes and waves meet at the end.
+struct PoolArgs {
+    const char *h, *hidden, *w;
+    const float *count, *mean_std, *a_pool, *c_pool;
+    char *out;                      // [N, 2 * wide], the next product's operand
+    int T, wide;
+};
+__device__ inline float row16_max(float x) {
+#pragma unroll
+    for (int k = 1; k < 16; k *= 2) x = __builtin_fmaxf(x, __shfl_xor(x, k));
+    return x;
+}
+__device__ inline float row16_sum(float x) {
+#pragma unroll
+    for (int k = 1; k < 16; k *= 2) x += __shfl_xor(x, k);
+    return x;
+}
+template <class DT>
+__global__ void __launch_bounds__(kThreads, 2)
+pool_kernel(PoolArgs a) {
+    constexpr int kSlack = 8;
+    __shared__ float meet[kWaves][64][4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
+    const int utt = blockIdx.y, c0 = blockIdx.x * 64, pitch = 2 * a.wide;
+    const Rsrc hs = make_rsrc(a.h + (int64_t)utt * a.T * pitch, a.T * pitch), ds = make_rsrc(a.hidden + (int64_t)utt * a.T * 256, a.T * 256);
+    const Rsrc ws = weight_rsrc(a.w, a.wide, 128);
+    const int valid = a.count ? max(0, min(a.T, (int)a.count[utt])) : a.T;
+    u32x4 w[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            w[j][s] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ws, lane * 16, ((c0 / 16 + j) * 4 + s) * kFrag, 0));
+    f32x4 mu[4], m[4], s0[4], s1[4], s2[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        mu[j] = *reinterpret_cast<const f32x4 *>(a.mean_std + (int64_t)utt * 2 * a.wide + c0 + 16 * j + 4 * g);
+        m[j] = f32x4{-1e30f, -1e30f, -1e30f, -1e30f};
+        s0[j] = s1[j] = s2[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const int tiles = (valid + 15) >> 4;
+    for (int t = wave; t < tiles; t += kWaves) {
+        const int row = 16 * t + n;
+        u32x4 d[4];
+        u32x2 xr[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) d[s] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ds, row * 256 + 64 * s + 16 * g, 0, 0));
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            xr[j] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(hs, row * pitch + 2 * (c0 + 16 * j + 4 * g), 0, 0));
+        f32x4 z[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            z[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < 4; ++s) z[j] = Mma<DT>::k32(w[j][s], d[s], z[j]);
+        }
+        bool outgrown = false;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                z[j][r] = row < valid ? z[j][r] * kLog2e : kNegInf;
+                outgrown |= z[j][r] > m[j][r] + kSlack;
+            }
+        if (__builtin_amdgcn_ballot_w64(outgrown)) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float up = __builtin_fmaxf(m[j][r], z[j][r]), f = __builtin_amdgcn_exp2f(m[j][r] - up);
+                    m[j][r] = up;
+                    s0[j][r] *= f;
+                    s1[j][r] *= f;
+                    s2[j][r] *= f;
+                }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const f32x4 v = widen4<DT>(xr[j]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float p = __builtin_amdgcn_exp2f(z[j][r] - m[j][r]), dx = v[r] - mu[j][r], pd = p * dx;
+                s0[j][r] += p;
+                s1[j][r] += pd;
+                s2[j][r] = __builtin_fmaf(pd, dx, s2[j][r]);
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float top = row16_max(m[j][r]), f = __builtin_amdgcn_exp2f(m[j][r] - top);
+            const float a0 = row16_sum(s0[j][r] * f), a1 = row16_sum(s1[j][r] * f), a2 = row16_sum(s2[j][r] * f);
+            if (n == 0) {
+                float *at = meet[wave][16 * j + 4 * g + r];
+                at[0] = top;
+                at[1] = a0;
+                at[2] = a1;
+                at[3] = a2;
+            }
+        }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int ch = threadIdx.x;
+    float top = meet[0][ch][0], a0 = 0.f, a1 = 0.f, a2 = 0.f;
+#pragma unroll
+    for (int k = 1; k < kWaves; ++k) top = __builtin_fmaxf(top, meet[k][ch][0]);
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k) {
+        const float f = __builtin_amdgcn_exp2f(meet[k][ch][0] - top);
+        a0 = __builtin_fmaf(f, meet[k][ch][1], a0);
+        a1 = __builtin_fmaf(f, meet[k][ch][2], a1);
+        a2 = __builtin_fmaf(f, meet[k][ch][3], a2);
+    }
+    const int64_t row = (int64_t)utt * 2 * a.wide;
+    const int c = c0 + ch;
+    const float dm = a1 / a0, mean = a.mean_std[row + c] + dm;
+    float var = a2 / a0 - dm * dm;
+    var = var < 1e-12f ? 1e-12f : var;
+    uint16_t *out = reinterpret_cast<uint16_t *>(a.out) + row;
+    out[c] = (uint16_t)Mma<DT>::pack(__builtin_fmaf(mean, a.a_pool[c], a.c_pool[c]), 0.f);
+    out[c + a.wide] = (uint16_t)Mma<DT>::pack(__builtin_fmaf(sqrtf(var), a.a_pool[c + a.wide], a.c_pool[c + a.wide]), 0.f);
+}
+
+// ----------------------------------------------------------------------------- launchers
+template <class DT, int MT, int NW, int PF>
+int launch_layer_mt(const LayerArgs &a, hipStream_t s) {
+    auto kern = layer_kernel<DT, MT, NW, PF>;
+    const size_t lds = (size_t)2 * 16 * MT * kRow;
+    if (!allow_lds(kern, lds)) return NA1D_ERR_LAUNCH;
+    const int64_t wgs = (a.M + 16 * MT - 1) / (16 * MT);
+    kern<<<(unsigned)wgs, 64 * NW, lds, s>>>(a);
+    return launch_status();
+}
+
+template <class DT> int launch_layer(const LayerArgs &a, hipStream_t s) {
+    // Fewer, larger tiles read the layer's weights fewer times; smaller ones spread few tokens over more CUs.
+    if (a.M <= 16 * 256) return launch_layer_mt<DT, 1, 8, 8>(a, s);
+    if (a.M <= 32 * 512) return launch_layer_mt<DT, 2, 8, 4>(a, s);
+    return launch_layer_mt<DT, 4, 4, 2>(a, s);
+}
+
+template <class DT, LinearEnd END> int launch_linear(const LinearArgs &a, hipStream_t s) {
+    if (a.inputs % 256 == 0 && a.M > 512) {
+        auto go = [&](auto kern, int mt, int ntw) {
+            const size_t lds = (size_t)2 * 16 * mt * kRow;
+            if (!allow_lds(kern, lds)) return (int)NA1D_ERR_LAUNCH;
+            const int cols = a.outputs / (64 * ntw);
+            kern<<<(unsigned)((a.M + 16 * mt - 1) / (16 * mt) * cols), kThreads, lds, s>>>(a, cols);
+            return launch_status();
+        };
+        if (a.outputs % 256 == 0 && a.M > 8192) return go(linear_kernel<DT, 4, 4, END>, 4, 4);
+        if (a.outputs % 128 == 0) return a.M > 8192 ? go(linear_kernel<DT, 4, 2, END>, 4, 2) : go(linear_kernel<DT, 2, 2, END>, 2, 2);
+    }
+    const int nt = a.outputs % 32 == 0 ? 2 : 1, cols = a.outputs / (16 * nt);
+    const unsigned wgs = (unsigned)((a.M + 15) / 16 * cols);
+    if (nt == 2)
+        linear_small_kernel<DT, 2, END><<<wgs, 512, 0, s>>>(a, cols);
+    else
+        linear_small_kernel<DT, 1, END><<<wgs, 512, 0, s>>>(a, cols);
+    return launch_status();
+}
+
+// The workspace's tensors, one behind the other.
+struct Buffers {
+    int64_t bytes = 0;
+    int64_t x, qkv, attn, blocks, patches, pos, h, hidden, stats, rounded, context, pooled, t_valid, count;
+    int64_t take(int64_t n) {
+        const int64_t at = bytes;
+        bytes += (n + 255) / 256 * 256;
+        return at;
+    }
+    Buffers(const na1d_encoder &e, int64_t N, int64_t T, int dense) {
+        const int64_t M = N * T;
+        x = take(M * kRow);
+        qkv = take(M * 3 * kRow);
+        attn = take(M * kRow);
+        blocks = take(M * e.blocks * kRow);
+        patches = take(M * e.in_chans * e.patch * 2);
+        pos = take(dense * T * kDim * 4);
+        h = take(M * e.wide * 2);
+        hidden = take(M * 256);
+        stats = take(N * 2 * e.wide * 4);
+        rounded = take(N * 2 * e.wide * 2);
+        context = take(N * 128 * 4);
+        pooled = take(N * 2 * e.wide * 2);
+        t_valid = take(N * 4);
+        count = take(N * 4);
+    }
+};
+inline int dense_layers(const na1d_encoder &e) {
+    int n = 0;
+    for (int i = 0; i < e.layers; ++i) n += e.layer[i].window == 0;
+    return n;
+}
+
+#define NA1D_TRY(...)                       \
+    do {                                    \
+        const int st_ = (__VA_ARGS__);      \
+        if (st_ != NA1D_OK) return st_;     \
+    } while (0)
+
+template <class DT>
+int encode(const na1d_encoder &e, char *out, const float *x, const float *lens, int64_t N, int64_t frames, char *ws, hipStream_t s) {
+    const int64_t T = (frames - e.patch) / e.patch + 1, M = N * T;
+    const int patch_width = 2 * e.in_chans * e.patch;
+    const Buffers b(e, N, T, dense_layers(e));
+    int32_t *t_valid = nullptr;
+    float *count = nullptr;
+    if (lens) {
+        t_valid = reinterpret_cast<int32_t *>(ws + b.t_valid);
+        count = reinterpret_cast<float *>(ws + b.count);
+        lengths_kernel<<<(unsigned)((N + 255) / 256), 256, 0, s>>>(t_valid, count, lens, (int)N, (int)frames, e.patch, (int)T);
+        NA1D_TRY(launch_status());
+    }
+    {
+        const size_t lds = (size_t)e.in_chans * (64 * e.patch + 1) * sizeof(float);
+        if (!allow_lds(patch_kernel<DT>, lds)) return NA1D_ERR_LAUNCH;
+        patch_kernel<DT><<<dim3((unsigned)((T + 63) / 64), (unsigned)N), 256, lds, s>>>(
+            reinterpret_cast<uint32_t *>(ws + b.patches), x, e.in_chans, (int)frames, e.patch, (int)T);
+        NA1D_TRY(launch_status());
+    }
+    int dense = 0;
+    for (int i = 0; i < e.layers; ++i) {
+        const na1d_encoder_layer &l = e.layer[i];
+        if (l.window) continue;
+        LinearArgs a{};
+        a.x = (const char *)e.pos;
+        a.w = (const char *)l.w_pos;
+        a.out = ws + b.pos + dense++ * T * kDim * 4;
+        a.bias = l.shift;
+        a.x_pitch = kRow;
+        a.out_pitch = 4 * kDim;
+        a.inputs = a.outputs = kDim;
+        a.M = (int)T;
+        NA1D_TRY(launch_linear<DT, kAffine>(a, s));
+    }
+    dense = 0;
+    int block = 0;
+    const char *x_in = nullptr;               // the residual stream of the layer before
+    int x_in_pitch = kRow;
+    for (int i = 0; i <= e.layers; ++i) {
+        LayerArgs a{};
+        a.M = (int)M;
+        a.T = (int)T;
+        a.T_magic = div_magic(T);
+        a.tail_groups = a.head_groups = 1;
+        if (i > 0) {
+            const na1d_encoder_layer &l = e.layer[i - 1];
+            a.attn = ws + b.attn;
+            a.x_in = x_in;
+            a.x_in_pitch = x_in_pitch;
+            a.w_proj = (const char *)l.w_proj, a.w_fc1 = (const char *)l.w_fc1, a.w_fc2 = (const char *)l.w_fc2;
+            a.b_proj = l.b_proj, a.b_fc1 = l.b_fc1, a.b_fc2 = l.b_fc2;
+            a.tail_groups = l.groups;
+            if (l.block_end) {
+                a.block_pitch = e.blocks * kRow;
+                a.block_out = ws + b.blocks + block++ * kRow;
+            }
+        }
+        if (i < e.layers) {
+            const na1d_encoder_layer &l = e.layer[i];
+            if (l.embeds) {
+                a.patches = ws + b.patches;
+                a.patch_width = patch_width;
+                a.w_embed = (const char *)l.w_embed;
+                a.b_embed = l.b_embed;
+            }
+            if (a.block_out && !l.embeds) {   // the block's output is the next layer's input as it is
+                x_in = a.block_out;
+                x_in_pitch = a.block_pitch;
+            } else {
+                a.x_out = ws + b.x;
+                x_in = a.x_out;
+                x_in_pitch = kRow;
+            }
+            a.qkv = ws + b.qkv;
+            a.w_qkv = (const char *)l.w_qkv;
+            a.b_qkv = l.b_qkv;
+            a.head_groups = l.groups;
+            if (!l.window) {
+                a.gain = l.gain;
+                a.posb = reinterpret_cast<const float *>(ws + b.pos + dense++ * T * kDim * 4);
+            }
+        }
+        NA1D_TRY(launch_layer<DT>(a, s));
+        if (i == e.layers) break;
+        const na1d_encoder_layer &l = e.layer[i];
+        Geom g;
+        g.B = N * l.heads;
+        g.T = T;
+        g.H = l.heads;
+        g.C = kDim / l.heads;
+        g.W = l.window ? l.window : 1;
+        g.L = l.window ? l.left : 0;
+        Layout in{T * 3 * kDim, g.C, 3 * kDim}, outl{T * kDim, g.C, kDim};
+        const char *q = ws + b.qkv, *k = q + kRow, *v = k + kRow;
+        if (l.window) {
+            set_dilation(g, l.dilation);
+            in.row *= g.dilation;
+            outl.row *= g.dilation;
+            int st = fused_fwd(ws + b.attn, nullptr, q, k, v, l.rpb, t_valid, g, in, outl, l.scale, DT::tag, s);
+            if (st == NA1D_ERR_UNSUPPORTED) st = wide_fwd(ws + b.attn, nullptr, q, k, v, l.rpb, t_valid, g, in, outl, l.scale, DT::tag, s);
+            NA1D_TRY(st);
+        } else {
+            NA1D_TRY(global_fwd(ws + b.attn, nullptr, q, k, v, t_valid, g, in, outl, l.scale, DT::tag, s));
+        }
+    }
+    LinearArgs a{};
+    a.x = ws + b.blocks, a.x_pitch = e.blocks * kRow, a.inputs = e.blocks * kDim, a.M = (int)M, a.T = (int)T;
+    a.w = (const char *)e.w_wide, a.bias = e.b_wide, a.scale = e.a_wide, a.offset = e.c_wide;
+    a.out = ws + b.h, a.out_pitch = 2 * e.wide, a.outputs = e.wide;
+    NA1D_TRY(launch_linear<DT, kReluNorm>(a, s));
+    stats_kernel<DT><<<dim3((unsigned)(e.wide / 64), (unsigned)N), 256, 0, s>>>(reinterpret_cast<float *>(ws + b.stats), ws + b.rounded,
+                                                                              ws + b.h, count, (int)T, e.wide);
+    NA1D_TRY(launch_status());
+    LinearArgs c{};
+    c.x = ws + b.rounded, c.x_pitch = 4 * e.wide, c.inputs = 2 * e.wide, c.M = (int)N;
+    c.w = (const char *)e.w_ctx, c.bias = e.b_att, c.out = ws + b.context, c.out_pitch = 4 * 128, c.outputs = 128;
+    NA1D_TRY(launch_linear<DT, kAffine>(c, s));
+    LinearArgs d{};
+    d.x = ws + b.h, d.x_pitch = 2 * e.wide, d.inputs = e.wide, d.M = (int)M, d.T = (int)T;
+    d.w = (const char *)e.w_att, d.bias = reinterpret_cast<const float *>(ws + b.context), d.scale = e.a_att, d.offset = e.c_att;
+    d.out = ws + b.hidden, d.out_pitch = 256, d.outputs = 128;
+    NA1D_TRY(launch_linear<DT, kTanhNorm>(d, s));
+    PoolArgs p{ws + b.h, ws + b.hidden, (const char *)e.w_logit, count, reinterpret_cast<const float *>(ws + b.stats), e.a_pool, e.c_pool,
+               ws + b.pooled, (int)T, e.wide};
+    pool_kernel<DT><<<dim3((unsigned)(e.wide / 64), (unsigned)N), kThreads, 0, s>>>(p);
+    NA1D_TRY(launch_status());
+    LinearArgs f{};
+    f.x = ws + b.pooled, f.x_pitch = 4 * e.wide, f.inputs = 2 * e.wide, f.M = (int)N;
+    f.w = (const char *)e.w_fc, f.bias = e.b_fc, f.out = out, f.out_pitch = 2 * e.emb, f.outputs = e.emb;
+    return launch_linear<DT, kEmbedding>(f, s);
+}
+
+// Sizes the kernels take (everything else is the caller's to run another way).
+bool encoder_ok(const na1d_encoder &e, int64_t N, int64_t frames) {
+    if (e.layers < 1 || e.blocks < 1 || e.patch < 1 || e.in_chans < 1 || e.wide < 256 || e.emb < 16 || frames < e.patch) return false;
+    if (e.in_chans > 4096 || e.patch > 256 || e.in_chans * e.patch % 32 || e.in_chans * e.patch > kDim || e.wide % 256 || e.emb % 16 || e.wide > (1 << 16) || e.emb > (1 << 16)) return false;
+    if ((size_t)e.in_chans * (64 * e.patch + 1) * sizeof(float) > 160 * 1024) return false;
+    const int64_t T = (frames - e.patch) / e.patch + 1;
+    // rows of an utterance stay in the reach of 31-bit offsets (the widest are those of the projection), launches of 31-bit ids
+    if (T > (1 << 29) / e.wide || N > 65535 || N * T > (1ll << 26) || frames > (1 << 24)) return false;
+    int blocks = 0;
+    for (int i = 0; i < e.layers; ++i) {
+        const na1d_encoder_layer &l = e.layer[i];
+        if (l.heads < 1 || kDim % l.heads || kDim / l.heads % 8 || kDim / l.heads > 128 || l.window < 0 || l.window > NA1D_MAX_WINDOW) return false;
+        if (l.window && (l.left < 0 || l.left >= l.window || l.dilation < 1)) return false;
+        if (!l.window && (!e.pos || e.pos_rows < T || !l.gain || !l.shift || !l.w_pos)) return false;
+        if (!l.w_qkv || !l.w_proj || !l.w_fc1 || !l.w_fc2 || (l.embeds && !l.w_embed)) return false;
+        blocks += l.block_end != 0;
+    }
+    return blocks == e.blocks && e.layer[0].embeds && e.layer[e.layers - 1].block_end;
+}
+int64_t workspace_bytes(const na1d_encoder &e, int64_t N, int64_t frames) {
+    return Buffers(e, N, (frames - e.patch) / e.patch + 1, dense_layers(e)).bytes;
+}
+int run(const na1d_encoder &e, void *out, const float *x, const float *lens, int64_t N, int64_t frames, void *ws, hipStream_t s) {
+    return e.dtype == NA1D_BF16 ? encode<BF16>(e, (char *)out, x, lens, N, frames, (char *)ws, s)
+                                : encode<FP16>(e, (char *)out, x, lens, N, frames, (char *)ws, s);
+}
+
+}  // namespace enc
+}  // namespace na1d
+

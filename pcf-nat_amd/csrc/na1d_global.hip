@@ -69,6 +69,7 @@ struct GlobalArgs {
     int pitch;                   // bytes per row = 2 * head_dim (packed rows)
     float scale;
     Dropout drop;                // attention dropout; its window slot is the key's row index
+    Strides in, outl;            // forward: where q, k, v and the output have their rows
 };
 
 // =============================================================================
@@ -90,7 +91,8 @@ global_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *_
                   uint32_t items, GlobalArgs a) {
     using LL = Lds<C>;
     constexpr int CT = C / 16;
-    fetch_args_now(out, lse, q, k, v, t_valid, items, a.T, a.H, a.strips, a.strips_magic, a.heads_magic, a.pitch, a.scale);
+    fetch_args_now(out, lse, q, k, v, t_valid, items, a.T, a.H, a.strips, a.strips_magic, a.heads_magic, a.scale, a.in.sample,
+                   a.in.head, a.in.pitch, a.in.width, a.outl.sample, a.outl.head, a.outl.pitch);
     if constexpr (DROP) fetch_args_now(a.drop.threshold, a.drop.seed_lo, a.drop.seed_hi, a.drop.inv_keep);
     constexpr int kStep = region_bytes<C>(kStripTiles);
     extern __shared__ __attribute__((aligned(16))) char smem[];          // 4 * kStep bytes: K and V of two chunks
@@ -105,19 +107,21 @@ global_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *_
     const uint32_t sample = div_by(b, a.H, a.heads_magic);
     const int T = a.T, tiles = (T + 15) >> 4;
 
-    const int64_t seq_off = (int64_t)b * T * a.pitch;
-    const Rsrc qs = make_rsrc(q + seq_off, T * a.pitch), ks = make_rsrc(k + seq_off, T * a.pitch);
-    const Rsrc vs = make_rsrc(v + seq_off, T * a.pitch), os = make_rsrc(out + seq_off, T * a.pitch);
+    const int64_t in_off = sample * a.in.sample + (b - sample * a.H) * a.in.head;
+    const int64_t out_off = sample * a.outl.sample + (b - sample * a.H) * a.outl.head;
+    const int pitch = a.in.pitch, width = a.in.width;
+    const Rsrc qs = make_rsrc(q + in_off, T * pitch), ks = make_rsrc(k + in_off, T * pitch);
+    const Rsrc vs = make_rsrc(v + in_off, T * pitch), os = make_rsrc(out + out_off, T * a.outl.pitch);
     const Rsrc ls = make_rsrc(lse ? lse + (int64_t)b * T : nullptr, lse ? T * 4 : 0);
-    const int lane_off = direct_lane_offset<C>(wave, lane, a.pitch, a.pitch);
-    stage_direct<C, kStripTiles, kReadShared>(ks, 0, kv_lds, kStripTiles, wave, lane_off, a.pitch);
-    stage_direct<C, kStripTiles, kReadShared>(vs, 0, kv_lds + kStep, kStripTiles, wave, lane_off, a.pitch);
+    const int lane_off = direct_lane_offset<C>(wave, lane, pitch, width);
+    stage_direct<C, kStripTiles, kReadShared>(ks, 0, kv_lds, kStripTiles, wave, lane_off, pitch);
+    stage_direct<C, kStripTiles, kReadShared>(vs, 0, kv_lds + kStep, kStripTiles, wave, lane_off, pitch);
     int qt[QT];                                             // this wave's query tiles
     RowOperand<C> qop[QT];
 #pragma unroll
     for (int h = 0; h < QT; ++h) {
         qt[h] = kStripTiles * (QT * strip + h) + wave;
-        load_rows<C, kReadShared>(qop[h], qs, 16 * qt[h] * a.pitch, a.pitch, a.pitch, lane);
+        load_rows<C, kReadShared>(qop[h], qs, 16 * qt[h] * pitch, pitch, width, lane);
     }
     int tv = T;
     if (t_valid) tv = max(0, min(T, t_valid[sample]));
@@ -240,8 +244,8 @@ global_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *_
         barrier_lds();      // this chunk has landed, and every wave is done with the one before, whose regions the next takes
         if (c0 + kStripTiles < tiles) {
             LDS_PTR(char) next = kv_lds + (at ^ 2 * kStep);
-            stage_direct<C, kStripTiles, kReadShared>(ks, 16 * (c0 + kStripTiles), next, kStripTiles, wave, lane_off, a.pitch);
-            stage_direct<C, kStripTiles, kReadShared>(vs, 16 * (c0 + kStripTiles), next + kStep, kStripTiles, wave, lane_off, a.pitch);
+            stage_direct<C, kStripTiles, kReadShared>(ks, 16 * (c0 + kStripTiles), next, kStripTiles, wave, lane_off, pitch);
+            stage_direct<C, kStripTiles, kReadShared>(vs, 16 * (c0 + kStripTiles), next + kStep, kStripTiles, wave, lane_off, pitch);
         }
         chunk(whole, c0, kv_lds + at, kv_lds + at + kStep);
         at ^= 2 * kStep;
@@ -258,7 +262,7 @@ global_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *_
         u32x2 ow[CT];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) ow[ct] = pack_acc<DT>(o[h][ct], inv);
-        store_tile<C>(os, qrow * a.pitch, ow, g, stores_whole_lines(a.pitch, C, 0), a.pitch);   // rows past T are dropped
+        store_tile<C>(os, qrow * a.outl.pitch, ow, g, stores_whole_lines(a.outl.pitch, C, 0), width);   // rows past T are dropped
         const float pad = qrow >= tv ? kMaskValue : 0.f;
         if (g == 0)
             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((m[h] + __builtin_amdgcn_logf(l[h])) * kLn2 + pad), ls, qrow * 4, 0, 0);
@@ -278,9 +282,10 @@ global_fwd_short_kernel(char *__restrict__ out, float *__restrict__ lse, const c
                         GlobalArgs a) {
     using LL = Lds<C>;
     constexpr int CT = C / 16, kW = TILES / QT;       // waves of the workgroup, QT query tiles each
-    fetch_args_now(out, lse, q, k, v, t_valid, a.T, a.H, a.heads_magic, a.pitch, a.scale);
+    fetch_args_now(out, lse, q, k, v, t_valid, a.T, a.H, a.heads_magic, a.scale, a.in.sample, a.in.head, a.in.pitch, a.in.width,
+                   a.outl.sample, a.outl.head, a.outl.pitch);
     if constexpr (DROP) fetch_args_now(a.drop.threshold, a.drop.seed_lo, a.drop.seed_hi, a.drop.inv_keep);
-    const int T = a.T, tiles = (T + 15) >> 4, pitch = a.pitch;      // rows of head_dim channels, zero-padded to C on the way in
+    const int T = a.T, tiles = (T + 15) >> 4, pitch = a.in.pitch, width = a.in.width;      // rows of head_dim channels, zero-padded to C on the way in
     extern __shared__ __attribute__((aligned(16))) char smem[];          // 2 * region_bytes<C>(tiles)
     LDS_PTR(char) k_lds = (LDS_PTR(char))smem;
     LDS_PTR(char) v_lds = k_lds + region_bytes<C>(tiles);
@@ -289,21 +294,22 @@ global_fwd_short_kernel(char *__restrict__ out, float *__restrict__ lse, const c
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, n = lane & 15;
     const uint32_t b = blockIdx.x;
-    const int64_t seq_off = (int64_t)((uint64_t)b * (uint32_t)(T * pitch));
-    const Rsrc ks = make_rsrc(k + seq_off, T * pitch), vs = make_rsrc(v + seq_off, T * pitch);
-    const Rsrc qs = make_rsrc(q + seq_off, T * pitch);
-    const int lane_off = direct_lane_offset<C>(wave, lane, pitch, pitch);
+    const uint32_t sample = div_by(b, a.H, a.heads_magic), head = b - sample * a.H;
+    const int64_t in_off = sample * a.in.sample + head * a.in.head;
+    const Rsrc ks = make_rsrc(k + in_off, T * pitch), vs = make_rsrc(v + in_off, T * pitch);
+    const Rsrc qs = make_rsrc(q + in_off, T * pitch);
+    const int lane_off = direct_lane_offset<C>(wave, lane, pitch, width);
     stage_direct<C, TILES, kReadOnce, kW>(ks, 0, k_lds, tiles, wave, lane_off, pitch);
     stage_direct<C, TILES, kReadOnce, kW>(vs, 0, v_lds, tiles, wave, lane_off, pitch);
     RowOperand<C> qop[QT];
 #pragma unroll
-    for (int h = 0; h < QT; ++h) load_rows<C, kReadOnce>(qop[h], qs, 16 * (wave + kW * h) * pitch, pitch, pitch, lane);
+    for (int h = 0; h < QT; ++h) load_rows<C, kReadOnce>(qop[h], qs, 16 * (wave + kW * h) * pitch, pitch, width, lane);
     __builtin_amdgcn_sched_barrier(0);
 
-    const uint32_t sample = div_by(b, a.H, a.heads_magic);
     int tv = T;
     if (t_valid) tv = max(0, min(T, t_valid[sample]));
-    const Rsrc os = make_rsrc(out + seq_off, T * pitch);
+    const int out_pitch = a.outl.pitch;
+    const Rsrc os = make_rsrc(out + sample * a.outl.sample + head * a.outl.head, T * out_pitch);
     const Rsrc ls = make_rsrc(lse ? lse + (int64_t)b * T : nullptr, lse ? T * 4 : 0);
     const float scale2 = a.scale * kLog2e, mask2 = kMaskValue * kLog2e;
     RowLane<C> row_lane;
@@ -434,7 +440,7 @@ global_fwd_short_kernel(char *__restrict__ out, float *__restrict__ lse, const c
         u32x2 ow[CT];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) ow[ct] = pack_acc<DT>(o[h][ct], inv);
-        store_tile<C>(os, qrow * pitch, ow, g, stores_whole_lines(pitch, C, 0), pitch);     // rows past T are dropped
+        store_tile<C>(os, qrow * out_pitch, ow, g, stores_whole_lines(out_pitch, C, 0), width);     // rows past T are dropped
         const float pad = qrow >= tv ? kMaskValue : 0.f;
         if (g == 0)
             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((m[h] + __builtin_amdgcn_logf(l[h])) * kLn2 + pad), ls, qrow * 4, 0, 0);
@@ -966,11 +972,13 @@ inline bool global_ok(const Geom &g, GlobalArgs &a, int64_t &items) {
 
 template <class DT, int C>
 int launch_global_fwd(void *out, float *lse, const void *q, const void *k, const void *v, const int32_t *t_valid,
-                      const Geom &g, float scale, hipStream_t s) {
+                      const Geom &g, const Layout &in, const Layout &outl, float scale, hipStream_t s) {
     GlobalArgs a;
     int64_t items;
-    if (!global_ok(g, a, items)) return NA1D_ERR_UNSUPPORTED;
+    if (!global_ok(g, a, items) || !strides_ok(in, g) || !strides_ok(outl, g)) return NA1D_ERR_UNSUPPORTED;
     a.scale = scale;
+    a.in = byte_strides(in, g);
+    a.outl = byte_strides(outl, g);
     const char *dt_name = DT::tag == NA1D_BF16 ? "BF16" : "FP16", *drop_name = g.drop.threshold ? "true" : "false";
     if (g.T <= 16 * kShortTiles) {
         // sequences of up to 4 tiles: a tile to each of the 4 waves; longer ones: two, which read every key and value
@@ -1062,8 +1070,8 @@ int launch_global_bwd(void *dq, void *dk, void *dv, float *delta, const void *q,
 }
 
 int global_fwd(void *out, float *lse, const void *q, const void *k, const void *v, const int32_t *t_valid,
-               const Geom &g, float scale, int dtype, hipStream_t s) {
-    NA1D_MFMA_DISPATCH(launch_global_fwd, out, lse, q, k, v, t_valid, g, scale, s);
+               const Geom &g, const Layout &in, const Layout &outl, float scale, int dtype, hipStream_t s) {
+    NA1D_MFMA_DISPATCH(launch_global_fwd, out, lse, q, k, v, t_valid, g, in, outl, scale, s);
 }
 
 int global_bwd(void *dq, void *dk, void *dv, float *delta, const void *q, const void *k, const void *v, const void *out,

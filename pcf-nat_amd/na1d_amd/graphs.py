@@ -7,6 +7,8 @@ from __future__ import annotations
 
 import torch
 
+from .encoder import plans_of
+
 
 class GraphedInference:
     """``model(x)`` (or ``model(x, lens)``) for one input shape, replayed from a captured graph.
@@ -32,6 +34,7 @@ class GraphedInference:
         self.graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(self.graph):
             self.out = self._eager(self.x, self.lens)
+        self.plans = plans_of(model)                               # the weights the graph reads live as long as it does
         for i in range(verify):
             x = example + 0.01 * (i + 1) * torch.randn_like(example)
             want = self._eager(x, lens)

@@ -31,6 +31,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .dense import global_attention
+from .encoder import embed as embed_natively
 from .fused import na1d_fused, na1d_fused_qkv
 from .nattn import getNA1dFunction
 
@@ -693,6 +694,9 @@ class _NATransformer(nn.Module):
         """x: [N, in_chans, frames]; lens: relative lengths in (0, 1] or None.  Returns [N, output_emb_size]."""
         tin = x.shape[-1]
         assert self.frames == tin or not self.training
+        out = embed_natively(self, x, lens)                           # inference at the published sizes: one native call
+        if out is not None:
+            return out
         padding = None
         if lens is not None:
             padding = ((tin - torch.round(lens * tin)) // self.patch_size).to(torch.int64)

@@ -339,3 +339,63 @@ def test_mfa_nat_4x4_full_batch_training_step_agrees_with_the_checked_small_batc
     grads = [p.grad for p in gpu.parameters() if p.grad is not None]
     assert len(grads) > 100 and all(torch.isfinite(gr).all() for gr in grads)
     assert sum(float(gr.abs().max() > 0) for gr in grads) > 0.9 * len(grads)
+
+
+# tokens of the batch: a single tile, tiles of 16 and their remainder, the first launch with tiles of 32 and of 64
+@pytest.mark.parametrize("batch,frames,lengths", [(1, 16, False), (3, 111, True), (65, 130, True), (130, 256, False)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("family", ["pcf", "mfa"])
+def test_native_encoder_at_tile_edges(family, dtype, batch, frames, lengths):
+    """The whole model in one native call (na1d_encode) against the CPU fp32 twin at every tile size of its kernels:
+    grouped projections (8, 4, 2, 1), narrow and wide windows, a dilated layer, dense layers, lengths.  The relative
+    error is four times what 16 bit shows over the depth of the full models (5e-3 / 6e-4)."""
+    kw = dict(depths=(2, 1, 2, 1), num_heads=[[16, 4], [16], [8, 16], [4]], win_size=[[27, 0], [27], [9, 33], [0]],
+              dilation=[[1, 1], 2, 1, 1])
+    if family == "pcf":
+        kw["groups"] = (8, 4, 2, 1)
+    factory = models.PCF_NATransformer if family == "pcf" else models.MFA_NATransformer
+    cpu = _twin(factory, dtype, seed=7, **kw).eval()
+    gpu = factory(na="fused_qkv", dtype=dtype, **kw)
+    gpu.load_state_dict(cpu.state_dict())
+    gpu = gpu.cuda().eval()
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(batch, 80, frames, generator=g)
+    lens = (0.3 + 0.7 * torch.rand(batch, generator=g)) if lengths else None
+    with torch.no_grad(), torch.autocast("cuda", dtype=dtype):
+        got = models.embed_natively(gpu, x.cuda(), None if lens is None else lens.cuda())
+        assert got is not None and got.dtype == dtype
+    with torch.no_grad():
+        want = cpu(x, lens)
+    assert O.rel_l2(got.float(), want) < (2e-2 if dtype == torch.bfloat16 else 2.5e-3)
+
+
+def test_native_encoder_follows_the_weights():
+    """The plan is made of the present weights: a changed parameter, statistic or submodule shows in the next call, and
+    two streams calling at once have workspaces of their own."""
+    torch.manual_seed(0)
+    kw = dict(depths=(1, 1), num_heads=[[16], [4]], win_size=[[27], [0]], groups=(8, 4))
+    model = models.PCF_NATransformer(na="fused_qkv", **kw).cuda().eval()
+    x = torch.randn(5, 80, 90, generator=torch.Generator().manual_seed(1)).cuda()
+
+    def run():
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+            return models.embed_natively(model, x).clone()
+    first = run()
+    assert torch.equal(first, run())
+    with torch.no_grad():
+        model.blocks[0].blocks[0].mlp.fc1.weight.mul_(1.5)
+    second = run()
+    assert not torch.equal(first, second)
+    with torch.no_grad():
+        model.norm.running_mean.add_(0.3)
+    third = run()
+    assert not torch.equal(second, third)
+    model.fc = torch.nn.Linear(model.fc.in_features, 64).cuda()
+    assert run().shape == (5, 64)
+    outs, streams = [], [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for s in streams * 3:
+        with torch.cuda.stream(s):
+            outs.append(run())
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, outs[0]) for o in outs)
