@@ -313,6 +313,43 @@ int na1d_encode(const na1d_encoder *e, void *out, const float *x, const float *l
                 void *workspace, int64_t workspace_bytes, void *stream);
 
 /*
+ * One windowed layer of those models in training (models/PCF_NATransformer.py:228-265, models/MFA_NATransformer.py:224-261),
+ * forward and backward, on token-major 16-bit activations x, out, dout, dx [N, T, dim]:
+ *   x1 = x + f_attn * proj(attention(qkv(norm1(x)))),   out = x1 + f_mlp * fc2(gelu(fc1(norm2(x1))))
+ * with batch norms over all N * T tokens (fp32 statistics; the running ones are updated by the forward), weights in fp32
+ * rounded to 16 bit for the products, sums in fp32.  Weights lie as [outputs, inputs / groups] (a linear layer, or a grouped
+ * 1x1 convolution); `ordered` says that the qkv projection's outputs are a channels-first model's (channel
+ * ((f % (dim / groups)) * groups + f / (dim / groups)) * 3 + which is q, k or v of head-major channel f).  dim and hidden are
+ * multiples of 256, groups have multiples of 32 channels; NA1D_ERR_UNSUPPORTED otherwise.
+ */
+typedef struct na1d_train_norm {
+    const float *weight, *bias;                 /* [dim] */
+    float *running_mean, *running_var;
+    int64_t *batches;                           /* one is added by a forward */
+    float *dweight, *dbias;                     /* written by the backward */
+    float eps, momentum;
+} na1d_train_norm;
+typedef struct na1d_train_layer {
+    int32_t dtype, dim, hidden, heads, window, left, dilation, groups, ordered;
+    float scale;
+    na1d_train_norm norm[2];
+    const float *w[4], *b[4];                   /* qkv, proj, fc1, fc2 */
+    float *dw[4], *db[4];                       /* written by the backward */
+    const float *rpb;                           /* [heads, window] */
+    float *drpb;                                /* added to */
+    const float *scale_attn, *scale_mlp;        /* f_attn, f_mlp: fp32 [N] (stochastic depth), NULL for 1 */
+} na1d_train_layer;
+
+/* `saved` is what a forward leaves for its backward; the workspaces are free again when the call's kernels are done. */
+int64_t na1d_train_layer_saved_bytes(const na1d_train_layer *l, int64_t N, int64_t T);
+int64_t na1d_train_layer_workspace_bytes(const na1d_train_layer *l, int64_t N, int64_t T, int backward);
+int na1d_train_layer_forward(const na1d_train_layer *l, void *out, const void *x, void *saved, int64_t saved_bytes,
+                             void *workspace, int64_t workspace_bytes, int64_t N, int64_t T, void *stream);
+int na1d_train_layer_backward(const na1d_train_layer *l, void *dx, const void *dout, const void *x, const void *saved,
+                              int64_t saved_bytes, void *workspace, int64_t workspace_bytes, int64_t N, int64_t T,
+                              void *stream);
+
+/*
  * Profiling hook; no counterpart in the reference.  From this call on, the matrix-core fused kernels that the
  * CALLING THREAD launches record `start` just before and `stop` just after the kernel itself (hipEvent_t handles,
  * recorded by hipExtLaunchKernel: the dispatch's own begin and end, i.e. what a profiler's kernel trace reports,

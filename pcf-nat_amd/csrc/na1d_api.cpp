@@ -445,6 +445,62 @@ int na1d_encode(const na1d_encoder *e, void *out, const float *x, const float *l
     return na1d::enc::run(*e, out, x, lens, N, frames, workspace, (hipStream_t)stream);
 }
 
+static int train_check(const na1d_train_layer *l, int64_t N, int64_t T) {
+    if (!l) return NA1D_ERR_NULL;
+    if (l->dtype != NA1D_BF16 && l->dtype != NA1D_FP16) return NA1D_ERR_DTYPE;
+    if (N < 0 || T < 0) return NA1D_ERR_SHAPE;
+    return mfma_allowed() && na1d::train::layer_ok(*l, N, T) ? NA1D_OK : NA1D_ERR_UNSUPPORTED;
+}
+static int train_pointers(const na1d_train_layer *l, bool backward) {
+    if (bad_scale(l->scale)) return NA1D_ERR_SCALE;
+    if (!l->rpb) return NA1D_ERR_NULL;
+    for (int j = 0; j < 4; ++j) {
+        const float *w = backward ? l->dw[j] : l->w[j], *b = backward ? l->db[j] : l->b[j];
+        if (!w || !b) return NA1D_ERR_NULL;
+        if (misaligned(w)) return NA1D_ERR_ALIGN;
+    }
+    for (int j = 0; j < 2; ++j) {
+        const na1d_train_norm &n = l->norm[j];
+        if (!n.weight || (backward ? !n.dweight || !n.dbias : !n.bias || !n.running_mean || !n.running_var || !n.batches))
+            return NA1D_ERR_NULL;
+    }
+    return NA1D_OK;
+}
+
+int64_t na1d_train_layer_saved_bytes(const na1d_train_layer *l, int64_t N, int64_t T) {
+    const int st = train_check(l, N, T);
+    return st == NA1D_OK ? na1d::train::saved_bytes(*l, N, T) : st;
+}
+
+int64_t na1d_train_layer_workspace_bytes(const na1d_train_layer *l, int64_t N, int64_t T, int backward) {
+    const int st = train_check(l, N, T);
+    return st == NA1D_OK ? na1d::train::scratch_bytes(*l, N, T, backward != 0) : st;
+}
+
+int na1d_train_layer_forward(const na1d_train_layer *l, void *out, const void *x, void *saved, int64_t saved_bytes, void *workspace,
+                             int64_t workspace_bytes, int64_t N, int64_t T, void *stream) {
+    int st = train_check(l, N, T);
+    if (st == NA1D_OK) st = train_pointers(l, false);
+    if (st != NA1D_OK) return st;
+    if (!out || !x || !saved || !workspace) return NA1D_ERR_NULL;
+    if (misaligned(out) || misaligned(x) || misaligned(saved) || misaligned(workspace)) return NA1D_ERR_ALIGN;
+    if (saved_bytes < na1d::train::saved_bytes(*l, N, T) || workspace_bytes < na1d::train::scratch_bytes(*l, N, T, false))
+        return NA1D_ERR_WORKSPACE;
+    return na1d::train::run_forward(*l, out, x, saved, workspace, N, T, (hipStream_t)stream);
+}
+
+int na1d_train_layer_backward(const na1d_train_layer *l, void *dx, const void *dout, const void *x, const void *saved,
+                              int64_t saved_bytes, void *workspace, int64_t workspace_bytes, int64_t N, int64_t T, void *stream) {
+    int st = train_check(l, N, T);
+    if (st == NA1D_OK) st = train_pointers(l, true);
+    if (st != NA1D_OK) return st;
+    if (!dx || !dout || !x || !saved || !workspace || !l->drpb) return NA1D_ERR_NULL;
+    if (misaligned(dx) || misaligned(dout) || misaligned(x) || misaligned(saved) || misaligned(workspace)) return NA1D_ERR_ALIGN;
+    if (saved_bytes < na1d::train::saved_bytes(*l, N, T) || workspace_bytes < na1d::train::scratch_bytes(*l, N, T, true))
+        return NA1D_ERR_WORKSPACE;
+    return na1d::train::run_backward(*l, dx, dout, x, saved, workspace, N, T, (hipStream_t)stream);
+}
+
 int na1d_fused_backward_noalloc(void *dq, void *dk, void *dv, float *drpb, const void *q, const void *k, const void *v,
                                 const void *out, const void *dout, const float *lse, const float *rpb,
                                 const int32_t *t_valid, int64_t B, int64_t H, int64_t T, int64_t C, int64_t W,

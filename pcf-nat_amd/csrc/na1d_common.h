@@ -214,4 +214,14 @@ int run(const na1d_encoder &e, void *out, const float *x, const float *lens, int
         hipStream_t s);
 }  // namespace enc
 
+// ---- a layer of those models in training: na1d_train.hip ------------------
+namespace train {
+bool layer_ok(const na1d_train_layer &l, int64_t N, int64_t T);
+int64_t saved_bytes(const na1d_train_layer &l, int64_t N, int64_t T);
+int64_t scratch_bytes(const na1d_train_layer &l, int64_t N, int64_t T, bool backward);
+int run_forward(const na1d_train_layer &l, void *out, const void *x, void *saved, void *ws, int64_t N, int64_t T, hipStream_t s);
+int run_backward(const na1d_train_layer &l, void *dx, const void *dout, const void *x, const void *saved, void *ws, int64_t N,
+                 int64_t T, hipStream_t s);
+}  // namespace train
+
 }  // namespace na1d

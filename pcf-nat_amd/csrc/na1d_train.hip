@@ -1,0 +1,815 @@
+// An encoder layer of the speaker-embedding models (models/PCF_NATransformer.py:228-265, models/MFA_NATransformer.py:
+// 224-261) in training, forward and backward, on token-major activations: batch norms with batch statistics, projections,
+// GELU, residuals and weight gradients around the attention kernels.
+//
+// A layer of 128 x 100 tokens, 256 channels, fp16, forward and backward: 29 launches of 215 us together, where the modules
+// took some 80 launches and 800 us (torch's batch norm of a transposed view with its copies, bias gradients as reductions of
+// their own, weight gradients through 16-bit sums of chunks).  Everything is launched by two calls, so the host keeps ahead.
+#include "na1d_encoder.h"
+
+namespace na1d {
+namespace train {
+
+using namespace enc;
+
+// =============================================================================
+// Batch norm over the rows of [M, C]
+// =============================================================================
+// Bound by memory: a pass over 12800 x 256 16-bit values is 6.5 MB.  A workgroup takes 64 channels (whole 128-byte lines)
+// of one of up to 64 chunks of rows; its sums are those of the differences to the chunk's first row, and the chunks meet
+// by their means (nothing cancels, however far the mean is from zero).  The kernel that uses the statistics combines the
+// chunks itself (32 KB from L2) instead of waiting for a third launch.  12800 x 256: sums 5.0 us and application 8.3 us
+// forward, 7.9 and 8.7 us backward, where torch took 31 and 54 us, and 13 us for each change of layout.
+constexpr int kBnCols = 64, kBnThreads = 256, kBnLanes = kBnThreads / 8, kBnChunks = 64;
+struct Chunks {
+    int rows, count;          // rows of a chunk (the last may have fewer), chunks
+};
+inline Chunks bn_chunks(int64_t M) {
+    const int64_t rows = std::max<int64_t>((M + kBnChunks - 1) / kBnChunks, kBnLanes);
+    return Chunks{(int)rows, (int)((M + rows - 1) / rows)};
+}
+template <class DT> __device__ inline void unpack(u32x4 w, float (&v)[8]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const f32x2 p = widen<DT>(w[i]);
+        v[2 * i] = p.x;
+        v[2 * i + 1] = p.y;
+    }
+}
+template <class DT> __device__ inline u32x4 repack(const float (&v)[8]) {
+    return u32x4{Mma<DT>::pack(v[0], v[1]), Mma<DT>::pack(v[2], v[3]), Mma<DT>::pack(v[4], v[5]), Mma<DT>::pack(v[6], v[7])};
+}
+// Sums over the 32 row lanes: a[channel of this thread's eight] -> total of channel `threadIdx.x & 63`, in threads below 64.
+__device__ inline void meet(float (*part)[kBnCols + 1], float (*quarter)[kBnCols], const float (&v)[8], float &total) {
+    const int c = threadIdx.x & 7, r = threadIdx.x >> 3, ch = threadIdx.x & 63, q = threadIdx.x >> 6;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) part[r][8 * c + i] = v[i];
+    __syncthreads();
+    float s = 0.f;
+#pragma unroll
+    for (int k = 0; k < kBnLanes / 4; ++k) s += part[q * (kBnLanes / 4) + k][ch];
+    quarter[q][ch] = s;
+    __syncthreads();
+    total = quarter[0][ch] + quarter[1][ch] + (quarter[2][ch] + quarter[3][ch]);
+}
+// The four groups of 64 threads' sums of one value per channel.
+__device__ inline float across_groups(float (*quarter)[kBnCols], float v) {
+    const int ch = threadIdx.x & 63, q = threadIdx.x >> 6;
+    __syncthreads();
+    quarter[q][ch] = v;
+    __syncthreads();
+    return quarter[0][ch] + quarter[1][ch] + (quarter[2][ch] + quarter[3][ch]);
+}
+
+template <class DT>
+__global__ void __launch_bounds__(kBnThreads)
+bn_stats_kernel(float *__restrict__ part_mean, float *__restrict__ part_m2, const char *__restrict__ x, int M, int C, int rows) {
+    __shared__ float part[kBnLanes][kBnCols + 1], quarter[4][kBnCols];
+    const int c = threadIdx.x & 7, r = threadIdx.x >> 3, c0 = blockIdx.x * kBnCols, r0 = blockIdx.y * rows, r1 = min(M, r0 + rows);
+    const char *src = x + 2 * (int64_t)(c0 + 8 * c);
+    const int64_t pitch = 2 * (int64_t)C;
+    float first[8], s1[8], s2[8];
+    unpack<DT>(*reinterpret_cast<const u32x4 *>(src + r0 * pitch), first);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s1[i] = s2[i] = 0.f;
+#pragma unroll 4
+    for (int t = r0 + r; t < r1; t += kBnLanes) {
+        float v[8];
+        unpack<DT>(*reinterpret_cast<const u32x4 *>(src + t * pitch), v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float d = v[i] - first[i];
+            s1[i] += d;
+            s2[i] = __builtin_fmaf(d, d, s2[i]);
+        }
+    }
+    float a, b;
+    meet(part, quarter, s1, a);
+    meet(part, quarter, s2, b);
+    if (threadIdx.x >= kBnCols) return;
+    const int ch = threadIdx.x;
+    const float x0 = widen<DT>((uint32_t)*reinterpret_cast<const uint16_t *>(x + r0 * pitch + 2 * (c0 + ch))).x;
+    const float m = a / (float)(r1 - r0);
+    part_mean[(int64_t)blockIdx.y * C + c0 + ch] = x0 + m;
+    part_m2[(int64_t)blockIdx.y * C + c0 + ch] = b - a * m;
+}
+
+struct BnApply {
+    char *y;
+    const char *x;
+    const float *part_mean, *part_m2, *weight, *bias;
+    float *mean, *rstd;                        // for the backward
+    float *running_mean, *running_var;
+    int64_t *batches;                          // counts the calls, as torch's module does
+    float eps, momentum;
+    int M, C, rows, chunks;
+};
+template <class DT>
+__global__ void __launch_bounds__(kBnThreads)
+bn_apply_kernel(BnApply a) {
+    __shared__ float quarter[4][kBnCols], s_mean[kBnCols], s_a[kBnCols], s_b[kBnCols];
+    const int c0 = blockIdx.x * kBnCols, ch = threadIdx.x & 63, q = threadIdx.x >> 6;
+    float s = 0.f;
+#pragma unroll 4
+    for (int k = q; k < a.chunks; k += 4) s = __builtin_fmaf((float)min(a.rows, a.M - k * a.rows), a.part_mean[(int64_t)k * a.C + c0 + ch], s);
+    const float mean = across_groups(quarter, s) / (float)a.M;
+    s = 0.f;
+#pragma unroll 4
+    for (int k = q; k < a.chunks; k += 4) {
+        const float d = a.part_mean[(int64_t)k * a.C + c0 + ch] - mean;
+        s += a.part_m2[(int64_t)k * a.C + c0 + ch] + (float)min(a.rows, a.M - k * a.rows) * d * d;
+    }
+    const float m2 = across_groups(quarter, s), rstd = rsqrtf(m2 / (float)a.M + a.eps);
+    if (threadIdx.x < kBnCols) {
+        s_mean[ch] = mean;
+        s_a[ch] = rstd * a.weight[c0 + ch];
+        s_b[ch] = a.bias[c0 + ch];
+        if (blockIdx.y == 0) {
+            a.mean[c0 + ch] = mean;
+            a.rstd[c0 + ch] = rstd;
+            a.running_mean[c0 + ch] += a.momentum * (mean - a.running_mean[c0 + ch]);
+            a.running_var[c0 + ch] += a.momentum * (m2 / (float)(a.M - 1) - a.running_var[c0 + ch]);
+            if (c0 == 0 && ch == 0) *a.batches += 1;
+        }
+    }
+    __syncthreads();
+    const int c = threadIdx.x & 7, r0 = blockIdx.y * a.rows, r1 = min(a.M, r0 + a.rows);
+    float m[8], k[8], b[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m[i] = s_mean[8 * c + i], k[i] = s_a[8 * c + i], b[i] = s_b[8 * c + i];
+    const int64_t pitch = 2 * (int64_t)a.C, at = 2 * (int64_t)(c0 + 8 * c);
+#pragma unroll 4
+    for (int t = r0 + (threadIdx.x >> 3); t < r1; t += kBnLanes) {
+        float v[8];
+        unpack<DT>(*reinterpret_cast<const u32x4 *>(a.x + t * pitch + at), v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = __builtin_fmaf(v[i] - m[i], k[i], b[i]);
+        *reinterpret_cast<u32x4 *>(a.y + t * pitch + at) = repack<DT>(v);
+    }
+}
+
+// Backward: sums of dy and of dy * (x - mean) over a chunk's rows, then
+// dx = weight * rstd * (dy - sum(dy) / M - (x - mean) * rstd^2 * sum(dy (x - mean)) / M) + `add`.
+template <class DT>
+__global__ void __launch_bounds__(kBnThreads)
+bn_bwd_sums_kernel(float *__restrict__ part_dy, float *__restrict__ part_dyx, const char *__restrict__ dy, const char *__restrict__ x,
+                   const float *__restrict__ mean, int M, int C, int rows) {
+    __shared__ float part[kBnLanes][kBnCols + 1], quarter[4][kBnCols];
+    const int c = threadIdx.x & 7, r = threadIdx.x >> 3, c0 = blockIdx.x * kBnCols, r0 = blockIdx.y * rows, r1 = min(M, r0 + rows);
+    const int64_t pitch = 2 * (int64_t)C, at = 2 * (int64_t)(c0 + 8 * c);
+    float m[8], s1[8], s2[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        m[i] = mean[c0 + 8 * c + i];
+        s1[i] = s2[i] = 0.f;
+    }
+#pragma unroll 4
+    for (int t = r0 + r; t < r1; t += kBnLanes) {
+        float v[8], d[8];
+        unpack<DT>(*reinterpret_cast<const u32x4 *>(x + t * pitch + at), v);
+        unpack<DT>(*reinterpret_cast<const u32x4 *>(dy + t * pitch + at), d);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            s1[i] += d[i];
+            s2[i] = __builtin_fmaf(d[i], v[i] - m[i], s2[i]);
+        }
+    }
+    float a, b;
+    meet(part, quarter, s1, a);
+    meet(part, quarter, s2, b);
+    if (threadIdx.x >= kBnCols) return;
+    part_dy[(int64_t)blockIdx.y * C + c0 + threadIdx.x] = a;
+    part_dyx[(int64_t)blockIdx.y * C + c0 + threadIdx.x] = b;
+}
+struct BnBackward {
+    char *dx;
+    const char *dy, *x, *add;
+    const float *part_dy, *part_dyx, *weight, *mean, *rstd;
+    float *dweight, *dbias;
+    int M, C, rows, chunks;
+};
+template <class DT>
+__global__ void __launch_bounds__(kBnThreads)
+bn_bwd_apply_kernel(BnBackward a) {
+    __shared__ float quarter[4][kBnCols], s_k1[kBnCols], s_k2[kBnCols], s_a[kBnCols];
+    const int c0 = blockIdx.x * kBnCols, ch = threadIdx.x & 63, q = threadIdx.x >> 6;
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll 4
+    for (int k = q; k < a.chunks; k += 4) {
+        s1 += a.part_dy[(int64_t)k * a.C + c0 + ch];
+        s2 += a.part_dyx[(int64_t)k * a.C + c0 + ch];
+    }
+    s1 = across_groups(quarter, s1);
+    s2 = across_groups(quarter, s2);
+    if (threadIdx.x < kBnCols) {
+        const float rstd = a.rstd[c0 + ch];
+        s_a[ch] = a.weight[c0 + ch] * rstd;
+        s_k1[ch] = s1 / (float)a.M;
+        s_k2[ch] = s2 * rstd * rstd / (float)a.M;
+        if (blockIdx.y == 0) {
+            a.dweight[c0 + ch] = s2 * rstd;
+            a.dbias[c0 + ch] = s1;
+        }
+    }
+    __syncthreads();
+    const int c = threadIdx.x & 7, r0 = blockIdx.y * a.rows, r1 = min(a.M, r0 + a.rows);
+    float m[8], k1[8], k2[8], f[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m[i] = a.mean[c0 + 8 * c + i], k1[i] = s_k1[8 * c + i], k2[i] = s_k2[8 * c + i], f[i] = s_a[8 * c + i];
+    const int64_t pitch = 2 * (int64_t)a.C, at = 2 * (int64_t)(c0 + 8 * c);
+#pragma unroll 4
+    for (int t = r0 + (threadIdx.x >> 3); t < r1; t += kBnLanes) {
+        float v[8], d[8], e[8];
+        unpack<DT>(*reinterpret_cast<const u32x4 *>(a.x + t * pitch + at), v);
+        unpack<DT>(*reinterpret_cast<const u32x4 *>(a.dy + t * pitch + at), d);
+        unpack<DT>(*reinterpret_cast<const u32x4 *>(a.add + t * pitch + at), e);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = __builtin_fmaf(f[i], d[i] - k1[i] - (v[i] - m[i]) * k2[i], e[i]);
+        *reinterpret_cast<u32x4 *>(a.dx + t * pitch + at) = repack<DT>(v);
+    }
+}
+
+// =============================================================================
+// Weights of a projection, packed
+// =============================================================================
+// A projection's weight lies in memory as [outputs, inputs / groups] (a linear layer or a grouped 1x1 convolution) and is
+// used as the dense [outputs, inputs] matrix with the groups' blocks on its diagonal.  Row r of a qkv projection of a
+// channels-first model is output channel ((f % per) * groups + f / per) * 3 + which, r = which * C + f, per = C / groups.
+struct Weight {
+    const float *w, *b;           // parameters
+    float *dw, *db;               // and their gradients
+    int outputs, inputs, groups, ordered;
+    __host__ __device__ inline int row(int r) const {
+        if (!ordered) return r;
+        const int C = outputs / 3, per = C / groups, which = r / C, f = r - which * C;
+        return ((f % per) * groups + f / per) * 3 + which;
+    }
+    // place of element (row r, input i) in the parameter, -1 off the diagonal
+    __host__ __device__ inline int64_t at(int r, int i) const {
+        const int o = row(r), in = inputs / groups, i0 = o / (outputs / groups) * in;
+        return i < i0 || i >= i0 + in ? -1 : (int64_t)o * in + (i - i0);
+    }
+};
+struct Pack {
+    Weight w[4];
+    char *plain[4], *turned[4];   // in fragment order: [outputs, inputs] and its transpose
+    float *bias[4];               // in the rows' order
+    int first[5];                 // blocks of 32 x 32 before each
+};
+template <class DT>
+__global__ void __launch_bounds__(256)
+pack_kernel(Pack p) {
+    __shared__ float tile[32][33];
+    int j = 0;
+    while (j < 3 && (int)blockIdx.x >= p.first[j + 1]) ++j;
+    const Weight &w = p.w[j];
+    const int block = (int)blockIdx.x - p.first[j], cols = w.inputs / 32, o0 = block / cols * 32, i0 = block % cols * 32;
+    {
+        const int r = threadIdx.x >> 3, c = (threadIdx.x & 7) * 4;
+        const int64_t at = w.at(o0 + r, i0 + c);           // groups have multiples of 32 inputs: four of a row are in or out together
+        const f32x4 v = at < 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4 *>(w.w + at);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) tile[r][c + k] = v[k];
+        if (i0 == 0 && c == 0) p.bias[j][o0 + r] = w.b[w.row(o0 + r)];
+    }
+    __syncthreads();
+    const int half = threadIdx.x >> 7, t = threadIdx.x & 127, frag = t >> 6, lane = t & 63, n = lane & 15, g = lane >> 4;
+    float v[8];
+    if (half == 0) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = tile[16 * frag + n][8 * g + k];
+        *reinterpret_cast<u32x4 *>(p.plain[j] + ((int64_t)(o0 / 16 + frag) * (w.inputs / 32) + i0 / 32) * kFrag + lane * 16) = repack<DT>(v);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = tile[8 * g + k][16 * frag + n];
+        *reinterpret_cast<u32x4 *>(p.turned[j] + ((int64_t)(i0 / 16 + frag) * (w.outputs / 32) + o0 / 32) * kFrag + lane * 16) = repack<DT>(v);
+    }
+}
+
+// =============================================================================
+// Products over all tokens
+// =============================================================================
+enum GemmEnd {
+    kStore,           // out = v
+    kBias,            // out = v + bias
+    kResidual,        // out = aux + sample_scale * (v + bias)
+    kGelu,            // out2 = v + bias, out = gelu(out2)
+    kGeluBack,        // out = v * gelu'(aux)
+};
+struct Gemm {
+    const char *x, *w;
+    char *out, *out2;
+    const char *aux;
+    const float *bias, *sample_scale;      // one factor per sample of T rows, or NULL
+    int inputs, outputs, M, T;
+    uint32_t T_magic;
+};
+// Phi(x) and x's density, the former by formula 7.1.26 of Abramowitz and Stegun as in gelu(); infinities come out as
+// x * Phi(x) gives them.
+__device__ inline void normal_of(float x, float &cdf, float &pdf) {
+    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_fabsf(x), 0.3275911f * 0.70710678f, 1.f));
+    float e = __builtin_fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
+    e = __builtin_fmaf(t, e, 0.5f * 1.421413741f);
+    e = __builtin_fmaf(t, e, 0.5f * -0.284496736f);
+    e = __builtin_fmaf(t, e, 0.5f * 0.254829592f);
+    const float ex = __builtin_amdgcn_exp2f(x * x * -0.72134752f), tail = t * e * ex;
+    cdf = x < 0.f ? tail : 1.f - tail;
+    pdf = ex * 0.3989422804f;
+}
+template <class DT, int MT, int NTW, GemmEnd END>
+__global__ void __launch_bounds__(kThreads, 2)
+gemm_kernel(Gemm a, int col_blocks) {
+    constexpr int PF = 4, NW = kWaves;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    LDS_PTR(char) lds = (LDS_PTR(char))smem;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
+    const uint32_t item = xcd_item(blockIdx.x, gridDim.x);           // neighbours share their rows' lines
+    const uint32_t row_block = item / (uint32_t)col_blocks;
+    const int64_t m0 = (int64_t)row_block * (16 * MT);
+    const int rows = (int)min((int64_t)(16 * MT), a.M - m0), x_pitch = 2 * a.inputs, pitch = 2 * a.outputs;
+    const int tile0 = ((int)(item - row_block * col_blocks) * NW + wave) * NTW;
+    const Rsrc xs = make_rsrc(a.x + m0 * x_pitch, rows * x_pitch), ws = weight_rsrc(a.w, a.outputs, a.inputs);
+    const int steps = a.inputs / 32, pieces = a.inputs / 256;
+    auto stage = [&](int piece) {
+        constexpr int kChunks = 16 * MT * kRow / kChunk;
+#pragma unroll
+        for (int j = 0; j < kChunks / NW; ++j) {
+            const int c = j * NW + wave, row = 2 * c + (lane >> 5);
+            load_to_lds<16, kReadShared>(xs, lds + (piece & 1) * (16 * MT * kRow) + c * kChunk, row * x_pitch + piece * kRow + ((lane & 31) ^ (row & 15)) * 16);
+        }
+    };
+    stage(0);
+    f32x4 acc[NTW][MT];
+    clear(acc);
+    Ring<NTW, PF> ring;
+    using P = Product<NTW, 8>;
+    const int lane16 = lane * 16;
+    ring.begin(P{ws, tile0 * steps, steps, 0}, lane16);
+#pragma unroll 1
+    for (int p = 0; p < pieces; ++p) {
+        wait_direct();
+        barrier_lds();
+        if (p + 1 < pieces) stage(p + 1);
+        const P now{ws, tile0 * steps + 8 * p, steps, 0}, next{ws, tile0 * steps + 8 * min(p + 1, pieces - 1), steps, 0};
+        multiply<DT, MT>(acc, 0, ring, now, next, lds + (p & 1) * (16 * MT * kRow), n, g, lane16);
+    }
+    const Rsrc os = make_rsrc(a.out + m0 * pitch, rows * pitch);
+    f32x4 bias[NTW];
+    if constexpr (END == kBias || END == kResidual || END == kGelu) {
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) bias[j] = *reinterpret_cast<const f32x4 *>(a.bias + 16 * (tile0 + j) + 4 * g);
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        u32x2 o[NTW];
+        const int row_byte = (16 * i + n) * pitch + 32 * tile0;
+        f32x4 aux[NTW];
+        if constexpr (END == kResidual || END == kGeluBack) {
+            const Rsrc as = make_rsrc(a.aux + m0 * pitch, rows * pitch);
+#pragma unroll
+            for (int j = 0; j < NTW; ++j)
+                aux[j] = widen4<DT>(__builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(as, row_byte + 32 * j + 8 * g, 0, 0)));
+        }
+        float f = 1.f;
+        if constexpr (END == kResidual)
+            if (a.sample_scale) {
+                const uint32_t m = (uint32_t)min(m0 + 16 * i + n, (int64_t)a.M - 1);
+                f = a.sample_scale[div_by(m, a.T, a.T_magic)];
+            }
+        if constexpr (END == kGelu) {
+            u32x2 h[NTW];
+#pragma unroll
+            for (int j = 0; j < NTW; ++j) {
+                h[j] = narrow4<DT>(acc[j][i] + bias[j]);
+                f32x4 v = widen4<DT>(h[j]);                  // of the value that the backward sees
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float cdf, pdf;
+                    normal_of(v[r], cdf, pdf);
+                    v[r] *= cdf;
+                }
+                o[j] = narrow4<DT>(v);
+            }
+            store_tile<16 * NTW, 0>(make_rsrc(a.out2 + m0 * pitch, rows * pitch), row_byte, h, g, 32 * NTW);
+        } else {
+#pragma unroll
+            for (int j = 0; j < NTW; ++j) {
+                f32x4 v = acc[j][i];
+                if constexpr (END == kBias) v += bias[j];
+                if constexpr (END == kResidual) v = aux[j] + f * (v + bias[j]);
+                if constexpr (END == kGeluBack) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        float cdf, pdf;
+                        normal_of(aux[j][r], cdf, pdf);
+                        v[r] *= __builtin_fmaf(aux[j][r], pdf, cdf);
+                    }
+                }
+                o[j] = narrow4<DT>(v);
+            }
+        }
+        store_tile<16 * NTW, 0>(os, row_byte, o, g, 32 * NTW);
+    }
+}
+
+// out[m, :] = x[m, :] * sample_scale[m / T]
+template <class DT>
+__global__ void __launch_bounds__(256)
+scale_kernel(char *__restrict__ out, const char *__restrict__ x, const float *__restrict__ sample_scale, int64_t units, int units_per_sample) {
+    for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < units; u += (int64_t)gridDim.x * 256) {
+        float v[8];
+        unpack<DT>(*reinterpret_cast<const u32x4 *>(x + u * 16), v);
+        const float f = sample_scale[u / units_per_sample];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] *= f;
+        *reinterpret_cast<u32x4 *>(out + u * 16) = repack<DT>(v);
+    }
+}
+
+// =============================================================================
+// Weight gradients of the layer's four projections in one launch
+// =============================================================================
+// dW[o, i] = sum over rows of dY[m, o] X[m, i], db[o] = sum of dY[m, o].  The contraction runs along the rows of both
+// operands, so both come out of LDS transposed (ds_read_b64_tr_b16).  A workgroup computes a 128 x 128 block of one dW
+// (each wave 64 x 64) over one of `splits` ranges of rows, 64 rows at a time, double buffered; the ranges' sums (fp32) are
+// folded in a fixed order by a second kernel, which also undoes the row order and drops what is off the diagonal.
+// 12800 tokens, 256 channels, 1024 hidden (20 GFLOP): 32 us, 620 TFLOP/s, and 7 us to fold ten ranges; as four library
+// products of chunks with four sums over the chunks and four bias sums it was 200 us.
+constexpr int kGradTile = 128, kGradRows = 64;
+struct GradJob {
+    const char *dy, *x;
+    int outputs, inputs, first;          // first: blocks of 128 x 128 before
+    int64_t part;                        // floats before: dW, then db
+};
+struct Grads {
+    GradJob job[4];
+    float *partial;
+    int64_t stride;                      // floats of one range
+    int M, rows, blocks;                 // rows of a range (a multiple of 64)
+};
+template <class DT>
+__global__ void __launch_bounds__(kThreads, 2)
+grad_kernel(Grads a) {
+    using L = Lds<kGradTile>;
+    constexpr int kPart = kGradRows * L::kRowBytes;            // 16 KB of dY, then of X
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    LDS_PTR(char) lds = (LDS_PTR(char))smem;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
+    const uint32_t item = xcd_item(blockIdx.x, gridDim.x);     // the blocks of a range read the same rows
+    const int split = (int)(item / (uint32_t)a.blocks), block = (int)item - split * a.blocks;
+    int jn = 0;
+    while (jn < 3 && block >= a.job[jn + 1].first) ++jn;
+    const GradJob &job = a.job[jn];
+    const int cols = job.inputs / kGradTile, o0 = (block - job.first) / cols * kGradTile, i0 = (block - job.first) % cols * kGradTile;
+    const int64_t m0 = (int64_t)split * a.rows;
+    const int rows = (int)min((int64_t)a.rows, a.M - m0), pieces = (rows + kGradRows - 1) / kGradRows;
+    const int y_pitch = 2 * job.outputs, x_pitch = 2 * job.inputs;
+    const Rsrc ys = make_rsrc(job.dy + m0 * y_pitch, rows * y_pitch), xs = make_rsrc(job.x + m0 * x_pitch, rows * x_pitch);
+    const int wo = wave & 1, wi = wave >> 1;
+    auto stage = [&](int piece) {
+        LDS_PTR(char) to = lds + (piece & 1) * (2 * kPart);
+#pragma unroll
+        for (int j = 0; j < kPart / kChunk / kWaves; ++j) {
+            const int c = j * kWaves + wave, r = 4 * c + (lane >> 4), unit = ((lane & 15) ^ (r & 15)) * 16, row = piece * kGradRows + r;
+            load_to_lds<16, kReadShared>(ys, to + c * kChunk, row * y_pitch + 2 * o0 + unit);
+            load_to_lds<16, kReadShared>(xs, to + kPart + c * kChunk, row * x_pitch + 2 * i0 + unit);
+        }
+    };
+    // byte of this lane's piece of channel tile t, rows 0 .. 15; tiles of 16 rows follow each other
+    int yo[4], xo[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        yo[t] = L::addr(4 * g + (n >> 2), 128 * wo + 32 * t + 8 * (n & 3));
+        xo[t] = kPart + L::addr(4 * g + (n >> 2), 128 * wi + 32 * t + 8 * (n & 3));
+    }
+    const bool sums = i0 == 0 && wi == 0;
+    const uint32_t one = Mma<DT>::pack(1.f, 1.f);
+    const u32x4 ones = {one, one, one, one};
+    f32x4 acc[4][4], db[4];                                    // [o tile][i tile]
+    clear(acc);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) db[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    stage(0);
+#pragma unroll 1
+    for (int p = 0; p < pieces; ++p) {
+        wait_direct();
+        barrier_lds();
+        if (p + 1 < pieces) stage(p + 1);
+        LDS_PTR(char) from = lds + (p & 1) * (2 * kPart);
+#pragma unroll
+        for (int s = 0; s < kGradRows / 32; ++s) {
+            u32x4 y[4], x[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const u32x2 y0 = read_tr(from + 2 * s * L::kTileBytes + yo[t]), y1 = read_tr(from + (2 * s + 1) * L::kTileBytes + yo[t]);
+                const u32x2 x0 = read_tr(from + 2 * s * L::kTileBytes + xo[t]), x1 = read_tr(from + (2 * s + 1) * L::kTileBytes + xo[t]);
+                y[t] = u32x4{y0.x, y0.y, y1.x, y1.y};
+                x[t] = u32x4{x0.x, x0.y, x1.x, x1.y};
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) acc[t][u] = Mma<DT>::k32(x[u], y[t], acc[t][u]);
+            if (sums)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) db[t] = Mma<DT>::k32(ones, y[t], db[t]);
+        }
+    }
+    float *part = a.partial + (int64_t)split * a.stride + job.part;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const int o = o0 + 64 * wo + 16 * t + n;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) *reinterpret_cast<f32x4 *>(part + (int64_t)o * job.inputs + i0 + 64 * wi + 16 * u + 4 * g) = acc[t][u];
+        if (sums && g == 0) part[(int64_t)job.outputs * job.inputs + o] = db[t][0];
+    }
+}
+struct Fold {
+    Weight w[4];
+    int64_t part[5];                     // floats before each projection's dW
+    const float *partial;
+    int64_t stride;
+    int splits;
+};
+__global__ void __launch_bounds__(256)
+grad_fold_kernel(Fold a) {
+    const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (e >= a.part[4]) return;
+    int j = 0;
+    while (j < 3 && e >= a.part[j + 1]) ++j;
+    const Weight &w = a.w[j];
+    const int64_t k = e - a.part[j], nw = (int64_t)w.outputs * w.inputs;
+    const int r = (int)(k / w.inputs), i = (int)(k - (int64_t)r * w.inputs);
+    const int64_t at = k < nw ? w.at(r, i) : 0;
+    if (at < 0) return;
+    f32x4 s = *reinterpret_cast<const f32x4 *>(a.partial + e);
+#pragma unroll 4
+    for (int p = 1; p < a.splits; ++p) s += *reinterpret_cast<const f32x4 *>(a.partial + p * a.stride + e);
+    if (k < nw) {
+        *reinterpret_cast<f32x4 *>(w.dw + at) = s;
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w.db[w.row((int)(k - nw) + q)] = s[q];
+    }
+}
+
+// ----------------------------------------------------------------------------- the layer
+inline Weight weight_of(const na1d_train_layer &l, int j) {
+    const int C = l.dim, outputs[4] = {3 * C, C, l.hidden, C}, inputs[4] = {C, C, C, l.hidden};
+    return Weight{l.w[j], l.b[j], l.dw[j], l.db[j], outputs[j], inputs[j], l.groups, j == 0 && l.ordered};
+}
+struct Buffers {
+    int64_t bytes = 0;
+    int64_t take(int64_t n) {
+        const int64_t at = bytes;
+        bytes += (n + 255) / 256 * 256;
+        return at;
+    }
+};
+// What the forward leaves for the backward.
+struct Saved : Buffers {
+    int64_t y1, qkv, lse, attn, x1, y2, h, g, stats[4], turned[4];
+    Saved(const na1d_train_layer &l, int64_t N, int64_t T) {
+        const int64_t M = N * T, row = M * l.dim * 2;
+        y1 = take(row), qkv = take(3 * row), lse = take(M * l.heads * 4), attn = take(row), x1 = take(row), y2 = take(row);
+        h = take(M * l.hidden * 2), g = take(M * l.hidden * 2);
+        for (int64_t &s : stats) s = take(l.dim * 4);
+        for (int j = 0; j < 4; ++j) {
+            const Weight w = weight_of(l, j);
+            turned[j] = take((int64_t)w.outputs * w.inputs * 2);
+        }
+    }
+};
+struct ForwardScratch : Buffers {
+    int64_t part, plain[4], bias[4];
+    explicit ForwardScratch(const na1d_train_layer &l) {
+        part = take((int64_t)2 * kBnChunks * l.dim * 4);
+        for (int j = 0; j < 4; ++j) {
+            const Weight w = weight_of(l, j);
+            plain[j] = take((int64_t)w.outputs * w.inputs * 2);
+            bias[j] = take(w.outputs * 4);
+        }
+    }
+};
+struct GradPlan {
+    int blocks = 0, splits, rows, first[4];
+    int64_t part[5] = {};
+    GradPlan(const na1d_train_layer &l, int64_t M) {
+        for (int j = 0; j < 4; ++j) {
+            const Weight w = weight_of(l, j);
+            first[j] = blocks;
+            blocks += (w.outputs / kGradTile) * (w.inputs / kGradTile);
+            part[j + 1] = part[j] + (int64_t)w.outputs * w.inputs + w.outputs;
+        }
+        // two workgroups on each CU; a range is worth a few pieces, and stays in the reach of 31-bit offsets
+        int64_t want = std::max<int64_t>(1, std::min<int64_t>(512 / blocks, (M + 255) / 256));
+        want = std::max(want, M * 2 * std::max(3 * l.dim, l.hidden) / (1 << 29) + 1);
+        rows = (int)(((M + want - 1) / want + kGradRows - 1) / kGradRows * kGradRows);
+        splits = (int)((M + rows - 1) / rows);
+    }
+};
+struct BackwardScratch : Buffers {
+    int64_t dz, dh, dy, dx1, ds, dattn, dqkv, part, grads;
+    BackwardScratch(const na1d_train_layer &l, int64_t N, int64_t T) {
+        const int64_t M = N * T, row = M * l.dim * 2;
+        const GradPlan p(l, M);
+        dz = take(l.scale_mlp ? row : 0), dh = take(M * l.hidden * 2), dy = take(row), dx1 = take(row), ds = take(l.scale_attn ? row : 0);
+        dattn = take(row), dqkv = take(3 * row), part = take((int64_t)2 * kBnChunks * l.dim * 4);
+        grads = take(p.splits * p.part[4] * 4);
+    }
+};
+
+#define NA1D_TRY(...)                       \
+    do {                                    \
+        const int st_ = (__VA_ARGS__);      \
+        if (st_ != NA1D_OK) return st_;     \
+    } while (0)
+
+// 64 rows x 256 outputs where that fills the chip (two workgroups on each CU); smaller blocks otherwise.
+template <class DT, GemmEnd END> int launch_gemm(const Gemm &a, hipStream_t s) {
+    auto go = [&](auto kern, int mt, int ntw) {
+        const size_t lds = (size_t)(a.inputs > 256 ? 2 : 1) * 16 * mt * kRow;
+        if (!allow_lds(kern, lds)) return (int)NA1D_ERR_LAUNCH;
+        const int cols = a.outputs / (64 * ntw);
+        kern<<<(unsigned)((a.M + 16 * mt - 1) / (16 * mt) * cols), kThreads, lds, s>>>(a, cols);
+        return launch_status();
+    };
+    const int64_t wide = ((int64_t)a.M + 63) / 64 * (a.outputs / 256);
+    if (wide >= 512) return go(gemm_kernel<DT, 4, 4, END>, 4, 4);
+    if (wide >= 128) return go(gemm_kernel<DT, 4, 2, END>, 4, 2);
+    return go(gemm_kernel<DT, 2, 2, END>, 2, 2);
+}
+template <class DT> int scale_rows(char *out, const char *x, const float *f, int64_t N, int64_t T, int dim, hipStream_t s) {
+    const int64_t units = N * T * dim / 8;
+    scale_kernel<DT><<<(unsigned)std::min<int64_t>((units + 255) / 256, 4096), 256, 0, s>>>(out, x, f, units, (int)(T * dim / 8));
+    return launch_status();
+}
+inline Geom attention_geom(const na1d_train_layer &l, int64_t N, int64_t T, Layout &in, Layout &out) {
+    Geom g;
+    const int64_t C = l.dim;
+    g.B = N * l.heads, g.T = T, g.H = l.heads, g.C = l.dim / l.heads, g.W = l.window, g.L = l.left;
+    in = Layout{T * 3 * C, g.C, 3 * C}, out = Layout{T * C, g.C, C};
+    set_dilation(g, l.dilation);
+    in.row *= g.dilation, out.row *= g.dilation;
+    return g;
+}
+
+template <class DT> int norm_forward(const na1d_train_layer &l, int which, char *y, const char *x, float *mean, float *rstd, float *part, int64_t M, hipStream_t s) {
+    const Chunks c = bn_chunks(M);
+    const dim3 grid((unsigned)(l.dim / kBnCols), (unsigned)c.count);
+    float *part_m2 = part + (int64_t)kBnChunks * l.dim;
+    bn_stats_kernel<DT><<<grid, kBnThreads, 0, s>>>(part, part_m2, x, (int)M, l.dim, c.rows);
+    NA1D_TRY(launch_status());
+    const na1d_train_norm &n = l.norm[which];
+    bn_apply_kernel<DT><<<grid, kBnThreads, 0, s>>>(BnApply{y, x, part, part_m2, n.weight, n.bias, mean, rstd, n.running_mean, n.running_var, n.batches,
+                                                            n.eps, n.momentum, (int)M, l.dim, c.rows, c.count});
+    return launch_status();
+}
+template <class DT>
+int norm_backward(const na1d_train_layer &l, int which, char *dx, const char *dy, const char *x, const char *add, const float *mean, const float *rstd, float *part,
+                  int64_t M, hipStream_t s) {
+    const Chunks c = bn_chunks(M);
+    const dim3 grid((unsigned)(l.dim / kBnCols), (unsigned)c.count);
+    float *part_dyx = part + (int64_t)kBnChunks * l.dim;
+    bn_bwd_sums_kernel<DT><<<grid, kBnThreads, 0, s>>>(part, part_dyx, dy, x, mean, (int)M, l.dim, c.rows);
+    NA1D_TRY(launch_status());
+    const na1d_train_norm &n = l.norm[which];
+    bn_bwd_apply_kernel<DT><<<grid, kBnThreads, 0, s>>>(BnBackward{dx, dy, x, add, part, part_dyx, n.weight, mean, rstd, n.dweight, n.dbias, (int)M, l.dim, c.rows, c.count});
+    return launch_status();
+}
+
+template <class DT> int forward(const na1d_train_layer &l, char *out, const char *x, char *saved, char *ws, int64_t N, int64_t T, hipStream_t s) {
+    const int64_t M = N * T;
+    const Saved o(l, N, T);
+    const ForwardScratch f(l);
+    auto stat = [&](int i) { return reinterpret_cast<float *>(saved + o.stats[i]); };
+    Pack p{};
+    for (int j = 0; j < 4; ++j) {
+        p.w[j] = weight_of(l, j);
+        p.plain[j] = ws + f.plain[j], p.turned[j] = saved + o.turned[j], p.bias[j] = reinterpret_cast<float *>(ws + f.bias[j]);
+        p.first[j + 1] = p.first[j] + p.w[j].outputs / 32 * (p.w[j].inputs / 32);
+    }
+    pack_kernel<DT><<<(unsigned)p.first[4], 256, 0, s>>>(p);
+    NA1D_TRY(launch_status());
+    float *part = reinterpret_cast<float *>(ws + f.part);
+    Gemm a{};
+    a.M = (int)M, a.T = (int)T, a.T_magic = div_magic(T);
+    auto product = [&](int j, const char *in, char *to) {
+        a.x = in, a.w = p.plain[j], a.bias = p.bias[j], a.out = to, a.inputs = p.w[j].inputs, a.outputs = p.w[j].outputs;
+    };
+    NA1D_TRY(norm_forward<DT>(l, 0, saved + o.y1, x, stat(0), stat(1), part, M, s));
+    product(0, saved + o.y1, saved + o.qkv);
+    NA1D_TRY(launch_gemm<DT, kBias>(a, s));
+    Layout in, outl;
+    const Geom g = attention_geom(l, N, T, in, outl);
+    const char *q = saved + o.qkv, *k = q + 2 * l.dim, *v = k + 2 * l.dim;
+    float *lse = reinterpret_cast<float *>(saved + o.lse);
+    int st = fused_fwd(saved + o.attn, lse, q, k, v, l.rpb, nullptr, g, in, outl, l.scale, DT::tag, s);
+    if (st == NA1D_ERR_UNSUPPORTED) st = wide_fwd(saved + o.attn, lse, q, k, v, l.rpb, nullptr, g, in, outl, l.scale, DT::tag, s);
+    NA1D_TRY(st);
+    product(1, saved + o.attn, saved + o.x1);
+    a.aux = x, a.sample_scale = l.scale_attn;
+    NA1D_TRY(launch_gemm<DT, kResidual>(a, s));
+    NA1D_TRY(norm_forward<DT>(l, 1, saved + o.y2, saved + o.x1, stat(2), stat(3), part, M, s));
+    product(2, saved + o.y2, saved + o.g);
+    a.out2 = saved + o.h;
+    NA1D_TRY(launch_gemm<DT, kGelu>(a, s));
+    product(3, saved + o.g, out);
+    a.aux = saved + o.x1, a.sample_scale = l.scale_mlp;
+    return launch_gemm<DT, kResidual>(a, s);
+}
+
+template <class DT>
+int backward(const na1d_train_layer &l, char *dx, const char *dout, const char *x, const char *saved, char *ws, int64_t N, int64_t T, hipStream_t s) {
+    const int64_t M = N * T;
+    const Saved o(l, N, T);
+    const BackwardScratch b(l, N, T);
+    auto stat = [&](int i) { return reinterpret_cast<const float *>(saved + o.stats[i]); };
+    float *part = reinterpret_cast<float *>(ws + b.part);
+    Gemm a{};
+    a.M = (int)M, a.T = (int)T, a.T_magic = div_magic(T);
+    auto turned = [&](int j, const char *dy, char *to) {
+        const Weight w = weight_of(l, j);
+        a.x = dy, a.w = saved + o.turned[j], a.out = to, a.inputs = w.outputs, a.outputs = w.inputs;
+    };
+    const char *dz = dout;
+    if (l.scale_mlp) {
+        NA1D_TRY(scale_rows<DT>(ws + b.dz, dout, l.scale_mlp, N, T, l.dim, s));
+        dz = ws + b.dz;
+    }
+    turned(3, dz, ws + b.dh);
+    a.aux = saved + o.h;
+    NA1D_TRY(launch_gemm<DT, kGeluBack>(a, s));
+    turned(2, ws + b.dh, ws + b.dy);
+    NA1D_TRY(launch_gemm<DT, kStore>(a, s));
+    NA1D_TRY(norm_backward<DT>(l, 1, ws + b.dx1, ws + b.dy, saved + o.x1, dout, stat(2), stat(3), part, M, s));
+    const char *ds = ws + b.dx1;
+    if (l.scale_attn) {
+        NA1D_TRY(scale_rows<DT>(ws + b.ds, ds, l.scale_attn, N, T, l.dim, s));
+        ds = ws + b.ds;
+    }
+    turned(1, ds, ws + b.dattn);
+    NA1D_TRY(launch_gemm<DT, kStore>(a, s));
+    Layout in, outl;
+    const Geom g = attention_geom(l, N, T, in, outl);
+    const int64_t step = 2 * l.dim;
+    const char *q = saved + o.qkv;
+    char *dq = ws + b.dqkv;
+    const float *lse = reinterpret_cast<const float *>(saved + o.lse);
+    int st = fused_bwd(dq, dq + step, dq + 2 * step, l.drpb, q, q + step, q + 2 * step, nullptr, ws + b.dattn, lse, l.rpb, nullptr, g, in, outl, l.scale, DT::tag,
+                       nullptr, 0, s);
+    if (st == NA1D_ERR_UNSUPPORTED)
+        st = wide_bwd(dq, dq + step, dq + 2 * step, l.drpb, q, q + step, q + 2 * step, ws + b.dattn, lse, l.rpb, nullptr, g, in, outl, l.scale, DT::tag, nullptr, 0, s);
+    NA1D_TRY(st);
+    turned(0, ws + b.dqkv, ws + b.dy);
+    NA1D_TRY(launch_gemm<DT, kStore>(a, s));
+    NA1D_TRY(norm_backward<DT>(l, 0, dx, ws + b.dy, x, ws + b.dx1, stat(0), stat(1), part, M, s));
+    const GradPlan plan(l, M);
+    Grads ga{};
+    Fold fo{};
+    const char *dys[4] = {ws + b.dqkv, ds, ws + b.dh, dz}, *xs[4] = {saved + o.y1, saved + o.attn, saved + o.y2, saved + o.g};
+    for (int j = 0; j < 4; ++j) {
+        fo.w[j] = weight_of(l, j);
+        ga.job[j] = GradJob{dys[j], xs[j], fo.w[j].outputs, fo.w[j].inputs, plan.first[j], plan.part[j]};
+        fo.part[j + 1] = plan.part[j + 1];
+    }
+    ga.partial = reinterpret_cast<float *>(ws + b.grads);
+    ga.stride = fo.stride = plan.part[4];
+    ga.M = (int)M, ga.rows = plan.rows, ga.blocks = plan.blocks;
+    fo.partial = ga.partial, fo.splits = plan.splits;
+    const size_t lds = (size_t)4 * kGradRows * kGradTile * 2;
+    if (!allow_lds(grad_kernel<DT>, lds)) return NA1D_ERR_LAUNCH;
+    grad_kernel<DT><<<(unsigned)(plan.blocks * plan.splits), kThreads, lds, s>>>(ga);
+    NA1D_TRY(launch_status());
+    grad_fold_kernel<<<(unsigned)((plan.part[4] / 4 + 255) / 256), 256, 0, s>>>(fo);
+    return launch_status();
+}
+
+bool layer_ok(const na1d_train_layer &l, int64_t N, int64_t T) {
+    if (l.dim < 256 || l.dim % 256 || l.dim > 2048 || l.hidden < 256 || l.hidden % 256 || l.hidden > 8192) return false;
+    if (l.heads < 1 || l.dim % l.heads || l.dim / l.heads % 8 || l.dim / l.heads > 128) return false;
+    if (l.groups < 1 || l.dim % l.groups || l.dim / l.groups % 32 || l.hidden % l.groups || l.hidden / l.groups % 32) return false;
+    if (l.window < 1 || l.window > NA1D_MAX_WINDOW || l.left < 0 || l.left >= l.window || l.dilation < 1) return false;
+    // offsets inside an utterance, and what the attention kernels' launches count, stay in the reach of 32 bits
+    if (N < 1 || T < 1 || N > (1 << 20) || T > (1 << 16) || N * T > (1 << 20)) return false;
+    const int64_t M = N * T, most = 1ll << 31;
+    if (T * 3 * l.dim > (1 << 29) || M * T >= most || l.dilation > 64) return false;
+    if (l.heads * M * l.heads >= most || l.heads * M * (T / 32 + 1) >= most || l.heads * M * l.dilation >= most) return false;
+    return N * T >= 2;          // variance of one row
+}
+int64_t saved_bytes(const na1d_train_layer &l, int64_t N, int64_t T) { return Saved(l, N, T).bytes; }
+int64_t scratch_bytes(const na1d_train_layer &l, int64_t N, int64_t T, bool backward) {
+    return backward ? BackwardScratch(l, N, T).bytes : ForwardScratch(l).bytes;
+}
+int run_forward(const na1d_train_layer &l, void *out, const void *x, void *saved, void *ws, int64_t N, int64_t T, hipStream_t s) {
+    return l.dtype == NA1D_BF16 ? forward<BF16>(l, (char *)out, (const char *)x, (char *)saved, (char *)ws, N, T, s)
+                                : forward<FP16>(l, (char *)out, (const char *)x, (char *)saved, (char *)ws, N, T, s);
+}
+int run_backward(const na1d_train_layer &l, void *dx, const void *dout, const void *x, const void *saved, void *ws, int64_t N, int64_t T, hipStream_t s) {
+    return l.dtype == NA1D_BF16 ? backward<BF16>(l, (char *)dx, (const char *)dout, (const char *)x, (const char *)saved, (char *)ws, N, T, s)
+                                : backward<FP16>(l, (char *)dx, (const char *)dout, (const char *)x, (const char *)saved, (char *)ws, N, T, s);
+}
+
+}  // namespace train
+}  // namespace na1d

@@ -34,6 +34,7 @@ from .dense import global_attention
 from .encoder import embed as embed_natively
 from .fused import na1d_fused, na1d_fused_qkv
 from .nattn import getNA1dFunction
+from .train import layer as train_layer
 
 MASK_VALUE = -100.0   # PCF_NATransformer.py:98
 
@@ -534,6 +535,10 @@ class NATFLayer(nn.Module):
         self.norm2 = norm(dim)
 
     def forward(self, x, padding=None, pos_emb=None, attn_mask_global=None):
+        if self.training:
+            out = train_layer(self, x)                  # one autograd node, native both ways
+            if out is not None:
+                return out
         y = self.norm1(x)
         if self.local:
             y = self.attn(y, padding=padding)

@@ -1,0 +1,158 @@
+"""A windowed encoder layer in training as one autograd node (``na1d_train_layer_*`` of the C ABI).
+
+:func:`layer` runs norm -> attention -> residual -> norm -> MLP -> residual of ``models.NATFLayer`` and its backward
+through the kernels of ``csrc/na1d_train.hip``, all launched from native code: the parameters, buffers, random draws and
+results are those of the modules, which stay what runs wherever something here does not fit.
+"""
+from __future__ import annotations
+
+import ctypes
+
+import torch
+import torch.nn as nn
+from torch.autograd.function import once_differentiable
+from torch.autograd.graph import increment_version
+
+from . import _lib
+
+_P, _I, _F = ctypes.c_void_p, ctypes.c_int32, ctypes.c_float
+
+
+class _Norm(ctypes.Structure):                     # na1d_train_norm
+    _fields_ = [(n, _P) for n in "weight bias running_mean running_var batches dweight dbias".split()] + [("eps", _F), ("momentum", _F)]
+
+
+class _Layer(ctypes.Structure):                    # na1d_train_layer
+    _fields_ = ([(n, _I) for n in "dtype dim hidden heads window left dilation groups ordered".split()] + [("scale", _F)]
+                + [("norm", _Norm * 2)] + [(n, _P * 4) for n in "w b dw db".split()]
+                + [(n, _P) for n in "rpb drpb scale_attn scale_mlp".split()])
+
+
+def _ptr(t):
+    return None if t is None else t.data_ptr()
+
+
+def _ptrs(ts):
+    return (_P * 4)(*(t.data_ptr() for t in ts))
+
+
+class _TrainLayer(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, geom, norms, scales, rpb, n1w, n1b, n2w, n2b, wq, bq, wp, bp, w1, b1, w2, b2):
+        lib = _lib.load()
+        n, t, dim = x.shape
+        weights, biases = (wq, wp, w1, w2), (bq, bp, b1, b2)
+        c = _Layer(*geom)
+        c.w, c.b = _ptrs(weights), _ptrs(biases)
+        for to, bn, w, b in zip(c.norm, norms, (n1w, n2w), (n1b, n2b)):
+            to.weight, to.bias, to.eps, to.momentum = w.data_ptr(), b.data_ptr(), bn.eps, bn.momentum
+            to.running_mean, to.running_var, to.batches = bn.running_mean.data_ptr(), bn.running_var.data_ptr(), bn.num_batches_tracked.data_ptr()
+        c.rpb, c.scale_attn, c.scale_mlp = rpb.data_ptr(), _ptr(scales[0]), _ptr(scales[1])
+        ref = ctypes.byref(c)
+        out = torch.empty_like(x)
+        with torch.cuda.device(x.device):
+            sizes = lib.na1d_train_layer_saved_bytes(ref, n, t), lib.na1d_train_layer_workspace_bytes(ref, n, t, 0)
+            _lib.check(min(*sizes, 0), "na1d_train_layer_saved_bytes")
+            saved, ws = (torch.empty(s, dtype=torch.uint8, device=x.device) for s in sizes)
+            _lib.check(lib.na1d_train_layer_forward(ref, out.data_ptr(), x.data_ptr(), saved.data_ptr(), sizes[0], ws.data_ptr(),
+                                                    sizes[1], n, t, torch.cuda.current_stream().cuda_stream),
+                       "na1d_train_layer_forward")
+        increment_version([b for bn in norms for b in (bn.running_mean, bn.running_var, bn.num_batches_tracked)])
+        ctx.save_for_backward(x, saved, rpb, n1w, n2w, *scales)
+        ctx.geom, ctx.shapes = geom, [p.shape for p in (rpb, n1w, n1b, n2w, n2b, wq, bq, wp, bp, w1, b1, w2, b2)]
+        return out
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dout):
+        lib = _lib.load()
+        x, saved, rpb, n1w, n2w, *scales = ctx.saved_tensors
+        n, t, dim = x.shape
+        dout = dout.contiguous()
+        dx = torch.empty_like(x)
+        grads = [torch.zeros(ctx.shapes[0], dtype=torch.float32, device=x.device)]       # the bias of the scores is added to
+        grads += [torch.empty(s, dtype=torch.float32, device=x.device) for s in ctx.shapes[1:]]
+        c = _Layer(*ctx.geom)
+        c.dw, c.db = _ptrs(grads[5::2]), _ptrs(grads[6::2])
+        for to, w, dw, db in zip(c.norm, (n1w, n2w), grads[1:5:2], grads[2:5:2]):
+            to.weight, to.dweight, to.dbias = w.data_ptr(), dw.data_ptr(), db.data_ptr()
+        c.rpb, c.drpb, c.scale_attn, c.scale_mlp = rpb.data_ptr(), grads[0].data_ptr(), _ptr(scales[0]), _ptr(scales[1])
+        ref = ctypes.byref(c)
+        with torch.cuda.device(x.device):
+            nbytes = lib.na1d_train_layer_workspace_bytes(ref, n, t, 1)
+            _lib.check(min(nbytes, 0), "na1d_train_layer_workspace_bytes")
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+            _lib.check(lib.na1d_train_layer_backward(ref, dx.data_ptr(), dout.data_ptr(), x.data_ptr(), saved.data_ptr(), saved.numel(),
+                                                     ws.data_ptr(), nbytes, n, t, torch.cuda.current_stream().cuda_stream),
+                       "na1d_train_layer_backward")
+        return (dx, None, None, None, *(g if need else None for g, need in zip(grads, ctx.needs_input_grad[4:])))
+
+
+def plain(m, *classes):
+    """Whether calling module ``m`` runs the forward of its class and nothing else."""
+    return (type(m) in classes and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+            and "forward" not in m.__dict__)
+
+
+def plain_call(x):
+    """Whether nothing but autograd looks at the operations on ``x``: no tracer, transform, subclass or dispatch mode."""
+    return (type(x) in (torch.Tensor, nn.Parameter) and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and not torch.nn.modules.module._has_any_global_hook() and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0)
+
+
+def _norm_fits(bn, dim):
+    return (bn.training and bn.track_running_stats and bn.affine and bn.momentum is not None and bn.num_features == dim
+            and bn.num_batches_tracked is not None)
+
+
+def _drop_path_scale(m, x):
+    """Stochastic depth's factor of each sample, drawn as ``models.DropPath`` draws it."""
+    if not getattr(m, "drop_prob", 0.0) or not m.training:
+        return None
+    keep = 1 - m.drop_prob
+    mask = (keep + torch.rand((x.shape[0], 1, 1), dtype=x.dtype, device=x.device)).floor_()
+    return mask.float().view(-1).div_(keep)
+
+
+def layer(m, x):
+    """``models.NATFLayer`` ``m`` in training on ``x`` ([N, T, C], or [N, C, T] for channels-first models), or ``None`` where
+    the kernels or their one autograd node would not be the same as the modules."""
+    from . import models as M
+    if not (x.is_cuda and m.training and m.local and torch.is_grad_enabled() and torch.is_autocast_enabled("cuda")
+            and x.dim() == 3 and x.dtype in (torch.bfloat16, torch.float16) and x.dtype == torch.get_autocast_dtype("cuda")):
+        return None
+    a, mlp = m.attn, m.mlp
+    cf = getattr(a, "channels_first", False)
+    linear, norm = (M.Conv1x1, M.BatchNorm1d) if cf else (M.TokenLinear, M.TokenBatchNorm)
+    if not (plain_call(x) and plain(a, M.NAttention) and plain(mlp, M.Mlp) and plain(m.norm1, norm) and plain(m.norm2, norm)
+            and plain(m.drop_path, nn.Identity, M.DropPath) and plain(mlp.act, nn.GELU) and mlp.act.approximate == "none"
+            and plain(mlp.drop, nn.Dropout) and plain(a.proj_drop, nn.Dropout)
+            and all(plain(p, linear) for p in (a.qkv, a.proj, mlp.fc1, mlp.fc2))):
+        return None
+    norms = (m.norm1, m.norm2) if cf else (m.norm1.norm, m.norm2.norm)
+    if a.na != "fused_qkv" or a.attn_drop or not a.training or a.proj_drop.p or mlp.drop.p or (not cf and not all(plain(b, M.BatchNorm1d) for b in norms)):
+        return None
+    xt = x.transpose(1, 2) if cf else x
+    n, t, dim = xt.shape
+    if dim != a.dim or t != a.attn_mask.shape[-2] or not all(_norm_fits(b, dim) for b in norms):
+        return None
+    groups = {getattr(p, "groups", 1) for p in (a.qkv, a.proj, mlp.fc1, mlp.fc2)}
+    params = (a.relative_position_bias, norms[0].weight, norms[0].bias, norms[1].weight, norms[1].bias, a.qkv.weight, a.qkv.bias,
+              a.proj.weight, a.proj.bias, mlp.fc1.weight, mlp.fc1.bias, mlp.fc2.weight, mlp.fc2.bias)
+    hidden = mlp.fc1.weight.shape[0]
+    sizes = (3 * dim, dim, dim, dim, hidden, dim, dim, hidden)
+    if len(groups) != 1 or any(p is None or type(p) is not nn.Parameter or p.dtype != torch.float32 or p.device != x.device
+                               or not p.is_contiguous() or p.data_ptr() % 16 for p in params):
+        return None
+    groups = groups.pop()
+    if any(p.numel() != o * i // groups for p, o, i in zip(params[5::2], sizes[::2], sizes[1::2])):
+        return None
+    geom = (_lib.dtype_tag(x.dtype), dim, hidden, a.num_heads, a.win_size, a.left, a.dilation, groups, int(cf), a.scale)
+    probe = _Layer(*geom)
+    if _lib.load().na1d_train_layer_saved_bytes(ctypes.byref(probe), n, t) < 0:
+        return None
+    xt = xt.contiguous()
+    scales = (_drop_path_scale(m.drop_path, xt), _drop_path_scale(m.drop_path, xt))
+    out = _TrainLayer.apply(xt, geom, norms, scales, *params)
+    return out.transpose(1, 2) if cf else out

@@ -1,0 +1,138 @@
+"""A windowed encoder layer in training as one native node (na1d_train_layer_*) against the fp32 module on the CPU."""
+import copy
+
+import pytest
+import torch
+
+from na1d_amd import models
+from oracle import na1d_oracle as O
+
+pytestmark = pytest.mark.gpu
+DT = {"bf16": torch.bfloat16, "fp16": torch.float16}
+
+
+def _cpu_attention(q, k, v, W, left, rpb=None, t_valid=None, num_heads=1, dilation=1):
+    """The operator in plain torch, differentiable: the keys of every window slot gathered by row."""
+    B, T, C = q.shape
+    t, j = torch.arange(T).unsqueeze(1), torch.arange(W)
+    key = t + (j - left) * dilation
+    inside = (key >= 0) & (key < T)
+    kk, vv = (z[:, key.clamp(0, T - 1)] for z in (k, v))                          # [B, T, W, C]
+    s = (q.unsqueeze(2) * kk).sum(-1) * inside
+    s = (s.view(-1, num_heads, T, W) + rpb.view(1, num_heads, 1, W)).view(B, T, W) + (~inside) * models.MASK_VALUE
+    p = torch.softmax(s, -1) * inside
+    return (p.unsqueeze(-1) * vv).sum(2)
+
+
+def _layers(family, groups, heads, window, dilation, frames, drop_path, seed, dim=256):
+    torch.manual_seed(seed)
+    layer = models.NATFLayer(frames, dim, heads, window, groups, drop_path, family == "pcf", torch.bfloat16, _cpu_attention,
+                             dilation=dilation)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.mul_(2.0)                                                              # far from the initial near-identity
+        for bn in (m for m in layer.modules() if isinstance(m, torch.nn.BatchNorm1d)):
+            bn.weight.uniform_(0.5, 1.5)
+            bn.bias.normal_(0, 0.3)
+    gpu = copy.deepcopy(layer).cuda()
+    gpu.attn.na = "fused_qkv"
+    return layer.train(), gpu.train()
+
+
+def _errors(cpu, gpu, x, g, dtype):
+    """Relative errors of the native layer's output, gradients and running statistics against the fp32 module."""
+    xg = x.cuda().to(dtype).requires_grad_(True)
+    torch.manual_seed(5)
+    with torch.autocast("cuda", dtype=dtype):
+        out = models.train_layer(gpu, xg)
+    assert out is not None, "not the native path"
+    gd = g.cuda().to(dtype)
+    out.backward(gd)
+    torch.manual_seed(5)
+    xc = x.to(dtype).float().requires_grad_(True)
+    want = cpu(xc)
+    want.backward(gd.float().cpu())
+    err = {"out": O.rel_l2(out.float(), want), "dx": O.rel_l2(xg.grad.float(), xc.grad)}
+    for (name, p), q in zip(cpu.named_parameters(), gpu.parameters()):
+        if name.endswith("proj.bias") or name.endswith("fc2.bias") or p.grad.norm() > 1e-3 * p.grad.numel() ** 0.5:
+            err["d " + name] = O.rel_l2(q.grad, p.grad)
+    for (name, p), q in zip(cpu.named_buffers(), gpu.buffers()):
+        if "running" in name:
+            err[name] = O.rel_l2(q, p)
+        elif name.endswith("batches_tracked"):
+            assert q.item() == p.item() == 1
+    return err
+
+
+# tokens: fewer than a tile (of two rows a norm makes +-1 whatever they hold: nothing to compare), one chunk of rows, remainders of every tile, the launch sizes of all three product tiles
+@pytest.mark.parametrize("batch,T", [(2, 5), (1, 33), (3, 50), (7, 101), (37, 100), (64, 260)])
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("family,groups,heads,window,dilation", [
+    ("mfa", 1, 16, 27, 1), ("mfa", 1, 4, 65, 1), ("pcf", 8, 16, 27, 1), ("pcf", 4, 8, 9, 2), ("pcf", 2, 16, 27, 1), ("pcf", 1, 32, 5, 3)])
+def test_native_training_layer(family, groups, heads, window, dilation, dtype, batch, T):
+    """16-bit rounding of weights, activations and gradients passes through six products and two norms: single results
+    are within a few units of eps (2^-9, 2^-12) in norm; a few rows leave the statistics of the gradients little to
+    average over, and what is left of sums that cancel (qkv's gradients behind the softmax) carries the most."""
+    if batch * T > 5000 and (dtype, family) not in (("fp16", "mfa"), ("bf16", "pcf")):
+        pytest.skip("the large batch once per family")
+    cpu, gpu = _layers(family, groups, heads, window, dilation, T, 0.0, seed=T)
+    gen = torch.Generator().manual_seed(batch)
+    shape = (batch, 256, T) if family == "pcf" else (batch, T, 256)
+    x = torch.randn(shape, generator=gen) + 0.5 * torch.randn((1,) + tuple(256 if s == 256 else 1 for s in shape[1:]), generator=gen)
+    err = _errors(cpu, gpu, x, torch.randn(shape, generator=gen), DT[dtype])
+    print("errors", {k: "%.1e" % v for k, v in err.items()})
+    eps = 2.0 ** -9 if dtype == "bf16" else 2.0 ** -12
+    for name, e in err.items():
+        # running statistics: norm1's come of exact inputs, norm2's of values rounded twice (a unit of eps each, averaged)
+        bound = 1e-5 if "norm1" in name and "running" in name else 2 * eps if "running" in name else 4 * eps if name == "out" else 32 * eps
+        assert e < bound, (name, e)
+
+
+def test_stochastic_depth_draws_like_the_modules():
+    cpu, gpu = _layers("mfa", 1, 16, 27, 1, 64, 0.4, seed=1)
+    gen = torch.Generator().manual_seed(0)
+    x, g = torch.randn(9, 64, 256, generator=gen).half().cuda(), torch.randn(9, 64, 256, generator=gen).half().cuda()
+    results = []
+    for native in (True, False):
+        layer = copy.deepcopy(gpu)
+        xg = x.clone().requires_grad_(True)
+        handle = None if native else layer.mlp.fc2.register_forward_hook(lambda *a: None)    # a hook keeps the modules in use
+        torch.manual_seed(3)
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert (models.train_layer(layer, xg) is not None) == native
+            torch.manual_seed(3)
+            out = layer(xg)
+        out.backward(g)
+        results.append((out.detach(), xg.grad, layer.mlp.fc2.weight.grad, layer.attn.qkv.weight.grad))
+    for a, b in zip(*results):
+        assert O.rel_l2(a.float(), b.float()) < 32 * 2.0 ** -12
+
+
+def test_what_the_node_does_not_cover_stays_with_the_modules():
+    _, gpu = _layers("mfa", 1, 16, 27, 1, 40, 0.0, seed=1)
+    x = torch.randn(4, 40, 256).half().cuda().requires_grad_(True)
+
+    def native(layer=gpu, x=x):
+        return models.train_layer(layer, x) is not None
+    assert not native()                                                              # no autocast
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert native()
+        assert not native(x=x.float())
+        assert not native(x=x[:, :39])                                              # the layer itself refuses this length
+        with pytest.raises(AssertionError):
+            gpu(x[:, :39])
+        with torch.no_grad():
+            assert not native()
+        for change in (lambda m: setattr(m.norm1.norm, "momentum", None), lambda m: m.norm2.norm.eval(),
+                       lambda m: setattr(m.mlp.drop, "p", 0.1), lambda m: setattr(m.attn, "attn_drop", 0.1),
+                       lambda m: setattr(m.mlp, "act", torch.nn.ReLU()), lambda m: m.attn.register_forward_hook(lambda *a: None),
+                       lambda m: setattr(m.mlp, "fc1", torch.nn.Sequential(m.mlp.fc1)), lambda m: m.half()):
+            layer = copy.deepcopy(gpu)
+            change(layer)
+            assert not native(layer)
+        layer = copy.deepcopy(gpu)
+        layer.mlp.fc1.weight.requires_grad_(False)
+        before = layer.norm1.norm.running_mean._version
+        layer(x).sum().backward()
+        assert layer.mlp.fc1.weight.grad is None and layer.mlp.fc2.weight.grad is not None
+        assert layer.norm1.norm.running_mean._version > before
