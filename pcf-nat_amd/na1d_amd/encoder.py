@@ -13,6 +13,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib
+from .train import plain, plain_call
 
 _P, _I, _F = ctypes.c_void_p, ctypes.c_int32, ctypes.c_float
 DIM, HIDDEN, POOL_HIDDEN = 256, 1024, 128          # channels the kernels are built for
@@ -120,8 +121,7 @@ class _Entry:
         self.children = [(m._modules, list(m._modules.values())) for m in mods if m._modules]
         self.tensors = [d for m in mods for d in (m._parameters, m._buffers) if d]
         self.attn = [layer.attn for block in model.blocks for layer in block.blocks] if hasattr(model, "blocks") else []
-        self.fits = _fits(model)
-        self.plans = {}                             # dtype -> (state of the tensors, plan)
+        self.plans = {}                             # dtype -> (state of the tensors, plan or None)
 
     def same_modules(self):
         return all(len(d) == len(c) and all(a is b for a, b in zip(d.values(), c)) for d, c in self.children)
@@ -132,7 +132,10 @@ class _Entry:
         if have is not None and len(have[0]) == len(state) and all(
                 a[0] is b[0] and a[1] == b[1] and a[2] == b[2] for a, b in zip(have[0], state)):
             return have[1]
-        plan = _Plan(model, dtype)
+        if torch.cuda.is_current_stream_capturing():          # it would record the preparation, not do it
+            return None
+        plan = _Plan(model, dtype) if _fits(model) else None
+        torch.cuda.current_stream().synchronize()             # the next call may come on another stream
         self.plans[dtype] = (state, plan)
         return plan
 
@@ -145,8 +148,10 @@ def _fits(model):
     from . import models as M
     layers = [layer for block in model.blocks for layer in block.blocks]
     conv = (model.patch_embeds[0] if model.channels_first else model.patch_embed).proj
-    return (model.embed_dim == DIM and isinstance(model.pool, M.AttentiveStatisticsPooling)
-            and isinstance(model.pool_norm, (nn.Identity, M.BatchNorm1d))
+    return (model.embed_dim == DIM and type(model.pool) is M.AttentiveStatisticsPooling
+            and type(model.fc) is nn.Linear and model.fc.bias is not None and model.fc.in_features == 2 * model.proj.conv.out_channels
+            and (type(model.pool_norm) is nn.Identity or type(model.pool_norm) is M.BatchNorm1d and model.pool_norm.affine
+                 and model.pool_norm.running_mean is not None)
             and all(layer.mlp.fc1.weight.shape[0] == HIDDEN for layer in layers)
             and model.pool.tdnn.conv.out_channels == POOL_HIDDEN and model.proj.conv.out_channels % 256 == 0
             and model.fc.out_features % 16 == 0 and conv.in_channels * model.patch_size % 32 == 0
@@ -159,14 +164,16 @@ def _fits(model):
 def plans_of(model):
     """The plans a captured graph of this model reads from (whoever keeps such a graph keeps them too)."""
     entry = _entries.get(model)
-    return [] if entry is None else [plan for _, plan in entry.plans.values()]
+    return [] if entry is None else [plan for _, plan in entry.plans.values() if plan is not None]
 
 
 def embed(model, x, lens=None):
     """``[N, emb]`` embeddings of ``x [N, in_chans, frames]`` under autocast without gradients, or ``None`` where the
     kernels do not cover the model, its inputs or the mode: the caller then takes another path."""
-    if model.training or not x.is_cuda or torch.is_grad_enabled() or not torch.is_autocast_enabled("cuda"):
+    if model.training or not x.is_cuda or torch.is_grad_enabled() or not torch.is_autocast_enabled("cuda") or not plain_call(x):
         return None
+    if not all(plain(m, type(m)) for m in (model.pool_norm, model.fc)):
+        return None                                 # called as modules otherwise: whatever hangs on them has to see the call
     dtype = torch.get_autocast_dtype("cuda")
     if dtype not in (torch.bfloat16, torch.float16) or x.dim() != 3 or x.dtype not in (torch.float32, torch.bfloat16, torch.float16):
         return None
@@ -175,11 +182,11 @@ def embed(model, x, lens=None):
     entry = _entries.get(model)
     if entry is None or not entry.same_modules():
         entry = _entries[model] = _Entry(model)
-    if not entry.fits or any((a.na != "fused_qkv") if hasattr(a, "na") else (a.dense != "native") for a in entry.attn):
+    if any((a.na != "fused_qkv") if hasattr(a, "na") else (a.dense != "native") for a in entry.attn):
         return None
     plan = entry.plan(model, dtype)
     n, chans, frames = x.shape
-    if chans != plan.encoder.in_chans or plan.keep[0].device != x.device:
+    if plan is None or chans != plan.encoder.in_chans or plan.keep[0].device != x.device:
         return None
     lib = _lib.load()
     if torch.cuda.current_device() != x.device.index:      # launches go to the device of the tensors

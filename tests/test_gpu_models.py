@@ -399,3 +399,41 @@ def test_native_encoder_follows_the_weights():
             outs.append(run())
     torch.cuda.synchronize()
     assert all(torch.equal(o, outs[0]) for o in outs)
+
+
+def test_native_encoder_leaves_changed_models_to_the_modules():
+    """A hook on the last modules sees the call, a head of another kind runs, and a capture without a pass before it
+    leaves nothing behind that a later call would take for prepared weights."""
+    torch.manual_seed(0)
+    kw = dict(depths=(1, 1), num_heads=[[16], [4]], win_size=[[27], [0]], groups=(8, 4))
+    model = models.PCF_NATransformer(na="fused_qkv", **kw).cuda().eval()
+    x = torch.randn(3, 80, 64, generator=torch.Generator().manual_seed(1)).cuda()
+
+    def run(natively=False):
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+            return models.embed_natively(model, x) if natively else model(x)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        unprepared = run(natively=True)
+        x.add_(0)
+    assert unprepared is None
+    want = run(natively=True).clone()
+    assert want.float().abs().sum() > 0
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        captured = run(natively=True)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, want) and torch.equal(run(natively=True), want)
+    seen = []
+    handles = [m.register_forward_hook(lambda m, a, out: seen.append(out.shape)) for m in (model.pool_norm, model.fc)]
+    assert run(natively=True) is None
+    run()
+    assert seen == [(3, 3072), (3, 192)]
+    for h in handles:
+        h.remove()
+    model.fc = torch.nn.Identity()
+    assert run(natively=True) is None and run().shape == (3, 3072)
