@@ -313,37 +313,43 @@ int na1d_encode(const na1d_encoder *e, void *out, const float *x, const float *l
                 void *workspace, int64_t workspace_bytes, void *stream);
 
 /*
- * One windowed layer of those models in training (models/PCF_NATransformer.py:228-265, models/MFA_NATransformer.py:224-261),
+ * One layer of those models in training (models/PCF_NATransformer.py:228-265, models/MFA_NATransformer.py:224-261),
  * forward and backward, on token-major 16-bit activations x, out, dout, dx [N, T, dim]:
  *   x1 = x + f_attn * proj(attention(qkv(norm1(x)))),   out = x1 + f_mlp * fc2(gelu(fc1(norm2(x1))))
- * with batch norms over all N * T tokens (fp32 statistics; the running ones are updated by the forward), weights in fp32
- * rounded to 16 bit for the products, sums in fp32.  Weights lie as [outputs, inputs / groups] (a linear layer, or a grouped
+ * with batch norms over all N * T tokens (the caller brings the batch's fp32 statistics), weights in fp32 rounded to 16 bit
+ * for the products, sums in fp32.  Weights lie as [outputs, inputs / groups] (a linear layer, or a grouped
  * 1x1 convolution); `ordered` says that the qkv projection's outputs are a channels-first model's (channel
  * ((f % (dim / groups)) * groups + f / (dim / groups)) * 3 + which is q, k or v of head-major channel f).  dim and hidden are
- * multiples of 256, groups have multiples of 32 channels; NA1D_ERR_UNSUPPORTED otherwise.
+ * multiples of 256, groups have multiples of 32 channels; NA1D_ERR_UNSUPPORTED otherwise.  window 0: a dense layer
+ * (models/PCF_NATransformer.py:181-225), whose qkv projection sees norm1(x) + linear_pos(pos).
  */
 typedef struct na1d_train_norm {
     const float *weight, *bias;                 /* [dim] */
-    float *running_mean, *running_var;
+    const float *batch_mean, *batch_var;        /* of the input, biased */
     int64_t *batches;                           /* one is added by a forward */
     float *dweight, *dbias;                     /* written by the backward */
-    float eps, momentum;
+    float eps;
 } na1d_train_norm;
 typedef struct na1d_train_layer {
     int32_t dtype, dim, hidden, heads, window, left, dilation, groups, ordered;
     float scale;
     na1d_train_norm norm[2];
-    const float *w[4], *b[4];                   /* qkv, proj, fc1, fc2 */
-    float *dw[4], *db[4];                       /* written by the backward */
+    const float *w[5], *b[5];                   /* qkv, proj, fc1, fc2; of a dense layer also linear_pos (no b) */
+    float *dw[5], *db[5];                       /* written by the backward */
     const float *rpb;                           /* [heads, window] */
     float *drpb;                                /* added to */
+    const void *pos;                            /* dense: 16-bit [T, dim] */
     const float *scale_attn, *scale_mlp;        /* f_attn, f_mlp: fp32 [N] (stochastic depth), NULL for 1 */
 } na1d_train_layer;
 
 /* `saved` is what a forward leaves for its backward; the workspaces are free again when the call's kernels are done. */
 int64_t na1d_train_layer_saved_bytes(const na1d_train_layer *l, int64_t N, int64_t T);
 int64_t na1d_train_layer_workspace_bytes(const na1d_train_layer *l, int64_t N, int64_t T, int backward);
-int na1d_train_layer_forward(const na1d_train_layer *l, void *out, const void *x, void *saved, int64_t saved_bytes,
+/* The forward comes in two parts, for the statistics that the caller works out between them.  part 0 (batch statistics of
+ * norm[0] given): up to x1, which it leaves in `out` as [N, dim, T]; part 1 (those of norm[1] given): the rest, into `out`
+ * [N, T, dim].  Both parts take the same x, saved and workspace.  na1d_train_to_channels: [N, T, dim] -> [N, dim, T]. */
+int na1d_train_to_channels(const na1d_train_layer *l, void *out, const void *x, int64_t N, int64_t T, void *stream);
+int na1d_train_layer_forward(const na1d_train_layer *l, int part, void *out, const void *x, void *saved, int64_t saved_bytes,
                              void *workspace, int64_t workspace_bytes, int64_t N, int64_t T, void *stream);
 int na1d_train_layer_backward(const na1d_train_layer *l, void *dx, const void *dout, const void *x, const void *saved,
                               int64_t saved_bytes, void *workspace, int64_t workspace_bytes, int64_t N, int64_t T,

@@ -420,8 +420,9 @@ int na1d_global_backward(void *dq, void *dk, void *dv, const void *q, const void
     if (workspace_bytes < g.B * g.T * (int64_t)sizeof(float)) return NA1D_ERR_SHAPE;
     if (!(p_drop >= 0.f && p_drop < 1.f)) return NA1D_ERR_SHAPE;
     g.drop = na1d::make_dropout(p_drop, seed);
-    return na1d::mfma::global_bwd(dq, dk, dv, (float *)workspace, q, k, v, out, dout, lse, t_valid, g, scale, dtype,
-                                  (hipStream_t)stream);
+    const na1d::Layout packed = na1d::packed_layout(g);
+    return na1d::mfma::global_bwd(dq, dk, dv, (float *)workspace, q, k, v, out, dout, lse, t_valid, g, packed, packed, scale,
+                                  dtype, (hipStream_t)stream);
 }
 
 int64_t na1d_encode_workspace_bytes(const na1d_encoder *e, int64_t N, int64_t frames) {
@@ -451,18 +452,19 @@ static int train_check(const na1d_train_layer *l, int64_t N, int64_t T) {
     if (N < 0 || T < 0) return NA1D_ERR_SHAPE;
     return mfma_allowed() && na1d::train::layer_ok(*l, N, T) ? NA1D_OK : NA1D_ERR_UNSUPPORTED;
 }
-static int train_pointers(const na1d_train_layer *l, bool backward) {
+static int train_pointers(const na1d_train_layer *l, bool backward, int part = 0) {
     if (bad_scale(l->scale)) return NA1D_ERR_SCALE;
-    if (!l->rpb) return NA1D_ERR_NULL;
-    for (int j = 0; j < 4; ++j) {
+    if (l->window ? !l->rpb : !l->pos) return NA1D_ERR_NULL;
+    if (!l->window && misaligned(l->pos)) return NA1D_ERR_ALIGN;
+    for (int j = 0; j < (l->window ? 4 : 5); ++j) {
         const float *w = backward ? l->dw[j] : l->w[j], *b = backward ? l->db[j] : l->b[j];
-        if (!w || !b) return NA1D_ERR_NULL;
+        if (!w || (j < 4 && !b)) return NA1D_ERR_NULL;
         if (misaligned(w)) return NA1D_ERR_ALIGN;
     }
     for (int j = 0; j < 2; ++j) {
         const na1d_train_norm &n = l->norm[j];
-        if (!n.weight || (backward ? !n.dweight || !n.dbias : !n.bias || !n.running_mean || !n.running_var || !n.batches))
-            return NA1D_ERR_NULL;
+        if (!n.weight || (backward ? !n.dweight || !n.dbias : !n.bias || !n.batches)) return NA1D_ERR_NULL;
+        if (!backward && j == part && (!n.batch_mean || !n.batch_var)) return NA1D_ERR_NULL;
     }
     return NA1D_OK;
 }
@@ -477,16 +479,25 @@ int64_t na1d_train_layer_workspace_bytes(const na1d_train_layer *l, int64_t N, i
     return st == NA1D_OK ? na1d::train::scratch_bytes(*l, N, T, backward != 0) : st;
 }
 
-int na1d_train_layer_forward(const na1d_train_layer *l, void *out, const void *x, void *saved, int64_t saved_bytes, void *workspace,
+int na1d_train_to_channels(const na1d_train_layer *l, void *out, const void *x, int64_t N, int64_t T, void *stream) {
+    const int st = train_check(l, N, T);
+    if (st != NA1D_OK) return st;
+    if (!out || !x) return NA1D_ERR_NULL;
+    if (misaligned(out) || misaligned(x)) return NA1D_ERR_ALIGN;
+    return na1d::train::to_channels(*l, out, x, N, T, (hipStream_t)stream);
+}
+
+int na1d_train_layer_forward(const na1d_train_layer *l, int part, void *out, const void *x, void *saved, int64_t saved_bytes, void *workspace,
                              int64_t workspace_bytes, int64_t N, int64_t T, void *stream) {
     int st = train_check(l, N, T);
-    if (st == NA1D_OK) st = train_pointers(l, false);
+    if (st == NA1D_OK && (part < 0 || part > 1)) st = NA1D_ERR_SHAPE;
+    if (st == NA1D_OK) st = train_pointers(l, false, part);
     if (st != NA1D_OK) return st;
     if (!out || !x || !saved || !workspace) return NA1D_ERR_NULL;
     if (misaligned(out) || misaligned(x) || misaligned(saved) || misaligned(workspace)) return NA1D_ERR_ALIGN;
     if (saved_bytes < na1d::train::saved_bytes(*l, N, T) || workspace_bytes < na1d::train::scratch_bytes(*l, N, T, false))
         return NA1D_ERR_WORKSPACE;
-    return na1d::train::run_forward(*l, out, x, saved, workspace, N, T, (hipStream_t)stream);
+    return na1d::train::run_forward(*l, part, out, x, saved, workspace, N, T, (hipStream_t)stream);
 }
 
 int na1d_train_layer_backward(const na1d_train_layer *l, void *dx, const void *dout, const void *x, const void *saved,
@@ -494,7 +505,7 @@ int na1d_train_layer_backward(const na1d_train_layer *l, void *dx, const void *d
     int st = train_check(l, N, T);
     if (st == NA1D_OK) st = train_pointers(l, true);
     if (st != NA1D_OK) return st;
-    if (!dx || !dout || !x || !saved || !workspace || !l->drpb) return NA1D_ERR_NULL;
+    if (!dx || !dout || !x || !saved || !workspace || (l->window && !l->drpb)) return NA1D_ERR_NULL;
     if (misaligned(dx) || misaligned(dout) || misaligned(x) || misaligned(saved) || misaligned(workspace)) return NA1D_ERR_ALIGN;
     if (saved_bytes < na1d::train::saved_bytes(*l, N, T) || workspace_bytes < na1d::train::scratch_bytes(*l, N, T, true))
         return NA1D_ERR_WORKSPACE;

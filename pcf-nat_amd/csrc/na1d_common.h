@@ -202,8 +202,8 @@ int64_t wide_bwd_workspace_bytes(const Geom &g);               // 0 when the sha
 int global_fwd(void *out, float *lse, const void *q, const void *k, const void *v, const int32_t *t_valid,
                const Geom &g, const Layout &in, const Layout &out_layout, float scale, int dtype, hipStream_t s);
 int global_bwd(void *dq, void *dk, void *dv, float *delta, const void *q, const void *k, const void *v, const void *out,
-               const void *dout, const float *lse, const int32_t *t_valid, const Geom &g, float scale, int dtype,
-               hipStream_t s);
+               const void *dout, const float *lse, const int32_t *t_valid, const Geom &g, const Layout &in,
+               const Layout &out_layout, float scale, int dtype, hipStream_t s);
 }  // namespace mfma
 
 // ---- the speaker-embedding models in inference: na1d_encoder.hip ------------------
@@ -219,7 +219,8 @@ namespace train {
 bool layer_ok(const na1d_train_layer &l, int64_t N, int64_t T);
 int64_t saved_bytes(const na1d_train_layer &l, int64_t N, int64_t T);
 int64_t scratch_bytes(const na1d_train_layer &l, int64_t N, int64_t T, bool backward);
-int run_forward(const na1d_train_layer &l, void *out, const void *x, void *saved, void *ws, int64_t N, int64_t T, hipStream_t s);
+int to_channels(const na1d_train_layer &l, void *out, const void *x, int64_t N, int64_t T, hipStream_t s);
+int run_forward(const na1d_train_layer &l, int half, void *out, const void *x, void *saved, void *ws, int64_t N, int64_t T, hipStream_t s);
 int run_backward(const na1d_train_layer &l, void *dx, const void *dout, const void *x, const void *saved, void *ws, int64_t N,
                  int64_t T, hipStream_t s);
 }  // namespace train

@@ -66,10 +66,9 @@ __device__ inline void scale_in_place(f32x4 &x, float a) {
 struct GlobalArgs {
     int T, H, strips;            // strips of kStripTiles tiles per sequence
     uint32_t strips_magic, heads_magic;
-    int pitch;                   // bytes per row = 2 * head_dim (packed rows)
     float scale;
     Dropout drop;                // attention dropout; its window slot is the key's row index
-    Strides in, outl;            // forward: where q, k, v and the output have their rows
+    Strides in, outl;            // where q, k, v (and their gradients), and the output (and its), have their rows
 };
 
 // =============================================================================
@@ -464,7 +463,7 @@ global_dq_kernel(char *__restrict__ dq, float *__restrict__ delta, const char *_
     constexpr int CT = C / 16;
     constexpr int kStep = region_bytes<C>(kStripTiles);
     fetch_args_now(dq, delta, q, k, v, out, dout, lse, t_valid, items, a.T, a.H, a.strips, a.strips_magic, a.heads_magic,
-                   a.pitch, a.scale);
+                   a.scale, a.in.sample, a.in.head, a.in.pitch, a.in.width, a.outl.sample, a.outl.head, a.outl.pitch);
     if constexpr (DROP) fetch_args_now(a.drop.threshold, a.drop.seed_lo, a.drop.seed_hi, a.drop.inv_keep);
     extern __shared__ __attribute__((aligned(16))) char smem[];          // 4 * kStep bytes: K and V of two chunks
     LDS_PTR(char) kv_lds = (LDS_PTR(char))smem;
@@ -478,24 +477,26 @@ global_dq_kernel(char *__restrict__ dq, float *__restrict__ delta, const char *_
     const uint32_t sample = div_by(b, a.H, a.heads_magic);
     const int T = a.T, tiles = (T + 15) >> 4;
 
-    const int64_t seq_off = (int64_t)b * T * a.pitch;
-    const Rsrc qs = make_rsrc(q + seq_off, T * a.pitch), ks = make_rsrc(k + seq_off, T * a.pitch);
-    const Rsrc vs = make_rsrc(v + seq_off, T * a.pitch), os = make_rsrc(out + seq_off, T * a.pitch);
-    const Rsrc gs = make_rsrc(dout + seq_off, T * a.pitch), dqs = make_rsrc(dq + seq_off, T * a.pitch);
+    const int64_t in_off = sample * a.in.sample + (b - sample * a.H) * a.in.head;
+    const int64_t out_off = sample * a.outl.sample + (b - sample * a.H) * a.outl.head;
+    const int pitch = a.in.pitch, out_pitch = a.outl.pitch, width = a.in.width;
+    const Rsrc qs = make_rsrc(q + in_off, T * pitch), ks = make_rsrc(k + in_off, T * pitch);
+    const Rsrc vs = make_rsrc(v + in_off, T * pitch), os = make_rsrc(out + out_off, T * out_pitch);
+    const Rsrc gs = make_rsrc(dout + out_off, T * out_pitch), dqs = make_rsrc(dq + in_off, T * pitch);
     const Rsrc ls = make_rsrc(lse + (int64_t)b * T, T * 4), ds = make_rsrc(delta + (int64_t)b * T, T * 4);
-    const int lane_off = direct_lane_offset<C>(wave, lane, a.pitch, a.pitch);
-    stage_direct<C, kStripTiles, kReadShared>(ks, 0, kv_lds, kStripTiles, wave, lane_off, a.pitch);
-    stage_direct<C, kStripTiles, kReadShared>(vs, 0, kv_lds + kStep, kStripTiles, wave, lane_off, a.pitch);
+    const int lane_off = direct_lane_offset<C>(wave, lane, pitch, width);
+    stage_direct<C, kStripTiles, kReadShared>(ks, 0, kv_lds, kStripTiles, wave, lane_off, pitch);
+    stage_direct<C, kStripTiles, kReadShared>(vs, 0, kv_lds + kStep, kStripTiles, wave, lane_off, pitch);
     int qt[QT];                                             // this wave's query tiles
     RowOperand<C> qop[QT], gop[QT], oop[QT];
     float lse_row[QT];
 #pragma unroll
     for (int h = 0; h < QT; ++h) {
         qt[h] = kStripTiles * (QT * strip + h) + wave;
-        const int at = 16 * qt[h] * a.pitch;
-        load_rows<C, kReadShared>(qop[h], qs, at, a.pitch, a.pitch, lane);
-        load_rows<C, kReadShared>(gop[h], gs, at, a.pitch, a.pitch, lane);
-        load_rows<C, kReadOnce>(oop[h], os, at, a.pitch, a.pitch, lane);
+        const int at = 16 * qt[h] * pitch, out_at = 16 * qt[h] * out_pitch;
+        load_rows<C, kReadShared>(qop[h], qs, at, pitch, width, lane);
+        load_rows<C, kReadShared>(gop[h], gs, out_at, out_pitch, width, lane);
+        load_rows<C, kReadOnce>(oop[h], os, out_at, out_pitch, width, lane);
         lse_row[h] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ls, (16 * qt[h] + n) * 4, 0, 0));
     }
     int tv = T;
@@ -577,8 +578,8 @@ global_dq_kernel(char *__restrict__ dq, float *__restrict__ delta, const char *_
         barrier_lds();      // this chunk has landed, and every wave is done with the one before, whose regions the next takes
         if (c0 + kStripTiles < tiles) {
             LDS_PTR(char) next = kv_lds + (at ^ 2 * kStep);
-            stage_direct<C, kStripTiles, kReadShared>(ks, 16 * (c0 + kStripTiles), next, kStripTiles, wave, lane_off, a.pitch);
-            stage_direct<C, kStripTiles, kReadShared>(vs, 16 * (c0 + kStripTiles), next + kStep, kStripTiles, wave, lane_off, a.pitch);
+            stage_direct<C, kStripTiles, kReadShared>(ks, 16 * (c0 + kStripTiles), next, kStripTiles, wave, lane_off, pitch);
+            stage_direct<C, kStripTiles, kReadShared>(vs, 16 * (c0 + kStripTiles), next + kStep, kStripTiles, wave, lane_off, pitch);
         }
         chunk(whole, c0, kv_lds + at, kv_lds + at + kStep);
         at ^= 2 * kStep;
@@ -594,7 +595,7 @@ global_dq_kernel(char *__restrict__ dq, float *__restrict__ delta, const char *_
         u32x2 qw[CT];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) qw[ct] = pack_acc<DT>(acc[h][ct], a.scale);
-        store_tile<C>(dqs, qrow * a.pitch, qw, g, stores_whole_lines(a.pitch, C, 0), a.pitch);
+        store_tile<C>(dqs, qrow * pitch, qw, g, stores_whole_lines(pitch, C, 0), width);
         if (g == 0) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(dl[h]), ds, qrow * 4, 0, 0);
     }
 }
@@ -617,7 +618,7 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
     constexpr int kRows = 16 * kStripTiles;                 // rows of a chunk: one lse / delta value each
     constexpr int kBuf = 2 * kStep + 2 * kRows * 4;         // Q, dO, lse, delta of one chunk
     fetch_args_now(dk, dv, q, k, v, dout, lse, delta, t_valid, items, a.T, a.H, a.strips, a.strips_magic, a.heads_magic,
-                   a.pitch, a.scale);
+                   a.scale, a.in.sample, a.in.head, a.in.pitch, a.in.width, a.outl.sample, a.outl.head, a.outl.pitch);
     if constexpr (DROP) fetch_args_now(a.drop.threshold, a.drop.seed_lo, a.drop.seed_hi, a.drop.inv_keep);
     extern __shared__ __attribute__((aligned(16))) char smem[];          // 2 * kBuf bytes
     LDS_PTR(char) buf_lds = (LDS_PTR(char))smem;
@@ -631,15 +632,17 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
     const uint32_t sample = div_by(b, a.H, a.heads_magic);
     const int T = a.T, tiles = (T + 15) >> 4;
 
-    const int64_t seq_off = (int64_t)b * T * a.pitch;
-    const Rsrc qs = make_rsrc(q + seq_off, T * a.pitch), ks = make_rsrc(k + seq_off, T * a.pitch);
-    const Rsrc vs = make_rsrc(v + seq_off, T * a.pitch), gs = make_rsrc(dout + seq_off, T * a.pitch);
-    const Rsrc dks = make_rsrc(dk + seq_off, T * a.pitch), dvs = make_rsrc(dv + seq_off, T * a.pitch);
+    const int64_t in_off = sample * a.in.sample + (b - sample * a.H) * a.in.head;
+    const int64_t out_off = sample * a.outl.sample + (b - sample * a.H) * a.outl.head;
+    const int pitch = a.in.pitch, out_pitch = a.outl.pitch, width = a.in.width;
+    const Rsrc qs = make_rsrc(q + in_off, T * pitch), ks = make_rsrc(k + in_off, T * pitch);
+    const Rsrc vs = make_rsrc(v + in_off, T * pitch), gs = make_rsrc(dout + out_off, T * out_pitch);
+    const Rsrc dks = make_rsrc(dk + in_off, T * pitch), dvs = make_rsrc(dv + in_off, T * pitch);
     const Rsrc ls = make_rsrc(lse + (int64_t)b * T, T * 4), ds = make_rsrc(delta + (int64_t)b * T, T * 4);
-    const int lane_off = direct_lane_offset<C>(wave, lane, a.pitch, a.pitch);
+    const int lane_off = direct_lane_offset<C>(wave, lane, pitch, width), out_lane_off = direct_lane_offset<C>(wave, lane, out_pitch, width);
     auto stage = [&](int c0, LDS_PTR(char) buf) {           // chunk of queries c0 .. c0 + 3 into one buffer
-        stage_direct<C, kStripTiles, kReadShared>(qs, 16 * c0, buf, kStripTiles, wave, lane_off, a.pitch);
-        stage_direct<C, kStripTiles, kReadShared>(gs, 16 * c0, buf + kStep, kStripTiles, wave, lane_off, a.pitch);
+        stage_direct<C, kStripTiles, kReadShared>(qs, 16 * c0, buf, kStripTiles, wave, lane_off, pitch);
+        stage_direct<C, kStripTiles, kReadShared>(gs, 16 * c0, buf + kStep, kStripTiles, wave, out_lane_off, out_pitch);
         if (wave == 0) load_to_lds<4, 0>(ls, buf + 2 * kStep, (16 * c0 + lane) * 4);            // rows past T: zeros
         if (wave == 1) load_to_lds<4, 0>(ds, buf + 2 * kStep + kRows * 4, (16 * c0 + lane) * 4);
     };
@@ -649,8 +652,8 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
 #pragma unroll
     for (int h = 0; h < QT; ++h) {
         kt_own[h] = kStripTiles * (QT * strip + h) + wave;
-        load_rows<C, kReadShared>(kop[h], ks, 16 * kt_own[h] * a.pitch, a.pitch, a.pitch, lane);
-        load_rows<C, kReadShared>(vop[h], vs, 16 * kt_own[h] * a.pitch, a.pitch, a.pitch, lane);
+        load_rows<C, kReadShared>(kop[h], ks, 16 * kt_own[h] * pitch, pitch, width, lane);
+        load_rows<C, kReadShared>(vop[h], vs, 16 * kt_own[h] * pitch, pitch, width, lane);
     }
     int tv = T;
     if (t_valid) tv = max(0, min(T, t_valid[sample]));
@@ -745,7 +748,7 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
     for (; 16 * (c0 + kStripTiles) <= whole_rows; c0 += kStripTiles) step(std::true_type{}, c0);
     for (; c0 < tiles; c0 += kStripTiles) step(std::false_type{}, c0);
 
-    const bool stream = stores_whole_lines(a.pitch, C, 0);
+    const bool stream = stores_whole_lines(pitch, C, 0);
 #pragma unroll
     for (int h = 0; h < QT; ++h) {
         if (kt_own[h] >= tiles) break;
@@ -756,8 +759,8 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
             kw[ct] = pack_acc<DT>(acck[h][ct], a.scale);
             vw[ct] = pack_acc<DT>(accv[h][ct], 1.f);
         }
-        store_tile<C>(dks, key * a.pitch, kw, g, stream, a.pitch);      // rows past T are dropped
-        store_tile<C>(dvs, key * a.pitch, vw, g, stream, a.pitch);
+        store_tile<C>(dks, key * pitch, kw, g, stream, width);      // rows past T are dropped
+        store_tile<C>(dvs, key * pitch, vw, g, stream, width);
     }
 }
 
@@ -776,9 +779,10 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
     using LL = Lds<C>;
     constexpr int CT = C / 16, kW = TILES / QT;       // waves of the workgroup, QT query / key tiles each
     constexpr int kRows = 16 * TILES;
-    fetch_args_now(dq, dk, dv, q, k, v, out, dout, lse, t_valid, a.T, a.H, a.heads_magic, a.pitch, a.scale);
+    fetch_args_now(dq, dk, dv, q, k, v, out, dout, lse, t_valid, a.T, a.H, a.heads_magic, a.scale, a.in.sample, a.in.head, a.in.pitch, a.in.width,
+                   a.outl.sample, a.outl.head, a.outl.pitch);
     if constexpr (DROP) fetch_args_now(a.drop.threshold, a.drop.seed_lo, a.drop.seed_hi, a.drop.inv_keep);
-    const int T = a.T, tiles = (T + 15) >> 4, pitch = a.pitch;
+    const int T = a.T, tiles = (T + 15) >> 4, pitch = a.in.pitch, out_pitch = a.outl.pitch, width = a.in.width;
     const int region = region_bytes<C>(tiles);
     extern __shared__ __attribute__((aligned(16))) char smem[];          // 4 * region + 2 * kRows * 4 bytes
     LDS_PTR(char) q_lds = (LDS_PTR(char))smem;
@@ -792,13 +796,15 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, n = lane & 15;
     const uint32_t b = blockIdx.x;
-    const int64_t seq_off = (int64_t)((uint64_t)b * (uint32_t)(T * pitch));
-    const Rsrc qs = make_rsrc(q + seq_off, T * pitch), gs = make_rsrc(dout + seq_off, T * pitch);
-    const Rsrc ks = make_rsrc(k + seq_off, T * pitch), vs = make_rsrc(v + seq_off, T * pitch);
-    const Rsrc os = make_rsrc(out + seq_off, T * pitch), ls = make_rsrc(lse + (int64_t)b * T, T * 4);
-    const int lane_off = direct_lane_offset<C>(wave, lane, pitch, pitch);
+    const uint32_t sample = div_by(b, a.H, a.heads_magic);
+    const int64_t in_off = sample * a.in.sample + (b - sample * a.H) * a.in.head;
+    const int64_t out_off = sample * a.outl.sample + (b - sample * a.H) * a.outl.head;
+    const Rsrc qs = make_rsrc(q + in_off, T * pitch), gs = make_rsrc(dout + out_off, T * out_pitch);
+    const Rsrc ks = make_rsrc(k + in_off, T * pitch), vs = make_rsrc(v + in_off, T * pitch);
+    const Rsrc os = make_rsrc(out + out_off, T * out_pitch), ls = make_rsrc(lse + (int64_t)b * T, T * 4);
+    const int lane_off = direct_lane_offset<C>(wave, lane, pitch, width), out_lane_off = direct_lane_offset<C>(wave, lane, out_pitch, width);
     stage_direct<C, TILES, kReadOnce, kW>(qs, 0, q_lds, tiles, wave, lane_off, pitch);
-    stage_direct<C, TILES, kReadOnce, kW>(gs, 0, g_lds, tiles, wave, lane_off, pitch);
+    stage_direct<C, TILES, kReadOnce, kW>(gs, 0, g_lds, tiles, wave, out_lane_off, out_pitch);
     stage_direct<C, TILES, kReadOnce, kW>(ks, 0, k_lds, tiles, wave, lane_off, pitch);
     stage_direct<C, TILES, kReadOnce, kW>(vs, 0, v_lds, tiles, wave, lane_off, pitch);
     if (wave < kRows / 64) load_to_lds<4, 0>(ls, (LDS_PTR(char))(lse_lds + 64 * wave), (64 * wave + lane) * 4);     // rows past T: zeros
@@ -808,11 +814,10 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
 #pragma unroll
     for (int h = 0; h < QT; ++h) {
         own[h] = min(wave + kW * h, tiles - 1);
-        load_rows<C, kReadOnce>(oop[h], os, 16 * own[h] * pitch, pitch, pitch, lane);
+        load_rows<C, kReadOnce>(oop[h], os, 16 * own[h] * out_pitch, out_pitch, width, lane);
     }
     __builtin_amdgcn_sched_barrier(0);
 
-    const uint32_t sample = div_by(b, a.H, a.heads_magic);
     int tv = T;
     if (t_valid) tv = max(0, min(T, t_valid[sample]));
     const float scale2 = a.scale * kLog2e, mask2 = kMaskValue * kLog2e;
@@ -874,14 +879,14 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
                 for (int h = 0; h < QT; ++h) acc[h][ct] = Mma<DT>::k16(kt_t, db[h], acc[h][ct]);
             }
         }
-        const Rsrc dqs = make_rsrc(dq + seq_off, T * pitch);
+        const Rsrc dqs = make_rsrc(dq + in_off, T * pitch);
 #pragma unroll
         for (int h = 0; h < QT; ++h) {
             if (wave + kW * h >= tiles) break;
             u32x2 qw[CT];
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) qw[ct] = pack_acc<DT>(acc[h][ct], a.scale);
-            store_tile<C>(dqs, (16 * own[h] + n) * pitch, qw, g, stores_whole_lines(pitch, C, 0), pitch);   // rows past T are dropped
+            store_tile<C>(dqs, (16 * own[h] + n) * pitch, qw, g, stores_whole_lines(pitch, C, 0), width);   // rows past T are dropped
         }
     }
     barrier_lds();                                          // every row's delta is in LDS
@@ -938,7 +943,7 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
             }
         }
     }
-    const Rsrc dks = make_rsrc(dk + seq_off, T * pitch), dvs = make_rsrc(dv + seq_off, T * pitch);
+    const Rsrc dks = make_rsrc(dk + in_off, T * pitch), dvs = make_rsrc(dv + in_off, T * pitch);
     const bool stream = stores_whole_lines(pitch, C, 0);
 #pragma unroll
     for (int h = 0; h < QT; ++h) {
@@ -949,8 +954,8 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
             kw[ct] = pack_acc<DT>(acck[h][ct], a.scale);
             vw[ct] = pack_acc<DT>(accv[h][ct], 1.f);
         }
-        store_tile<C>(dks, (16 * own[h] + n) * pitch, kw, g, stream, pitch);      // rows past T are dropped
-        store_tile<C>(dvs, (16 * own[h] + n) * pitch, vw, g, stream, pitch);
+        store_tile<C>(dks, (16 * own[h] + n) * pitch, kw, g, stream, width);      // rows past T are dropped
+        store_tile<C>(dvs, (16 * own[h] + n) * pitch, vw, g, stream, width);
     }
 }
 
@@ -965,7 +970,6 @@ inline bool global_ok(const Geom &g, GlobalArgs &a, int64_t &items) {
     if (items > 0x7fffff00LL || !div_magic_ok(items, a.strips) || !div_magic_ok(g.B, g.H)) return false;
     a.strips_magic = div_magic(a.strips);
     a.heads_magic = div_magic(g.H);
-    a.pitch = 2 * g.C;
     a.drop = g.drop;
     return true;
 }
@@ -1020,11 +1024,13 @@ int launch_global_fwd(void *out, float *lse, const void *q, const void *k, const
 template <class DT, int C>
 int launch_global_bwd(void *dq, void *dk, void *dv, float *delta, const void *q, const void *k, const void *v,
                       const void *out, const void *dout, const float *lse, const int32_t *t_valid, const Geom &g,
-                      float scale, hipStream_t s) {
+                      const Layout &in, const Layout &outl, float scale, hipStream_t s) {
     GlobalArgs a;
     int64_t items;
-    if (!global_ok(g, a, items)) return NA1D_ERR_UNSUPPORTED;
+    if (!global_ok(g, a, items) || !strides_ok(in, g) || !strides_ok(outl, g)) return NA1D_ERR_UNSUPPORTED;
     a.scale = scale;
+    a.in = byte_strides(in, g);
+    a.outl = byte_strides(outl, g);
     if (g.T <= 16 * kShortTiles) {
         const int tiles_max = g.T <= 64 ? 4 : 8;            // a wave per tile either way
         const size_t lds = 4 * (size_t)region_bytes<C>((int)(g.T + 15) / 16) + 2 * 16 * tiles_max * sizeof(float);
@@ -1075,9 +1081,9 @@ int global_fwd(void *out, float *lse, const void *q, const void *k, const void *
 }
 
 int global_bwd(void *dq, void *dk, void *dv, float *delta, const void *q, const void *k, const void *v, const void *out,
-               const void *dout, const float *lse, const int32_t *t_valid, const Geom &g, float scale, int dtype,
-               hipStream_t s) {
-    NA1D_MFMA_DISPATCH(launch_global_bwd, dq, dk, dv, delta, q, k, v, out, dout, lse, t_valid, g, scale, s);
+               const void *dout, const float *lse, const int32_t *t_valid, const Geom &g, const Layout &in,
+               const Layout &outl, float scale, int dtype, hipStream_t s) {
+    NA1D_MFMA_DISPATCH(launch_global_bwd, dq, dk, dv, delta, q, k, v, out, dout, lse, t_valid, g, in, outl, scale, s);
 }
 
 }  // namespace mfma

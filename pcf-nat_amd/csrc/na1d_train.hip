@@ -2,9 +2,12 @@
 // 224-261) in training, forward and backward, on token-major activations: batch norms with batch statistics, projections,
 // GELU, residuals and weight gradients around the attention kernels.
 //
-// A layer of 128 x 100 tokens, 256 channels, fp16, forward and backward: 29 launches of 215 us together, where the modules
-// took some 80 launches and 800 us (torch's batch norm of a transposed view with its copies, bias gradients as reductions of
-// their own, weight gradients through 16-bit sums of chunks).  Everything is launched by two calls, so the host keeps ahead.
+// A layer of 128 x 100 tokens, 256 channels, fp16, forward and backward: 33 launches of 250 us together, where the modules
+// took some 80 launches and 800 us (torch's batch norm with its copies, bias gradients as reductions of their own, weight
+// gradients through 16-bit sums of chunks).  Everything else than the batch statistics is launched from native code, so the
+// host keeps ahead.  The forward rounds where the modules round and is theirs to the bit: training amplifies a difference
+// anywhere in it, by way of the rounding of sixteen layers, to what 16 bits give (1.2e-3 of the embeddings, 3 % of the
+// gradients).  The backward's gradients are within 4e-4 of the modules'.
 #include "na1d_encoder.h"
 
 namespace na1d {
@@ -15,11 +18,11 @@ using namespace enc;
 // =============================================================================
 // Batch norm over the rows of [M, C]
 // =============================================================================
-// Bound by memory: a pass over 12800 x 256 16-bit values is 6.5 MB.  A workgroup takes 64 channels (whole 128-byte lines)
-// of one of up to 64 chunks of rows; its sums are those of the differences to the chunk's first row, and the chunks meet
-// by their means (nothing cancels, however far the mean is from zero).  The kernel that uses the statistics combines the
-// chunks itself (32 KB from L2) instead of waiting for a third launch.  12800 x 256: sums 5.0 us and application 8.3 us
-// forward, 7.9 and 8.7 us backward, where torch took 31 and 54 us, and 13 us for each change of layout.
+// The sums of the forward are torch's (batch_norm_update_stats on [N, C, T]), to the bit.
+// What uses the statistics, and the backward, is bound by memory: a pass over 12800 x 256 16-bit values is 6.5 MB.  A
+// workgroup takes 64 channels (whole 128-byte lines) of one of up to 64 chunks of rows; the kernel that uses the backward's
+// sums adds up the chunks itself (32 KB from L2) instead of waiting for a third launch.  12800 x 256: 7.9 and 8.7 us
+// backward, where torch took 54 us, and 13 us for each change of layout.
 constexpr int kBnCols = 64, kBnThreads = 256, kBnLanes = kBnThreads / 8, kBnChunks = 64;
 struct Chunks {
     int rows, count;          // rows of a chunk (the last may have fewer), chunks
@@ -36,6 +39,9 @@ template <class DT> __device__ inline void unpack(u32x4 w, float (&v)[8]) {
         v[2 * i + 1] = p.y;
     }
 }
+// Sums round where the modules round: a projection's output before the residual takes it, a norm's gradient before the
+// residual's.
+template <class DT> __device__ inline f32x4 rounded(f32x4 v) { return widen4<DT>(narrow4<DT>(v)); }
 template <class DT> __device__ inline u32x4 repack(const float (&v)[8]) {
     return u32x4{Mma<DT>::pack(v[0], v[1]), Mma<DT>::pack(v[2], v[3]), Mma<DT>::pack(v[4], v[5]), Mma<DT>::pack(v[6], v[7])};
 }
@@ -62,90 +68,88 @@ __device__ inline float across_groups(float (*quarter)[kBnCols], float v) {
     return quarter[0][ch] + quarter[1][ch] + (quarter[2][ch] + quarter[3][ch]);
 }
 
-template <class DT>
-__global__ void __launch_bounds__(kBnThreads)
-bn_stats_kernel(float *__restrict__ part_mean, float *__restrict__ part_m2, const char *__restrict__ x, int M, int C, int rows) {
-    __shared__ float part[kBnLanes][kBnCols + 1], quarter[4][kBnCols];
-    const int c = threadIdx.x & 7, r = threadIdx.x >> 3, c0 = blockIdx.x * kBnCols, r0 = blockIdx.y * rows, r1 = min(M, r0 + rows);
-    const char *src = x + 2 * (int64_t)(c0 + 8 * c);
-    const int64_t pitch = 2 * (int64_t)C;
-    float first[8], s1[8], s2[8];
-    unpack<DT>(*reinterpret_cast<const u32x4 *>(src + r0 * pitch), first);
+// [N, T, C] -> [N, C, T], 64 x 64 at a time through LDS: the layout in which torch sums the statistics.
+__global__ void __launch_bounds__(256)
+to_channels_kernel(uint16_t *__restrict__ out, const char *__restrict__ x, int T, int C) {
+    __shared__ uint16_t tile[64][64 + 2];
+    const int t0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
+    const char *src = x + ((int64_t)blockIdx.z * T * C + c0) * 2;
+    uint16_t *dst = out + ((int64_t)blockIdx.z * C + c0) * T;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) s1[i] = s2[i] = 0.f;
-#pragma unroll 4
-    for (int t = r0 + r; t < r1; t += kBnLanes) {
-        float v[8];
-        unpack<DT>(*reinterpret_cast<const u32x4 *>(src + t * pitch), v);
+    for (int i = 0; i < 2; ++i) {
+        const int u = i * 256 + threadIdx.x, t = u >> 3, c = (u & 7) * 8;
+        if (t0 + t < T) {
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(src + ((int64_t)(t0 + t) * C + c) * 2);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float d = v[i] - first[i];
-            s1[i] += d;
-            s2[i] = __builtin_fmaf(d, d, s2[i]);
+            for (int k = 0; k < 4; ++k) {
+                tile[t][c + 2 * k] = (uint16_t)v[k];
+                tile[t][c + 2 * k + 1] = (uint16_t)(v[k] >> 16);
+            }
         }
     }
-    float a, b;
-    meet(part, quarter, s1, a);
-    meet(part, quarter, s2, b);
-    if (threadIdx.x >= kBnCols) return;
-    const int ch = threadIdx.x;
-    const float x0 = widen<DT>((uint32_t)*reinterpret_cast<const uint16_t *>(x + r0 * pitch + 2 * (c0 + ch))).x;
-    const float m = a / (float)(r1 - r0);
-    part_mean[(int64_t)blockIdx.y * C + c0 + ch] = x0 + m;
-    part_m2[(int64_t)blockIdx.y * C + c0 + ch] = b - a * m;
+    __syncthreads();
+    const int t = threadIdx.x & 63;
+    if (t0 + t >= T) return;
+#pragma unroll 4
+    for (int c = threadIdx.x >> 6; c < 64; c += 4) dst[(int64_t)c * T + t0 + t] = tile[t][c];
 }
 
+// weight * (x - mean) * rstd + bias of two channels, each rounded once (as torch's kernel rounds: fp16 through the mixed
+// multiply-add, which rounds its exact result).
+template <class DT> __device__ inline uint32_t normal_pair(const float *x, const float *m, const float *w, const float *r, const float *b);
+template <> __device__ inline uint32_t normal_pair<FP16>(const float *x, const float *m, const float *w, const float *r, const float *b) {
+    uint32_t v;
+    const float lo = w[0] * (x[0] - m[0]), hi = w[1] * (x[1] - m[1]);
+    asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(v) : "v"(lo), "v"(r[0]), "v"(b[0]));
+    asm("v_fma_mixhi_f16 %0, %1, %2, %3" : "+v"(v) : "v"(hi), "v"(r[1]), "v"(b[1]));
+    return v;
+}
+template <> __device__ inline uint32_t normal_pair<BF16>(const float *x, const float *m, const float *w, const float *r, const float *b) {
+    return Mma<BF16>::pack(__builtin_fmaf(w[0] * (x[0] - m[0]), r[0], b[0]), __builtin_fmaf(w[1] * (x[1] - m[1]), r[1], b[1]));
+}
 struct BnApply {
     char *y;
     const char *x;
-    const float *part_mean, *part_m2, *weight, *bias;
+    const float *batch_mean, *batch_var, *weight, *bias;
     float *mean, *rstd;                        // for the backward
-    float *running_mean, *running_var;
     int64_t *batches;                          // counts the calls, as torch's module does
-    float eps, momentum;
-    int M, C, rows, chunks;
+    float eps;
+    int M, C, rows;
+    const char *add;                           // 16-bit [T, C], added to every sample's rows, or NULL
+    int T;
 };
 template <class DT>
 __global__ void __launch_bounds__(kBnThreads)
 bn_apply_kernel(BnApply a) {
-    __shared__ float quarter[4][kBnCols], s_mean[kBnCols], s_a[kBnCols], s_b[kBnCols];
-    const int c0 = blockIdx.x * kBnCols, ch = threadIdx.x & 63, q = threadIdx.x >> 6;
-    float s = 0.f;
-#pragma unroll 4
-    for (int k = q; k < a.chunks; k += 4) s = __builtin_fmaf((float)min(a.rows, a.M - k * a.rows), a.part_mean[(int64_t)k * a.C + c0 + ch], s);
-    const float mean = across_groups(quarter, s) / (float)a.M;
-    s = 0.f;
-#pragma unroll 4
-    for (int k = q; k < a.chunks; k += 4) {
-        const float d = a.part_mean[(int64_t)k * a.C + c0 + ch] - mean;
-        s += a.part_m2[(int64_t)k * a.C + c0 + ch] + (float)min(a.rows, a.M - k * a.rows) * d * d;
-    }
-    const float m2 = across_groups(quarter, s), rstd = rsqrtf(m2 / (float)a.M + a.eps);
-    if (threadIdx.x < kBnCols) {
-        s_mean[ch] = mean;
-        s_a[ch] = rstd * a.weight[c0 + ch];
-        s_b[ch] = a.bias[c0 + ch];
-        if (blockIdx.y == 0) {
-            a.mean[c0 + ch] = mean;
-            a.rstd[c0 + ch] = rstd;
-            a.running_mean[c0 + ch] += a.momentum * (mean - a.running_mean[c0 + ch]);
-            a.running_var[c0 + ch] += a.momentum * (m2 / (float)(a.M - 1) - a.running_var[c0 + ch]);
-            if (c0 == 0 && ch == 0) *a.batches += 1;
-        }
-    }
-    __syncthreads();
-    const int c = threadIdx.x & 7, r0 = blockIdx.y * a.rows, r1 = min(a.M, r0 + a.rows);
-    float m[8], k[8], b[8];
+    const int c = threadIdx.x & 7, c0 = blockIdx.x * kBnCols + 8 * c, r0 = blockIdx.y * a.rows, r1 = min(a.M, r0 + a.rows);
+    float m[8], w[8], b[8], r[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) m[i] = s_mean[8 * c + i], k[i] = s_a[8 * c + i], b[i] = s_b[8 * c + i];
-    const int64_t pitch = 2 * (int64_t)a.C, at = 2 * (int64_t)(c0 + 8 * c);
+    for (int i = 0; i < 8; ++i) {
+        m[i] = a.batch_mean[c0 + i], w[i] = a.weight[c0 + i], b[i] = a.bias[c0 + i];
+        r[i] = __builtin_amdgcn_rsqf(a.batch_var[c0 + i] + a.eps);
+    }
+    if (blockIdx.y == 0 && threadIdx.x < 8) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a.mean[c0 + i] = m[i], a.rstd[c0 + i] = r[i];
+        if (c0 == 0) *a.batches += 1;
+    }
+    const int64_t pitch = 2 * (int64_t)a.C, at = 2 * (int64_t)c0;
 #pragma unroll 4
     for (int t = r0 + (threadIdx.x >> 3); t < r1; t += kBnLanes) {
         float v[8];
         unpack<DT>(*reinterpret_cast<const u32x4 *>(a.x + t * pitch + at), v);
+        u32x4 y;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = __builtin_fmaf(v[i] - m[i], k[i], b[i]);
-        *reinterpret_cast<u32x4 *>(a.y + t * pitch + at) = repack<DT>(v);
+        for (int i = 0; i < 4; ++i) y[i] = normal_pair<DT>(v + 2 * i, m + 2 * i, w + 2 * i, r + 2 * i, b + 2 * i);
+        if (a.add) {
+            float e[8];
+            unpack<DT>(y, v);
+            unpack<DT>(*reinterpret_cast<const u32x4 *>(a.add + t % a.T * pitch + at), e);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] += e[i];
+            y = repack<DT>(v);
+        }
+        *reinterpret_cast<u32x4 *>(a.y + t * pitch + at) = y;
     }
 }
 
@@ -225,7 +229,10 @@ bn_bwd_apply_kernel(BnBackward a) {
         unpack<DT>(*reinterpret_cast<const u32x4 *>(a.dy + t * pitch + at), d);
         unpack<DT>(*reinterpret_cast<const u32x4 *>(a.add + t * pitch + at), e);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = __builtin_fmaf(f[i], d[i] - k1[i] - (v[i] - m[i]) * k2[i], e[i]);
+        for (int i = 0; i < 8; ++i) v[i] = f[i] * (d[i] - k1[i] - (v[i] - m[i]) * k2[i]);
+        unpack<DT>(repack<DT>(v), v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] += e[i];
         *reinterpret_cast<u32x4 *>(a.dx + t * pitch + at) = repack<DT>(v);
     }
 }
@@ -251,18 +258,19 @@ struct Weight {
         return i < i0 || i >= i0 + in ? -1 : (int64_t)o * in + (i - i0);
     }
 };
+constexpr int kWeights = 5;       // qkv, proj, fc1, fc2; linear_pos of dense layers, otherwise empty
 struct Pack {
-    Weight w[4];
-    char *plain[4], *turned[4];   // in fragment order: [outputs, inputs] and its transpose
-    float *bias[4];               // in the rows' order
-    int first[5];                 // blocks of 32 x 32 before each
+    Weight w[kWeights];
+    char *plain[kWeights], *turned[kWeights];   // in fragment order: [outputs, inputs] and its transpose
+    float *bias[kWeights];                      // in the rows' order
+    int first[kWeights + 1];                    // blocks of 32 x 32 before each
 };
 template <class DT>
 __global__ void __launch_bounds__(256)
 pack_kernel(Pack p) {
     __shared__ float tile[32][33];
     int j = 0;
-    while (j < 3 && (int)blockIdx.x >= p.first[j + 1]) ++j;
+    while (j < kWeights - 1 && (int)blockIdx.x >= p.first[j + 1]) ++j;
     const Weight &w = p.w[j];
     const int block = (int)blockIdx.x - p.first[j], cols = w.inputs / 32, o0 = block / cols * 32, i0 = block % cols * 32;
     {
@@ -271,7 +279,7 @@ pack_kernel(Pack p) {
         const f32x4 v = at < 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4 *>(w.w + at);
 #pragma unroll
         for (int k = 0; k < 4; ++k) tile[r][c + k] = v[k];
-        if (i0 == 0 && c == 0) p.bias[j][o0 + r] = w.b[w.row(o0 + r)];
+        if (w.b && i0 == 0 && c == 0) p.bias[j][o0 + r] = widen<DT>(Mma<DT>::pack(w.b[w.row(o0 + r)], 0.f)).x;     // autocast's
     }
     __syncthreads();
     const int half = threadIdx.x >> 7, t = threadIdx.x & 127, frag = t >> 6, lane = t & 63, n = lane & 15, g = lane >> 4;
@@ -280,7 +288,7 @@ pack_kernel(Pack p) {
 #pragma unroll
         for (int k = 0; k < 8; ++k) v[k] = tile[16 * frag + n][8 * g + k];
         *reinterpret_cast<u32x4 *>(p.plain[j] + ((int64_t)(o0 / 16 + frag) * (w.inputs / 32) + i0 / 32) * kFrag + lane * 16) = repack<DT>(v);
-    } else {
+    } else if (p.turned[j]) {
 #pragma unroll
         for (int k = 0; k < 8; ++k) v[k] = tile[8 * g + k][16 * frag + n];
         *reinterpret_cast<u32x4 *>(p.turned[j] + ((int64_t)(i0 / 16 + frag) * (w.outputs / 32) + o0 / 32) * kFrag + lane * 16) = repack<DT>(v);
@@ -304,6 +312,7 @@ struct Gemm {
     const float *bias, *sample_scale;      // one factor per sample of T rows, or NULL
     int inputs, outputs, M, T;
     uint32_t T_magic;
+    int late;                              // the sum is rounded before the bias is added (a product and an addition in torch)
 };
 // Phi(x) and x's density, the former by formula 7.1.26 of Abramowitz and Stegun as in gelu(); infinities come out as
 // x * Phi(x) gives them.
@@ -381,14 +390,10 @@ gemm_kernel(Gemm a, int col_blocks) {
             u32x2 h[NTW];
 #pragma unroll
             for (int j = 0; j < NTW; ++j) {
-                h[j] = narrow4<DT>(acc[j][i] + bias[j]);
+                h[j] = narrow4<DT>((a.late ? rounded<DT>(acc[j][i]) : acc[j][i]) + bias[j]);
                 f32x4 v = widen4<DT>(h[j]);                  // of the value that the backward sees
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float cdf, pdf;
-                    normal_of(v[r], cdf, pdf);
-                    v[r] *= cdf;
-                }
+                for (int r = 0; r < 4; ++r) v[r] = v[r] * 0.5f * (1.f + erff(v[r] * 0.70710678118654752f));
                 o[j] = narrow4<DT>(v);
             }
             store_tile<16 * NTW, 0>(make_rsrc(a.out2 + m0 * pitch, rows * pitch), row_byte, h, g, 32 * NTW);
@@ -396,9 +401,10 @@ gemm_kernel(Gemm a, int col_blocks) {
 #pragma unroll
             for (int j = 0; j < NTW; ++j) {
                 f32x4 v = acc[j][i];
-                if constexpr (END == kBias) v += bias[j];
-                if constexpr (END == kResidual) v = aux[j] + f * (v + bias[j]);
+                if constexpr (END == kBias) v = (a.late ? rounded<DT>(v) : v) + bias[j];
+                if constexpr (END == kResidual) v = aux[j] + rounded<DT>(f * rounded<DT>((a.late ? rounded<DT>(v) : v) + bias[j]));
                 if constexpr (END == kGeluBack) {
+                    v = rounded<DT>(v);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         float cdf, pdf;
@@ -427,8 +433,35 @@ scale_kernel(char *__restrict__ out, const char *__restrict__ x, const float *__
     }
 }
 
+// out[t, :] = sum over the samples of x[n, t, :]: 32 units of eight channels to a workgroup, a sample to each of its eight lanes.
+template <class DT>
+__global__ void __launch_bounds__(256)
+sum_samples_kernel(char *__restrict__ out, const char *__restrict__ x, int N, int64_t units) {
+    __shared__ float part[8][32][9];
+    const int k = threadIdx.x & 31, lane = threadIdx.x >> 5;
+    const int64_t u = (int64_t)blockIdx.x * 32 + k;
+    float s[8] = {};
+    if (u < units)
+#pragma unroll 4
+        for (int n = lane; n < N; n += 8) {
+            float v[8];
+            unpack<DT>(*reinterpret_cast<const u32x4 *>(x + (n * units + u) * 16), v);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s[i] += v[i];
+        }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) part[lane][k][i] = s[i];
+    __syncthreads();
+    if (lane || u >= units) return;
+#pragma unroll
+    for (int l = 1; l < 8; ++l)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s[i] += part[l][k][i];
+    *reinterpret_cast<u32x4 *>(out + u * 16) = repack<DT>(s);
+}
+
 // =============================================================================
-// Weight gradients of the layer's four projections in one launch
+// Weight gradients of the layer's projections in one launch
 // =============================================================================
 // dW[o, i] = sum over rows of dY[m, o] X[m, i], db[o] = sum of dY[m, o].  The contraction runs along the rows of both
 // operands, so both come out of LDS transposed (ds_read_b64_tr_b16).  A workgroup computes a 128 x 128 block of one dW
@@ -439,14 +472,14 @@ scale_kernel(char *__restrict__ out, const char *__restrict__ x, const float *__
 constexpr int kGradTile = 128, kGradRows = 64;
 struct GradJob {
     const char *dy, *x;
-    int outputs, inputs, first;          // first: blocks of 128 x 128 before
+    int outputs, inputs, M, first;       // M: rows; first: blocks of 128 x 128 before
     int64_t part;                        // floats before: dW, then db
 };
 struct Grads {
-    GradJob job[4];
+    GradJob job[kWeights];
     float *partial;
     int64_t stride;                      // floats of one range
-    int M, rows, blocks;                 // rows of a range (a multiple of 64)
+    int rows, blocks;                    // rows of a range (a multiple of 64)
 };
 template <class DT>
 __global__ void __launch_bounds__(kThreads, 2)
@@ -459,11 +492,11 @@ grad_kernel(Grads a) {
     const uint32_t item = xcd_item(blockIdx.x, gridDim.x);     // the blocks of a range read the same rows
     const int split = (int)(item / (uint32_t)a.blocks), block = (int)item - split * a.blocks;
     int jn = 0;
-    while (jn < 3 && block >= a.job[jn + 1].first) ++jn;
+    while (jn < kWeights - 1 && block >= a.job[jn + 1].first) ++jn;
     const GradJob &job = a.job[jn];
     const int cols = job.inputs / kGradTile, o0 = (block - job.first) / cols * kGradTile, i0 = (block - job.first) % cols * kGradTile;
     const int64_t m0 = (int64_t)split * a.rows;
-    const int rows = (int)min((int64_t)a.rows, a.M - m0), pieces = (rows + kGradRows - 1) / kGradRows;
+    const int rows = (int)max((int64_t)0, min((int64_t)a.rows, job.M - m0)), pieces = (rows + kGradRows - 1) / kGradRows;
     const int y_pitch = 2 * job.outputs, x_pitch = 2 * job.inputs;
     const Rsrc ys = make_rsrc(job.dy + m0 * y_pitch, rows * y_pitch), xs = make_rsrc(job.x + m0 * x_pitch, rows * x_pitch);
     const int wo = wave & 1, wi = wave >> 1;
@@ -490,7 +523,7 @@ grad_kernel(Grads a) {
     clear(acc);
 #pragma unroll
     for (int t = 0; t < 4; ++t) db[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    stage(0);
+    if (pieces) stage(0);                                      // a projection of few rows has ranges without any: zeros
 #pragma unroll 1
     for (int p = 0; p < pieces; ++p) {
         wait_direct();
@@ -526,8 +559,8 @@ grad_kernel(Grads a) {
     }
 }
 struct Fold {
-    Weight w[4];
-    int64_t part[5];                     // floats before each projection's dW
+    Weight w[kWeights];
+    int64_t part[kWeights + 1];          // floats before each projection's dW
     const float *partial;
     int64_t stride;
     int splits;
@@ -535,9 +568,9 @@ struct Fold {
 __global__ void __launch_bounds__(256)
 grad_fold_kernel(Fold a) {
     const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (e >= a.part[4]) return;
+    if (e >= a.part[kWeights]) return;
     int j = 0;
-    while (j < 3 && e >= a.part[j + 1]) ++j;
+    while (j < kWeights - 1 && e >= a.part[j + 1]) ++j;
     const Weight &w = a.w[j];
     const int64_t k = e - a.part[j], nw = (int64_t)w.outputs * w.inputs;
     const int r = (int)(k / w.inputs), i = (int)(k - (int64_t)r * w.inputs);
@@ -548,7 +581,7 @@ grad_fold_kernel(Fold a) {
     for (int p = 1; p < a.splits; ++p) s += *reinterpret_cast<const f32x4 *>(a.partial + p * a.stride + e);
     if (k < nw) {
         *reinterpret_cast<f32x4 *>(w.dw + at) = s;
-    } else {
+    } else if (w.db) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) w.db[w.row((int)(k - nw) + q)] = s[q];
     }
@@ -556,7 +589,7 @@ grad_fold_kernel(Fold a) {
 
 // ----------------------------------------------------------------------------- the layer
 inline Weight weight_of(const na1d_train_layer &l, int j) {
-    const int C = l.dim, outputs[4] = {3 * C, C, l.hidden, C}, inputs[4] = {C, C, C, l.hidden};
+    const int C = l.dim, outputs[kWeights] = {3 * C, C, l.hidden, C, l.window ? 0 : C}, inputs[kWeights] = {C, C, C, l.hidden, C};
     return Weight{l.w[j], l.b[j], l.dw[j], l.db[j], outputs[j], inputs[j], l.groups, j == 0 && l.ordered};
 }
 struct Buffers {
@@ -582,10 +615,10 @@ struct Saved : Buffers {
     }
 };
 struct ForwardScratch : Buffers {
-    int64_t part, plain[4], bias[4];
-    explicit ForwardScratch(const na1d_train_layer &l) {
-        part = take((int64_t)2 * kBnChunks * l.dim * 4);
-        for (int j = 0; j < 4; ++j) {
+    int64_t plain[kWeights], bias[kWeights], pos;
+    ForwardScratch(const na1d_train_layer &l, int64_t T) {
+        pos = take(l.window ? 0 : T * l.dim * 2);
+        for (int j = 0; j < kWeights; ++j) {
             const Weight w = weight_of(l, j);
             plain[j] = take((int64_t)w.outputs * w.inputs * 2);
             bias[j] = take(w.outputs * 4);
@@ -593,10 +626,10 @@ struct ForwardScratch : Buffers {
     }
 };
 struct GradPlan {
-    int blocks = 0, splits, rows, first[4];
-    int64_t part[5] = {};
+    int blocks = 0, splits, rows, first[kWeights];
+    int64_t part[kWeights + 1] = {};
     GradPlan(const na1d_train_layer &l, int64_t M) {
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < kWeights; ++j) {
             const Weight w = weight_of(l, j);
             first[j] = blocks;
             blocks += (w.outputs / kGradTile) * (w.inputs / kGradTile);
@@ -610,13 +643,14 @@ struct GradPlan {
     }
 };
 struct BackwardScratch : Buffers {
-    int64_t dz, dh, dy, dx1, ds, dattn, dqkv, part, grads;
+    int64_t dz, dh, dy, dx1, ds, dattn, dqkv, part, grads, delta, dpos;
     BackwardScratch(const na1d_train_layer &l, int64_t N, int64_t T) {
         const int64_t M = N * T, row = M * l.dim * 2;
         const GradPlan p(l, M);
         dz = take(l.scale_mlp ? row : 0), dh = take(M * l.hidden * 2), dy = take(row), dx1 = take(row), ds = take(l.scale_attn ? row : 0);
         dattn = take(row), dqkv = take(3 * row), part = take((int64_t)2 * kBnChunks * l.dim * 4);
-        grads = take(p.splits * p.part[4] * 4);
+        grads = take(p.splits * p.part[kWeights] * 4);
+        delta = take(l.window ? 0 : M * l.heads * 4), dpos = take(l.window ? 0 : T * l.dim * 2);
     }
 };
 
@@ -648,22 +682,22 @@ template <class DT> int scale_rows(char *out, const char *x, const float *f, int
 inline Geom attention_geom(const na1d_train_layer &l, int64_t N, int64_t T, Layout &in, Layout &out) {
     Geom g;
     const int64_t C = l.dim;
-    g.B = N * l.heads, g.T = T, g.H = l.heads, g.C = l.dim / l.heads, g.W = l.window, g.L = l.left;
+    g.B = N * l.heads, g.T = T, g.H = l.heads, g.C = l.dim / l.heads, g.W = l.window ? l.window : 1, g.L = l.window ? l.left : 0;
     in = Layout{T * 3 * C, g.C, 3 * C}, out = Layout{T * C, g.C, C};
-    set_dilation(g, l.dilation);
+    if (l.window) set_dilation(g, l.dilation);
     in.row *= g.dilation, out.row *= g.dilation;
     return g;
 }
 
-template <class DT> int norm_forward(const na1d_train_layer &l, int which, char *y, const char *x, float *mean, float *rstd, float *part, int64_t M, hipStream_t s) {
+template <class DT> int norm_apply(const na1d_train_layer &l, int which, char *y, const char *x, float *mean, float *rstd, int64_t M, const char *add, int64_t T, hipStream_t s) {
     const Chunks c = bn_chunks(M);
-    const dim3 grid((unsigned)(l.dim / kBnCols), (unsigned)c.count);
-    float *part_m2 = part + (int64_t)kBnChunks * l.dim;
-    bn_stats_kernel<DT><<<grid, kBnThreads, 0, s>>>(part, part_m2, x, (int)M, l.dim, c.rows);
-    NA1D_TRY(launch_status());
     const na1d_train_norm &n = l.norm[which];
-    bn_apply_kernel<DT><<<grid, kBnThreads, 0, s>>>(BnApply{y, x, part, part_m2, n.weight, n.bias, mean, rstd, n.running_mean, n.running_var, n.batches,
-                                                            n.eps, n.momentum, (int)M, l.dim, c.rows, c.count});
+    bn_apply_kernel<DT><<<dim3((unsigned)(l.dim / kBnCols), (unsigned)c.count), kBnThreads, 0, s>>>(
+        BnApply{y, x, n.batch_mean, n.batch_var, n.weight, n.bias, mean, rstd, n.batches, n.eps, (int)M, l.dim, c.rows, add, (int)T});
+    return launch_status();
+}
+int to_channels(const na1d_train_layer &l, void *out, const void *x, int64_t N, int64_t T, hipStream_t s) {
+    to_channels_kernel<<<dim3((unsigned)((T + 63) / 64), (unsigned)(l.dim / 64), (unsigned)N), 256, 0, s>>>((uint16_t *)out, (const char *)x, (int)T, l.dim);
     return launch_status();
 }
 template <class DT>
@@ -679,45 +713,56 @@ int norm_backward(const na1d_train_layer &l, int which, char *dx, const char *dy
     return launch_status();
 }
 
-template <class DT> int forward(const na1d_train_layer &l, char *out, const char *x, char *saved, char *ws, int64_t N, int64_t T, hipStream_t s) {
+// part 0: up to x1, which also goes to `out` as [N, dim, T]; part 1: from x1 and its statistics on
+template <class DT> int forward(const na1d_train_layer &l, int half, char *out, const char *x, char *saved, char *ws, int64_t N, int64_t T, hipStream_t s) {
     const int64_t M = N * T;
     const Saved o(l, N, T);
-    const ForwardScratch f(l);
+    const ForwardScratch f(l, T);
     auto stat = [&](int i) { return reinterpret_cast<float *>(saved + o.stats[i]); };
     Pack p{};
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < kWeights; ++j) {
         p.w[j] = weight_of(l, j);
-        p.plain[j] = ws + f.plain[j], p.turned[j] = saved + o.turned[j], p.bias[j] = reinterpret_cast<float *>(ws + f.bias[j]);
+        p.plain[j] = ws + f.plain[j], p.turned[j] = j < 4 ? saved + o.turned[j] : nullptr, p.bias[j] = reinterpret_cast<float *>(ws + f.bias[j]);
         p.first[j + 1] = p.first[j] + p.w[j].outputs / 32 * (p.w[j].inputs / 32);
     }
-    pack_kernel<DT><<<(unsigned)p.first[4], 256, 0, s>>>(p);
-    NA1D_TRY(launch_status());
-    float *part = reinterpret_cast<float *>(ws + f.part);
     Gemm a{};
     a.M = (int)M, a.T = (int)T, a.T_magic = div_magic(T);
     auto product = [&](int j, const char *in, char *to) {
         a.x = in, a.w = p.plain[j], a.bias = p.bias[j], a.out = to, a.inputs = p.w[j].inputs, a.outputs = p.w[j].outputs;
+        a.late = l.ordered || j % 2 == 0;
     };
-    NA1D_TRY(norm_forward<DT>(l, 0, saved + o.y1, x, stat(0), stat(1), part, M, s));
+    if (half) {
+        NA1D_TRY(norm_apply<DT>(l, 1, saved + o.y2, saved + o.x1, stat(2), stat(3), M, nullptr, T, s));
+        product(2, saved + o.y2, saved + o.g);
+        a.out2 = saved + o.h;
+        NA1D_TRY(launch_gemm<DT, kGelu>(a, s));
+        product(3, saved + o.g, out);
+        a.aux = saved + o.x1, a.sample_scale = l.scale_mlp;
+        return launch_gemm<DT, kResidual>(a, s);
+    }
+    pack_kernel<DT><<<(unsigned)p.first[kWeights], 256, 0, s>>>(p);
+    NA1D_TRY(launch_status());
+    if (!l.window) {
+        a.M = (int)T;
+        product(4, (const char *)l.pos, ws + f.pos);
+        NA1D_TRY(launch_gemm<DT, kStore>(a, s));
+        a.M = (int)M;
+    }
+    NA1D_TRY(norm_apply<DT>(l, 0, saved + o.y1, x, stat(0), stat(1), M, l.window ? nullptr : ws + f.pos, T, s));
     product(0, saved + o.y1, saved + o.qkv);
     NA1D_TRY(launch_gemm<DT, kBias>(a, s));
     Layout in, outl;
     const Geom g = attention_geom(l, N, T, in, outl);
     const char *q = saved + o.qkv, *k = q + 2 * l.dim, *v = k + 2 * l.dim;
     float *lse = reinterpret_cast<float *>(saved + o.lse);
-    int st = fused_fwd(saved + o.attn, lse, q, k, v, l.rpb, nullptr, g, in, outl, l.scale, DT::tag, s);
-    if (st == NA1D_ERR_UNSUPPORTED) st = wide_fwd(saved + o.attn, lse, q, k, v, l.rpb, nullptr, g, in, outl, l.scale, DT::tag, s);
+    int st = !l.window ? global_fwd(saved + o.attn, lse, q, k, v, nullptr, g, in, outl, l.scale, DT::tag, s)
+                       : fused_fwd(saved + o.attn, lse, q, k, v, l.rpb, nullptr, g, in, outl, l.scale, DT::tag, s);
+    if (st == NA1D_ERR_UNSUPPORTED && l.window) st = wide_fwd(saved + o.attn, lse, q, k, v, l.rpb, nullptr, g, in, outl, l.scale, DT::tag, s);
     NA1D_TRY(st);
     product(1, saved + o.attn, saved + o.x1);
     a.aux = x, a.sample_scale = l.scale_attn;
     NA1D_TRY(launch_gemm<DT, kResidual>(a, s));
-    NA1D_TRY(norm_forward<DT>(l, 1, saved + o.y2, saved + o.x1, stat(2), stat(3), part, M, s));
-    product(2, saved + o.y2, saved + o.g);
-    a.out2 = saved + o.h;
-    NA1D_TRY(launch_gemm<DT, kGelu>(a, s));
-    product(3, saved + o.g, out);
-    a.aux = saved + o.x1, a.sample_scale = l.scale_mlp;
-    return launch_gemm<DT, kResidual>(a, s);
+    return to_channels(l, out, saved + o.x1, N, T, s);
 }
 
 template <class DT>
@@ -757,32 +802,40 @@ int backward(const na1d_train_layer &l, char *dx, const char *dout, const char *
     const char *q = saved + o.qkv;
     char *dq = ws + b.dqkv;
     const float *lse = reinterpret_cast<const float *>(saved + o.lse);
-    int st = fused_bwd(dq, dq + step, dq + 2 * step, l.drpb, q, q + step, q + 2 * step, nullptr, ws + b.dattn, lse, l.rpb, nullptr, g, in, outl, l.scale, DT::tag,
+    int st = !l.window ? global_bwd(dq, dq + step, dq + 2 * step, reinterpret_cast<float *>(ws + b.delta), q, q + step, q + 2 * step, saved + o.attn, ws + b.dattn,
+                                    lse, nullptr, g, in, outl, l.scale, DT::tag, s)
+                       : fused_bwd(dq, dq + step, dq + 2 * step, l.drpb, q, q + step, q + 2 * step, nullptr, ws + b.dattn, lse, l.rpb, nullptr, g, in, outl, l.scale, DT::tag,
                        nullptr, 0, s);
-    if (st == NA1D_ERR_UNSUPPORTED)
+    if (st == NA1D_ERR_UNSUPPORTED && l.window)
         st = wide_bwd(dq, dq + step, dq + 2 * step, l.drpb, q, q + step, q + 2 * step, ws + b.dattn, lse, l.rpb, nullptr, g, in, outl, l.scale, DT::tag, nullptr, 0, s);
     NA1D_TRY(st);
     turned(0, ws + b.dqkv, ws + b.dy);
     NA1D_TRY(launch_gemm<DT, kStore>(a, s));
     NA1D_TRY(norm_backward<DT>(l, 0, dx, ws + b.dy, x, ws + b.dx1, stat(0), stat(1), part, M, s));
+    if (!l.window) {
+        const int64_t units = T * l.dim / 8;
+        sum_samples_kernel<DT><<<(unsigned)((units + 31) / 32), 256, 0, s>>>(ws + b.dpos, ws + b.dy, (int)N, units);
+        NA1D_TRY(launch_status());
+    }
     const GradPlan plan(l, M);
     Grads ga{};
     Fold fo{};
-    const char *dys[4] = {ws + b.dqkv, ds, ws + b.dh, dz}, *xs[4] = {saved + o.y1, saved + o.attn, saved + o.y2, saved + o.g};
-    for (int j = 0; j < 4; ++j) {
+    const char *dys[kWeights] = {ws + b.dqkv, ds, ws + b.dh, dz, ws + b.dpos};
+    const char *xs[kWeights] = {saved + o.y1, saved + o.attn, saved + o.y2, saved + o.g, (const char *)l.pos};
+    for (int j = 0; j < kWeights; ++j) {
         fo.w[j] = weight_of(l, j);
-        ga.job[j] = GradJob{dys[j], xs[j], fo.w[j].outputs, fo.w[j].inputs, plan.first[j], plan.part[j]};
+        ga.job[j] = GradJob{dys[j], xs[j], fo.w[j].outputs, fo.w[j].inputs, (int)(j < 4 ? M : T), plan.first[j], plan.part[j]};
         fo.part[j + 1] = plan.part[j + 1];
     }
     ga.partial = reinterpret_cast<float *>(ws + b.grads);
-    ga.stride = fo.stride = plan.part[4];
-    ga.M = (int)M, ga.rows = plan.rows, ga.blocks = plan.blocks;
+    ga.stride = fo.stride = plan.part[kWeights];
+    ga.rows = plan.rows, ga.blocks = plan.blocks;
     fo.partial = ga.partial, fo.splits = plan.splits;
     const size_t lds = (size_t)4 * kGradRows * kGradTile * 2;
     if (!allow_lds(grad_kernel<DT>, lds)) return NA1D_ERR_LAUNCH;
     grad_kernel<DT><<<(unsigned)(plan.blocks * plan.splits), kThreads, lds, s>>>(ga);
     NA1D_TRY(launch_status());
-    grad_fold_kernel<<<(unsigned)((plan.part[4] / 4 + 255) / 256), 256, 0, s>>>(fo);
+    grad_fold_kernel<<<(unsigned)((plan.part[kWeights] / 4 + 255) / 256), 256, 0, s>>>(fo);
     return launch_status();
 }
 
@@ -790,7 +843,7 @@ bool layer_ok(const na1d_train_layer &l, int64_t N, int64_t T) {
     if (l.dim < 256 || l.dim % 256 || l.dim > 2048 || l.hidden < 256 || l.hidden % 256 || l.hidden > 8192) return false;
     if (l.heads < 1 || l.dim % l.heads || l.dim / l.heads % 8 || l.dim / l.heads > 128) return false;
     if (l.groups < 1 || l.dim % l.groups || l.dim / l.groups % 32 || l.hidden % l.groups || l.hidden / l.groups % 32) return false;
-    if (l.window < 1 || l.window > NA1D_MAX_WINDOW || l.left < 0 || l.left >= l.window || l.dilation < 1) return false;
+    if (l.window < 0 || l.window > NA1D_MAX_WINDOW || (l.window && (l.left < 0 || l.left >= l.window)) || l.dilation < 1 || (!l.window && l.dilation > 1)) return false;
     // offsets inside an utterance, and what the attention kernels' launches count, stay in the reach of 32 bits
     if (N < 1 || T < 1 || N > (1 << 20) || T > (1 << 16) || N * T > (1 << 20)) return false;
     const int64_t M = N * T, most = 1ll << 31;
@@ -800,11 +853,11 @@ bool layer_ok(const na1d_train_layer &l, int64_t N, int64_t T) {
 }
 int64_t saved_bytes(const na1d_train_layer &l, int64_t N, int64_t T) { return Saved(l, N, T).bytes; }
 int64_t scratch_bytes(const na1d_train_layer &l, int64_t N, int64_t T, bool backward) {
-    return backward ? BackwardScratch(l, N, T).bytes : ForwardScratch(l).bytes;
+    return backward ? BackwardScratch(l, N, T).bytes : ForwardScratch(l, T).bytes;
 }
-int run_forward(const na1d_train_layer &l, void *out, const void *x, void *saved, void *ws, int64_t N, int64_t T, hipStream_t s) {
-    return l.dtype == NA1D_BF16 ? forward<BF16>(l, (char *)out, (const char *)x, (char *)saved, (char *)ws, N, T, s)
-                                : forward<FP16>(l, (char *)out, (const char *)x, (char *)saved, (char *)ws, N, T, s);
+int run_forward(const na1d_train_layer &l, int half, void *out, const void *x, void *saved, void *ws, int64_t N, int64_t T, hipStream_t s) {
+    return l.dtype == NA1D_BF16 ? forward<BF16>(l, half, (char *)out, (const char *)x, (char *)saved, (char *)ws, N, T, s)
+                                : forward<FP16>(l, half, (char *)out, (const char *)x, (char *)saved, (char *)ws, N, T, s);
 }
 int run_backward(const na1d_train_layer &l, void *dx, const void *dout, const void *x, const void *saved, void *ws, int64_t N, int64_t T, hipStream_t s) {
     return l.dtype == NA1D_BF16 ? backward<BF16>(l, (char *)dx, (const char *)dout, (const char *)x, (const char *)saved, (char *)ws, N, T, s)

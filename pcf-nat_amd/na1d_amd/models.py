@@ -536,7 +536,7 @@ class NATFLayer(nn.Module):
 
     def forward(self, x, padding=None, pos_emb=None, attn_mask_global=None):
         if self.training:
-            out = train_layer(self, x)                  # one autograd node, native both ways
+            out = train_layer(self, x, pos_emb, attn_mask_global)                  # one autograd node, native both ways
             if out is not None:
                 return out
         y = self.norm1(x)

@@ -1,4 +1,4 @@
-"""A windowed encoder layer in training as one autograd node (``na1d_train_layer_*`` of the C ABI).
+"""An encoder layer in training as one autograd node (``na1d_train_layer_*`` of the C ABI).
 
 :func:`layer` runs norm -> attention -> residual -> norm -> MLP -> residual of ``models.NATFLayer`` and its backward
 through the kernels of ``csrc/na1d_train.hip``, all launched from native code: the parameters, buffers, random draws and
@@ -19,13 +19,13 @@ _P, _I, _F = ctypes.c_void_p, ctypes.c_int32, ctypes.c_float
 
 
 class _Norm(ctypes.Structure):                     # na1d_train_norm
-    _fields_ = [(n, _P) for n in "weight bias running_mean running_var batches dweight dbias".split()] + [("eps", _F), ("momentum", _F)]
+    _fields_ = [(n, _P) for n in "weight bias batch_mean batch_var batches dweight dbias".split()] + [("eps", _F)]
 
 
 class _Layer(ctypes.Structure):                    # na1d_train_layer
     _fields_ = ([(n, _I) for n in "dtype dim hidden heads window left dilation groups ordered".split()] + [("scale", _F)]
-                + [("norm", _Norm * 2)] + [(n, _P * 4) for n in "w b dw db".split()]
-                + [(n, _P) for n in "rpb drpb scale_attn scale_mlp".split()])
+                + [("norm", _Norm * 2)] + [(n, _P * 5) for n in "w b dw db".split()]
+                + [(n, _P) for n in "rpb drpb pos scale_attn scale_mlp".split()])
 
 
 def _ptr(t):
@@ -33,50 +33,57 @@ def _ptr(t):
 
 
 def _ptrs(ts):
-    return (_P * 4)(*(t.data_ptr() for t in ts))
+    return (_P * 5)(*map(_ptr, ts))
 
 
 class _TrainLayer(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, geom, norms, scales, rpb, n1w, n1b, n2w, n2b, wq, bq, wp, bp, w1, b1, w2, b2):
+    def forward(ctx, x, by_channel, geom, norms, scales, pos, extra, n1w, n1b, n2w, n2b, wq, bq, wp, bp, w1, b1, w2, b2):
         lib = _lib.load()
         n, t, dim = x.shape
-        weights, biases = (wq, wp, w1, w2), (bq, bp, b1, b2)
+        dense = pos is not None                     # extra: linear_pos' weight, or the bias of a window's scores
+        weights, biases = (wq, wp, w1, w2, extra if dense else None), (bq, bp, b1, b2)
         c = _Layer(*geom)
         c.w, c.b = _ptrs(weights), _ptrs(biases)
         for to, bn, w, b in zip(c.norm, norms, (n1w, n2w), (n1b, n2b)):
-            to.weight, to.bias, to.eps, to.momentum = w.data_ptr(), b.data_ptr(), bn.eps, bn.momentum
-            to.running_mean, to.running_var, to.batches = bn.running_mean.data_ptr(), bn.running_var.data_ptr(), bn.num_batches_tracked.data_ptr()
-        c.rpb, c.scale_attn, c.scale_mlp = rpb.data_ptr(), _ptr(scales[0]), _ptr(scales[1])
+            to.weight, to.bias, to.eps, to.batches = w.data_ptr(), b.data_ptr(), bn.eps, bn.num_batches_tracked.data_ptr()
+        c.rpb, c.pos, c.scale_attn, c.scale_mlp = None if dense else extra.data_ptr(), _ptr(pos), _ptr(scales[0]), _ptr(scales[1])
         ref = ctypes.byref(c)
         out = torch.empty_like(x)
         with torch.cuda.device(x.device):
+            stream = torch.cuda.current_stream().cuda_stream
             sizes = lib.na1d_train_layer_saved_bytes(ref, n, t), lib.na1d_train_layer_workspace_bytes(ref, n, t, 0)
             _lib.check(min(*sizes, 0), "na1d_train_layer_saved_bytes")
             saved, ws = (torch.empty(s, dtype=torch.uint8, device=x.device) for s in sizes)
-            _lib.check(lib.na1d_train_layer_forward(ref, out.data_ptr(), x.data_ptr(), saved.data_ptr(), sizes[0], ws.data_ptr(),
-                                                    sizes[1], n, t, torch.cuda.current_stream().cuda_stream),
-                       "na1d_train_layer_forward")
+            if by_channel is None:
+                by_channel = x.new_empty((n, dim, t))
+                _lib.check(lib.na1d_train_to_channels(ref, by_channel.data_ptr(), x.data_ptr(), n, t, stream), "na1d_train_to_channels")
+            x1 = x.new_empty((n, dim, t))
+            for part, (of, to) in enumerate(((by_channel, x1), (x1, out))):
+                stats = torch.batch_norm_update_stats(of, norms[part].running_mean, norms[part].running_var, norms[part].momentum)
+                c.norm[part].batch_mean, c.norm[part].batch_var = map(_ptr, stats)
+                _lib.check(lib.na1d_train_layer_forward(ref, part, to.data_ptr(), x.data_ptr(), saved.data_ptr(), sizes[0], ws.data_ptr(),
+                                                        sizes[1], n, t, stream), "na1d_train_layer_forward")
         increment_version([b for bn in norms for b in (bn.running_mean, bn.running_var, bn.num_batches_tracked)])
-        ctx.save_for_backward(x, saved, rpb, n1w, n2w, *scales)
-        ctx.geom, ctx.shapes = geom, [p.shape for p in (rpb, n1w, n1b, n2w, n2b, wq, bq, wp, bp, w1, b1, w2, b2)]
+        ctx.save_for_backward(x, saved, pos, None if dense else extra, n1w, n2w, *scales)
+        ctx.geom, ctx.shapes = geom, [p.shape for p in (extra, n1w, n1b, n2w, n2b, wq, bq, wp, bp, w1, b1, w2, b2)]
         return out
 
     @staticmethod
     @once_differentiable
     def backward(ctx, dout):
         lib = _lib.load()
-        x, saved, rpb, n1w, n2w, *scales = ctx.saved_tensors
+        x, saved, pos, rpb, n1w, n2w, *scales = ctx.saved_tensors
         n, t, dim = x.shape
         dout = dout.contiguous()
         dx = torch.empty_like(x)
         grads = [torch.zeros(ctx.shapes[0], dtype=torch.float32, device=x.device)]       # the bias of the scores is added to
         grads += [torch.empty(s, dtype=torch.float32, device=x.device) for s in ctx.shapes[1:]]
         c = _Layer(*ctx.geom)
-        c.dw, c.db = _ptrs(grads[5::2]), _ptrs(grads[6::2])
+        c.dw, c.db = _ptrs(grads[5::2] + ([] if pos is None else grads[:1])), _ptrs(grads[6::2])
         for to, w, dw, db in zip(c.norm, (n1w, n2w), grads[1:5:2], grads[2:5:2]):
             to.weight, to.dweight, to.dbias = w.data_ptr(), dw.data_ptr(), db.data_ptr()
-        c.rpb, c.drpb, c.scale_attn, c.scale_mlp = rpb.data_ptr(), grads[0].data_ptr(), _ptr(scales[0]), _ptr(scales[1])
+        c.rpb, c.drpb, c.pos, c.scale_attn, c.scale_mlp = _ptr(rpb), grads[0].data_ptr(), _ptr(pos), _ptr(scales[0]), _ptr(scales[1])
         ref = ctypes.byref(c)
         with torch.cuda.device(x.device):
             nbytes = lib.na1d_train_layer_workspace_bytes(ref, n, t, 1)
@@ -85,7 +92,7 @@ class _TrainLayer(torch.autograd.Function):
             _lib.check(lib.na1d_train_layer_backward(ref, dx.data_ptr(), dout.data_ptr(), x.data_ptr(), saved.data_ptr(), saved.numel(),
                                                      ws.data_ptr(), nbytes, n, t, torch.cuda.current_stream().cuda_stream),
                        "na1d_train_layer_backward")
-        return (dx, None, None, None, *(g if need else None for g, need in zip(grads, ctx.needs_input_grad[4:])))
+        return (dx, None, None, None, None, None, *(g if need else None for g, need in zip(grads, ctx.needs_input_grad[6:])))
 
 
 def plain(m, *classes):
@@ -115,30 +122,37 @@ def _drop_path_scale(m, x):
     return mask.float().view(-1).div_(keep)
 
 
-def layer(m, x):
+def layer(m, x, pos_emb=None, attn_mask_global=None):
     """``models.NATFLayer`` ``m`` in training on ``x`` ([N, T, C], or [N, C, T] for channels-first models), or ``None`` where
     the kernels or their one autograd node would not be the same as the modules."""
     from . import models as M
-    if not (x.is_cuda and m.training and m.local and torch.is_grad_enabled() and torch.is_autocast_enabled("cuda")
+    if not (x.is_cuda and m.training and torch.is_grad_enabled() and torch.is_autocast_enabled("cuda")
             and x.dim() == 3 and x.dtype in (torch.bfloat16, torch.float16) and x.dtype == torch.get_autocast_dtype("cuda")):
         return None
     a, mlp = m.attn, m.mlp
     cf = getattr(a, "channels_first", False)
     linear, norm = (M.Conv1x1, M.BatchNorm1d) if cf else (M.TokenLinear, M.TokenBatchNorm)
-    if not (plain_call(x) and plain(a, M.NAttention) and plain(mlp, M.Mlp) and plain(m.norm1, norm) and plain(m.norm2, norm)
+    if not (plain_call(x) and plain(a, M.NAttention if m.local else M.GlobalAttention) and plain(mlp, M.Mlp) and plain(m.norm1, norm) and plain(m.norm2, norm)
             and plain(m.drop_path, nn.Identity, M.DropPath) and plain(mlp.act, nn.GELU) and mlp.act.approximate == "none"
             and plain(mlp.drop, nn.Dropout) and plain(a.proj_drop, nn.Dropout)
             and all(plain(p, linear) for p in (a.qkv, a.proj, mlp.fc1, mlp.fc2))):
         return None
     norms = (m.norm1, m.norm2) if cf else (m.norm1.norm, m.norm2.norm)
-    if a.na != "fused_qkv" or a.attn_drop or not a.training or a.proj_drop.p or mlp.drop.p or (not cf and not all(plain(b, M.BatchNorm1d) for b in norms)):
+    if (a.na != "fused_qkv" if m.local else a.dense != "native") or a.attn_drop or not a.training or a.proj_drop.p or mlp.drop.p or (not cf and not all(plain(b, M.BatchNorm1d) for b in norms)):
         return None
     xt = x.transpose(1, 2) if cf else x
     n, t, dim = xt.shape
-    if dim != a.dim or t != a.attn_mask.shape[-2] or not all(_norm_fits(b, dim) for b in norms):
+    if (t != a.attn_mask.shape[-2] if m.local else attn_mask_global is not None) or not all(_norm_fits(b, dim) for b in norms):
         return None
-    groups = {getattr(p, "groups", 1) for p in (a.qkv, a.proj, mlp.fc1, mlp.fc2)}
-    params = (a.relative_position_bias, norms[0].weight, norms[0].bias, norms[1].weight, norms[1].bias, a.qkv.weight, a.qkv.bias,
+    projections = [a.qkv, a.proj, mlp.fc1, mlp.fc2]
+    pos = None
+    if not m.local:
+        if (pos_emb is None or type(pos_emb) is not torch.Tensor or pos_emb.requires_grad or pos_emb.device != x.device
+                or pos_emb.shape != ((1, dim, t) if cf else (1, t, dim)) or not plain(a.linear_pos, linear) or a.linear_pos.bias is not None):
+            return None
+        projections.append(a.linear_pos)
+    groups = {getattr(p, "groups", 1) for p in projections}
+    params = (a.relative_position_bias if m.local else a.linear_pos.weight, norms[0].weight, norms[0].bias, norms[1].weight, norms[1].bias, a.qkv.weight, a.qkv.bias,
               a.proj.weight, a.proj.bias, mlp.fc1.weight, mlp.fc1.bias, mlp.fc2.weight, mlp.fc2.bias)
     hidden = mlp.fc1.weight.shape[0]
     sizes = (3 * dim, dim, dim, dim, hidden, dim, dim, hidden)
@@ -148,11 +162,18 @@ def layer(m, x):
     groups = groups.pop()
     if any(p.numel() != o * i // groups for p, o, i in zip(params[5::2], sizes[::2], sizes[1::2])):
         return None
-    geom = (_lib.dtype_tag(x.dtype), dim, hidden, a.num_heads, a.win_size, a.left, a.dilation, groups, int(cf), a.scale)
+    if params[0].numel() != (a.num_heads * a.win_size if m.local else dim * dim // groups):
+        return None
+    window = (a.win_size, a.left, a.dilation) if m.local else (0, 0, 1)
+    geom = (_lib.dtype_tag(x.dtype), dim, hidden, a.num_heads, *window, groups, int(cf), a.scale)
     probe = _Layer(*geom)
     if _lib.load().na1d_train_layer_saved_bytes(ctypes.byref(probe), n, t) < 0:
         return None
+    by_channel = xt.detach().transpose(1, 2)
+    by_channel = by_channel if by_channel.is_contiguous() else None       # [N, C, T], the layout of the statistics, is there already
     xt = xt.contiguous()
+    if not m.local:
+        pos = (pos_emb.transpose(1, 2) if cf else pos_emb).to(x.dtype).contiguous()
     scales = (_drop_path_scale(m.drop_path, xt), _drop_path_scale(m.drop_path, xt))
-    out = _TrainLayer.apply(xt, geom, norms, scales, *params)
+    out = _TrainLayer.apply(xt, by_channel, geom, norms, scales, pos, *params)
     return out.transpose(1, 2) if cf else out

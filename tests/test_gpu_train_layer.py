@@ -35,22 +35,23 @@ def _layers(family, groups, heads, window, dilation, frames, drop_path, seed, di
             bn.weight.uniform_(0.5, 1.5)
             bn.bias.normal_(0, 0.3)
     gpu = copy.deepcopy(layer).cuda()
-    gpu.attn.na = "fused_qkv"
+    if window:
+        gpu.attn.na = "fused_qkv"
     return layer.train(), gpu.train()
 
 
-def _errors(cpu, gpu, x, g, dtype):
+def _errors(cpu, gpu, x, g, dtype, pos=None):
     """Relative errors of the native layer's output, gradients and running statistics against the fp32 module."""
     xg = x.cuda().to(dtype).requires_grad_(True)
     torch.manual_seed(5)
     with torch.autocast("cuda", dtype=dtype):
-        out = models.train_layer(gpu, xg)
+        out = models.train_layer(gpu, xg, None if pos is None else pos.cuda())
     assert out is not None, "not the native path"
     gd = g.cuda().to(dtype)
     out.backward(gd)
     torch.manual_seed(5)
     xc = x.to(dtype).float().requires_grad_(True)
-    want = cpu(xc)
+    want = cpu(xc, pos_emb=None if pos is None else pos.to(dtype).float())
     want.backward(gd.float().cpu())
     err = {"out": O.rel_l2(out.float(), want), "dx": O.rel_l2(xg.grad.float(), xc.grad)}
     for (name, p), q in zip(cpu.named_parameters(), gpu.parameters()):
@@ -68,7 +69,8 @@ def _errors(cpu, gpu, x, g, dtype):
 @pytest.mark.parametrize("batch,T", [(2, 5), (1, 33), (3, 50), (7, 101), (37, 100), (64, 260)])
 @pytest.mark.parametrize("dtype", ["bf16", "fp16"])
 @pytest.mark.parametrize("family,groups,heads,window,dilation", [
-    ("mfa", 1, 16, 27, 1), ("mfa", 1, 4, 65, 1), ("pcf", 8, 16, 27, 1), ("pcf", 4, 8, 9, 2), ("pcf", 2, 16, 27, 1), ("pcf", 1, 32, 5, 3)])
+    ("mfa", 1, 16, 27, 1), ("mfa", 1, 4, 65, 1), ("pcf", 8, 16, 27, 1), ("pcf", 4, 8, 9, 2), ("pcf", 2, 16, 27, 1), ("pcf", 1, 32, 5, 3),
+    ("mfa", 1, 4, 0, 1), ("mfa", 1, 16, 0, 1), ("pcf", 8, 4, 0, 1), ("pcf", 1, 2, 0, 1)])
 def test_native_training_layer(family, groups, heads, window, dilation, dtype, batch, T):
     """16-bit rounding of weights, activations and gradients passes through six products and two norms: single results
     are within a few units of eps (2^-9, 2^-12) in norm; a few rows leave the statistics of the gradients little to
@@ -79,12 +81,14 @@ def test_native_training_layer(family, groups, heads, window, dilation, dtype, b
     gen = torch.Generator().manual_seed(batch)
     shape = (batch, 256, T) if family == "pcf" else (batch, T, 256)
     x = torch.randn(shape, generator=gen) + 0.5 * torch.randn((1,) + tuple(256 if s == 256 else 1 for s in shape[1:]), generator=gen)
-    err = _errors(cpu, gpu, x, torch.randn(shape, generator=gen), DT[dtype])
+    pos = None if window else models.sinusoid_table(256, T, family == "pcf")
+    err = _errors(cpu, gpu, x, torch.randn(shape, generator=gen), DT[dtype], pos)
     print("errors", {k: "%.1e" % v for k, v in err.items()})
     eps = 2.0 ** -9 if dtype == "bf16" else 2.0 ** -12
     for name, e in err.items():
-        # running statistics: norm1's come of exact inputs, norm2's of values rounded twice (a unit of eps each, averaged)
-        bound = 1e-5 if "norm1" in name and "running" in name else 2 * eps if "running" in name else 4 * eps if name == "out" else 32 * eps
+        # running statistics: norm1's come of exact inputs; norm2's are means of the attention half's outputs, and of few
+        # rows no better than a single one
+        bound = 1e-5 if "norm1" in name and "running" in name else 4 * eps if "running" in name or name == "out" else 32 * eps
         assert e < bound, (name, e)
 
 
