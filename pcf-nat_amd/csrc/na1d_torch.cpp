@@ -1,0 +1,317 @@
+// The attention operators' autograd nodes for torch in C++: what fused.py, dense.py and nattn.py do per call, without the
+// interpreter.  A windowed layer's forward and backward at a training batch are 45 us of kernels; the same host path in
+// Python took 115 us (allocations, context managers, ctypes, and the engine's thread waiting for the interpreter lock).
+//
+// Every function here returns nothing (None) for calls it does not take as they are - other devices, types, layouts,
+// tensor subclasses, transforms, tracers, forward-mode gradients - and the Python implementation then serves or refuses
+// them as before.
+#include <torch/extension.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/DeviceGuard.h>
+
+#include "na1d.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+using MaybeTensor = std::optional<Tensor>;
+
+void check(int status, const char *name) {
+    if (status != NA1D_OK) throw std::runtime_error(std::string(name) + " failed: " + na1d_status_string(status) + " (status " + std::to_string(status) + ")");
+}
+void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream(); }
+void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
+int tag(const Tensor &t) { return t.scalar_type() == at::kBFloat16 ? NA1D_BF16 : NA1D_FP16; }
+
+// A plain GPU tensor that nothing but autograd looks at.
+bool plain(const Tensor &t) {
+    const auto keys = t.key_set();
+    return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.is_conj() && !t.is_neg() &&
+           !keys.has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                              c10::DispatchKey::Functionalize, c10::DispatchKey::Batched, c10::DispatchKey::FuncTorchVmapMode})) &&
+           !t._fw_grad(0).defined();
+}
+bool plain_call() {
+    const auto tls = c10::impl::tls_local_dispatch_key_set().included_;
+    return !torch::jit::tracer::isTracing() && !c10::impl::dispatch_mode_enabled() &&
+           !tls.has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::FuncTorchDynamicLayerBackMode,
+                                             c10::DispatchKey::FuncTorchVmapMode, c10::DispatchKey::Functionalize, c10::DispatchKey::Python}));
+}
+bool half_type(const Tensor &t) { return t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kHalf; }
+// [B, T, C] operands of one kind.
+bool same_operands(const Tensor &q, const Tensor &k, const Tensor &v) {
+    for (const Tensor &t : {q, k, v})
+        if (!plain(t) || t.dim() != 3 || !t.is_contiguous() || t.scalar_type() != q.scalar_type() || t.sizes() != q.sizes() || t.device() != q.device())
+            return false;
+    return half_type(q) && q.numel() > 0;
+}
+struct Dropout {
+    double p;
+    uint64_t seed;
+};
+
+// ------------------------------------------------------------------------------------------------ the fused operator
+struct Geometry {
+    int64_t N, H, T, C, W, left, dilation;
+    double scale;
+    Dropout drop;
+    bool in_place;                                    // q, k, v inside a projection's output [N, T, 3, H, C]
+};
+struct Strides {
+    int64_t in[3], out[3];
+};
+Strides strides_of(const Geometry &g) {
+    if (g.in_place) return Strides{{g.T * 3 * g.H * g.C, g.C, 3 * g.H * g.C}, {g.T * g.H * g.C, g.C, g.H * g.C}};
+    return Strides{{g.H * g.T * g.C, g.T * g.C, g.C}, {g.H * g.T * g.C, g.T * g.C, g.C}};
+}
+int forward_kernel(const Geometry &g, const Tensor &out, const Tensor &lse, const void *q, const void *k, const void *v, const Tensor &rpb, const Tensor &t_valid,
+                   int dtype, void *stream) {
+    const float *bias = (const float *)ptr(rpb);
+    const int32_t *valid = (const int32_t *)ptr(t_valid);
+    if (g.dilation == 1 && !g.in_place) {
+        if (g.drop.p > 0)
+            return na1d_fused_forward_dropout(ptr(out), (float *)ptr(lse), q, k, v, bias, valid, g.N * g.H, g.H, g.T, g.C, g.W, g.left, (float)g.scale, dtype,
+                                              (float)g.drop.p, g.drop.seed, stream);
+        return na1d_fused_forward(ptr(out), (float *)ptr(lse), q, k, v, bias, valid, g.N * g.H, g.H, g.T, g.C, g.W, g.left, (float)g.scale, dtype, stream);
+    }
+    const Strides s = strides_of(g);
+    return na1d_fused_forward_dilated(ptr(out), (float *)ptr(lse), q, k, v, bias, valid, g.N, g.H, g.T, g.C, g.W, g.left, g.dilation, (float)g.scale, dtype, s.in, s.out,
+                                      (float)g.drop.p, g.drop.seed, stream);
+}
+int backward_kernel(const Geometry &g, void *dq, void *dk, void *dv, const Tensor &drpb, const void *q, const void *k, const void *v, const Tensor &out,
+                    const Tensor &dout, const Tensor &lse, const Tensor &rpb, const Tensor &t_valid, int dtype, void *stream) {
+    const float *bias = (const float *)ptr(rpb);
+    const int32_t *valid = (const int32_t *)ptr(t_valid);
+    if (g.dilation == 1 && !g.in_place) {
+        if (g.drop.p > 0)
+            return na1d_fused_backward_dropout(dq, dk, dv, (float *)ptr(drpb), q, k, v, ptr(out), ptr(dout), (const float *)ptr(lse), bias, valid, g.N * g.H, g.H, g.T,
+                                               g.C, g.W, g.left, (float)g.scale, dtype, (float)g.drop.p, g.drop.seed, nullptr, 0, stream);
+        return na1d_fused_backward(dq, dk, dv, (float *)ptr(drpb), q, k, v, ptr(out), ptr(dout), (const float *)ptr(lse), bias, valid, g.N * g.H, g.H, g.T, g.C, g.W,
+                                   g.left, (float)g.scale, dtype, nullptr, 0, stream);
+    }
+    const Strides s = strides_of(g);
+    return na1d_fused_backward_dilated(dq, dk, dv, (float *)ptr(drpb), q, k, v, ptr(dout), (const float *)ptr(lse), bias, valid, g.N, g.H, g.T, g.C, g.W, g.left,
+                                       g.dilation, (float)g.scale, dtype, s.in, s.out, (float)g.drop.p, g.drop.seed, nullptr, 0, stream);
+}
+void remember(AutogradContext *ctx, const Geometry &g, const MaybeTensor &rpb) {
+    ctx->saved_data["geometry"] = std::vector<int64_t>{g.N, g.H, g.T, g.C, g.W, g.left, g.dilation, (int64_t)g.drop.seed, g.in_place};
+    ctx->saved_data["scale"] = g.scale;
+    ctx->saved_data["p"] = g.drop.p;
+    ctx->saved_data["bias"] = rpb && rpb->requires_grad();
+    ctx->saved_data["bias_shape"] = rpb ? rpb->sizes().vec() : std::vector<int64_t>{};
+}
+Geometry recall(AutogradContext *ctx) {
+    const auto v = ctx->saved_data["geometry"].toIntVector();
+    return Geometry{v[0], v[1], v[2], v[3], v[4], v[5], v[6], ctx->saved_data["scale"].toDouble(), {ctx->saved_data["p"].toDouble(), (uint64_t)v[7]}, v[8] != 0};
+}
+Tensor bias_of(const MaybeTensor &rpb, const Geometry &g) {
+    return rpb ? rpb->detach().reshape({g.H, g.W}).to(at::kFloat).contiguous() : Tensor();
+}
+Tensor lengths_of(const MaybeTensor &t_valid, const Tensor &like) { return t_valid ? t_valid->to(like.device(), at::kInt).contiguous() : Tensor(); }
+
+struct Fused : torch::autograd::Function<Fused> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const MaybeTensor &rpb, const MaybeTensor &t_valid,
+                          const Geometry &g) {
+        const Tensor bias = bias_of(rpb, g), valid = lengths_of(t_valid, q), out = at::empty_like(q);
+        const Tensor lse = at::empty({g.N * g.H, g.T}, q.options().dtype(at::kFloat));
+        check(forward_kernel(g, out, lse, ptr(q), ptr(k), ptr(v), bias, valid, tag(q), stream_of(q)), "na1d_fused_forward");
+        ctx->save_for_backward({q, k, v, out, bias, valid, lse});
+        remember(ctx, g, rpb);
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const Geometry g = recall(ctx);
+        const Tensor &q = s[0];
+        const c10::DeviceGuard guard(q.device());
+        const Tensor dout = grads[0].contiguous(), dq = at::empty_like(q), dk = at::empty_like(q), dv = at::empty_like(q);
+        Tensor drpb;
+        if (ctx->saved_data["bias"].toBool()) drpb = at::zeros(ctx->saved_data["bias_shape"].toIntVector(), q.options().dtype(at::kFloat));
+        check(backward_kernel(g, ptr(dq), ptr(dk), ptr(dv), drpb, ptr(q), ptr(s[1]), ptr(s[2]), s[3], dout, s[6], s[4], s[5], tag(q), stream_of(q)),
+              "na1d_fused_backward");
+        return {dq, dk, dv, drpb, Tensor(), Tensor()};
+    }
+};
+struct FusedQKV : torch::autograd::Function<FusedQKV> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &qkv, const MaybeTensor &rpb, const MaybeTensor &t_valid, const Geometry &g) {
+        const Tensor bias = bias_of(rpb, g), valid = lengths_of(t_valid, qkv), out = at::empty({g.N, g.T, g.H * g.C}, qkv.options());
+        const Tensor lse = at::empty({g.N * g.H, g.T}, qkv.options().dtype(at::kFloat));
+        const char *q = (const char *)ptr(qkv);
+        const int64_t step = 2 * g.H * g.C;
+        check(forward_kernel(g, out, lse, q, q + step, q + 2 * step, bias, valid, tag(qkv), stream_of(qkv)), "na1d_fused_forward");
+        ctx->save_for_backward({qkv, bias, valid, lse});
+        remember(ctx, g, rpb);
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const Geometry g = recall(ctx);
+        const Tensor &qkv = s[0];
+        const c10::DeviceGuard guard(qkv.device());
+        const Tensor dout = grads[0].contiguous(), dqkv = at::empty_like(qkv);
+        Tensor drpb;
+        if (ctx->saved_data["bias"].toBool()) drpb = at::zeros(ctx->saved_data["bias_shape"].toIntVector(), qkv.options().dtype(at::kFloat));
+        const int64_t step = 2 * g.H * g.C;
+        char *dq = (char *)ptr(dqkv);
+        const char *q = (const char *)ptr(qkv);
+        check(backward_kernel(g, dq, dq + step, dq + 2 * step, drpb, q, q + step, q + 2 * step, Tensor(), dout, s[3], s[1], s[2], tag(qkv), stream_of(qkv)),
+              "na1d_fused_backward");
+        return {dqkv, drpb, Tensor(), Tensor()};
+    }
+};
+// Whether bias and lengths are what the Python path takes without complaint, and the sizes what the one-launch kernels cover.
+bool covered(const Geometry &g, const Tensor &like, const MaybeTensor &rpb, const MaybeTensor &t_valid) {
+    if (g.H < 1 || g.W < 1 || g.W > NA1D_MAX_WINDOW || g.left < 0 || g.left >= g.W || g.dilation < 1 || g.C % 8 || g.C > 128 || !(g.drop.p >= 0 && g.drop.p < 1))
+        return false;
+    if (rpb && (!plain(*rpb) || rpb->device() != like.device() || rpb->numel() != g.H * g.W || !rpb->is_floating_point())) return false;
+    if (t_valid && (!plain(*t_valid) || t_valid->numel() != g.N || t_valid->device() != like.device())) return false;
+    return na1d_fused_backward_dilated_workspace_bytes(g.N, g.H, g.T, g.C, g.W, g.left, g.dilation, tag(like)) > 0;
+}
+
+bool needs_grad(std::initializer_list<Tensor> operands, const MaybeTensor &rpb) {
+    if (!at::GradMode::is_enabled()) return false;
+    for (const Tensor &t : operands)
+        if (t.requires_grad()) return true;
+    return rpb && rpb->requires_grad();
+}
+
+MaybeTensor fused(const Tensor &q, const Tensor &k, const Tensor &v, const MaybeTensor &rpb, const MaybeTensor &t_valid, int64_t H, int64_t W, int64_t left,
+                  double scale, int64_t dilation, double p, uint64_t seed) {
+    if (!plain_call() || !same_operands(q, k, v) || H < 1 || q.size(0) % H) return std::nullopt;
+    const Geometry g{q.size(0) / H, H, q.size(1), q.size(2), W, left, dilation, scale, {p, seed}, false};
+    if (!covered(g, q, rpb, t_valid)) return std::nullopt;
+    const c10::DeviceGuard guard(q.device());
+    if (!needs_grad({q, k, v}, rpb)) {                 // no node, no log-sum-exp
+        const Tensor out = at::empty_like(q);
+        check(forward_kernel(g, out, Tensor(), ptr(q), ptr(k), ptr(v), bias_of(rpb, g), lengths_of(t_valid, q), tag(q), stream_of(q)), "na1d_fused_forward");
+        return out;
+    }
+    return Fused::apply(q, k, v, rpb, t_valid, g);
+}
+MaybeTensor fused_qkv(const Tensor &qkv, const MaybeTensor &rpb, const MaybeTensor &t_valid, int64_t W, int64_t left, double scale, int64_t dilation, double p,
+                      uint64_t seed) {
+    if (!plain_call() || !plain(qkv) || qkv.dim() != 5 || qkv.size(2) != 3 || !qkv.is_contiguous() || !half_type(qkv) || !qkv.numel()) return std::nullopt;
+    const Geometry g{qkv.size(0), qkv.size(3), qkv.size(1), qkv.size(4), W, left, dilation, scale, {p, seed}, true};
+    if (!covered(g, qkv, rpb, t_valid)) return std::nullopt;
+    const c10::DeviceGuard guard(qkv.device());
+    if (!needs_grad({qkv}, rpb)) {
+        const Tensor out = at::empty({g.N, g.T, g.H * g.C}, qkv.options());
+        const char *q = (const char *)ptr(qkv);
+        const int64_t step = 2 * g.H * g.C;
+        check(forward_kernel(g, out, Tensor(), q, q + step, q + 2 * step, bias_of(rpb, g), lengths_of(t_valid, qkv), tag(qkv), stream_of(qkv)), "na1d_fused_forward");
+        return out;
+    }
+    return FusedQKV::apply(qkv, rpb, t_valid, g);
+}
+
+// ------------------------------------------------------------------------------------------------ dense attention
+struct Dense : torch::autograd::Function<Dense> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const MaybeTensor &t_valid, int64_t H, double scale, double p,
+                          uint64_t seed) {
+        const Tensor out = at::empty_like(q), lse = at::empty({q.size(0), q.size(1)}, q.options().dtype(at::kFloat)), valid = t_valid ? *t_valid : Tensor();
+        check(na1d_global_forward(ptr(out), (float *)ptr(lse), ptr(q), ptr(k), ptr(v), (const int32_t *)ptr(valid), q.size(0), H, q.size(1), q.size(2), (float)scale,
+                                  tag(q), (float)p, seed, stream_of(q)),
+              "na1d_global_forward");
+        ctx->save_for_backward({q, k, v, out, lse, valid});
+        ctx->saved_data["heads"] = H;
+        ctx->saved_data["scale"] = scale;
+        ctx->saved_data["p"] = p;
+        ctx->saved_data["seed"] = (int64_t)seed;
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const Tensor &q = s[0];
+        const c10::DeviceGuard guard(q.device());
+        const int64_t B = q.size(0), T = q.size(1), C = q.size(2), H = ctx->saved_data["heads"].toInt();
+        const Tensor dout = grads[0].contiguous(), dq = at::empty_like(q), dk = at::empty_like(q), dv = at::empty_like(q);
+        const int64_t nbytes = na1d_global_backward_workspace_bytes(B, H, T, C, tag(q));
+        check((int)std::min<int64_t>(nbytes, 0), "na1d_global_backward_workspace_bytes");
+        const Tensor ws = at::empty({nbytes}, q.options().dtype(at::kByte));
+        check(na1d_global_backward(ptr(dq), ptr(dk), ptr(dv), ptr(q), ptr(s[1]), ptr(s[2]), ptr(s[3]), ptr(dout), (const float *)ptr(s[4]), (const int32_t *)ptr(s[5]),
+                                   B, H, T, C, (float)ctx->saved_data["scale"].toDouble(), tag(q), (float)ctx->saved_data["p"].toDouble(),
+                                   (uint64_t)ctx->saved_data["seed"].toInt(), ptr(ws), nbytes, stream_of(q)),
+              "na1d_global_backward");
+        return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+MaybeTensor dense(const Tensor &q, const Tensor &k, const Tensor &v, const MaybeTensor &t_valid, int64_t H, double scale, double p, uint64_t seed) {
+    if (!plain_call() || !same_operands(q, k, v) || H < 1 || q.size(0) % H || q.size(2) % 8 || q.size(2) > 128) return std::nullopt;
+    if (t_valid && (!plain(*t_valid) || t_valid->scalar_type() != at::kInt || t_valid->numel() != q.size(0) / H || !t_valid->is_contiguous() ||
+                    t_valid->device() != q.device()))
+        return std::nullopt;
+    const c10::DeviceGuard guard(q.device());
+    return Dense::apply(q, k, v, t_valid, H, scale, p, seed);
+}
+
+// ------------------------------------------------------------------------------------------------ the two-call operator
+using Band = int(void *, const void *, const void *, int64_t, int64_t, int64_t, int64_t, int64_t, int, void *);
+void band(Band *f, const char *name, const Tensor &out, const Tensor &a, const Tensor &b, const Tensor &like, int64_t W, int64_t left) {
+    check(f(ptr(out), ptr(a), ptr(b), like.size(0), like.size(1), like.size(2), W, left, tag(like), stream_of(like)), name);
+}
+struct QK : torch::autograd::Function<QK> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, int64_t W, int64_t left) {
+        const Tensor attn = at::empty({q.size(0), q.size(1), W}, q.options().dtype(at::kFloat));
+        band(na1d_qk_forward, "na1d_qk_forward", attn, q, k, q, W, left);
+        ctx->save_for_backward({q, k});
+        ctx->saved_data["W"] = W;
+        ctx->saved_data["left"] = left;
+        return attn;
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const int64_t W = ctx->saved_data["W"].toInt(), left = ctx->saved_data["left"].toInt();
+        const c10::DeviceGuard guard(s[0].device());
+        const Tensor g = grads[0].contiguous(), dq = at::empty_like(s[0]), dk = at::empty_like(s[0]);
+        band(na1d_q_backward, "na1d_q_backward", dq, g, s[1], s[0], W, left);
+        band(na1d_k_backward, "na1d_k_backward", dk, g, s[0], s[0], W, left);
+        return {dq, dk, Tensor(), Tensor()};
+    }
+};
+struct AV : torch::autograd::Function<AV> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &attn, const Tensor &v, int64_t W, int64_t left) {
+        const Tensor out = at::empty_like(v);
+        band(na1d_av_forward, "na1d_av_forward", out, attn, v, v, W, left);
+        ctx->save_for_backward({attn, v});
+        ctx->saved_data["W"] = W;
+        ctx->saved_data["left"] = left;
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const int64_t W = ctx->saved_data["W"].toInt(), left = ctx->saved_data["left"].toInt();
+        const c10::DeviceGuard guard(s[1].device());
+        const Tensor g = grads[0].contiguous(), dattn = at::empty_like(s[0]), dv = at::empty_like(s[1]);
+        band(na1d_a_backward, "na1d_a_backward", dattn, g, s[1], s[1], W, left);
+        band(na1d_v_backward, "na1d_v_backward", dv, s[0], g, s[1], W, left);
+        return {dattn, dv, Tensor(), Tensor()};
+    }
+};
+bool band_window(int64_t W, int64_t left) { return W >= 1 && W <= NA1D_MAX_WINDOW && left >= 0 && left < W; }
+MaybeTensor qk(const Tensor &q, const Tensor &k, int64_t W, int64_t left) {
+    if (!plain_call() || !same_operands(q, k, k) || q.size(2) % 8 || !band_window(W, left)) return std::nullopt;
+    const c10::DeviceGuard guard(q.device());
+    return QK::apply(q, k, W, left);
+}
+MaybeTensor av(const Tensor &attn, const Tensor &v, int64_t W, int64_t left) {
+    if (!plain_call() || !same_operands(v, v, v) || v.size(2) % 8 || !band_window(W, left)) return std::nullopt;
+    if (!plain(attn) || attn.scalar_type() != at::kFloat || !attn.is_contiguous() || attn.device() != v.device() || attn.dim() != 3 || attn.size(0) != v.size(0) ||
+        attn.size(1) != v.size(1) || attn.size(2) != W)
+        return std::nullopt;
+    const c10::DeviceGuard guard(v.device());
+    return AV::apply(attn, v, W, left);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    m.def("fused", &fused);
+    m.def("fused_qkv", &fused_qkv);
+    m.def("dense", &dense);
+    m.def("qk", &qk);
+    m.def("av", &av);
+}

@@ -7,6 +7,7 @@ call fails, a Python exception is raised.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 
 import torch
@@ -34,6 +35,8 @@ SYMBOLS = _UNFUSED + ("na1d_fused_forward", "na1d_fused_backward", "na1d_fused_b
 UNSUPPORTED = -8
 
 _lib = None
+_nodes = None
+_other_build = "NA1D_LIB" in os.environ
 
 
 class NA1DError(RuntimeError):
@@ -117,6 +120,24 @@ def load():
     lib.na1d_status_string.argtypes = [_int]
     _lib = lib
     return lib
+
+
+def nodes():
+    """The operators' autograd nodes in C++ (``csrc/na1d_torch.cpp``).  They call the library beside them: with
+    another build named by NA1D_LIB, and under ``torch.compile``, the Python implementations serve (``None``)."""
+    global _nodes
+    if _other_build or torch.compiler.is_compiling():
+        return None
+    if _nodes is None:
+        load()
+        path = os.path.join(os.path.dirname(LIB_PATH), "na1d_torch.so")
+        if not os.path.exists(path):
+            raise NA1DError(build_hint().replace(LIB_PATH, path).replace("libna1d.so", "na1d_torch.so"))
+        spec = importlib.util.spec_from_file_location("na1d_torch", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _nodes = module
+    return _nodes
 
 
 def dtype_tag(dtype: torch.dtype) -> int:

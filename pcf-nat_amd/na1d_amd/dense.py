@@ -59,4 +59,10 @@ def global_attention(q, k, v, num_heads, t_valid=None, scale=None, dropout_p=0.0
     if dropout_p > 0.0:
         assert dropout_p < 1.0
         dropout = (float(dropout_p), int(torch.randint(0, 2 ** 62, (1,)).item()) if seed is None else int(seed))
+    if q.is_cuda:
+        nodes = _lib.nodes()
+        p, seed = dropout or (0.0, 0)
+        out = None if nodes is None else nodes.dense(q, k, v, t_valid, num_heads, float(scale), p, seed & (2 ** 64 - 1))
+        if out is not None:
+            return out
     return _GlobalAttention.apply(q, k, v, t_valid, num_heads, float(scale), dropout)

@@ -138,6 +138,10 @@ class _FusedNA1D(torch.autograd.Function):
         return dq, dk, dv, drpb, None, None, None, None, None, None, None, None
 
 
+def _native_dropout(dropout):
+    return (0.0, 0) if dropout is None else (dropout[0], dropout[1] & (2 ** 64 - 1))
+
+
 def na1d_fused(q, k, v, win_size, left, rpb=None, t_valid=None, num_heads=1, scale=1.0, deterministic=False,
                dilation=1, dropout_p=0.0, seed=None):
     """Fused neighbourhood attention.
@@ -167,6 +171,12 @@ def na1d_fused(q, k, v, win_size, left, rpb=None, t_valid=None, num_heads=1, sca
         if seed is None:
             seed = int(torch.randint(0, 2 ** 62, (1,)).item())
         dropout = (float(dropout_p), int(seed))
+    if not deterministic and q.is_cuda:
+        nodes = _lib.nodes()
+        out = None if nodes is None else nodes.fused(q, k, v, rpb, t_valid, num_heads, win_size, left, float(scale), int(dilation),
+                                                     *_native_dropout(dropout))
+        if out is not None:
+            return out
     return _FusedNA1D.apply(q, k, v, rpb, t_valid, num_heads, win_size, left, float(scale), bool(deterministic),
                             int(dilation), dropout)
 
@@ -244,6 +254,12 @@ def na1d_fused_qkv(qkv, win_size, left, rpb=None, t_valid=None, scale=1.0, deter
         if seed is None:
             seed = int(torch.randint(0, 2 ** 62, (1,)).item())
         dropout = (float(dropout_p), int(seed))
+    if not deterministic and qkv.is_cuda:
+        nodes = _lib.nodes()
+        out = None if nodes is None else nodes.fused_qkv(qkv, rpb, t_valid, win_size, left, float(scale), int(dilation),
+                                                         *_native_dropout(dropout))
+        if out is not None:
+            return out
     if dropout is None and dilation == 1 and not (torch.is_grad_enabled() and (qkv.requires_grad or (rpb is not None and rpb.requires_grad))):
         # inference: one library call, no views, no log-sum-exp
         assert qkv.dim() == 5 and qkv.shape[2] == 3 and qkv.is_contiguous()

@@ -82,6 +82,18 @@ def _make_functions(dtype: torch.dtype, prefix: str):
             _lib.call_unfused("na1d_v_backward", v_gd, attn, result_gd, B, T, C, ctx.win_size, ctx.left, dtype)
             return (attn_gd, v_gd, None, None, None)
 
+    # what ``apply`` does for calls that the C++ nodes take as they are; everything else goes through the classes
+    def qk_apply(q, k, win_size, left, dilation=1, python=QK.apply):
+        nodes = _lib.nodes() if q.is_cuda and q.dtype == dtype else None
+        out = None if nodes is None else nodes.qk(q, k, win_size, left)
+        return python(q, k, win_size, left, dilation) if out is None else out
+
+    def av_apply(attn, v, win_size, left, dilation=1, python=AV.apply):
+        nodes = _lib.nodes() if v.is_cuda and v.dtype == dtype else None
+        out = None if nodes is None else nodes.av(attn, v, win_size, left)
+        return python(attn, v, win_size, left, dilation) if out is None else out
+
+    QK.apply, AV.apply = staticmethod(qk_apply), staticmethod(av_apply)
     QK.__name__ = QK.__qualname__ = prefix + "_ANA1d_QK_Function"
     AV.__name__ = AV.__qualname__ = prefix + "_ANA1d_AV_Function"
     return QK, AV
