@@ -411,24 +411,28 @@ __global__ void lengths_kernel(int32_t *t_valid, float *count, const float *lens
 }
 
 // [N, in_chans, frames] fp32 -> patch rows [N * T, in_chans * patch] of 16 bit, element (c, j) of token t = x[c][t * patch + j].
-// 64 tokens to a workgroup through LDS: reads run along the frames, writes along the rows.
+// kPatchTokens tokens of `chans` channels to a workgroup through LDS: a wave reads along the frames of a channel, the
+// writes run along the rows.  Bound by memory; the work is split over the channels too, or a single utterance is a handful
+// of workgroups (3 s: 19.5 us in three workgroups of whole rows that divided twice for every value).
+constexpr int kPatchTokens = 32;
 template <class DT>
 __global__ void __launch_bounds__(256)
-patch_kernel(uint32_t *__restrict__ out, const float *__restrict__ x, int in_chans, int frames, int patch, int T) {
+patch_kernel(uint32_t *__restrict__ out, const float *__restrict__ x, int in_chans, int chans, int frames, int patch, int T, uint32_t patch_magic,
+             uint32_t width_magic) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    float *tile = reinterpret_cast<float *>(smem);               // [in_chans][64 * patch + 1]
-    const int span = 64 * patch, pitch = span + 1, t0 = blockIdx.x * 64, nt = min(64, T - t0), width = in_chans * patch;
-    const float *src = x + (int64_t)blockIdx.y * in_chans * frames + (int64_t)t0 * patch;
-    for (int i = threadIdx.x; i < in_chans * span; i += 256) {
-        const int c = i / span, f = i - c * span;
-        tile[c * pitch + f] = f < nt * patch ? src[(int64_t)c * frames + f] : 0.f;
-    }
+    float *tile = reinterpret_cast<float *>(smem);               // [chans][kPatchTokens * patch + 1]
+    const int span = kPatchTokens * patch, pitch = span + 1, t0 = blockIdx.x * kPatchTokens, nt = min(kPatchTokens, T - t0), c_first = blockIdx.z * chans;
+    const float *src = x + ((int64_t)blockIdx.y * in_chans + c_first) * frames + (int64_t)t0 * patch;
+#pragma unroll 4
+    for (int c = threadIdx.x >> 6; c < chans; c += 4)
+        for (int f = threadIdx.x & 63; f < nt * patch; f += 64) tile[c * pitch + f] = src[(int64_t)c * frames + f];
     __syncthreads();
-    uint32_t *dst = out + ((int64_t)blockIdx.y * T + t0) * (width / 2);
-    for (int i = threadIdx.x; i < nt * (width / 2); i += 256) {
-        const int t = i / (width / 2), e = 2 * (i - t * (width / 2));
-        const int c0 = e / patch, j0 = e - c0 * patch, c1 = (e + 1) / patch, j1 = e + 1 - c1 * patch;
-        dst[i] = Mma<DT>::pack(tile[c0 * pitch + t * patch + j0], tile[c1 * pitch + t * patch + j1]);
+    const int half = chans * patch / 2, row = in_chans * patch / 2;                // pairs of a row here and in all
+    uint32_t *dst = out + ((int64_t)blockIdx.y * T + t0) * row + c_first * patch / 2;
+    for (int i = threadIdx.x; i < nt * half; i += 256) {
+        const int t = div_by(i, half, width_magic), k = i - t * half, e = 2 * k;
+        const int c0 = div_by(e, patch, patch_magic), j0 = e - c0 * patch, c1 = div_by(e + 1, patch, patch_magic), j1 = e + 1 - c1 * patch;
+        dst[(int64_t)t * row + k] = Mma<DT>::pack(tile[c0 * pitch + t * patch + j0], tile[c1 * pitch + t * patch + j1]);
     }
 }
 
@@ -503,15 +507,23 @@ struct PoolArgs {
     char *out;                      // [N, 2 * wide], the next product's operand
     int T, wide;
 };
+// Over the 16 lanes of a row, in all of them, without LDS: by neighbours, by pairs, then mirrored within 8 and 16 lanes
+// (whose quarters are equal by then).  256 of these steps close a wave's work; as shuffles through LDS they were half of
+// the kernel's time at 100 tokens.
+template <int CTRL> __device__ inline float row_step(float x) {
+    return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), CTRL, 0xf, 0xf, true));
+}
 __device__ inline float row16_max(float x) {
-#pragma unroll
-    for (int k = 1; k < 16; k *= 2) x = __builtin_fmaxf(x, __shfl_xor(x, k));
-    return x;
+    x = __builtin_fmaxf(x, row_step<0xb1>(x));
+    x = __builtin_fmaxf(x, row_step<0x4e>(x));
+    x = __builtin_fmaxf(x, row_step<0x141>(x));
+    return __builtin_fmaxf(x, row_step<0x140>(x));
 }
 __device__ inline float row16_sum(float x) {
-#pragma unroll
-    for (int k = 1; k < 16; k *= 2) x += __shfl_xor(x, k);
-    return x;
+    x += row_step<0xb1>(x);
+    x += row_step<0x4e>(x);
+    x += row_step<0x141>(x);
+    return x + row_step<0x140>(x);
 }
 template <class DT>
 __global__ void __launch_bounds__(kThreads, 2)
@@ -714,10 +726,11 @@ int encode(const na1d_encoder &e, char *out, const float *x, const float *lens, 
         NA1D_TRY(launch_status());
     }
     {
-        const size_t lds = (size_t)e.in_chans * (64 * e.patch + 1) * sizeof(float);
+        const int chans = e.in_chans % 16 == 0 ? 16 : e.in_chans, half = chans * e.patch / 2;
+        const size_t lds = (size_t)chans * (kPatchTokens * e.patch + 1) * sizeof(float);
         if (!allow_lds(patch_kernel<DT>, lds)) return NA1D_ERR_LAUNCH;
-        patch_kernel<DT><<<dim3((unsigned)((T + 63) / 64), (unsigned)N), 256, lds, s>>>(
-            reinterpret_cast<uint32_t *>(ws + b.patches), x, e.in_chans, (int)frames, e.patch, (int)T);
+        patch_kernel<DT><<<dim3((unsigned)((T + kPatchTokens - 1) / kPatchTokens), (unsigned)N, (unsigned)(e.in_chans / chans)), 256, lds, s>>>(
+            reinterpret_cast<uint32_t *>(ws + b.patches), x, e.in_chans, chans, (int)frames, e.patch, (int)T, div_magic(e.patch), div_magic(half));
         NA1D_TRY(launch_status());
     }
     int dense = 0;

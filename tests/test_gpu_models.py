@@ -437,3 +437,21 @@ def test_native_encoder_leaves_changed_models_to_the_modules():
         h.remove()
     model.fc = torch.nn.Identity()
     assert run(natively=True) is None and run().shape == (3, 3072)
+
+
+@pytest.mark.parametrize("in_chans,patch,frames", [(24, 4, 103), (64, 3, 100), (160, 1, 33), (80, 2, 64), (16, 16, 1030)])
+def test_native_encoder_patches(in_chans, patch, frames):
+    """Patch rows of every shape the kernel splits differently: channels in sixteens or all at once, odd patches, frames
+    that do not fill the last patch or the last block of 32 tokens.  Tolerance as at the tile edges."""
+    kw = dict(depths=(1,), num_heads=[[16]], win_size=[[27]], in_chans=in_chans, patch_size=patch)
+    cpu = _twin(models.MFA_NATransformer, torch.float16, seed=3, **kw).eval()
+    gpu = models.MFA_NATransformer(na="fused_qkv", dtype=torch.float16, **kw)
+    gpu.load_state_dict(cpu.state_dict())
+    gpu = gpu.cuda().eval()
+    x = torch.randn(3, in_chans, frames, generator=torch.Generator().manual_seed(2))
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+        got = models.embed_natively(gpu, x.cuda())
+    assert got is not None
+    with torch.no_grad():
+        want = cpu(x)
+    assert O.rel_l2(got.float(), want) < 2.5e-3
