@@ -29,6 +29,8 @@ struct LayerArgs {
     int x_in_pitch, block_pitch, patch_width, M, T;
     uint32_t T_magic;
     int tail_groups, head_groups;     // block-diagonal weights: 8, 4, 2; otherwise 1
+    char *x1;                         // split layers (part_kernel): [M, 256] ...
+    float *parts;                     // ... and what each quarter of the hidden channels adds, [4, M, 256]
 };
 
 // Grouped projections (PCF-NAT: blocks of 8, 4, 2 and 1 groups) have block-diagonal weights; which 32-input steps of an
@@ -87,17 +89,16 @@ template <class DT, int MT, int NW, int PF> struct LayerWave {
     }
     __device__ inline f32x4 bias(const float *b, int c) const { return *reinterpret_cast<const f32x4 *>(b + c + 4 * g); }
 
-    // attention rows in p_lds, x in q_lds (on their way) -> x2 in q_lds
-    template <int G> __device__ inline void tail() {
+    // attention rows in p_lds, x in q_lds (on their way) -> x1 in q_lds; the ring holds the start of fc1's chunk c
+    template <int G> __device__ inline void project(Rsrc w1, int first_chunk) {
         using S = Groups<G, NW>;
-        const Rsrc w1 = weight_rsrc(a.w_fc1, kHidden, kDim), w2 = weight_rsrc(a.w_fc2, kDim, kHidden);
         const auto proj = S::proj(weight_rsrc(a.w_proj, kDim, kDim), wave);
         ring.begin(proj, lane16);
         f32x4 hid[NTW][MT];
         clear(hid);
         wait_direct();
         barrier_lds();
-        multiply<DT, MT>(hid, 0, ring, proj, S::fc1(w1, 0, wave), p_lds, n, g, lane16);
+        multiply<DT, MT>(hid, 0, ring, proj, S::fc1(w1, first_chunk, wave), p_lds, n, g, lane16);
 #pragma unroll
         for (int j = 0; j < NTW; ++j) {
             const int c = CW * wave + 16 * j;
@@ -105,39 +106,47 @@ template <class DT, int MT, int NW, int PF> struct LayerWave {
 #pragma unroll
             for (int i = 0; i < MT; ++i) *at(q_lds, c, i) = narrow4<DT>(hid[j][i] + b + widen4<DT>(*at(q_lds, c, i)));
         }
+    }
+    // 256 hidden channels: x1 in q_lds -> their share of the output in acc[a0 ..] (a0 a constant)
+    template <int G, int NA> __device__ inline void chunk(f32x4 (&acc)[NA][MT], Rsrc w1, Rsrc w2, int c, int a0, bool last) {
+        using S = Groups<G, NW>;
+        f32x4 hid[NTW][MT];
+        clear(hid);
+        barrier_lds();                           // x1 is whole (first round); every wave is done with the hidden channels before
+        multiply<DT, MT>(hid, 0, ring, S::fc1(w1, c, wave), S::fc2(w2, c, wave), q_lds, n, g, lane16);
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) {
+            const int ch = CW * wave + 16 * j;
+            const f32x4 b = bias(a.b_fc1, 256 * c + ch);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                f32x4 h = hid[j][i] + b;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) h[r] = gelu(h[r]);
+                *at(p_lds, ch, i) = narrow4<DT>(h);
+            }
+        }
+        barrier_lds();
+        if (wave < S::kActive)
+            multiply<DT, MT>(acc, a0, ring, S::fc2(w2, c, wave), S::fc1(w1, last ? 0 : c + 1, wave), p_lds, n, g, lane16);
+        else
+            ring.begin(S::fc1(w1, last ? 0 : c + 1, wave), lane16);
+    }
+    // the rest of the layer: -> x2 in q_lds
+    template <int G> __device__ inline void tail() {
+        using S = Groups<G, NW>;
+        const Rsrc w1 = weight_rsrc(a.w_fc1, kHidden, kDim), w2 = weight_rsrc(a.w_fc2, kDim, kHidden);
+        project<G>(w1, 0);
         f32x4 acc[S::kAcc][MT];
         clear(acc);
-        const bool active = wave < S::kActive;
-        auto chunk = [&](int c, int a0, bool last) {      // a0: the chunk's output tiles in acc, a constant
-            clear(hid);
-            barrier_lds();                           // x1 is whole (first round); every wave is done with the hidden channels before
-            multiply<DT, MT>(hid, 0, ring, S::fc1(w1, c, wave), S::fc2(w2, c, wave), q_lds, n, g, lane16);
-#pragma unroll
-            for (int j = 0; j < NTW; ++j) {
-                const int ch = CW * wave + 16 * j;
-                const f32x4 b = bias(a.b_fc1, 256 * c + ch);
-#pragma unroll
-                for (int i = 0; i < MT; ++i) {
-                    f32x4 h = hid[j][i] + b;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) h[r] = gelu(h[r]);
-                    *at(p_lds, ch, i) = narrow4<DT>(h);
-                }
-            }
-            barrier_lds();
-            if (active)
-                multiply<DT, MT>(acc, a0, ring, S::fc2(w2, c, wave), S::fc1(w1, last ? 0 : c + 1, wave), p_lds, n, g, lane16);
-            else
-                ring.begin(S::fc1(w1, last ? 0 : c + 1, wave), lane16);
-        };
         if constexpr (S::kSets == 1) {
 #pragma unroll 1
-            for (int c = 0; c < 4; ++c) chunk(c, 0, c == 3);
+            for (int c = 0; c < 4; ++c) chunk<G>(acc, w1, w2, c, 0, c == 3);
         } else {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) chunk(c, c * S::kSets / 4 * S::kPer, c == 3);
+            for (int c = 0; c < 4; ++c) chunk<G>(acc, w1, w2, c, c * S::kSets / 4 * S::kPer, c == 3);
         }
-        if (active) {
+        if (wave < S::kActive) {
 #pragma unroll
             for (int t = 0; t < S::kAcc; ++t) {
                 const int c = 16 * (t / S::kPer * S::kOutTiles + wave * S::kPer + t % S::kPer);
@@ -148,14 +157,58 @@ template <class DT, int MT, int NW, int PF> struct LayerWave {
         }
     }
 
-    template <int G> __device__ inline void head(int64_t m0, int rows) {
+    // a quarter of it: x1 to memory (the first quarter's), the hidden channels' share of the output to `parts`
+    template <int G> __device__ inline void tail_part(int c, int64_t m0, int rows) {
+        using S = Groups<G, NW>;
+        const Rsrc w1 = weight_rsrc(a.w_fc1, kHidden, kDim), w2 = weight_rsrc(a.w_fc2, kDim, kHidden);
+        project<G>(w1, c);
+        f32x4 acc[S::kPer][MT];
+        clear(acc);
+        chunk<G>(acc, w1, w2, c, 0, true);
+        const Rsrc d = make_rsrc(a.parts + ((int64_t)c * a.M + m0) * kDim, rows * kDim * 4);
+        if (wave < S::kActive) {
+#pragma unroll
+            for (int t = 0; t < S::kPer; ++t) {
+                const int ch = 16 * (c * S::kSets / 4 * S::kOutTiles + wave * S::kPer + t) + 4 * g;
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[t][i]), d, (16 * i + n) * kDim * 4 + ch * 4, 0, 0);
+            }
+        }
+        if (c == 0) write_rows(a.x1, m0, rows, kRow);
+    }
+    // and the quarters put together: -> x2 in q_lds.  A quarter reaches all outputs (one group), half of them (two) or its own quarter.
+    __device__ inline void join(int64_t m0, int rows) {
+        const int per = a.tail_groups == 1 ? 4 : a.tail_groups == 2 ? 2 : 1;
+        const Rsrc xs = make_rsrc(a.x1 + m0 * kRow, rows * kRow);
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) {
+            const int c = CW * wave + 16 * j, first = c / (64 * per) * per;
+            const f32x4 b = bias(a.b_fc2, c);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                const int row = 16 * i + n;
+                const f32x4 x = widen4<DT>(__builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(xs, row * kRow + 2 * c + 8 * g, 0, 0)));
+                f32x4 v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (k < per) {
+                        const Rsrc ps = make_rsrc(a.parts + ((int64_t)(first + k) * a.M + m0) * kDim, rows * kDim * 4);
+                        v += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ps, row * kDim * 4 + 4 * c + 16 * g, 0, 0));
+                    }
+                *at(q_lds, c, i) = narrow4<DT>(v + b + x);
+            }
+        }
+    }
+
+    template <int G> __device__ inline void head(int64_t m0, int rows, int from, int to) {
         using S = Groups<G, NW>;
         const Rsrc w = weight_rsrc(a.w_qkv, 3 * kDim, kDim);
-        ring.begin(S::qkv(w, 0, wave), lane16);
+        ring.begin(S::qkv(w, from, wave), lane16);
         barrier_lds();
         const Rsrc qs = make_rsrc(a.qkv + m0 * (3 * kRow), rows * (3 * kRow));
 #pragma unroll 1
-        for (int which = 0; which < 3; ++which) {
+        for (int which = from; which < to; ++which) {
             f32x4 acc[NTW][MT];
             clear(acc);
             multiply<DT, MT>(acc, 0, ring, S::qkv(w, which, wave), S::qkv(w, min(which + 1, 2), wave), q_lds, n, g, lane16);
@@ -184,7 +237,33 @@ template <class DT, int MT, int NW, int PF> struct LayerWave {
     }
 };
 
-template <class DT, int MT, int NW, int PF>
+// Few tokens: a layer's weights (up to 1.6 MB) take a CU 21 us to read, so each 16 tokens go to four workgroups, one for
+// every 256 hidden channels (each works out the output projection), and then to three, one each for q, k and v
+// (layer_kernel with SPLIT, which puts the quarters together).  One 3 s utterance through the 4x4 model: 340 -> 276 us.
+template <class DT, int NW, int PF>
+__global__ void __launch_bounds__(64 * NW, 2)
+part_kernel(LayerArgs a) {
+    using W = LayerWave<DT, 1, NW, PF>;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    W w{a, (LDS_PTR(char))smem, (LDS_PTR(char))smem + 16 * kRow, wave, lane, lane & 15, lane >> 4, lane * 16};
+    const int c = (int)(blockIdx.x & 3);
+    const int64_t m0 = (int64_t)(blockIdx.x >> 2) * 16;
+    const int rows = (int)min((int64_t)16, a.M - m0);
+    const Rsrc as = make_rsrc(a.attn + m0 * kRow, rows * kRow), xs = make_rsrc(a.x_in + m0 * a.x_in_pitch, rows * a.x_in_pitch);
+    stage_tokens<16, NW, kReadShared>(as, w.p_lds, kRow, kRow, wave, lane);
+    stage_tokens<16, NW, kReadShared>(xs, w.q_lds, a.x_in_pitch, kRow, wave, lane);
+    switch (a.tail_groups) {
+        case 8: w.template tail_part<8>(c, m0, rows); break;
+        case 4: w.template tail_part<4>(c, m0, rows); break;
+        case 2: w.template tail_part<2>(c, m0, rows); break;
+        default: w.template tail_part<1>(c, m0, rows);
+    }
+}
+
+// SPLIT: one workgroup to each of q, k and v of a tile (or one where there is no projection behind); the layer before
+// comes in quarters
+template <class DT, int MT, int NW, int PF, bool SPLIT>
 __global__ void __launch_bounds__(64 * NW, MT == 2 ? 3 : 2)
 layer_kernel(LayerArgs a) {
     using W = LayerWave<DT, MT, NW, PF>;
@@ -193,9 +272,16 @@ layer_kernel(LayerArgs a) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // p_lds: attention rows, then 256 hidden channels at a time, then patches; q_lds: x, then x1, then x2
     W w{a, (LDS_PTR(char))smem, (LDS_PTR(char))smem + 16 * MT * kRow, wave, lane, lane & 15, lane >> 4, lane * 16};
-    const int64_t m0 = (int64_t)blockIdx.x * (16 * MT);
+    const int each = SPLIT && a.qkv ? 3 : 1, mine = each == 3 ? (int)(blockIdx.x % 3u) : 0;
+    const int64_t m0 = (int64_t)(blockIdx.x / (uint32_t)each) * (16 * MT);
     const int rows = (int)min((int64_t)(16 * MT), a.M - m0);
-    if (a.attn) {
+    if (SPLIT && a.attn) {
+        w.join(m0, rows);
+        if (a.block_out && mine == 0) {
+            barrier_lds();
+            w.write_rows(a.block_out, m0, rows, a.block_pitch);
+        }
+    } else if (a.attn) {
         const Rsrc as = make_rsrc(a.attn + m0 * kRow, rows * kRow), xs = make_rsrc(a.x_in + m0 * a.x_in_pitch, rows * a.x_in_pitch);
         stage_tokens<16 * MT, NW, kReadOnce>(as, w.p_lds, kRow, kRow, wave, lane);
         stage_tokens<16 * MT, NW, kReadOnce>(xs, w.q_lds, a.x_in_pitch, kRow, wave, lane);
@@ -212,7 +298,7 @@ layer_kernel(LayerArgs a) {
     }
     if (!a.qkv) return;
     if (a.patches) {
-        if (a.attn) barrier_lds();                   // every wave is done with the hidden channels
+        if (a.attn && !SPLIT) barrier_lds();         // every wave is done with the hidden channels
         const Rsrc es = make_rsrc(a.patches + m0 * a.patch_width, rows * a.patch_width);
         stage_tokens<16 * MT, NW, kReadShared>(es, w.p_lds, a.patch_width, a.patch_width, wave, lane);
         const int ks_all = a.patch_width / 64;       // steps of 32 inputs
@@ -238,7 +324,7 @@ layer_kernel(LayerArgs a) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) *w.at(w.q_lds, CW * wave + 16 * j, i) = narrow4<DT>(acc[j][i]);
     }
-    if (a.x_out) {
+    if (a.x_out && mine == 0) {
         barrier_lds();
         w.write_rows(a.x_out, m0, rows, kRow);
     }
@@ -258,10 +344,10 @@ layer_kernel(LayerArgs a) {
         }
     }
     switch (a.head_groups) {
-        case 8: w.template head<8>(m0, rows); break;
-        case 4: w.template head<4>(m0, rows); break;
-        case 2: w.template head<2>(m0, rows); break;
-        default: w.template head<1>(m0, rows);
+        case 8: w.template head<8>(m0, rows, mine, each == 3 ? mine + 1 : 3); break;
+        case 4: w.template head<4>(m0, rows, mine, each == 3 ? mine + 1 : 3); break;
+        case 2: w.template head<2>(m0, rows, mine, each == 3 ? mine + 1 : 3); break;
+        default: w.template head<1>(m0, rows, mine, each == 3 ? mine + 1 : 3);
     }
 }
 
@@ -637,7 +723,7 @@ pool_kernel(PoolArgs a) {
 // ----------------------------------------------------------------------------- launchers
 template <class DT, int MT, int NW, int PF>
 int launch_layer_mt(const LayerArgs &a, hipStream_t s) {
-    auto kern = layer_kernel<DT, MT, NW, PF>;
+    auto kern = layer_kernel<DT, MT, NW, PF, false>;
     const size_t lds = (size_t)2 * 16 * MT * kRow;
     if (!allow_lds(kern, lds)) return NA1D_ERR_LAUNCH;
     const int64_t wgs = (a.M + 16 * MT - 1) / (16 * MT);
@@ -645,7 +731,23 @@ int launch_layer_mt(const LayerArgs &a, hipStream_t s) {
     return launch_status();
 }
 
+// Up to this many tokens the four quarters of every tile find a CU of their own.  A PCF 4x4 pass with and without:
+// 125 tokens 273 and 336 us, 500: 295 and 344, 1000: 335 and 352; 1500: 426 and 370, 4000: 634 and 454.
+constexpr int64_t kSplitTokens = 16 * 64;
+template <class DT> int launch_layer_split(const LayerArgs &a, hipStream_t s) {
+    const size_t lds = (size_t)2 * 16 * kRow;
+    const unsigned tiles = (unsigned)((a.M + 15) / 16);
+    if (a.attn) {
+        part_kernel<DT, 8, 8><<<4 * tiles, 512, lds, s>>>(a);
+        const int st = launch_status();
+        if (st != NA1D_OK) return st;
+    }
+    layer_kernel<DT, 1, 8, 8, true><<<(a.qkv ? 3 : 1) * tiles, 512, lds, s>>>(a);
+    return launch_status();
+}
+
 template <class DT> int launch_layer(const LayerArgs &a, hipStream_t s) {
+    if (a.M <= kSplitTokens) return launch_layer_split<DT>(a, s);
     // Fewer, larger tiles read the layer's weights fewer times; smaller ones spread few tokens over more CUs.
     if (a.M <= 16 * 256) return launch_layer_mt<DT, 1, 8, 8>(a, s);
     if (a.M <= 32 * 512) return launch_layer_mt<DT, 2, 8, 4>(a, s);
@@ -676,7 +778,7 @@ template <class DT, LinearEnd END> int launch_linear(const LinearArgs &a, hipStr
 // The workspace's tensors, one behind the other.
 struct Buffers {
     int64_t bytes = 0;
-    int64_t x, qkv, attn, blocks, patches, pos, h, hidden, stats, rounded, context, pooled, t_valid, count;
+    int64_t x, qkv, attn, blocks, patches, pos, h, hidden, stats, rounded, context, pooled, t_valid, count, x1, parts;
     int64_t take(int64_t n) {
         const int64_t at = bytes;
         bytes += (n + 255) / 256 * 256;
@@ -698,6 +800,8 @@ struct Buffers {
         pooled = take(N * 2 * e.wide * 2);
         t_valid = take(N * 4);
         count = take(N * 4);
+        x1 = take(M <= kSplitTokens ? M * kRow : 0);
+        parts = take(M <= kSplitTokens ? 4 * M * kDim * 4 : 0);
     }
 };
 inline int dense_layers(const na1d_encoder &e) {
@@ -758,6 +862,8 @@ int encode(const na1d_encoder &e, char *out, const float *x, const float *lens, 
         a.T = (int)T;
         a.T_magic = div_magic(T);
         a.tail_groups = a.head_groups = 1;
+        a.x1 = ws + b.x1;
+        a.parts = reinterpret_cast<float *>(ws + b.parts);
         if (i > 0) {
             const na1d_encoder_layer &l = e.layer[i - 1];
             a.attn = ws + b.attn;

@@ -341,8 +341,9 @@ def test_mfa_nat_4x4_full_batch_training_step_agrees_with_the_checked_small_batc
     assert sum(float(gr.abs().max() > 0) for gr in grads) > 0.9 * len(grads)
 
 
-# tokens of the batch: a single tile, tiles of 16 and their remainder, the first launch with tiles of 32 and of 64
-@pytest.mark.parametrize("batch,frames,lengths", [(1, 16, False), (3, 111, True), (65, 130, True), (130, 256, False)])
+# tokens of the batch: a single tile, tiles of 16 and their remainder, the last launch in quarters and the first without,
+# the first with tiles of 32 and of 64
+@pytest.mark.parametrize("batch,frames,lengths", [(1, 16, False), (3, 111, True), (16, 128, True), (17, 122, False), (65, 130, True), (130, 256, False)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("family", ["pcf", "mfa"])
 def test_native_encoder_at_tile_edges(family, dtype, batch, frames, lengths):
