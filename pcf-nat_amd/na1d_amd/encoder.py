@@ -179,6 +179,11 @@ def embed(model, x, lens=None):
         return None
     if lens is not None and (lens.dtype != torch.float32 or lens.device != x.device or lens.shape != (x.shape[0],)):
         return None
+    if next(model.parameters()).device != x.device:
+        return None
+    if torch.cuda.current_device() != x.device.index:      # plans are made, and launches go, where the tensors are
+        with torch.cuda.device(x.device):
+            return embed(model, x, lens)
     entry = _entries.get(model)
     if entry is None or not entry.same_modules():
         entry = _entries[model] = _Entry(model)
@@ -189,9 +194,6 @@ def embed(model, x, lens=None):
     if plan is None or chans != plan.encoder.in_chans or plan.keep[0].device != x.device:
         return None
     lib = _lib.load()
-    if torch.cuda.current_device() != x.device.index:      # launches go to the device of the tensors
-        with torch.cuda.device(x.device):
-            return embed(model, x, lens)
     ref = ctypes.byref(plan.encoder)
     nbytes = lib.na1d_encode_workspace_bytes(ref, n, frames)
     if nbytes == _lib.UNSUPPORTED:
