@@ -34,7 +34,7 @@ struct LayerArgs {
 };
 
 // Grouped projections (PCF-NAT: blocks of 8, 4, 2 and 1 groups) have block-diagonal weights; which 32-input steps of an
-// output tile are not zero follows from the number of groups G alone:
+// output tile are not zero follows from the number of groups G alone (any other number: all of them, as with one group):
 //   output projection, fc1   outputs of a group see the 256 / G inputs of the same group
 //   fc2                      256 hidden channels (chunk c) reach kOut outputs, from kOut * (c * kOut / 256 ...) on
 //   qkv                      output f (head-major order, see _qkv_channel_order) sees group (f mod 256/G) / (256/G^2)
@@ -73,6 +73,9 @@ template <int G, int NW> struct Groups {
         return Qkv{w, (16 * which + wave * NTW) * 8 + k0, 8, k0};
     }
 };
+
+// The number of groups as the kernels know it: every switch over it and every sum over its parts starts from this.
+inline int known_groups(int groups) { return groups == 2 || groups == 4 || groups == 8 ? groups : 1; }
 
 template <class DT, int MT, int NW, int PF> struct LayerWave {
     static constexpr int NTW = 16 / NW, CW = 16 * NTW;
@@ -179,7 +182,9 @@ template <class DT, int MT, int NW, int PF> struct LayerWave {
     }
     // and the quarters put together: -> x2 in q_lds.  A quarter reaches all outputs (one group), half of them (two) or its own quarter.
     __device__ inline void join(int64_t m0, int rows) {
-        const int per = a.tail_groups == 1 ? 4 : a.tail_groups == 2 ? 2 : 1;
+        const int sets = a.tail_groups == 8 ? Groups<8, NW>::kSets : a.tail_groups == 4 ? Groups<4, NW>::kSets : a.tail_groups == 2 ? Groups<2, NW>::kSets
+                                                                                                                            : Groups<1, NW>::kSets;
+        const int per = 4 / sets;
         const Rsrc xs = make_rsrc(a.x1 + m0 * kRow, rows * kRow);
 #pragma unroll
         for (int j = 0; j < NTW; ++j) {
@@ -871,7 +876,7 @@ int encode(const na1d_encoder &e, char *out, const float *x, const float *lens, 
             a.x_in_pitch = x_in_pitch;
             a.w_proj = (const char *)l.w_proj, a.w_fc1 = (const char *)l.w_fc1, a.w_fc2 = (const char *)l.w_fc2;
             a.b_proj = l.b_proj, a.b_fc1 = l.b_fc1, a.b_fc2 = l.b_fc2;
-            a.tail_groups = l.groups;
+            a.tail_groups = known_groups(l.groups);
             if (l.block_end) {
                 a.block_pitch = e.blocks * kRow;
                 a.block_out = ws + b.blocks + block++ * kRow;
@@ -896,7 +901,7 @@ int encode(const na1d_encoder &e, char *out, const float *x, const float *lens, 
             a.qkv = ws + b.qkv;
             a.w_qkv = (const char *)l.w_qkv;
             a.b_qkv = l.b_qkv;
-            a.head_groups = l.groups;
+            a.head_groups = known_groups(l.groups);
             if (!l.window) {
                 a.gain = l.gain;
                 a.posb = reinterpret_cast<const float *>(ws + b.pos + dense++ * T * kDim * 4);

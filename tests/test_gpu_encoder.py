@@ -1,0 +1,57 @@
+"""Embedding models in one native call: what it shares with the modules beyond ordinary inputs."""
+import copy
+
+import pytest
+import torch
+
+from na1d_amd import models
+from oracle import na1d_oracle as O
+
+pytestmark = pytest.mark.gpu
+SMALL = dict(depths=(1, 1), num_heads=[[16], [4]], win_size=[[27], [0]], groups=(8, 4))
+
+
+def _model(family="pcf", dtype=torch.bfloat16, seed=0, **kw):
+    torch.manual_seed(seed)
+    kw = dict(SMALL, **kw)
+    if family == "mfa":
+        kw.pop("groups")
+    model = (models.PCF_NATransformer if family == "pcf" else models.MFA_NATransformer)(na="fused_qkv", dtype=dtype, **kw).cuda().eval()
+    gen = torch.Generator().manual_seed(seed)
+    with torch.no_grad():
+        for m in model.modules():
+            if isinstance(m, torch.nn.BatchNorm1d):                                     # statistics as training leaves them
+                m.running_mean.copy_(0.1 * torch.randn(m.num_features, generator=gen))
+                m.running_var.copy_(0.75 + 0.5 * torch.rand(m.num_features, generator=gen))
+    return model
+
+
+def _input(batch, frames, seed=1, chans=80):
+    return torch.randn(batch, chans, frames, generator=torch.Generator().manual_seed(seed)).cuda()
+
+
+def _both(model, x, lens=None, dtype=torch.bfloat16):
+    """The native call's embeddings (None where it leaves the model to the modules), and the modules'."""
+    with torch.no_grad(), torch.autocast("cuda", dtype=dtype):
+        native = models.embed_natively(model, x, lens)
+        handle = model.fc.register_forward_hook(lambda *a: None)                        # a hook keeps the modules in use
+        try:
+            modules = model(x, lens)
+        finally:
+            handle.remove()
+    return native, modules
+
+
+def _near(a, b, dtype=torch.bfloat16):
+    """Two 16-bit evaluations of a few layers: each is within a few units of eps of the exact value."""
+    return O.rel_l2(a.float(), b.float()) < (2e-2 if dtype == torch.bfloat16 else 2.5e-3)
+
+
+@pytest.mark.parametrize("groups", [16, 32])
+@pytest.mark.parametrize("batch,frames", [(3, 111), (16, 128), (17, 122), (80, 128)])
+def test_group_counts_without_kernels_of_their_own(groups, batch, frames):
+    """Weights in blocks of any number of groups but 2, 4 and 8 are multiplied as the dense matrices they are, in the split
+    launches of up to 1024 tokens as in the larger ones."""
+    model = _model(groups=(groups, 8), in_chans=64)
+    native, modules = _both(model, _input(batch, frames, chans=64))
+    assert native is not None and _near(native, modules)
