@@ -390,7 +390,7 @@ __device__ inline void finish(const LinearArgs &a, Rsrc out, int64_t m0, int row
         const f32x4 sc = *reinterpret_cast<const f32x4 *>(a.scale + c), of = *reinterpret_cast<const f32x4 *>(a.offset + c);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            v[r] = __builtin_fmaf(__builtin_fmaxf(v[r], 0.f), sc[r], of[r]);
+            v[r] = __builtin_fmaf(v[r] < 0.f ? 0.f : v[r], sc[r], of[r]);        // NaN stays
             if constexpr (END == kTanhNorm) v[r] = tanh_of(v[r]);
         }
     }

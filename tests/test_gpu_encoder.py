@@ -55,3 +55,28 @@ def test_group_counts_without_kernels_of_their_own(groups, batch, frames):
     model = _model(groups=(groups, 8), in_chans=64)
     native, modules = _both(model, _input(batch, frames, chans=64))
     assert native is not None and _near(native, modules)
+
+
+@pytest.mark.parametrize("batch,frames", [(3, 64), (40, 128), (180, 100)])
+@pytest.mark.parametrize("family", ["pcf", "mfa"])
+def test_nan_stays_in_its_utterance_and_is_not_lost(family, batch, frames):
+    """A frame without a number makes its utterance's embedding so, as in the modules; the others' stay what they were."""
+    model = _model(family, dtype=torch.float16)
+    x = _input(batch, frames)
+    clean, _ = _both(model, x, dtype=torch.float16)
+    broken = x.clone()
+    broken[1, 5, 7] = float("nan")
+    native, modules = _both(model, broken, dtype=torch.float16)
+    assert torch.isnan(modules[1]).all() and torch.isnan(native[1]).all()
+    rest = [i for i in range(batch) if i != 1]
+    assert torch.equal(native[rest], clean[rest])
+
+
+def test_overflow_is_not_lost():
+    """Values beyond fp16 become infinities, and what is made of them not a number, exactly where the modules' do."""
+    model = _model("mfa", dtype=torch.float16)
+    x = _input(4, 64)
+    x[2] *= 1e9
+    native, modules = _both(model, x, dtype=torch.float16)
+    assert not torch.isfinite(modules[2]).all()
+    assert torch.equal(torch.isfinite(native), torch.isfinite(modules))
