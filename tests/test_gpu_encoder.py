@@ -57,6 +57,21 @@ def test_group_counts_without_kernels_of_their_own(groups, batch, frames):
     assert native is not None and _near(native, modules)
 
 
+@pytest.mark.parametrize("groups", [0, 3, 16])
+@pytest.mark.parametrize("batch,frames", [(3, 111), (80, 128)])
+def test_layers_of_the_c_interface_are_dense_unless_2_4_or_8(groups, batch, frames):
+    """na1d_encoder_layer.groups: any other number says nothing about the weights.  (The models' own 16 or 32 groups have
+    zeros where the quarters of the hidden layer do not meet; dense weights do not.)"""
+    from na1d_amd import encoder
+    model = _model("mfa")
+    x = _input(batch, frames)
+    want, _ = _both(model, x)
+    for l in encoder._entries[model].plans[torch.bfloat16][1].layers:
+        l.groups = groups
+    got, _ = _both(model, x)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("batch,frames", [(3, 64), (40, 128), (180, 100)])
 @pytest.mark.parametrize("family", ["pcf", "mfa"])
 def test_nan_stays_in_its_utterance_and_is_not_lost(family, batch, frames):
