@@ -172,6 +172,8 @@ def embed(model, x, lens=None):
     kernels do not cover the model, its inputs or the mode: the caller then takes another path."""
     if model.training or not x.is_cuda or torch.is_grad_enabled() or not torch.is_autocast_enabled("cuda") or not plain_call(x):
         return None
+    if getattr(model, "_is_replica", False):        # of DataParallel: lives for one call and holds plain tensors, no parameters
+        return None
     if not all(plain(m, type(m)) for m in (model.pool_norm, model.fc)):
         return None                                 # called as modules otherwise: whatever hangs on them has to see the call
     dtype = torch.get_autocast_dtype("cuda")

@@ -95,3 +95,13 @@ def test_overflow_is_not_lost():
     native, modules = _both(model, x, dtype=torch.float16)
     assert not torch.isfinite(modules[2]).all()
     assert torch.equal(torch.isfinite(native), torch.isfinite(modules))
+
+
+def test_replicas_run():
+    """What DataParallel makes of a model for each call: copies whose weights are plain tensors."""
+    model = _model()
+    x = _input(3, 64)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        replica = torch.nn.parallel.replicate(model, [0])[0]
+        assert not list(replica.parameters())
+        assert _near(replica(x), model(x))
