@@ -118,47 +118,100 @@ class _Entry:
 
     def __init__(self, model):
         mods = list(model.modules())
-        self.children = [(m._modules, list(m._modules.values())) for m in mods if m._modules]
+        self.children = [(m._modules, list(m._modules.values())) for m in mods]
+        self.kinds = [(m, type(m)) for m in mods]
+        self.methods = [m.__dict__ for m in mods if hasattr(m, "forward_tokens")]
         self.tensors = [d for m in mods for d in (m._parameters, m._buffers) if d]
         self.attn = [layer.attn for block in model.blocks for layer in block.blocks] if hasattr(model, "blocks") else []
-        self.plans = {}                             # dtype -> (state of the tensors, plan or None)
+        self.plans = {}                             # (dtype, device) -> (state of the tensors, plan or None)
 
     def same_modules(self):
-        return all(len(d) == len(c) and all(a is b for a, b in zip(d.values(), c)) for d, c in self.children)
+        return (all(len(d) == len(c) and all(a is b for a, b in zip(d.values(), c)) for d, c in self.children)
+                and all(type(m) is k for m, k in self.kinds) and not any("forward_tokens" in d for d in self.methods))
 
-    def plan(self, model, dtype):
+    def plan(self, model, dtype, device):
         state = [(t, t._version, t.data_ptr()) for d in self.tensors for t in d.values() if t is not None]
-        have = self.plans.get(dtype)
+        have = self.plans.get((dtype, device))
         if have is not None and len(have[0]) == len(state) and all(
                 a[0] is b[0] and a[1] == b[1] and a[2] == b[2] for a, b in zip(have[0], state)):
             return have[1]
         if torch.cuda.is_current_stream_capturing():          # it would record the preparation, not do it
             return None
-        plan = _Plan(model, dtype) if _fits(model) else None
+        plan = _Plan(model, dtype) if _fits(model, device) else None
         torch.cuda.current_stream().synchronize()             # the next call may come on another stream
-        self.plans[dtype] = (state, plan)
+        self.plans[dtype, device] = (state, plan)
         return plan
 
 
 _entries = weakref.WeakKeyDictionary()              # model -> _Entry
 
 
-def _fits(model):
-    """Whether the kernels cover the model's sizes (they are built for the sizes of the published models)."""
+def _own(m, *classes):
+    """Whether module ``m`` is of these classes, with their way through tokens and no other."""
+    return type(m) in classes and "forward_tokens" not in m.__dict__
+
+
+def _as_built(model):
+    """Whether the model's pass over tokens is the one that the kernels compute."""
+    from .models import _NATransformer as base
+    return all(getattr(type(model), n) is getattr(base, n) and n not in model.__dict__ for n in ("_forward_tokens", "_tokens_path"))
+
+
+def _fits(model, device):
+    """Whether the kernels compute what the modules would: their own classes, at the sizes of the published models (those
+    the kernels are built for), with parameters of their own in fp32 on the input's device."""
     from . import models as M
-    layers = [layer for block in model.blocks for layer in block.blocks]
-    conv = (model.patch_embeds[0] if model.channels_first else model.patch_embed).proj
-    return (model.embed_dim == DIM and type(model.pool) is M.AttentiveStatisticsPooling
-            and type(model.fc) is nn.Linear and model.fc.bias is not None and model.fc.in_features == 2 * model.proj.conv.out_channels
-            and (type(model.pool_norm) is nn.Identity or type(model.pool_norm) is M.BatchNorm1d and model.pool_norm.affine
-                 and model.pool_norm.running_mean is not None)
-            and all(layer.mlp.fc1.weight.shape[0] == HIDDEN for layer in layers)
-            and model.pool.tdnn.conv.out_channels == POOL_HIDDEN and model.proj.conv.out_channels % 256 == 0
-            and model.fc.out_features % 16 == 0 and conv.in_channels * model.patch_size % 32 == 0
-            and conv.in_channels * model.patch_size <= DIM
-            and all(layer.attn.num_heads and DIM % (8 * layer.attn.num_heads) == 0 and DIM // layer.attn.num_heads <= 128
-                    for layer in layers)
-            and all(p.dtype == torch.float32 for p in model.parameters()))
+    def held(t, *shape):
+        return t is not None and t.dtype == torch.float32 and t.device == device and t.shape == shape
+
+    def norm(bn, channels):
+        return (_own(bn, M.BatchNorm1d) and all(held(bn._parameters.get(n), channels) for n in ("weight", "bias"))
+                and all(held(bn._buffers.get(n), channels) for n in ("running_mean", "running_var")))
+
+    def projection(p, outputs, inputs, kernel=(), bias=True):
+        """`kernel`: () for a linear layer, else the length of a convolution's."""
+        if not _own(p, *((M.PatchConv, M.Conv1x1) if kernel else (M.TokenLinear, nn.Linear))):
+            return False
+        groups = p.groups if kernel else 1
+        return (outputs % groups == 0 and inputs % groups == 0 and held(p._parameters.get("weight"), outputs, inputs // groups, *kernel)
+                and (held(p._parameters.get("bias"), outputs) if bias else p._parameters.get("bias") is None))
+
+    cf = model.channels_first
+    token = (1,) if cf else ()
+    if model.embed_dim != DIM or not all(_own(block, M.NATFBlock) for block in model.blocks):
+        return False
+    for layer in (layer for block in model.blocks for layer in block.blocks):
+        if not (_own(layer, M.NATFLayer) and _own(layer.attn, M.NAttention if layer.local else M.GlobalAttention) and _own(layer.mlp, M.Mlp)):
+            return False
+        a, mlp, norms = layer.attn, layer.mlp, (layer.norm1, layer.norm2)
+        if not cf:
+            if not all(_own(n, M.TokenBatchNorm) for n in norms):
+                return False
+            norms = tuple(n.norm for n in norms)
+        if not (a.channels_first == cf and a.num_heads >= 1 and DIM % (8 * a.num_heads) == 0 and DIM // a.num_heads <= 128
+                and all(norm(n, DIM) for n in norms) and projection(a.qkv, 3 * DIM, DIM, token) and projection(a.proj, DIM, DIM, token)
+                and projection(mlp.fc1, HIDDEN, DIM, token) and projection(mlp.fc2, DIM, HIDDEN, token)):
+            return False
+        if not (held(a._parameters.get("relative_position_bias"), 1, a.num_heads, 1, a.win_size) if layer.local
+                else projection(a.linear_pos, DIM, DIM, token, bias=False)):
+            return False
+    embeds = list(model.patch_embeds) if cf else [model.patch_embed]
+    if len(embeds) != (len(model.blocks) if cf else 1) or not all(_own(e, M.PatchEmbed) and norm(e.norm, DIM) for e in embeds):
+        return False
+    chans, patch = embeds[0].proj.in_channels, model.patch_size
+    if chans * patch % 32 or chans * patch > DIM or not all(projection(e.proj, DIM, chans, (patch,)) for e in embeds):
+        return False
+    pool, wide = model.pool, model.proj.conv.out_channels
+    if not (wide % 256 == 0 and norm(model.norm, DIM * len(model.blocks)) and _own(model.proj, M.TDNNBlock)
+            and projection(model.proj.conv, wide, DIM * len(model.blocks), (1,)) and norm(model.proj.norm, wide)):
+        return False
+    if not (_own(pool, M.AttentiveStatisticsPooling) and pool.eps == 1e-12 and _own(pool.tdnn, M.TDNNBlock)
+            and projection(pool.tdnn.conv, POOL_HIDDEN, 3 * wide, (1,)) and norm(pool.tdnn.norm, POOL_HIDDEN)
+            and projection(pool.conv, wide, POOL_HIDDEN, (1,))):
+        return False
+    if not (type(model.pool_norm) is nn.Identity or norm(model.pool_norm, 2 * wide) and not model.pool_norm.training):
+        return False
+    return type(model.fc) is nn.Linear and model.fc.out_features % 16 == 0 and projection(model.fc, model.fc.out_features, 2 * wide)
 
 
 def plans_of(model):
@@ -176,12 +229,12 @@ def embed(model, x, lens=None):
         return None
     if not all(plain(m, type(m)) for m in (model.pool_norm, model.fc)):
         return None                                 # called as modules otherwise: whatever hangs on them has to see the call
+    if not _as_built(model):
+        return None
     dtype = torch.get_autocast_dtype("cuda")
     if dtype not in (torch.bfloat16, torch.float16) or x.dim() != 3 or x.dtype not in (torch.float32, torch.bfloat16, torch.float16):
         return None
     if lens is not None and (lens.dtype != torch.float32 or lens.device != x.device or lens.shape != (x.shape[0],)):
-        return None
-    if next(model.parameters()).device != x.device:
         return None
     if torch.cuda.current_device() != x.device.index:      # plans are made, and launches go, where the tensors are
         with torch.cuda.device(x.device):
@@ -191,9 +244,9 @@ def embed(model, x, lens=None):
         entry = _entries[model] = _Entry(model)
     if any((a.na != "fused_qkv") if hasattr(a, "na") else (a.dense != "native") for a in entry.attn):
         return None
-    plan = entry.plan(model, dtype)
+    plan = entry.plan(model, dtype, x.device)
     n, chans, frames = x.shape
-    if plan is None or chans != plan.encoder.in_chans or plan.keep[0].device != x.device:
+    if plan is None or chans != plan.encoder.in_chans:
         return None
     lib = _lib.load()
     ref = ctypes.byref(plan.encoder)

@@ -1,0 +1,93 @@
+"""Which models the native embedding call takes: decided on the host, so checked without a GPU."""
+import copy
+import types
+
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.utils.parametrize  # noqa: F401
+
+from na1d_amd import encoder, models
+
+CPU = torch.device("cpu")
+SMALL = dict(depths=(1, 1), num_heads=[[16], [4]], win_size=[[27], [0]], na="fused_qkv")
+
+
+def _model(family="pcf", **kw):
+    torch.manual_seed(0)
+    kw = dict(SMALL, **kw)
+    return (models.PCF_NATransformer(groups=(8, 4), **kw) if family == "pcf" else models.MFA_NATransformer(**kw)).eval()
+
+
+def _subclass(cls, **methods):
+    return type("Sub" + cls.__name__, (cls,), methods)
+
+
+def _reclass(m, **methods):
+    m.__class__ = _subclass(type(m), **methods)
+
+
+def _weight_norm(m):
+    """What torch.nn.utils.weight_norm leaves: the weight is a plain attribute that a hook works out."""
+    w = m.weight.detach()
+    del m._parameters["weight"]
+    m.weight = w
+
+
+CHANGES = {
+    "layer of another class": lambda m: _reclass(m.blocks[0].blocks[0], forward_tokens=lambda self, x, *a: x),
+    "block of another class": lambda m: _reclass(m.blocks[1], forward_tokens=lambda self, x, *a: x),
+    "attention of another class": lambda m: _reclass(m.blocks[1].blocks[0].attn),
+    "MLP of another class": lambda m: _reclass(m.blocks[0].blocks[0].mlp),
+    "patch embedding of another class": lambda m: _reclass((m.patch_embeds[0] if m.channels_first else m.patch_embed)),
+    "a layer's own method": lambda m: setattr(m.blocks[0].blocks[0], "forward_tokens", lambda x, *a: x),
+    "a model's own method": lambda m: setattr(m, "_forward_tokens", types.MethodType(lambda self, *a: None, m)),
+    "model of another class": lambda m: _reclass(m, _forward_tokens=lambda self, *a: None),
+    "projection of another kind": lambda m: setattr(m.blocks[0].blocks[0].mlp, "fc1", nn.Sequential(m.blocks[0].blocks[0].mlp.fc1)),
+    "projection without a bias": lambda m: setattr(m.blocks[0].blocks[0].mlp.fc2, "bias", None),
+    "attention's projection without a bias": lambda m: setattr(m.blocks[1].blocks[0].attn.proj, "bias", None),
+    "pooling without a bias": lambda m: setattr(m.pool.tdnn.conv, "bias", None),
+    "head without a bias": lambda m: setattr(m.fc, "bias", None),
+    "projection of another size": lambda m: setattr(m.blocks[0].blocks[0].mlp, "fc2", type(m.blocks[0].blocks[0].mlp.fc2)(512, 256)),
+    "norm without statistics": lambda m: setattr(m.norm, "running_mean", None),
+    "norm without weights": lambda m: setattr(m.proj.norm, "weight", None),
+    "pooled norm in training": lambda m: m.pool_norm.train(),
+    "pooled norm of another kind": lambda m: setattr(m, "pool_norm", nn.LayerNorm(m.fc.in_features)),
+    "pooling of another class": lambda m: _reclass(m.pool),
+    "pooling's threshold": lambda m: setattr(m.pool, "eps", 1e-6),
+    "window without its bias": lambda m: setattr(m.blocks[0].blocks[0].attn, "win_size", 25),
+    "weight that is no parameter": lambda m: _weight_norm(m.blocks[0].blocks[0].attn.qkv),
+    "16-bit parameters": lambda m: m.blocks[0].blocks[0].attn.qkv.to(torch.bfloat16),
+    "double statistics": lambda m: m.pool_norm.double(),
+    "a layer on another device": lambda m: m.fc.to("meta"),
+    "statistics on another device": lambda m: m.norm._buffers.update(running_var=m.norm.running_var.to("meta")),
+}
+
+
+@pytest.mark.parametrize("family", ["pcf", "mfa"])
+def test_models_as_constructed_fit(family):
+    model = _model(family)
+    assert encoder._as_built(model) and encoder._fits(model, CPU) and not encoder._fits(model, torch.device("cuda", 0))
+    assert encoder._fits(_model(family, poolnorm=False), CPU) and not encoder._fits(_model(family, asp=False), CPU)
+    assert not encoder._fits(_model(family, embed_dim=128), CPU) and not encoder._fits(_model(family, patch_size=5), CPU)
+    assert encoder._fits(copy.deepcopy(model), CPU)
+
+
+@pytest.mark.parametrize("family", ["pcf", "mfa"])
+@pytest.mark.parametrize("change", sorted(CHANGES))
+def test_what_the_kernels_do_not_know_stays_with_the_modules(change, family):
+    model = _model(family)
+    CHANGES[change](model)
+    assert not (encoder._as_built(model) and encoder._fits(model, CPU))
+
+
+@pytest.mark.parametrize("change", ["layer of another class", "a layer's own method", "projection of another kind", "parametrized weight"])
+def test_changes_after_the_first_call_are_seen(change):
+    model = _model()
+    entry = encoder._Entry(model)
+    assert entry.same_modules()
+    if change in CHANGES:
+        CHANGES[change](model)
+    else:
+        nn.utils.parametrize.register_parametrization(model.blocks[0].blocks[0].attn.qkv, "weight", nn.Identity())
+    assert not entry.same_modules()

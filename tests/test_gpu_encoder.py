@@ -66,7 +66,7 @@ def test_layers_of_the_c_interface_are_dense_unless_2_4_or_8(groups, batch, fram
     model = _model("mfa")
     x = _input(batch, frames)
     want, _ = _both(model, x)
-    for l in encoder._entries[model].plans[torch.bfloat16][1].layers:
+    for l in encoder.plans_of(model)[0].layers:
         l.groups = groups
     got, _ = _both(model, x)
     assert torch.equal(got, want)
@@ -105,3 +105,26 @@ def test_replicas_run():
         replica = torch.nn.parallel.replicate(model, [0])[0]
         assert not list(replica.parameters())
         assert _near(replica(x), model(x))
+
+
+def test_models_that_do_not_fit_run_as_they_did():
+    """A layer of a class of its own is called, a projection without a bias runs, tensors on two devices are refused."""
+    x = _input(3, 64)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        model = _model()
+        before = model(x)
+        layer = model.blocks[1].blocks[0]
+        layer.__class__ = type("Skipped", (models.NATFLayer,), {"forward_tokens": lambda self, x, *a: 0.5 * x})
+        assert models.embed_natively(model, x) is None and not _near(model(x), before)
+        model = _model()
+        model.blocks[0].blocks[0].mlp.fc2.bias = None
+        assert models.embed_natively(model, x) is None
+        a = model(x)
+        model.blocks[0].blocks[0].mlp.fc2.bias = torch.nn.Parameter(torch.zeros(256, device="cuda"))
+        assert models.embed_natively(model, x) is not None and _near(model(x), a)
+        model.fc.cpu()
+        assert models.embed_natively(model, x) is None
+        with pytest.raises(RuntimeError):
+            model(x)
+        model.fc.cuda()
+        assert _near(model(x), a)
