@@ -113,6 +113,11 @@ class _Plan:
         return t.data_ptr()
 
 
+# The modules' numbers that a plan is made of.
+_NUMBERS = ("channels_first", "embed_dim", "patch_size", "attn_global", "local", "num_heads", "scale", "groups", "win_size", "left", "dilation",
+            "eps", "training")
+
+
 class _Entry:
     """What is kept for a model: where its tensors are found, and the plans made of their present values."""
 
@@ -122,8 +127,9 @@ class _Entry:
         self.kinds = [(m, type(m)) for m in mods]
         self.methods = [m.__dict__ for m in mods if hasattr(m, "forward_tokens")]
         self.tensors = [d for m in mods for d in (m._parameters, m._buffers) if d]
+        self.numbers = [(m.__dict__, n) for m in mods for n in _NUMBERS if n in m.__dict__]
         self.attn = [layer.attn for block in model.blocks for layer in block.blocks] if hasattr(model, "blocks") else []
-        self.plans = {}                             # (dtype, device) -> (state of the tensors, plan or None)
+        self.plans = {}                             # (dtype, device) -> (state of the tensors, numbers, plan or None)
 
     def same_modules(self):
         return (all(len(d) == len(c) and all(a is b for a, b in zip(d.values(), c)) for d, c in self.children)
@@ -131,15 +137,16 @@ class _Entry:
 
     def plan(self, model, dtype, device):
         state = [(t, t._version, t.data_ptr()) for d in self.tensors for t in d.values() if t is not None]
+        numbers = [d.get(n) for d, n in self.numbers]
         have = self.plans.get((dtype, device))
-        if have is not None and len(have[0]) == len(state) and all(
+        if have is not None and have[1] == numbers and len(have[0]) == len(state) and all(
                 a[0] is b[0] and a[1] == b[1] and a[2] == b[2] for a, b in zip(have[0], state)):
-            return have[1]
+            return have[2]
         if torch.cuda.is_current_stream_capturing():          # it would record the preparation, not do it
             return None
         plan = _Plan(model, dtype) if _fits(model, device) else None
         torch.cuda.current_stream().synchronize()             # the next call may come on another stream
-        self.plans[dtype, device] = (state, plan)
+        self.plans[dtype, device] = (state, numbers, plan)
         return plan
 
 
@@ -217,7 +224,7 @@ def _fits(model, device):
 def plans_of(model):
     """The plans a captured graph of this model reads from (whoever keeps such a graph keeps them too)."""
     entry = _entries.get(model)
-    return [] if entry is None else [plan for _, plan in entry.plans.values() if plan is not None]
+    return [] if entry is None else [plan for *_, plan in entry.plans.values() if plan is not None]
 
 
 def embed(model, x, lens=None):

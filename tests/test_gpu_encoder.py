@@ -128,3 +128,47 @@ def test_models_that_do_not_fit_run_as_they_did():
             model(x)
         model.fc.cuda()
         assert _near(model(x), a)
+
+
+def _dilation(m):
+    m.blocks[0].blocks[0].attn.dilation = 2
+
+
+def _scale(m):
+    m.blocks[0].blocks[0].attn.scale *= 1.5
+
+
+def _dense_scale(m):
+    m.blocks[1].blocks[0].attn.scale *= 3.0
+
+
+def _left(m):
+    m.blocks[0].blocks[0].attn.left = 3
+
+
+def _heads(m):
+    m.blocks[1].blocks[0].attn.num_heads = 16
+
+
+def _eps(m):
+    m.norm.eps = 0.5
+
+
+def _head_eps(m):
+    m.pool_norm.eps = 0.5
+
+
+@pytest.mark.parametrize("change", [_dilation, _scale, _dense_scale, _left, _heads, _eps, _head_eps])
+def test_numbers_are_read_at_each_call(change):
+    """Scales, windows, dilations, heads and a norm's eps are attributes that a program may set between two calls; the copy is a
+    model made with them."""
+    model, x = _model(), _input(5, 90)
+    with torch.no_grad():                                                               # attentions that tell their keys apart
+        for block in model.blocks:
+            block.blocks[0].attn.qkv.weight.mul_(4.0)
+    before, _ = _both(model, x)
+    change(model)
+    fresh = copy.deepcopy(model)
+    native, _ = _both(model, x)
+    again, modules = _both(fresh, x)
+    assert _near(native, modules) and torch.equal(native, again) and not torch.equal(native, before)
