@@ -271,7 +271,9 @@ int64_t na1d_global_backward_workspace_bytes(int64_t B, int64_t H, int64_t T, in
  * A whole speaker-embedding model in inference (models/PCF_NATransformer.py:402-462, models/MFA_NATransformer.py:
  * 400-466): patch embeddings, encoder layers, the projection of all blocks' outputs, attentive statistics pooling
  * (models/Pooling.py:16-59) and the final linear layer, launched back to back on `stream` without a host decision or an
- * allocation in between.  Batch norms are given folded: into the projection behind them, or as an affine map per channel.
+ * allocation in between.  Batch norms are given folded into the projection behind them or as an affine map per channel,
+ * except those of dense layers' inputs and of the pooled vector, which come as they are, and the last layer's weight, which is
+ * the parameter itself: what a program changes there the next call sees.
  *
  * Weights are 16-bit (`dtype`) matrices [outputs, inputs] in fragment order: element (o, i) lies at
  *     ((o / 16 * (inputs / 32) + i / 32) * 64 + i % 32 / 8 * 16 + o % 16) * 8 + i % 8
@@ -279,6 +281,10 @@ int64_t na1d_global_backward_workspace_bytes(int64_t B, int64_t H, int64_t T, in
  * Tokens have 256 channels, the MLP 1024, the attention of the pooling 128; `wide` (channels of the projection) is a
  * multiple of 256, in_chans * patch a multiple of 32 and at most 256, `emb` a multiple of 16.
  */
+typedef struct na1d_encoder_norm {              /* (x - mean) / sqrt(var + eps) * weight + bias */
+    const float *weight, *bias, *mean, *var;
+    float eps;
+} na1d_encoder_norm;
 typedef struct na1d_encoder_layer {
     int32_t heads, window, left, dilation;      /* window 0: dense attention */
     int32_t groups;                             /* 2, 4, 8: the projections' weights are block-diagonal; else 1 */
@@ -290,7 +296,7 @@ typedef struct na1d_encoder_layer {
     const void *w_embed;                        /* [256, in_chans * patch] */
     const float *b_embed;
     const void *w_pos;                          /* dense: [256, 256] on the positions' rows; the layer's */
-    const float *gain, *shift;                  /* qkv projection reads x * gain + shift + w_pos . pos[t] */
+    na1d_encoder_norm norm;                     /* qkv projection reads norm(x) + w_pos . pos[t] */
 } na1d_encoder_layer;
 typedef struct na1d_encoder {
     int32_t dtype, layers, blocks, in_chans, patch, wide, emb;
@@ -301,9 +307,8 @@ typedef struct na1d_encoder {
     const float *b_wide, *a_wide, *c_wide;
     const void *w_att, *w_ctx, *w_logit;        /* pooling: [128, wide] on tokens, [128, 2 * wide] on (mean, std), [wide, 128] */
     const float *b_att, *a_att, *c_att;         /* tanh(relu(. + b_att) * a_att + c_att); the logits need no bias: softmax */
-    const float *a_pool, *c_pool;               /* affine map of the pooled (mean, std) [2 * wide] */
-    const void *w_fc;                           /* [emb, 2 * wide] */
-    const float *b_fc;
+    na1d_encoder_norm pool_norm;                /* of the pooled (mean, std) [2 * wide]; weight NULL: none */
+    const float *w_fc, *b_fc;                   /* [emb, 2 * wide] in fp32, rows of inputs; [emb] */
 } na1d_encoder;
 
 /* x: fp32 [N, in_chans, frames]; lens: fp32 [N] relative lengths in (0, 1] or NULL; out: 16-bit [N, emb].  The workspace

@@ -5,6 +5,16 @@
 namespace na1d {
 namespace enc {
 
+// What a batch norm with running statistics multiplies channels c .. c+3 by.  The few norms that no weight has been folded
+// with are read as the module holds them, so that the next call sees what a program writes there.
+__device__ inline f32x4 norm_gain(const na1d_encoder_norm &n, int c) {
+    const f32x4 w = *reinterpret_cast<const f32x4 *>(n.weight + c), v = *reinterpret_cast<const f32x4 *>(n.var + c);
+    f32x4 gain;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) gain[r] = w[r] * __builtin_amdgcn_rsqf(v[r] + n.eps);
+    return gain;
+}
+
 // =============================================================================
 // Between two attentions
 // =============================================================================
@@ -25,7 +35,8 @@ struct LayerArgs {
     const char *w_qkv;
     const float *b_qkv;
     char *qkv;
-    const float *gain, *posb;         // dense layers: qkv of x * gain + posb[token's place]
+    na1d_encoder_norm norm;           // dense layers: qkv of x * gain(norm) + posb[token's place] (posb != null)
+    const float *posb;
     int x_in_pitch, block_pitch, patch_width, M, T;
     uint32_t T_magic;
     int tail_groups, head_groups;     // block-diagonal weights: 8, 4, 2; otherwise 1
@@ -333,7 +344,10 @@ layer_kernel(LayerArgs a) {
         barrier_lds();
         w.write_rows(a.x_out, m0, rows, kRow);
     }
-    if (a.gain) {
+    if (a.posb) {
+        f32x4 gain[NTW];
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) gain[j] = norm_gain(a.norm, CW * wave + 16 * j + 4 * w.g);
         barrier_lds();
         const uint32_t first = (uint32_t)m0 % (uint32_t)a.T;     // place of the tile's first token in its utterance
 #pragma unroll
@@ -344,7 +358,7 @@ layer_kernel(LayerArgs a) {
 #pragma unroll
             for (int j = 0; j < NTW; ++j) {
                 const int c = CW * wave + 16 * j;
-                *w.at(w.q_lds, c, i) = narrow4<DT>(widen4<DT>(*w.at(w.q_lds, c, i)) * w.bias(a.gain, c) + w.bias(pos, c));
+                *w.at(w.q_lds, c, i) = narrow4<DT>(widen4<DT>(*w.at(w.q_lds, c, i)) * gain[j] + w.bias(pos, c));
             }
         }
     }
@@ -368,6 +382,7 @@ __device__ inline float tanh_of(float x) {
 // =============================================================================
 enum LinearEnd {
     kAffine,          // + bias, as fp32
+    kShift,           // + what a norm adds, as fp32
     kEmbedding,       // + bias, 16-bit
     kReluNorm,        // relu(. + bias) * scale + offset, 16-bit
     kTanhNorm,        // tanh(relu(. + add[m / T]) * scale + offset), 16-bit
@@ -377,12 +392,15 @@ struct LinearArgs {
     char *out;
     const float *bias, *scale, *offset;
     int x_pitch, out_pitch, inputs, outputs, M, T;      // T: rows that share a row of `bias` (kTanhNorm)
+    na1d_encoder_norm norm;                             // kShift
 };
 template <class DT, LinearEnd END>
 __device__ inline void finish(const LinearArgs &a, Rsrc out, int64_t m0, int row, int c, f32x4 v) {
     if constexpr (END == kTanhNorm) {
         const uint32_t u = (uint32_t)(m0 + row) / (uint32_t)a.T;
         v += *reinterpret_cast<const f32x4 *>(a.bias + (int64_t)u * a.outputs + c);
+    } else if constexpr (END == kShift) {
+        v += *reinterpret_cast<const f32x4 *>(a.norm.bias + c) - *reinterpret_cast<const f32x4 *>(a.norm.mean + c) * norm_gain(a.norm, c);
     } else {
         v += *reinterpret_cast<const f32x4 *>(a.bias + c);
     }
@@ -394,7 +412,7 @@ __device__ inline void finish(const LinearArgs &a, Rsrc out, int64_t m0, int row
             if constexpr (END == kTanhNorm) v[r] = tanh_of(v[r]);
         }
     }
-    if constexpr (END == kAffine)
+    if constexpr (END == kAffine || END == kShift)
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), out, row * a.out_pitch + 4 * c, 0, 0);
     else
         __builtin_amdgcn_raw_buffer_store_b64(narrow4<DT>(v), out, row * a.out_pitch + 2 * c, 0, 0);
@@ -505,11 +523,41 @@ __global__ void lengths_kernel(int32_t *t_valid, float *count, const float *lens
 // kPatchTokens tokens of `chans` channels to a workgroup through LDS: a wave reads along the frames of a channel, the
 // writes run along the rows.  Bound by memory; the work is split over the channels too, or a single utterance is a handful
 // of workgroups (3 s: 19.5 us in three workgroups of whole rows that divided twice for every value).
+// The launch's last slices bring the last layer's weight into fragment order and the pooled norm into an affine map, from
+// the module's own tensors at each call.  A single utterance takes 278 us so, 281 with the last product rounding the fp32
+// rows itself, 275 where both were kept from call to call and a write that no version counts went unseen.
 constexpr int kPatchTokens = 32;
+struct Head {
+    char *w;                        // 16-bit fragments of ...
+    const float *w_fc;              // ... [emb, inputs]
+    float *a_pool, *c_pool;         // [inputs]
+    na1d_encoder_norm norm;         // weight NULL: none
+    int emb, inputs, slices;        // slices of the launch before these
+};
+template <class DT>
+__device__ inline void prepare_head(const Head &h) {
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int64_t blocks = (int64_t)(gridDim.z - h.slices) * gridDim.y * gridDim.x;
+    const int64_t block = ((int64_t)(blockIdx.z - h.slices) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    const int steps = h.inputs / 32;
+    for (int64_t f = 4 * block + (threadIdx.x >> 6); f < (int64_t)h.emb / 16 * steps; f += 4 * blocks) {
+        const float *from = h.w_fc + (f / steps * 16 + n) * h.inputs + f % steps * 32 + 8 * g;
+        u32x4 w;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = Mma<DT>::pack(from[2 * k], from[2 * k + 1]);
+        *reinterpret_cast<u32x4 *>(h.w + f * kFrag + lane * 16) = w;
+    }
+    for (int64_t c = block * 256 + threadIdx.x; c < h.inputs; c += blocks * 256) {
+        const float gain = h.norm.weight ? h.norm.weight[c] * __builtin_amdgcn_rsqf(h.norm.var[c] + h.norm.eps) : 1.f;
+        h.a_pool[c] = gain;
+        h.c_pool[c] = h.norm.weight ? __builtin_fmaf(-h.norm.mean[c], gain, h.norm.bias[c]) : 0.f;
+    }
+}
 template <class DT>
 __global__ void __launch_bounds__(256)
 patch_kernel(uint32_t *__restrict__ out, const float *__restrict__ x, int in_chans, int chans, int frames, int patch, int T, uint32_t patch_magic,
-             uint32_t width_magic) {
+             uint32_t width_magic, Head head) {
+    if ((int)blockIdx.z >= head.slices) return prepare_head<DT>(head);
     extern __shared__ __attribute__((aligned(16))) char smem[];
     float *tile = reinterpret_cast<float *>(smem);               // [chans][kPatchTokens * patch + 1]
     const int span = kPatchTokens * patch, pitch = span + 1, t0 = blockIdx.x * kPatchTokens, nt = min(kPatchTokens, T - t0), c_first = blockIdx.z * chans;
@@ -783,7 +831,7 @@ template <class DT, LinearEnd END> int launch_linear(const LinearArgs &a, hipStr
 // The workspace's tensors, one behind the other.
 struct Buffers {
     int64_t bytes = 0;
-    int64_t x, qkv, attn, blocks, patches, pos, h, hidden, stats, rounded, context, pooled, t_valid, count, x1, parts;
+    int64_t x, qkv, attn, blocks, patches, pos, h, hidden, stats, rounded, context, pooled, t_valid, count, x1, parts, w_fc, pool_map;
     int64_t take(int64_t n) {
         const int64_t at = bytes;
         bytes += (n + 255) / 256 * 256;
@@ -807,6 +855,8 @@ struct Buffers {
         count = take(N * 4);
         x1 = take(M <= kSplitTokens ? M * kRow : 0);
         parts = take(M <= kSplitTokens ? 4 * M * kDim * 4 : 0);
+        w_fc = take((int64_t)e.emb * 2 * e.wide * 2);
+        pool_map = take((int64_t)2 * 2 * e.wide * 4);
     }
 };
 inline int dense_layers(const na1d_encoder &e) {
@@ -838,8 +888,12 @@ int encode(const na1d_encoder &e, char *out, const float *x, const float *lens, 
         const int chans = e.in_chans % 16 == 0 ? 16 : e.in_chans, half = chans * e.patch / 2;
         const size_t lds = (size_t)chans * (kPatchTokens * e.patch + 1) * sizeof(float);
         if (!allow_lds(patch_kernel<DT>, lds)) return NA1D_ERR_LAUNCH;
-        patch_kernel<DT><<<dim3((unsigned)((T + kPatchTokens - 1) / kPatchTokens), (unsigned)N, (unsigned)(e.in_chans / chans)), 256, lds, s>>>(
-            reinterpret_cast<uint32_t *>(ws + b.patches), x, e.in_chans, chans, (int)frames, e.patch, (int)T, div_magic(e.patch), div_magic(half));
+        const int slices = e.in_chans / chans, inputs = 2 * e.wide;
+        const int64_t x_blocks = (T + kPatchTokens - 1) / kPatchTokens, packing = ((int64_t)e.emb / 16 * (inputs / 32) + 3) / 4;     // a fragment to a wave
+        const unsigned more = (unsigned)std::min<int64_t>(1024, (packing + x_blocks * N - 1) / (x_blocks * N));
+        patch_kernel<DT><<<dim3((unsigned)x_blocks, (unsigned)N, slices + more), 256, lds, s>>>(
+            reinterpret_cast<uint32_t *>(ws + b.patches), x, e.in_chans, chans, (int)frames, e.patch, (int)T, div_magic(e.patch), div_magic(half),
+            Head{ws + b.w_fc, e.w_fc, reinterpret_cast<float *>(ws + b.pool_map), reinterpret_cast<float *>(ws + b.pool_map) + inputs, e.pool_norm, e.emb, inputs, slices});
         NA1D_TRY(launch_status());
     }
     int dense = 0;
@@ -850,12 +904,12 @@ int encode(const na1d_encoder &e, char *out, const float *x, const float *lens, 
         a.x = (const char *)e.pos;
         a.w = (const char *)l.w_pos;
         a.out = ws + b.pos + dense++ * T * kDim * 4;
-        a.bias = l.shift;
+        a.norm = l.norm;
         a.x_pitch = kRow;
         a.out_pitch = 4 * kDim;
         a.inputs = a.outputs = kDim;
         a.M = (int)T;
-        NA1D_TRY(launch_linear<DT, kAffine>(a, s));
+        NA1D_TRY(launch_linear<DT, kShift>(a, s));
     }
     dense = 0;
     int block = 0;
@@ -903,7 +957,7 @@ int encode(const na1d_encoder &e, char *out, const float *x, const float *lens, 
             a.b_qkv = l.b_qkv;
             a.head_groups = known_groups(l.groups);
             if (!l.window) {
-                a.gain = l.gain;
+                a.norm = l.norm;
                 a.posb = reinterpret_cast<const float *>(ws + b.pos + dense++ * T * kDim * 4);
             }
         }
@@ -947,16 +1001,17 @@ int encode(const na1d_encoder &e, char *out, const float *x, const float *lens, 
     d.w = (const char *)e.w_att, d.bias = reinterpret_cast<const float *>(ws + b.context), d.scale = e.a_att, d.offset = e.c_att;
     d.out = ws + b.hidden, d.out_pitch = 256, d.outputs = 128;
     NA1D_TRY(launch_linear<DT, kTanhNorm>(d, s));
-    PoolArgs p{ws + b.h, ws + b.hidden, (const char *)e.w_logit, count, reinterpret_cast<const float *>(ws + b.stats), e.a_pool, e.c_pool,
-               ws + b.pooled, (int)T, e.wide};
+    PoolArgs p{ws + b.h, ws + b.hidden, (const char *)e.w_logit, count, reinterpret_cast<const float *>(ws + b.stats),
+               reinterpret_cast<const float *>(ws + b.pool_map), reinterpret_cast<const float *>(ws + b.pool_map) + 2 * e.wide, ws + b.pooled, (int)T, e.wide};
     pool_kernel<DT><<<dim3((unsigned)(e.wide / 64), (unsigned)N), kThreads, 0, s>>>(p);
     NA1D_TRY(launch_status());
     LinearArgs f{};
     f.x = ws + b.pooled, f.x_pitch = 4 * e.wide, f.inputs = 2 * e.wide, f.M = (int)N;
-    f.w = (const char *)e.w_fc, f.bias = e.b_fc, f.out = out, f.out_pitch = 2 * e.emb, f.outputs = e.emb;
+    f.w = ws + b.w_fc, f.bias = e.b_fc, f.out = out, f.out_pitch = 2 * e.emb, f.outputs = e.emb;
     return launch_linear<DT, kEmbedding>(f, s);
 }
 
+inline bool norm_whole(const na1d_encoder_norm &n) { return n.weight && n.bias && n.mean && n.var; }
 // Sizes the kernels take (everything else is the caller's to run another way).
 bool encoder_ok(const na1d_encoder &e, int64_t N, int64_t frames) {
     if (e.layers < 1 || e.blocks < 1 || e.patch < 1 || e.in_chans < 1 || e.wide < 256 || e.emb < 16 || frames < e.patch) return false;
@@ -970,10 +1025,11 @@ bool encoder_ok(const na1d_encoder &e, int64_t N, int64_t frames) {
         const na1d_encoder_layer &l = e.layer[i];
         if (l.heads < 1 || kDim % l.heads || kDim / l.heads % 8 || kDim / l.heads > 128 || l.window < 0 || l.window > NA1D_MAX_WINDOW) return false;
         if (l.window && (l.left < 0 || l.left >= l.window || l.dilation < 1)) return false;
-        if (!l.window && (!e.pos || e.pos_rows < T || !l.gain || !l.shift || !l.w_pos)) return false;
+        if (!l.window && (!e.pos || e.pos_rows < T || !norm_whole(l.norm) || !l.w_pos)) return false;
         if (!l.w_qkv || !l.w_proj || !l.w_fc1 || !l.w_fc2 || (l.embeds && !l.w_embed)) return false;
         blocks += l.block_end != 0;
     }
+    if (e.pool_norm.weight && !norm_whole(e.pool_norm)) return false;
     return blocks == e.blocks && e.layer[0].embeds && e.layer[e.layers - 1].block_end;
 }
 int64_t workspace_bytes(const na1d_encoder &e, int64_t N, int64_t frames) {

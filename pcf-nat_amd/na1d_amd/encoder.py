@@ -19,17 +19,21 @@ _P, _I, _F = ctypes.c_void_p, ctypes.c_int32, ctypes.c_float
 DIM, HIDDEN, POOL_HIDDEN = 256, 1024, 128          # channels the kernels are built for
 
 
+class _Norm(ctypes.Structure):                     # na1d_encoder_norm
+    _fields_ = [(n, _P) for n in "weight bias mean var".split()] + [("eps", _F)]
+
+
 class _Layer(ctypes.Structure):                    # na1d_encoder_layer
     _fields_ = ([(n, _I) for n in "heads window left dilation groups embeds block_end".split()] + [("scale", _F)]
-                + [(n, _P) for n in ("w_qkv w_proj w_fc1 w_fc2 b_qkv b_proj b_fc1 b_fc2 rpb w_embed b_embed w_pos gain "
-                                     "shift").split()])
+                + [(n, _P) for n in ("w_qkv w_proj w_fc1 w_fc2 b_qkv b_proj b_fc1 b_fc2 rpb w_embed b_embed "
+                                     "w_pos").split()] + [("norm", _Norm)])
 
 
 class _Encoder(ctypes.Structure):                  # na1d_encoder
     _fields_ = ([(n, _I) for n in "dtype layers blocks in_chans patch wide emb".split()]
                 + [("layer", ctypes.POINTER(_Layer)), ("pos", _P), ("pos_rows", ctypes.c_int64)]
-                + [(n, _P) for n in ("w_wide b_wide a_wide c_wide w_att w_ctx w_logit b_att a_att c_att a_pool c_pool w_fc "
-                                     "b_fc").split()])
+                + [(n, _P) for n in ("w_wide b_wide a_wide c_wide w_att w_ctx w_logit b_att a_att c_att").split()]
+                + [("pool_norm", _Norm), ("w_fc", _P), ("b_fc", _P)])
 
 
 def fragment_order(w, dtype):
@@ -72,8 +76,7 @@ class _Plan:
                 wq, bq = M._dense_weight(attn.qkv), attn.qkv.bias
                 if order is not None:
                     wq, bq = wq.index_select(0, order), bq.index_select(0, order)
-                gain, shift = M._bn_affine(bn[0])
-                l.gain, l.shift, l.w_pos = vector(gain), vector(shift), matrix(M._dense_weight(attn.linear_pos))
+                l.norm, l.w_pos = self._norm(bn[0]), matrix(M._dense_weight(attn.linear_pos))
             l.w_qkv, l.b_qkv = matrix(wq), vector(bq)
             l.w_proj, l.b_proj = matrix(M._dense_weight(attn.proj)), vector(attn.proj.bias)
             w1, b1 = M._fold_norm(bn[1], layer.mlp.fc1)
@@ -102,11 +105,13 @@ class _Plan:
         w, (a, c) = M._dense_weight(tdnn.conv), M._bn_affine(tdnn.norm)
         e.w_att, e.w_ctx, e.b_att = matrix(w[:, :wide]), matrix(w[:, wide:]), vector(tdnn.conv.bias)
         e.a_att, e.c_att, e.w_logit = vector(a), vector(c), matrix(M._dense_weight(model.pool.conv))
-        if isinstance(model.pool_norm, nn.Identity):
-            a, c = torch.ones(2 * wide, device=w.device), torch.zeros(2 * wide, device=w.device)
-        else:
-            a, c = M._bn_affine(model.pool_norm)
-        e.a_pool, e.c_pool, e.w_fc, e.b_fc = vector(a), vector(c), matrix(model.fc.weight), vector(model.fc.bias)
+        if not isinstance(model.pool_norm, nn.Identity):
+            e.pool_norm = self._norm(model.pool_norm)
+        e.w_fc, e.b_fc = vector(model.fc.weight), vector(model.fc.bias)          # the parameters themselves
+
+    def _norm(self, bn):
+        """A norm's own tensors."""
+        return _Norm(*(self._hold(t.detach()) for t in (bn.weight, bn.bias, bn.running_mean, bn.running_var)), bn.eps)
 
     def _hold(self, t):
         self.keep.append(t)
@@ -169,7 +174,7 @@ def _fits(model, device):
     the kernels are built for), with parameters of their own in fp32 on the input's device."""
     from . import models as M
     def held(t, *shape):
-        return t is not None and t.dtype == torch.float32 and t.device == device and t.shape == shape
+        return t is not None and t.dtype == torch.float32 and t.device == device and t.shape == shape and t.is_contiguous()
 
     def norm(bn, channels):
         return (_own(bn, M.BatchNorm1d) and all(held(bn._parameters.get(n), channels) for n in ("weight", "bias"))

@@ -172,3 +172,38 @@ def test_numbers_are_read_at_each_call(change):
     native, _ = _both(model, x)
     again, modules = _both(fresh, x)
     assert _near(native, modules) and torch.equal(native, again) and not torch.equal(native, before)
+
+
+@pytest.mark.parametrize("name", ["fc.weight", "fc.bias", "pool_norm.weight", "pool_norm.bias", "pool_norm.running_mean", "pool_norm.running_var",
+                                  "blocks.1.blocks.0.norm1.weight", "blocks.1.blocks.0.norm1.bias", "blocks.1.blocks.0.norm1.running_mean",
+                                  "blocks.1.blocks.0.norm1.running_var", "blocks.0.blocks.0.attn.relative_position_bias"])
+@pytest.mark.parametrize("batch,frames", [(3, 64), (40, 128), (600, 16)])
+def test_what_the_modules_read_at_each_call_is_read_at_each_call(name, batch, frames):
+    """The head, the pooled norm, a dense layer's first norm and a window's bias are never copied: a write that torch counts
+    no version for (through .data) shows in the next call, and in the next replay of a graph."""
+    model, x = _model(), _input(batch, frames)
+    before, _ = _both(model, x)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16), torch.cuda.graph(graph):
+        captured = models.embed_natively(model, x)
+    t = model.get_parameter(name) if not name.rpartition(".")[2].startswith("running") else model.get_buffer(name)
+    version = t._version
+    t.data.mul_(1.5).add_(0.5 * torch.randn(t.shape, generator=torch.Generator().manual_seed(2)).cuda().abs())
+    assert t._version == version
+    native, modules = _both(model, x)
+    assert _near(native, modules) and not torch.equal(native, before)
+    for _ in range(2):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, native)
+
+
+@pytest.mark.parametrize("emb", [16, 64, 208, 256])
+@pytest.mark.parametrize("batch", [1, 17, 513])
+def test_embedding_sizes(emb, batch):
+    """The last layer at every remainder of its tiles of 16 rows and of the rounds of inputs."""
+    for poolnorm in (True, False):
+        model = _model("mfa", dtype=torch.float16, output_emb_size=emb, proj_channel=256 * (1 + emb % 3), poolnorm=poolnorm)
+        native, modules = _both(model, _input(batch, 16), dtype=torch.float16)
+        assert native.shape == (batch, emb) and _near(native, modules, torch.float16)
