@@ -129,7 +129,7 @@ class _Entry:
     def __init__(self, model):
         mods = list(model.modules())
         self.children = [(m._modules, list(m._modules.values())) for m in mods]
-        self.kinds = [(m, type(m)) for m in mods]
+        self.kinds = [(m, type(m)) for m in mods if m is not model]       # nothing here may keep the model itself
         self.methods = [m.__dict__ for m in mods if hasattr(m, "forward_tokens")]
         self.tensors = [d for m in mods for d in (m._parameters, m._buffers) if d]
         self.numbers = [(m.__dict__, n) for m in mods for n in _NUMBERS if n in m.__dict__]

@@ -1,6 +1,8 @@
 """Which models the native embedding call takes: decided on the host, so checked without a GPU."""
 import copy
+import gc
 import types
+import weakref
 
 import pytest
 import torch
@@ -91,3 +93,12 @@ def test_changes_after_the_first_call_are_seen(change):
     else:
         nn.utils.parametrize.register_parametrization(model.blocks[0].blocks[0].attn.qkv, "weight", nn.Identity())
     assert not entry.same_modules()
+
+
+def test_what_is_kept_for_a_model_does_not_keep_the_model():
+    model = _model()
+    encoder._entries[model] = encoder._Entry(model)
+    gone, held = weakref.ref(model), len(encoder._entries)
+    del model
+    gc.collect()
+    assert gone() is None and len(encoder._entries) == held - 1
