@@ -42,80 +42,106 @@ def fragment_order(w, dtype):
     return w.to(dtype).view(o // 16, 16, i // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
 
 
+def _stamps(tensors):
+    return [(t, t._version, t.data_ptr()) for t in tensors if t is not None]
+
+
+def _same(a, b):
+    return len(a) == len(b) and all(x[0] is y[0] and x[1] == y[1] and x[2] == y[2] for x, y in zip(a, b))
+
+
 class _Plan:
-    """The C structures of one model in one dtype, and the tensors they point into."""
+    """The C structures of one model in one dtype, and the tensors they point into.  What is derived from tensors that are
+    as they were for the plan `before` is taken over from there: a changed tensor costs what was made of it."""
 
-    def __init__(self, model, dtype):
+    def __init__(self, model, dtype, before=None):
         from . import models as M
-        self.keep = []
-        self.dtype = dtype
+        self.dtype, self.keep = dtype, []
+        self.made = {}                              # name -> (stamps of its sources, tensors made of them)
+        known = {} if before is None else before.made
 
-        def matrix(w):
-            return self._hold(fragment_order(w.detach(), dtype))
+        def derive(name, sources, build):
+            now = _stamps(sources)
+            have = known.get(name)
+            if have is None or not _same(have[0], now):
+                have = (now, build())
+            self.made[name] = have
+            return (t.data_ptr() for t in have[1])
 
-        def vector(v):
-            return self._hold(v.detach().float().contiguous())
+        def matrices(name, sources, build):         # build() -> weights [outputs, inputs]
+            return derive(name, sources, lambda: [fragment_order(w.detach(), dtype) for w in build()])
+
+        def product(name, sources, build):          # build() -> a weight and its bias
+            def both():
+                w, b = build()
+                return fragment_order(w.detach(), dtype), b.detach().float().contiguous()
+            return derive(name, sources, both)
+
+        def affine(name, bn):
+            return derive(name, M._bn_tensors(bn), lambda: [v.detach().contiguous() for v in M._bn_affine(bn)])
+
+        def own(p):                                 # a parameter itself
+            self.keep.append(p.detach())
+            return p.data_ptr()
+
+        def norm(bn):                               # a norm's own tensors
+            return _Norm(*map(own, M._bn_tensors(bn)), bn.eps)
 
         flat = [(block, i, layer) for block in model.blocks for i, layer in enumerate(block.blocks)]
         self.layers = (_Layer * len(flat))()
         for at, (l, (block, i, layer)) in enumerate(zip(self.layers, flat)):
-            attn, dim, cf = layer.attn, DIM, layer.attn.channels_first
+            attn, mlp, cf = layer.attn, layer.mlp, layer.attn.channels_first
             bn = [n.norm if isinstance(n, M.TokenBatchNorm) else n for n in (layer.norm1, layer.norm2)]
-            order = M._qkv_channel_order(dim, attn.groups, bn[0].weight.device) if cf else None
-            projections = (attn.qkv, attn.proj, layer.mlp.fc1, layer.mlp.fc2)
-            groups = {getattr(p, "groups", 1) for p in projections}
+            order = (lambda: M._qkv_channel_order(DIM, attn.groups, attn.qkv.weight.device)) if cf else lambda: None
+            groups = {getattr(p, "groups", 1) for p in (attn.qkv, attn.proj, mlp.fc1, mlp.fc2)}
             l.groups = groups.pop() if len(groups) == 1 else 1
             l.heads, l.scale = attn.num_heads, attn.scale
             l.block_end = i == len(block.blocks) - 1
+            qkv = [attn.qkv.weight, attn.qkv.bias]
             if layer.local:
                 l.window, l.left, l.dilation = attn.win_size, attn.left, attn.dilation
-                l.rpb = vector(attn.relative_position_bias.reshape(attn.num_heads, attn.win_size))
-                wq, bq = M._fold_norm(bn[0], attn.qkv, order)
+                l.rpb = own(attn.relative_position_bias)
+                l.w_qkv, l.b_qkv = product((at, "qkv"), qkv + M._bn_tensors(bn[0]), lambda: M._fold_norm(bn[0], attn.qkv, order()))
             else:
                 l.dilation = 1
-                wq, bq = M._dense_weight(attn.qkv), attn.qkv.bias
-                if order is not None:
-                    wq, bq = wq.index_select(0, order), bq.index_select(0, order)
-                l.norm, l.w_pos = self._norm(bn[0]), matrix(M._dense_weight(attn.linear_pos))
-            l.w_qkv, l.b_qkv = matrix(wq), vector(bq)
-            l.w_proj, l.b_proj = matrix(M._dense_weight(attn.proj)), vector(attn.proj.bias)
-            w1, b1 = M._fold_norm(bn[1], layer.mlp.fc1)
-            l.w_fc1, l.b_fc1 = matrix(w1), vector(b1)
-            l.w_fc2, l.b_fc2 = matrix(M._dense_weight(layer.mlp.fc2)), vector(layer.mlp.fc2.bias)
+                l.norm, (l.w_pos,) = norm(bn[0]), matrices((at, "pos"), [attn.linear_pos.weight], lambda: [M._dense_weight(attn.linear_pos)])
+                def reordered():
+                    w, b = M._dense_weight(attn.qkv), attn.qkv.bias
+                    return (w.index_select(0, order()), b.index_select(0, order())) if cf else (w, b)
+                l.w_qkv, l.b_qkv = product((at, "qkv"), qkv, reordered)
+            (l.w_proj,), l.b_proj = matrices((at, "proj"), [attn.proj.weight], lambda: [M._dense_weight(attn.proj)]), own(attn.proj.bias)
+            l.w_fc1, l.b_fc1 = product((at, "fc1"), [mlp.fc1.weight, mlp.fc1.bias] + M._bn_tensors(bn[1]), lambda: M._fold_norm(bn[1], mlp.fc1))
+            (l.w_fc2,), l.b_fc2 = matrices((at, "fc2"), [mlp.fc2.weight], lambda: [M._dense_weight(mlp.fc2)]), own(mlp.fc2.bias)
             if i == 0 and (model.channels_first or at == 0):
                 embed = model.patch_embeds[list(model.blocks).index(block)] if model.channels_first else model.patch_embed
                 conv = embed.proj
-                w = conv.weight.reshape(conv.out_channels, -1).float()
-                if conv.groups > 1:
-                    w = torch.block_diag(*w.view(conv.groups, conv.out_channels // conv.groups, -1))
-                a, b = M._bn_affine(embed.norm)
-                l.embeds, l.w_embed, l.b_embed = 1, matrix(w * a.unsqueeze(1)), vector(conv.bias.float() * a + b)
+                def patches():
+                    w = conv.weight.reshape(conv.out_channels, -1).float()
+                    if conv.groups > 1:
+                        w = torch.block_diag(*w.view(conv.groups, conv.out_channels // conv.groups, -1))
+                    a, b = M._bn_affine(embed.norm)
+                    return w * a.unsqueeze(1), conv.bias.float() * a + b
+                l.embeds = 1
+                l.w_embed, l.b_embed = product((at, "embed"), [conv.weight, conv.bias] + M._bn_tensors(embed.norm), patches)
         e = self.encoder = _Encoder()
-        conv = (model.patch_embeds[0] if model.channels_first else model.patch_embed).proj
+        conv, device = (model.patch_embeds[0] if model.channels_first else model.patch_embed).proj, model.fc.weight.device
         wide = model.proj.conv.out_channels
         e.dtype, e.layers, e.blocks, e.layer = _lib.dtype_tag(dtype), len(flat), len(model.blocks), self.layers
         e.in_chans, e.patch, e.wide, e.emb = conv.in_channels, model.patch_size, wide, model.fc.out_features
         if model.attn_global:
-            pos = M.sinusoid_table(DIM, 40000, False)[0].to(conv.weight.device)
-            e.pos, e.pos_rows = self._hold(pos.to(dtype).contiguous()), pos.shape[0]
-        w, b = M._fold_norm(model.norm, model.proj.conv)
-        a, c = M._bn_affine(model.proj.norm)
-        e.w_wide, e.b_wide, e.a_wide, e.c_wide = matrix(w), vector(b), vector(a), vector(c)
-        tdnn = model.pool.tdnn
-        w, (a, c) = M._dense_weight(tdnn.conv), M._bn_affine(tdnn.norm)
-        e.w_att, e.w_ctx, e.b_att = matrix(w[:, :wide]), matrix(w[:, wide:]), vector(tdnn.conv.bias)
-        e.a_att, e.c_att, e.w_logit = vector(a), vector(c), matrix(M._dense_weight(model.pool.conv))
+            table = model.eval_positions(device)
+            (e.pos,) = derive("positions", [] if table.is_inference() else [table], lambda: [(table[0].t() if model.channels_first else table[0]).to(dtype).contiguous()])
+            e.pos_rows = table.shape[2 if model.channels_first else 1]
+        w = model.proj.conv
+        e.w_wide, e.b_wide = product("wide", [w.weight, w.bias] + M._bn_tensors(model.norm), lambda: M._fold_norm(model.norm, w))
+        e.a_wide, e.c_wide = affine("wide norm", model.proj.norm)
+        tdnn, logit = model.pool.tdnn, model.pool.conv
+        e.w_att, e.w_ctx = matrices("pooling", [tdnn.conv.weight], lambda: M._dense_weight(tdnn.conv).split([wide, 2 * wide], 1))
+        e.b_att, (e.a_att, e.c_att) = own(tdnn.conv.bias), affine("pooling norm", tdnn.norm)
+        (e.w_logit,) = matrices("logits", [logit.weight], lambda: [M._dense_weight(logit)])
         if not isinstance(model.pool_norm, nn.Identity):
-            e.pool_norm = self._norm(model.pool_norm)
-        e.w_fc, e.b_fc = vector(model.fc.weight), vector(model.fc.bias)          # the parameters themselves
-
-    def _norm(self, bn):
-        """A norm's own tensors."""
-        return _Norm(*(self._hold(t.detach()) for t in (bn.weight, bn.bias, bn.running_mean, bn.running_var)), bn.eps)
-
-    def _hold(self, t):
-        self.keep.append(t)
-        return t.data_ptr()
+            e.pool_norm = norm(model.pool_norm)
+        e.w_fc, e.b_fc = own(model.fc.weight), own(model.fc.bias)
 
 
 # The modules' numbers that a plan is made of.
@@ -141,15 +167,14 @@ class _Entry:
                 and all(type(m) is k for m, k in self.kinds) and not any("forward_tokens" in d for d in self.methods))
 
     def plan(self, model, dtype, device):
-        state = [(t, t._version, t.data_ptr()) for d in self.tensors for t in d.values() if t is not None]
+        state = _stamps(t for d in self.tensors for t in d.values())
         numbers = [d.get(n) for d, n in self.numbers]
         have = self.plans.get((dtype, device))
-        if have is not None and have[1] == numbers and len(have[0]) == len(state) and all(
-                a[0] is b[0] and a[1] == b[1] and a[2] == b[2] for a, b in zip(have[0], state)):
+        if have is not None and have[1] == numbers and _same(have[0], state):
             return have[2]
         if torch.cuda.is_current_stream_capturing():          # it would record the preparation, not do it
             return None
-        plan = _Plan(model, dtype) if _fits(model, device) else None
+        plan = _Plan(model, dtype, have[2] if have is not None and have[1] == numbers else None) if _fits(model, device) else None
         torch.cuda.current_stream().synchronize()             # the next call may come on another stream
         self.plans[dtype, device] = (state, numbers, plan)
         return plan

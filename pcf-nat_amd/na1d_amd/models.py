@@ -695,6 +695,12 @@ class _NATransformer(nn.Module):
                 if m.bias is not None:
                     nn.init.constant_(m.bias, 0)
 
+    def eval_positions(self, device):
+        """The dense layers' positions in inference: a table for any length, made once."""
+        if self.pos_emb_eval is None or self.pos_emb_eval.device != device:
+            self.pos_emb_eval = sinusoid_table(self.embed_dim, 40000, self.channels_first).to(device)
+        return self.pos_emb_eval
+
     def forward(self, x, lens=None):
         """x: [N, in_chans, frames]; lens: relative lengths in (0, 1] or None.  Returns [N, output_emb_size]."""
         tin = x.shape[-1]
@@ -711,9 +717,8 @@ class _NATransformer(nn.Module):
             if self.training:
                 pos_emb = self.pos_emb
             else:
-                if self.pos_emb_eval is None or self.pos_emb_eval.device != x.device:
-                    self.pos_emb_eval = sinusoid_table(self.embed_dim, 40000, self.channels_first).to(x.device)
-                pos_emb = self.pos_emb_eval[:, :, :t] if self.channels_first else self.pos_emb_eval[:, :t, :]
+                table = self.eval_positions(x.device)
+                pos_emb = table[:, :, :t] if self.channels_first else table[:, :t, :]
                 if padding is not None:
                     pad = torch.arange(t, device=x.device).unsqueeze(0) >= (t - padding.to(x.device)).unsqueeze(1)
                     both = pad.unsqueeze(-1) | pad.unsqueeze(-2)

@@ -102,3 +102,28 @@ def test_what_is_kept_for_a_model_does_not_keep_the_model():
     del model
     gc.collect()
     assert gone() is None and len(encoder._entries) == held - 1
+
+
+@pytest.mark.parametrize("family", ["pcf", "mfa"])
+def test_a_changed_tensor_costs_what_was_made_of_it(family, monkeypatch):
+    """A plan takes over what the plan before made of unchanged tensors, the table of positions among it; what it holds of
+    the others is what a plan made from nothing holds."""
+    model = _model(family)
+    calls = []
+    table = models.sinusoid_table
+    monkeypatch.setattr(models, "sinusoid_table", lambda *a: calls.append(a) or table(*a))
+    plan = encoder._Plan(model, torch.bfloat16)
+    for change, renewed in ((lambda: model.blocks[0].blocks[0].mlp.fc1.weight.mul_(2), {(0, "fc1")}),
+                            (lambda: model.blocks[0].blocks[0].norm2.load_state_dict(model.blocks[0].blocks[0].norm2.state_dict()), {(0, "fc1")}),
+                            (lambda: model.norm.running_var.mul_(2), {"wide"}),
+                            (lambda: model.blocks[1].blocks[0].attn.linear_pos.weight.mul_(2), {(1, "pos")}),
+                            (lambda: model.fc.weight.mul_(2), set()),
+                            (lambda: setattr(model.pool.conv, "weight", nn.Parameter(2 * model.pool.conv.weight)), {"logits"})):
+        with torch.no_grad():
+            change()
+        after, fresh = encoder._Plan(model, torch.bfloat16, plan), encoder._Plan(model, torch.bfloat16)
+        assert {n for n in after.made if after.made[n] is not plan.made[n]} == renewed
+        assert all(torch.equal(a, b) for n in fresh.made for a, b in zip(after.made[n][1], fresh.made[n][1]))
+        plan = after
+    assert len(calls) == 1
+    assert len(plan.made) == len(encoder._Plan(model, torch.float16, None).made)

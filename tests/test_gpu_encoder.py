@@ -207,3 +207,18 @@ def test_embedding_sizes(emb, batch):
         model = _model("mfa", dtype=torch.float16, output_emb_size=emb, proj_channel=256 * (1 + emb % 3), poolnorm=poolnorm)
         native, modules = _both(model, _input(batch, 16), dtype=torch.float16)
         assert native.shape == (batch, emb) and _near(native, modules, torch.float16)
+
+
+def test_first_calls_and_changes_in_inference_mode():
+    """Plans and the table of positions may be made while torch tracks no versions of new tensors."""
+    model, x = _model(), _input(3, 64)
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.bfloat16):
+        first = models.embed_natively(model, x)
+    native, _ = _both(model, x)
+    assert torch.equal(first, native)
+    with torch.no_grad():
+        model.blocks[0].blocks[0].mlp.fc1.weight.mul_(2.0)
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.bfloat16):
+        second = models.embed_natively(model, x)
+    native, modules = _both(model, x)
+    assert torch.equal(second, native) and _near(native, modules) and not torch.equal(first, second)
