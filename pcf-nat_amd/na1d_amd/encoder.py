@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import weakref
+from operator import is_
 
 import torch
 import torch.nn as nn
@@ -146,37 +147,46 @@ class _Plan:
 
 # The modules' numbers that a plan is made of.
 _NUMBERS = ("channels_first", "embed_dim", "patch_size", "attn_global", "local", "num_heads", "scale", "groups", "win_size", "left", "dilation",
-            "eps", "training")
+            "eps")
 
 
 class _Entry:
     """What is kept for a model: where its tensors are found, and the plans made of their present values."""
 
     def __init__(self, model):
-        mods = list(model.modules())
-        self.children = [(m._modules, list(m._modules.values())) for m in mods]
-        self.kinds = [(m, type(m)) for m in mods if m is not model]       # nothing here may keep the model itself
+        mods = [m for m in model.modules() if m is not model]             # nothing here may keep the model itself
+        self.mods, self.kinds = mods, list(map(type, mods))
+        self.children = [m._modules for m in [model] + mods]
+        self.present = [list(d.values()) for d in self.children]
         self.methods = [m.__dict__ for m in mods if hasattr(m, "forward_tokens")]
-        self.tensors = [d for m in mods for d in (m._parameters, m._buffers) if d]
-        self.numbers = [(m.__dict__, n) for m in mods for n in _NUMBERS if n in m.__dict__]
+        self.parameters = [m._parameters for m in mods if m._parameters]
+        self.statistics = [m._buffers for m in mods if "running_mean" in m._buffers]
+        self.numbers = [(m.__dict__, n) for m in [model] + mods if not isinstance(m, nn.Conv1d)
+                        for n in _NUMBERS if n in m.__dict__]
         self.attn = [layer.attn for block in model.blocks for layer in block.blocks] if hasattr(model, "blocks") else []
-        self.plans = {}                             # (dtype, device) -> (state of the tensors, numbers, plan or None)
+        self.plans = {}                             # (dtype, device) -> (state, plan or None)
 
     def same_modules(self):
-        return (all(len(d) == len(c) and all(a is b for a, b in zip(d.values(), c)) for d, c in self.children)
-                and all(type(m) is k for m, k in self.kinds) and not any("forward_tokens" in d for d in self.methods))
+        return ([list(d.values()) for d in self.children] == self.present and list(map(type, self.mods)) == self.kinds
+                and not any("forward_tokens" in d for d in self.methods))
+
+    def state(self):
+        """Everything that a plan is made of, as it is now."""
+        tensors = [t for d in self.parameters for t in d.values()]
+        tensors += [d.get(n) for d in self.statistics for n in ("running_mean", "running_var")]
+        tensors = [t for t in tensors if t is not None]
+        return tensors, [t._version for t in tensors], [t.data_ptr() for t in tensors], [d.get(n) for d, n in self.numbers]
 
     def plan(self, model, dtype, device):
-        state = _stamps(t for d in self.tensors for t in d.values())
-        numbers = [d.get(n) for d, n in self.numbers]
-        have = self.plans.get((dtype, device))
-        if have is not None and have[1] == numbers and _same(have[0], state):
-            return have[2]
+        now = self.state()
+        before, plan = self.plans.get((dtype, device), (None, None))
+        if before is not None and now[1:] == before[1:] and len(now[0]) == len(before[0]) and all(map(is_, now[0], before[0])):
+            return plan
         if torch.cuda.is_current_stream_capturing():          # it would record the preparation, not do it
             return None
-        plan = _Plan(model, dtype, have[2] if have is not None and have[1] == numbers else None) if _fits(model, device) else None
+        plan = _Plan(model, dtype, plan if before is not None and now[3] == before[3] else None) if _fits(model, device) else None
         torch.cuda.current_stream().synchronize()             # the next call may come on another stream
-        self.plans[dtype, device] = (state, numbers, plan)
+        self.plans[dtype, device] = (now, plan)
         return plan
 
 
@@ -246,7 +256,7 @@ def _fits(model, device):
             and projection(pool.tdnn.conv, POOL_HIDDEN, 3 * wide, (1,)) and norm(pool.tdnn.norm, POOL_HIDDEN)
             and projection(pool.conv, wide, POOL_HIDDEN, (1,))):
         return False
-    if not (type(model.pool_norm) is nn.Identity or norm(model.pool_norm, 2 * wide) and not model.pool_norm.training):
+    if not (type(model.pool_norm) is nn.Identity or norm(model.pool_norm, 2 * wide)):
         return False
     return type(model.fc) is nn.Linear and model.fc.out_features % 16 == 0 and projection(model.fc, model.fc.out_features, 2 * wide)
 
@@ -254,7 +264,7 @@ def _fits(model, device):
 def plans_of(model):
     """The plans a captured graph of this model reads from (whoever keeps such a graph keeps them too)."""
     entry = _entries.get(model)
-    return [] if entry is None else [plan for *_, plan in entry.plans.values() if plan is not None]
+    return [] if entry is None else [plan for _, plan in entry.plans.values() if plan is not None]
 
 
 def embed(model, x, lens=None):
@@ -266,7 +276,7 @@ def embed(model, x, lens=None):
         return None
     if not all(plain(m, type(m)) for m in (model.pool_norm, model.fc)):
         return None                                 # called as modules otherwise: whatever hangs on them has to see the call
-    if not _as_built(model):
+    if not _as_built(model) or model.pool_norm.training:
         return None
     dtype = torch.get_autocast_dtype("cuda")
     if dtype not in (torch.bfloat16, torch.float16) or x.dim() != 3 or x.dtype not in (torch.float32, torch.bfloat16, torch.float16):

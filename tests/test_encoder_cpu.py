@@ -53,7 +53,6 @@ CHANGES = {
     "projection of another size": lambda m: setattr(m.blocks[0].blocks[0].mlp, "fc2", type(m.blocks[0].blocks[0].mlp.fc2)(512, 256)),
     "norm without statistics": lambda m: setattr(m.norm, "running_mean", None),
     "norm without weights": lambda m: setattr(m.proj.norm, "weight", None),
-    "pooled norm in training": lambda m: m.pool_norm.train(),
     "pooled norm of another kind": lambda m: setattr(m, "pool_norm", nn.LayerNorm(m.fc.in_features)),
     "pooling of another class": lambda m: _reclass(m.pool),
     "pooling's threshold": lambda m: setattr(m.pool, "eps", 1e-6),

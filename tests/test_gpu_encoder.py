@@ -128,6 +128,8 @@ def test_models_that_do_not_fit_run_as_they_did():
             model(x)
         model.fc.cuda()
         assert _near(model(x), a)
+        model.pool_norm.train()
+        assert models.embed_natively(model, x) is None and not _near(model(x), a)      # statistics of the batch
 
 
 def _dilation(m):
