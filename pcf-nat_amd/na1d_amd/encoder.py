@@ -59,6 +59,7 @@ class _Plan:
         from . import models as M
         self.dtype, self.keep = dtype, []
         self.made = {}                              # name -> (stamps of its sources, tensors made of them)
+        self.streams = set()                        # that have been told to the tensors' allocator
         known = {} if before is None else before.made
 
         def derive(name, sources, build):
@@ -143,6 +144,15 @@ class _Plan:
         if not isinstance(model.pool_norm, nn.Identity):
             e.pool_norm = norm(model.pool_norm)
         e.w_fc, e.b_fc = own(model.fc.weight), own(model.fc.bias)
+
+
+    def use_on(self, stream):
+        """A plan that is replaced gives its memory back, also while another stream than the one that made it still reads."""
+        if stream.cuda_stream not in self.streams:
+            for _, tensors in self.made.values():
+                for t in tensors:
+                    t.record_stream(stream)
+            self.streams.add(stream.cuda_stream)
 
 
 # The modules' numbers that a plan is made of.
@@ -301,11 +311,13 @@ def embed(model, x, lens=None):
     if nbytes == _lib.UNSUPPORTED:
         return None
     _lib.check(min(nbytes, 0), "na1d_encode_workspace_bytes")
-    x = x.float().contiguous()
+    stream = torch.cuda.current_stream(x.device)
+    plan.use_on(stream)
+    x, lens = x.float().contiguous(), None if lens is None else lens.contiguous()
     out = torch.empty((n, plan.encoder.emb), dtype=dtype, device=x.device)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    st = lib.na1d_encode(ref, out.data_ptr(), x.data_ptr(), None if lens is None else lens.contiguous().data_ptr(), n, frames,
-                         ws.data_ptr(), nbytes, torch.cuda.current_stream(x.device).cuda_stream)
+    st = lib.na1d_encode(ref, out.data_ptr(), x.data_ptr(), None if lens is None else lens.data_ptr(), n, frames,
+                         ws.data_ptr(), nbytes, stream.cuda_stream)
     if st == _lib.UNSUPPORTED:
         return None
     _lib.check(st, "na1d_encode")

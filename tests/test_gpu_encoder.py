@@ -224,3 +224,25 @@ def test_first_calls_and_changes_in_inference_mode():
         second = models.embed_natively(model, x)
     native, modules = _both(model, x)
     assert torch.equal(second, native) and _near(native, modules) and not torch.equal(first, second)
+
+
+def test_a_plan_outlives_its_use_on_other_streams():
+    """Weights change, and another stream makes the new plan, while a queue of passes still reads the old one: the memory of
+    the old one is not handed out before they are done."""
+    model, x = _model("mfa"), _input(64, 600)
+    want, _ = _both(model, x)
+    side, outs = torch.cuda.Stream(), []
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(20):
+            with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+                outs.append(models.embed_natively(model, x))
+    with torch.no_grad():
+        for block in model.blocks:
+            for m in (block.blocks[0].attn.proj, block.blocks[0].mlp.fc1, block.blocks[0].mlp.fc2):
+                m.weight = torch.nn.Parameter(torch.zeros_like(m.weight))              # the passes read biases, not these
+    after, _ = _both(model, x[:1])
+    filled = [torch.full((n,), float("nan"), dtype=torch.bfloat16, device="cuda") for n in (256 * 256, 256 * 1024) * 40]
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, want) for o in outs) and not _near(after, want[:1])
+    del filled
