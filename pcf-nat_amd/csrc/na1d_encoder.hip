@@ -1017,6 +1017,8 @@ bool encoder_ok(const na1d_encoder &e, int64_t N, int64_t frames) {
     if (e.layers < 1 || e.blocks < 1 || e.patch < 1 || e.in_chans < 1 || e.wide < 256 || e.emb < 16 || frames < e.patch) return false;
     if (e.in_chans > 4096 || e.patch > 256 || e.in_chans * e.patch % 32 || e.in_chans * e.patch > kDim || e.wide % 256 || e.emb % 16 || e.wide > (1 << 16) || e.emb > (1 << 16)) return false;
     if ((size_t)e.in_chans * (64 * e.patch + 1) * sizeof(float) > 160 * 1024) return false;
+    // a weight's bytes are counted in 31 bits
+    if ((int64_t)e.emb * e.wide >= (1 << 29) || (int64_t)e.blocks * e.wide >= (1 << 22)) return false;
     const int64_t T = (frames - e.patch) / e.patch + 1;
     // rows of an utterance stay in the reach of 31-bit offsets (the widest are those of the projection), launches of 31-bit ids
     if (T > (1 << 29) / e.wide || N > 65535 || N * T > (1ll << 26) || frames > (1 << 24)) return false;

@@ -1,5 +1,6 @@
 """Which models the native embedding call takes: decided on the host, so checked without a GPU."""
 import copy
+import ctypes
 import gc
 import types
 import weakref
@@ -9,7 +10,7 @@ import torch
 import torch.nn as nn
 import torch.nn.utils.parametrize  # noqa: F401
 
-from na1d_amd import encoder, models
+from na1d_amd import _lib, encoder, models
 
 CPU = torch.device("cpu")
 SMALL = dict(depths=(1, 1), num_heads=[[16], [4]], win_size=[[27], [0]], na="fused_qkv")
@@ -126,3 +127,16 @@ def test_a_changed_tensor_costs_what_was_made_of_it(family, monkeypatch):
         plan = after
     assert len(calls) == 1
     assert len(plan.made) == len(encoder._Plan(model, torch.float16, None).made)
+
+
+@pytest.mark.parametrize("wide,emb,blocks,taken", [(1536, 192, 2, True), (65536, 8176, 2, True), (65536, 8192, 2, False), (65536, 65536, 2, False),
+                                                   (65536, 16, 63, True), (65536, 16, 64, False)])
+def test_weights_beyond_31_bits_are_refused(wide, emb, blocks, taken):
+    plan = encoder._Plan(_model(), torch.bfloat16)
+    e = plan.encoder
+    e.wide, e.emb, e.blocks = wide, emb, blocks
+    layers = (encoder._Layer * blocks)(*[plan.layers[0]] * blocks)
+    for l in layers:
+        l.block_end = 1
+    e.layers, e.layer = blocks, layers
+    assert (_lib.load().na1d_encode_workspace_bytes(ctypes.byref(e), 4, 100) > 0) == taken
