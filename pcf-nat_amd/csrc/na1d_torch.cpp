@@ -3,8 +3,8 @@
 // Python took 115 us (allocations, context managers, ctypes, and the engine's thread waiting for the interpreter lock).
 //
 // Every function here returns nothing (None) for calls it does not take as they are - other devices, types, layouts,
-// tensor subclasses, transforms, tracers, forward-mode gradients - and the Python implementation then serves or refuses
-// them as before.
+// tensor subclasses, transforms, tracers, forward-mode gradients - and for those that the library refuses (the kernels are
+// launched before a node is built).  The Python implementation then serves or refuses them as before.
 #include <torch/extension.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
@@ -113,15 +113,17 @@ Tensor bias_of(const MaybeTensor &rpb, const Geometry &g) {
 }
 Tensor lengths_of(const MaybeTensor &t_valid, const Tensor &like) { return t_valid ? t_valid->to(like.device(), at::kInt).contiguous() : Tensor(); }
 
+// A forward whose kernels are launched: what its node is built around.
+struct Done {
+    Tensor out, lse, bias, valid;
+};
+
 struct Fused : torch::autograd::Function<Fused> {
-    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const MaybeTensor &rpb, const MaybeTensor &t_valid,
-                          const Geometry &g) {
-        const Tensor bias = bias_of(rpb, g), valid = lengths_of(t_valid, q), out = at::empty_like(q);
-        const Tensor lse = at::empty({g.N * g.H, g.T}, q.options().dtype(at::kFloat));
-        check(forward_kernel(g, out, lse, ptr(q), ptr(k), ptr(v), bias, valid, tag(q), stream_of(q)), "na1d_fused_forward");
-        ctx->save_for_backward({q, k, v, out, bias, valid, lse});
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const MaybeTensor &rpb, const MaybeTensor &,
+                          const Geometry &g, const Done &done) {
+        ctx->save_for_backward({q, k, v, done.out, done.bias, done.valid, done.lse});
         remember(ctx, g, rpb);
-        return out;
+        return done.out;
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
         const variable_list s = ctx->get_saved_variables();
@@ -133,19 +135,14 @@ struct Fused : torch::autograd::Function<Fused> {
         if (ctx->saved_data["bias"].toBool()) drpb = at::zeros(ctx->saved_data["bias_shape"].toIntVector(), q.options().dtype(at::kFloat));
         check(backward_kernel(g, ptr(dq), ptr(dk), ptr(dv), drpb, ptr(q), ptr(s[1]), ptr(s[2]), s[3], dout, s[6], s[4], s[5], tag(q), stream_of(q)),
               "na1d_fused_backward");
-        return {dq, dk, dv, drpb, Tensor(), Tensor()};
+        return {dq, dk, dv, drpb, Tensor(), Tensor(), Tensor()};
     }
 };
 struct FusedQKV : torch::autograd::Function<FusedQKV> {
-    static Tensor forward(AutogradContext *ctx, const Tensor &qkv, const MaybeTensor &rpb, const MaybeTensor &t_valid, const Geometry &g) {
-        const Tensor bias = bias_of(rpb, g), valid = lengths_of(t_valid, qkv), out = at::empty({g.N, g.T, g.H * g.C}, qkv.options());
-        const Tensor lse = at::empty({g.N * g.H, g.T}, qkv.options().dtype(at::kFloat));
-        const char *q = (const char *)ptr(qkv);
-        const int64_t step = 2 * g.H * g.C;
-        check(forward_kernel(g, out, lse, q, q + step, q + 2 * step, bias, valid, tag(qkv), stream_of(qkv)), "na1d_fused_forward");
-        ctx->save_for_backward({qkv, bias, valid, lse});
+    static Tensor forward(AutogradContext *ctx, const Tensor &qkv, const MaybeTensor &rpb, const MaybeTensor &, const Geometry &g, const Done &done) {
+        ctx->save_for_backward({qkv, done.bias, done.valid, done.lse});
         remember(ctx, g, rpb);
-        return out;
+        return done.out;
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
         const variable_list s = ctx->get_saved_variables();
@@ -160,7 +157,7 @@ struct FusedQKV : torch::autograd::Function<FusedQKV> {
         const char *q = (const char *)ptr(qkv);
         check(backward_kernel(g, dq, dq + step, dq + 2 * step, drpb, q, q + step, q + 2 * step, Tensor(), dout, s[3], s[1], s[2], tag(qkv), stream_of(qkv)),
               "na1d_fused_backward");
-        return {dqkv, drpb, Tensor(), Tensor()};
+        return {dqkv, drpb, Tensor(), Tensor(), Tensor()};
     }
 };
 // Whether bias and lengths are what the Python path takes without complaint, and the sizes what the one-launch kernels cover.
@@ -185,12 +182,10 @@ MaybeTensor fused(const Tensor &q, const Tensor &k, const Tensor &v, const Maybe
     const Geometry g{q.size(0) / H, H, q.size(1), q.size(2), W, left, dilation, scale, {p, seed}, false};
     if (!covered(g, q, rpb, t_valid)) return std::nullopt;
     const c10::DeviceGuard guard(q.device());
-    if (!needs_grad({q, k, v}, rpb)) {                 // no node, no log-sum-exp
-        const Tensor out = at::empty_like(q);
-        check(forward_kernel(g, out, Tensor(), ptr(q), ptr(k), ptr(v), bias_of(rpb, g), lengths_of(t_valid, q), tag(q), stream_of(q)), "na1d_fused_forward");
-        return out;
-    }
-    return Fused::apply(q, k, v, rpb, t_valid, g);
+    const bool node = needs_grad({q, k, v}, rpb);      // otherwise no log-sum-exp either
+    const Done done{at::empty_like(q), node ? at::empty({g.N * g.H, g.T}, q.options().dtype(at::kFloat)) : Tensor(), bias_of(rpb, g), lengths_of(t_valid, q)};
+    if (forward_kernel(g, done.out, done.lse, ptr(q), ptr(k), ptr(v), done.bias, done.valid, tag(q), stream_of(q)) != NA1D_OK) return std::nullopt;
+    return node ? Fused::apply(q, k, v, rpb, t_valid, g, done) : done.out;
 }
 MaybeTensor fused_qkv(const Tensor &qkv, const MaybeTensor &rpb, const MaybeTensor &t_valid, int64_t W, int64_t left, double scale, int64_t dilation, double p,
                       uint64_t seed) {
@@ -198,30 +193,25 @@ MaybeTensor fused_qkv(const Tensor &qkv, const MaybeTensor &rpb, const MaybeTens
     const Geometry g{qkv.size(0), qkv.size(3), qkv.size(1), qkv.size(4), W, left, dilation, scale, {p, seed}, true};
     if (!covered(g, qkv, rpb, t_valid)) return std::nullopt;
     const c10::DeviceGuard guard(qkv.device());
-    if (!needs_grad({qkv}, rpb)) {
-        const Tensor out = at::empty({g.N, g.T, g.H * g.C}, qkv.options());
-        const char *q = (const char *)ptr(qkv);
-        const int64_t step = 2 * g.H * g.C;
-        check(forward_kernel(g, out, Tensor(), q, q + step, q + 2 * step, bias_of(rpb, g), lengths_of(t_valid, qkv), tag(qkv), stream_of(qkv)), "na1d_fused_forward");
-        return out;
-    }
-    return FusedQKV::apply(qkv, rpb, t_valid, g);
+    const bool node = needs_grad({qkv}, rpb);
+    const Done done{at::empty({g.N, g.T, g.H * g.C}, qkv.options()), node ? at::empty({g.N * g.H, g.T}, qkv.options().dtype(at::kFloat)) : Tensor(),
+                    bias_of(rpb, g), lengths_of(t_valid, qkv)};
+    const char *q = (const char *)ptr(qkv);
+    const int64_t step = 2 * g.H * g.C;
+    if (forward_kernel(g, done.out, done.lse, q, q + step, q + 2 * step, done.bias, done.valid, tag(qkv), stream_of(qkv)) != NA1D_OK) return std::nullopt;
+    return node ? FusedQKV::apply(qkv, rpb, t_valid, g, done) : done.out;
 }
 
 // ------------------------------------------------------------------------------------------------ dense attention
 struct Dense : torch::autograd::Function<Dense> {
-    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const MaybeTensor &t_valid, int64_t H, double scale, double p,
-                          uint64_t seed) {
-        const Tensor out = at::empty_like(q), lse = at::empty({q.size(0), q.size(1)}, q.options().dtype(at::kFloat)), valid = t_valid ? *t_valid : Tensor();
-        check(na1d_global_forward(ptr(out), (float *)ptr(lse), ptr(q), ptr(k), ptr(v), (const int32_t *)ptr(valid), q.size(0), H, q.size(1), q.size(2), (float)scale,
-                                  tag(q), (float)p, seed, stream_of(q)),
-              "na1d_global_forward");
-        ctx->save_for_backward({q, k, v, out, lse, valid});
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, int64_t H, double scale, double p, uint64_t seed,
+                          const Done &done) {
+        ctx->save_for_backward({q, k, v, done.out, done.lse, done.valid});
         ctx->saved_data["heads"] = H;
         ctx->saved_data["scale"] = scale;
         ctx->saved_data["p"] = p;
         ctx->saved_data["seed"] = (int64_t)seed;
-        return out;
+        return done.out;
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
         const variable_list s = ctx->get_saved_variables();
@@ -245,57 +235,59 @@ MaybeTensor dense(const Tensor &q, const Tensor &k, const Tensor &v, const Maybe
                     t_valid->device() != q.device()))
         return std::nullopt;
     const c10::DeviceGuard guard(q.device());
-    return Dense::apply(q, k, v, t_valid, H, scale, p, seed);
+    const Done done{at::empty_like(q), at::empty({q.size(0), q.size(1)}, q.options().dtype(at::kFloat)), Tensor(), t_valid ? *t_valid : Tensor()};
+    if (na1d_global_forward(ptr(done.out), (float *)ptr(done.lse), ptr(q), ptr(k), ptr(v), (const int32_t *)ptr(done.valid), q.size(0), H, q.size(1), q.size(2),
+                            (float)scale, tag(q), (float)p, seed, stream_of(q)) != NA1D_OK)
+        return std::nullopt;
+    return Dense::apply(q, k, v, H, scale, p, seed, done);
 }
 
 // ------------------------------------------------------------------------------------------------ the two-call operator
 using Band = int(void *, const void *, const void *, int64_t, int64_t, int64_t, int64_t, int64_t, int, void *);
-void band(Band *f, const char *name, const Tensor &out, const Tensor &a, const Tensor &b, const Tensor &like, int64_t W, int64_t left) {
-    check(f(ptr(out), ptr(a), ptr(b), like.size(0), like.size(1), like.size(2), W, left, tag(like), stream_of(like)), name);
+int band(Band *f, const Tensor &out, const Tensor &a, const Tensor &b, const Tensor &like, int64_t W, int64_t left) {
+    return f(ptr(out), ptr(a), ptr(b), like.size(0), like.size(1), like.size(2), W, left, tag(like), stream_of(like));
 }
 struct QK : torch::autograd::Function<QK> {
-    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, int64_t W, int64_t left) {
-        const Tensor attn = at::empty({q.size(0), q.size(1), W}, q.options().dtype(at::kFloat));
-        band(na1d_qk_forward, "na1d_qk_forward", attn, q, k, q, W, left);
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, int64_t W, int64_t left, const Done &done) {
         ctx->save_for_backward({q, k});
         ctx->saved_data["W"] = W;
         ctx->saved_data["left"] = left;
-        return attn;
+        return done.out;
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
         const variable_list s = ctx->get_saved_variables();
         const int64_t W = ctx->saved_data["W"].toInt(), left = ctx->saved_data["left"].toInt();
         const c10::DeviceGuard guard(s[0].device());
         const Tensor g = grads[0].contiguous(), dq = at::empty_like(s[0]), dk = at::empty_like(s[0]);
-        band(na1d_q_backward, "na1d_q_backward", dq, g, s[1], s[0], W, left);
-        band(na1d_k_backward, "na1d_k_backward", dk, g, s[0], s[0], W, left);
-        return {dq, dk, Tensor(), Tensor()};
+        check(band(na1d_q_backward, dq, g, s[1], s[0], W, left), "na1d_q_backward");
+        check(band(na1d_k_backward, dk, g, s[0], s[0], W, left), "na1d_k_backward");
+        return {dq, dk, Tensor(), Tensor(), Tensor()};
     }
 };
 struct AV : torch::autograd::Function<AV> {
-    static Tensor forward(AutogradContext *ctx, const Tensor &attn, const Tensor &v, int64_t W, int64_t left) {
-        const Tensor out = at::empty_like(v);
-        band(na1d_av_forward, "na1d_av_forward", out, attn, v, v, W, left);
+    static Tensor forward(AutogradContext *ctx, const Tensor &attn, const Tensor &v, int64_t W, int64_t left, const Done &done) {
         ctx->save_for_backward({attn, v});
         ctx->saved_data["W"] = W;
         ctx->saved_data["left"] = left;
-        return out;
+        return done.out;
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
         const variable_list s = ctx->get_saved_variables();
         const int64_t W = ctx->saved_data["W"].toInt(), left = ctx->saved_data["left"].toInt();
         const c10::DeviceGuard guard(s[1].device());
         const Tensor g = grads[0].contiguous(), dattn = at::empty_like(s[0]), dv = at::empty_like(s[1]);
-        band(na1d_a_backward, "na1d_a_backward", dattn, g, s[1], s[1], W, left);
-        band(na1d_v_backward, "na1d_v_backward", dv, s[0], g, s[1], W, left);
-        return {dattn, dv, Tensor(), Tensor()};
+        check(band(na1d_a_backward, dattn, g, s[1], s[1], W, left), "na1d_a_backward");
+        check(band(na1d_v_backward, dv, s[0], g, s[1], W, left), "na1d_v_backward");
+        return {dattn, dv, Tensor(), Tensor(), Tensor()};
     }
 };
 bool band_window(int64_t W, int64_t left) { return W >= 1 && W <= NA1D_MAX_WINDOW && left >= 0 && left < W; }
 MaybeTensor qk(const Tensor &q, const Tensor &k, int64_t W, int64_t left) {
     if (!plain_call() || !same_operands(q, k, k) || q.size(2) % 8 || !band_window(W, left)) return std::nullopt;
     const c10::DeviceGuard guard(q.device());
-    return QK::apply(q, k, W, left);
+    const Done done{at::empty({q.size(0), q.size(1), W}, q.options().dtype(at::kFloat)), Tensor(), Tensor(), Tensor()};
+    if (band(na1d_qk_forward, done.out, q, k, q, W, left) != NA1D_OK) return std::nullopt;
+    return QK::apply(q, k, W, left, done);
 }
 MaybeTensor av(const Tensor &attn, const Tensor &v, int64_t W, int64_t left) {
     if (!plain_call() || !same_operands(v, v, v) || v.size(2) % 8 || !band_window(W, left)) return std::nullopt;
@@ -303,7 +295,9 @@ MaybeTensor av(const Tensor &attn, const Tensor &v, int64_t W, int64_t left) {
         attn.size(1) != v.size(1) || attn.size(2) != W)
         return std::nullopt;
     const c10::DeviceGuard guard(v.device());
-    return AV::apply(attn, v, W, left);
+    const Done done{at::empty_like(v), Tensor(), Tensor(), Tensor()};
+    if (band(na1d_av_forward, done.out, attn, v, v, W, left) != NA1D_OK) return std::nullopt;
+    return AV::apply(attn, v, W, left, done);
 }
 
 }  // namespace
