@@ -6,6 +6,7 @@
 // tensor subclasses, transforms, tracers, forward-mode gradients - and for those that the library refuses (the kernels are
 // launched before a node is built).  The Python implementation then serves or refuses them as before.
 #include <torch/extension.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -20,8 +21,16 @@ using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 using MaybeTensor = std::optional<Tensor>;
 
+PyObject *error_class = PyExc_RuntimeError;             // the package's exception, which lives as long as this module
+
+// In a backward, on a thread of torch's: its engine carries a Python error to the caller.
 void check(int status, const char *name) {
-    if (status != NA1D_OK) throw std::runtime_error(std::string(name) + " failed: " + na1d_status_string(status) + " (status " + std::to_string(status) + ")");
+    if (status == NA1D_OK) return;
+    const pybind11::gil_scoped_acquire gil;
+    PyErr_Format(error_class, "%s failed: %s (status %d)", name, na1d_status_string(status), status);
+    python_error error;
+    error.persist();
+    throw error;
 }
 void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream(); }
 void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
@@ -303,6 +312,7 @@ MaybeTensor av(const Tensor &attn, const Tensor &v, int64_t W, int64_t left) {
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    m.def("raise_as", [](pybind11::object c) { error_class = c.inc_ref().ptr(); });
     m.def("fused", &fused);
     m.def("fused_qkv", &fused_qkv);
     m.def("dense", &dense);

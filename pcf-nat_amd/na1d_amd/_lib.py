@@ -136,6 +136,7 @@ def nodes():
         spec = importlib.util.spec_from_file_location("na1d_torch", path)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
+        module.raise_as(NA1DError)
         _nodes = module
     return _nodes
 

@@ -52,3 +52,16 @@ def test_refusals_are_na1d_errors():
                      lambda: QK.apply(qg, bad, 5, 2, 1), lambda: AV.apply(attn, bad, 5, 2, 1)):
             with pytest.raises(_lib.NA1DError):
                 call()
+
+
+def test_refusals_in_the_backward_are_na1d_errors():
+    q, k, v = (_rand(2, 20, 16, seed=i).requires_grad_(True) for i in range(3))
+    QK, AV = getNA1dFunction(16, 1, torch.float16)
+    attn = torch.rand(2, 20, 5, device="cuda", requires_grad=True)
+    grads = _misaligned(2, 20, 16)
+    for out in (na1d_fused(q, k, v, 5, 2), na1d_fused(q, k, v, 5, 2, dilation=2), global_attention(q, k, v, 1), AV.apply(attn, v, 5, 2, 1)):
+        with pytest.raises(_lib.NA1DError, match="failed"):
+            out.backward(grads)
+        assert q.grad is None
+    na1d_fused(q, k, v, 5, 2).backward(grads.clone())
+    assert torch.isfinite(q.grad).all()
