@@ -845,7 +845,7 @@ bool layer_ok(const na1d_train_layer &l, int64_t N, int64_t T) {
     if (l.groups < 1 || l.dim % l.groups || l.dim / l.groups % 32 || l.hidden % l.groups || l.hidden / l.groups % 32) return false;
     if (l.window < 0 || l.window > NA1D_MAX_WINDOW || (l.window && (l.left < 0 || l.left >= l.window)) || l.dilation < 1 || (!l.window && l.dilation > 1)) return false;
     // offsets inside an utterance, and what the attention kernels' launches count, stay in the reach of 32 bits
-    if (N < 1 || T < 1 || N > (1 << 20) || T > (1 << 16) || N * T > (1 << 20)) return false;
+    if (N < 1 || T < 1 || N > 65535 || T > (1 << 16) || N * T > (1 << 20)) return false;     // samples: a grid's third dimension
     const int64_t M = N * T, most = 1ll << 31;
     if (T * 3 * l.dim > (1 << 29) || M * T >= most || l.dilation > 64) return false;
     if (l.heads * M * l.heads >= most || l.heads * M * (T / 32 + 1) >= most || l.heads * M * l.dilation >= most) return false;
