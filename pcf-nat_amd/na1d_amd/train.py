@@ -108,9 +108,10 @@ def plain_call(x):
             and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0)
 
 
-def _norm_fits(bn, dim):
+def _norm_fits(bn, dim, device):
     return (bn.training and bn.track_running_stats and bn.affine and bn.momentum is not None and bn.num_features == dim
-            and bn.num_batches_tracked is not None)
+            and all(s is not None and s.dtype == torch.float32 and s.device == device and s.shape == (dim,) for s in (bn.running_mean, bn.running_var))
+            and bn.num_batches_tracked is not None and bn.num_batches_tracked.dtype == torch.int64 and bn.num_batches_tracked.device == device)
 
 
 def _drop_path_scale(m, x):
@@ -142,7 +143,7 @@ def layer(m, x, pos_emb=None, attn_mask_global=None):
         return None
     xt = x.transpose(1, 2) if cf else x
     n, t, dim = xt.shape
-    if (t != a.attn_mask.shape[-2] if m.local else attn_mask_global is not None) or not all(_norm_fits(b, dim) for b in norms):
+    if (t != a.attn_mask.shape[-2] if m.local else attn_mask_global is not None) or not all(_norm_fits(b, dim, x.device) for b in norms):
         return None
     projections = [a.qkv, a.proj, mlp.fc1, mlp.fc2]
     pos = None
