@@ -36,6 +36,11 @@ def _ptrs(ts):
     return (_P * 5)(*map(_ptr, ts))
 
 
+def _aligned(t):
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
+
+
 class _TrainLayer(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, by_channel, geom, norms, scales, pos, extra, n1w, n1b, n2w, n2b, wq, bq, wp, bp, w1, b1, w2, b2):
@@ -75,7 +80,7 @@ class _TrainLayer(torch.autograd.Function):
         lib = _lib.load()
         x, saved, pos, rpb, n1w, n2w, *scales = ctx.saved_tensors
         n, t, dim = x.shape
-        dout = dout.contiguous()
+        dout = _aligned(dout)
         dx = torch.empty_like(x)
         grads = [torch.zeros(ctx.shapes[0], dtype=torch.float32, device=x.device)]       # the bias of the scores is added to
         grads += [torch.empty(s, dtype=torch.float32, device=x.device) for s in ctx.shapes[1:]]
@@ -142,6 +147,8 @@ def layer(m, x, pos_emb=None, attn_mask_global=None):
     if (a.na != "fused_qkv" if m.local else a.dense != "native") or a.attn_drop or not a.training or a.proj_drop.p or mlp.drop.p or (not cf and not all(plain(b, M.BatchNorm1d) for b in norms)):
         return None
     xt = x.transpose(1, 2) if cf else x
+    if xt.is_contiguous() and xt.data_ptr() % 16:
+        return None
     n, t, dim = xt.shape
     if (t != a.attn_mask.shape[-2] if m.local else attn_mask_global is not None) or not all(_norm_fits(b, dim, x.device) for b in norms):
         return None
@@ -174,7 +181,7 @@ def layer(m, x, pos_emb=None, attn_mask_global=None):
     by_channel = by_channel if by_channel.is_contiguous() else None       # [N, C, T], the layout of the statistics, is there already
     xt = xt.contiguous()
     if not m.local:
-        pos = (pos_emb.transpose(1, 2) if cf else pos_emb).to(x.dtype).contiguous()
+        pos = _aligned((pos_emb.transpose(1, 2) if cf else pos_emb).to(x.dtype))
     scales = (_drop_path_scale(m.drop_path, xt), _drop_path_scale(m.drop_path, xt))
     out = _TrainLayer.apply(xt, by_channel, geom, norms, scales, pos, *params)
     return out.transpose(1, 2) if cf else out

@@ -140,3 +140,32 @@ def test_what_the_node_does_not_cover_stays_with_the_modules():
         layer(x).sum().backward()
         assert layer.mlp.fc1.weight.grad is None and layer.mlp.fc2.weight.grad is not None
         assert layer.norm1.norm.running_mean._version > before
+
+
+def _off_alignment(t):
+    return torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)[1:t.numel() + 1].view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("window", [27, 0])
+def test_tensors_off_their_alignment(window):
+    """An input that starts anywhere goes to the modules, a gradient and positions that do are copied."""
+    _, gpu = _layers("mfa", 1, 16, window, 1, 40, 0.0, seed=1)
+    gen = torch.Generator().manual_seed(2)
+    x, g = (torch.randn(4, 40, 256, generator=gen).half().cuda() for _ in range(2))
+    pos = None if window else models.sinusoid_table(256, 40, False).half().cuda()
+    results = []
+    for move in (lambda t: t, _off_alignment):
+        layer = copy.deepcopy(gpu)
+        xg = x.clone().requires_grad_(True)
+        with torch.autocast("cuda", dtype=torch.float16):
+            out = layer(xg, pos_emb=None if pos is None else move(pos))
+        assert type(out.grad_fn).__name__ == "_TrainLayerBackward"
+        out.backward(move(g))
+        results.append((out.detach(), xg.grad, layer.mlp.fc1.weight.grad, layer.attn.qkv.weight.grad))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+    off = _off_alignment(x).requires_grad_(True)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert models.train_layer(copy.deepcopy(gpu), off, pos) is None
+        out = copy.deepcopy(gpu)(off, pos_emb=pos)
+    out.backward(g)
+    assert O.rel_l2(off.grad.float(), results[0][1].float()) < 32 * 2.0 ** -12
