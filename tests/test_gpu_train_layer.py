@@ -169,3 +169,31 @@ def test_tensors_off_their_alignment(window):
         out = copy.deepcopy(gpu)(off, pos_emb=pos)
     out.backward(g)
     assert O.rel_l2(off.grad.float(), results[0][1].float()) < 32 * 2.0 ** -12
+
+
+# both product tiles (64 rows from 128 blocks of 64 rows x 256 outputs on, else 32), remainders of either, one sample
+@pytest.mark.parametrize("batch,T", [(1, 33), (7, 101), (37, 100), (128, 100), (64, 260)])
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("family,groups,heads,window,dilation", [
+    ("mfa", 1, 16, 27, 1), ("mfa", 1, 4, 65, 1), ("pcf", 8, 16, 27, 1), ("pcf", 4, 8, 9, 2), ("pcf", 2, 16, 27, 1), ("pcf", 1, 32, 5, 3),
+    ("mfa", 1, 4, 0, 1), ("mfa", 1, 16, 0, 1), ("pcf", 8, 4, 0, 1), ("pcf", 1, 2, 0, 1)])
+def test_forward_is_the_modules_to_the_bit(family, groups, heads, window, dilation, dtype, batch, T):
+    """Output and running statistics, at these sizes: training amplifies a difference in the last bit of a forward over its
+    layers.  The residual stream lies in memory as it does in the models, channels first in both families (torch sums
+    statistics and adds biases in another way for the other layout)."""
+    _, gpu = _layers(family, groups, heads, window, dilation, T, 0.3, seed=T)
+    gen = torch.Generator().manual_seed(batch)
+    x = torch.randn(batch, 256, T, generator=gen).cuda().to(DT[dtype])
+    x = x if family == "pcf" else x.transpose(1, 2)
+    pos = None if window else models.sinusoid_table(256, T, family == "pcf").cuda()
+    results = []
+    for native in (True, False):
+        layer = copy.deepcopy(gpu)
+        if not native:
+            layer.mlp.fc2.register_forward_hook(lambda *a: None)
+        torch.manual_seed(3)
+        with torch.autocast("cuda", dtype=DT[dtype]):
+            out = layer(x.clone().requires_grad_(True), pos_emb=pos)
+        assert ("_TrainLayer" in repr(out.grad_fn) or "_TrainLayer" in repr(out.grad_fn.next_functions)) == native
+        results.append([out.detach()] + [b for n, b in layer.named_buffers() if "running" in n or "batches" in n])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
