@@ -338,6 +338,7 @@ typedef struct na1d_train_norm {
 typedef struct na1d_train_layer {
     int32_t dtype, dim, hidden, heads, window, left, dilation, groups, ordered;
     float scale;
+    int32_t late;                               /* qkv and fc1: sums are rounded before the bias is added (always if ordered) */
     na1d_train_norm norm[2];
     const float *w[5], *b[5];                   /* qkv, proj, fc1, fc2; of a dense layer also linear_pos (no b) */
     float *dw[5], *db[5];                       /* written by the backward */

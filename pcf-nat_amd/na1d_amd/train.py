@@ -24,7 +24,7 @@ class _Norm(ctypes.Structure):                     # na1d_train_norm
 
 class _Layer(ctypes.Structure):                    # na1d_train_layer
     _fields_ = ([(n, _I) for n in "dtype dim hidden heads window left dilation groups ordered".split()] + [("scale", _F)]
-                + [("norm", _Norm * 2)] + [(n, _P * 5) for n in "w b dw db".split()]
+                + [("late", _I), ("norm", _Norm * 2)] + [(n, _P * 5) for n in "w b dw db".split()]
                 + [(n, _P) for n in "rpb drpb pos scale_attn scale_mlp".split()])
 
 
@@ -71,6 +71,7 @@ class _TrainLayer(torch.autograd.Function):
                                                         sizes[1], n, t, stream), "na1d_train_layer_forward")
         increment_version([b for bn in norms for b in (bn.running_mean, bn.running_var, bn.num_batches_tracked)])
         ctx.save_for_backward(x, saved, pos, None if dense else extra, n1w, n2w, *scales)
+        ctx.late = c.late
         ctx.geom, ctx.shapes = geom, [p.shape for p in (extra, n1w, n1b, n2w, n2b, wq, bq, wp, bp, w1, b1, w2, b2)]
         return out
 
@@ -173,7 +174,10 @@ def layer(m, x, pos_emb=None, attn_mask_global=None):
     if params[0].numel() != (a.num_heads * a.win_size if m.local else dim * dim // groups):
         return None
     window = (a.win_size, a.left, a.dilation) if m.local else (0, 0, 1)
-    geom = (_lib.dtype_tag(x.dtype), dim, hidden, a.num_heads, *window, groups, int(cf), a.scale)
+    # The modules' products of a stream that lies channels first in memory (a model's, from the patch embedding on) round
+    # before the bias is added, those of a tokens-first tensor after.  The node's own output lies tokens first either way.
+    late = cf or not x.is_contiguous() or getattr(x.grad_fn, "late", 0)
+    geom = (_lib.dtype_tag(x.dtype), dim, hidden, a.num_heads, *window, groups, int(cf), a.scale, int(late))
     probe = _Layer(*geom)
     if _lib.load().na1d_train_layer_saved_bytes(ctypes.byref(probe), n, t) < 0:
         return None

@@ -197,3 +197,48 @@ def test_forward_is_the_modules_to_the_bit(family, groups, heads, window, dilati
         assert ("_TrainLayer" in repr(out.grad_fn) or "_TrainLayer" in repr(out.grad_fn.next_functions)) == native
         results.append([out.detach()] + [b for n, b in layer.named_buffers() if "running" in n or "batches" in n])
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+def test_layers_behind_each_other_are_the_modules_to_the_bit(dtype):
+    """The tokens-first model's stream: channels first in the modules' memory, tokens first between two native layers."""
+    stack = torch.nn.ModuleList(_layers("mfa", 1, heads, window, 1, 100, 0.2, seed=i)[1] for i, (heads, window) in enumerate(((16, 27), (4, 0), (16, 27))))
+    x = torch.randn(24, 256, 100, generator=torch.Generator().manual_seed(0)).cuda().to(DT[dtype]).transpose(1, 2)
+    pos = models.sinusoid_table(256, 100, False).cuda()
+    results = []
+    for native in (True, False):
+        layers = copy.deepcopy(stack)
+        torch.manual_seed(3)
+        y = x.clone().requires_grad_(True)
+        with torch.autocast("cuda", dtype=DT[dtype]):
+            for layer in layers:
+                if not native:
+                    layer.mlp.fc2.register_forward_hook(lambda *a: None)
+                y = layer(y, pos_emb=pos)
+        results.append([y.detach()] + [b for n, b in layers.named_buffers() if "running" in n])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("heads,window", [(16, 27), (4, 0)])
+def test_tokens_first_inputs_lose_nothing(heads, window, dtype):
+    """A layer called by itself on tokens that lie one behind the other is as near to 64 bits as the modules are."""
+    cpu, gpu = _layers("mfa", 1, heads, window, 1, 100, 0.0, seed=2)
+    gen = torch.Generator().manual_seed(0)
+    x, g = (torch.randn(24, 100, 256, generator=gen).to(DT[dtype]) for _ in range(2))
+    pos = None if window else models.sinusoid_table(256, 100, False)
+    exact, xc = copy.deepcopy(cpu).double(), x.double().requires_grad_(True)
+    want = exact(xc, pos_emb=None if pos is None else pos.to(DT[dtype]).double())
+    want.backward(g.double())
+    errors = []
+    for native in (True, False):
+        layer, xg = copy.deepcopy(gpu), x.cuda().requires_grad_(True)
+        if not native:
+            layer.mlp.fc2.register_forward_hook(lambda *a: None)
+        with torch.autocast("cuda", dtype=DT[dtype]):
+            out = layer(xg, pos_emb=None if pos is None else pos.cuda())
+        assert (type(out.grad_fn).__name__ == "_TrainLayerBackward") == native
+        out.backward(g.cuda())
+        errors.append([O.rel_l2(out.float(), want.float()), O.rel_l2(xg.grad.float(), xc.grad.float())])
+    print(errors)
+    assert all(a < 1.02 * b for a, b in zip(*errors))
