@@ -65,7 +65,7 @@ def _errors(cpu, gpu, x, g, dtype, pos=None):
     return err
 
 
-# tokens: fewer than a tile (of two rows a norm makes +-1 whatever they hold: nothing to compare), one chunk of rows, remainders of every tile, the launch sizes of all three product tiles
+# tokens: fewer than a tile (of two rows a norm makes +-1 whatever they hold: nothing to compare), one chunk of rows, remainders of every tile, the launch sizes of both product tiles
 @pytest.mark.parametrize("batch,T", [(2, 5), (1, 33), (3, 50), (7, 101), (37, 100), (64, 260)])
 @pytest.mark.parametrize("dtype", ["bf16", "fp16"])
 @pytest.mark.parametrize("family,groups,heads,window,dilation", [
