@@ -3,6 +3,7 @@
 // kernel-family switch, and the per-GPU scratch array of na1d_fused_backward_noalloc (na1d_mfma.hip).
 #include <atomic>
 #include <cstdlib>
+#include <initializer_list>
 
 #include "na1d_common.h"
 
@@ -433,12 +434,26 @@ int64_t na1d_encode_workspace_bytes(const na1d_encoder *e, int64_t N, int64_t fr
     return na1d::enc::workspace_bytes(*e, N, frames);
 }
 
+static bool encoder_whole(const na1d_encoder &e) {
+    auto all = [](std::initializer_list<const void *> ps) {
+        for (const void *p : ps)
+            if (!p) return false;
+        return true;
+    };
+    for (int i = 0; i < e.layers; ++i) {
+        const na1d_encoder_layer &l = e.layer[i];
+        if (!all({l.w_qkv, l.w_proj, l.w_fc1, l.w_fc2, l.b_qkv, l.b_proj, l.b_fc1, l.b_fc2})) return false;
+        if (l.embeds && !all({l.w_embed, l.b_embed})) return false;
+    }
+    return all({e.w_wide, e.b_wide, e.a_wide, e.c_wide, e.w_att, e.w_ctx, e.w_logit, e.b_att, e.a_att, e.c_att, e.w_fc, e.b_fc});
+}
+
 int na1d_encode(const na1d_encoder *e, void *out, const float *x, const float *lens, int64_t N, int64_t frames,
                 void *workspace, int64_t workspace_bytes, void *stream) {
     const int64_t need = na1d_encode_workspace_bytes(e, N, frames);
     if (need < 0) return (int)need;
     if (N == 0) return NA1D_OK;
-    if (!out || !x || !workspace) return NA1D_ERR_NULL;
+    if (!out || !x || !workspace || !encoder_whole(*e)) return NA1D_ERR_NULL;
     if (misaligned(out) || misaligned(workspace)) return NA1D_ERR_ALIGN;
     if (workspace_bytes < need) return NA1D_ERR_WORKSPACE;
     for (int i = 0; i < e->layers; ++i)

@@ -140,3 +140,21 @@ def test_weights_beyond_31_bits_are_refused(wide, emb, blocks, taken):
         l.block_end = 1
     e.layers, e.layer = blocks, layers
     assert (_lib.load().na1d_encode_workspace_bytes(ctypes.byref(e), 4, 100) > 0) == taken
+
+
+_POINTERS = [n for n, t in encoder._Layer._fields_ if t is ctypes.c_void_p and n not in ("rpb", "w_pos")]
+
+
+@pytest.mark.parametrize("name", _POINTERS + [n for n, t in encoder._Encoder._fields_ if t is ctypes.c_void_p and n != "pos"] + ["out", "x", "workspace"])
+def test_missing_pointers_are_refused(name):
+    """Before anything is launched: every argument but one is in order."""
+    plan = encoder._Plan(_model(), torch.bfloat16)
+    lib, e, args = _lib.load(), plan.encoder, {"out": 4096, "x": 4096, "workspace": 4096}
+    need = lib.na1d_encode_workspace_bytes(ctypes.byref(e), 2, 64)
+    assert need > 0
+    if name in args:
+        args[name] = None
+    else:
+        setattr(plan.layers[0] if name in _POINTERS else e, name, None)
+    st = lib.na1d_encode(ctypes.byref(e), args["out"], args["x"], None, 2, 64, args["workspace"], need, None)
+    assert st in (-1, _lib.UNSUPPORTED)                     # a weight's absence already says that nothing covers the call
