@@ -2,7 +2,9 @@
 
 :func:`embed` runs the models of ``models.py`` through the token-local kernels of ``csrc/na1d_encoder.hip`` and the
 attention kernels, launched back to back from native code.  Its plan holds the weights in the kernels' order with the
-batch norms folded into them; it is rebuilt when a parameter or a running statistic changes.
+batch norms folded into them; what is made of a parameter or running statistic is made again when it changes (torch counts
+the versions of a tensor; writes through ``.data`` are seen in the last layer, the pooled norm, dense layers' first norms and
+the biases of scores and outputs, which the kernels read from the modules).
 """
 from __future__ import annotations
 
