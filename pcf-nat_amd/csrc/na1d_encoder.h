@@ -121,18 +121,21 @@ template <class DT> __device__ inline f32x4 widen4(u32x2 w) {
 }
 template <class DT> __device__ inline u32x2 narrow4(f32x4 v) { return u32x2{Mma<DT>::pack(v[0], v[1]), Mma<DT>::pack(v[2], v[3])}; }
 
-// x * Phi(x), the exact (erf) GELU, by formula 7.1.26 of Abramowitz and Stegun's handbook (error of erf below 1.5e-7):
-// with t = 1 / (1 + p z), z = |x| / sqrt 2, erfc(z) = t (a1 + t (a2 + ...)) exp(-z^2), and
-// gelu(x) = max(x, 0) - |x| erfc(z) / 2 for either sign.
+// x * Phi(x), the exact (erf) GELU, as max(x, 0) - |x| Phi(-|x|) for either sign.  The base-2 logarithm of Phi(-a) is a smooth
+// function that a polynomial of degree 7 follows (least weighted maximum over 0 .. 12; its leading coefficient is negative, so
+// the tail vanishes beyond): the whole is within 2.7e-7 of the exact value at fp32, most of it the result's own rounding (3.3e-7
+// by formula 7.1.26 of Abramowitz and Stegun's handbook, which takes a reciprocal too).  The layers' kernels are bound by vector
+// instructions where the blocks are grouped; passes of 25600, 64000 and 10000 tokens: 1272 -> 1211, 3702 -> 3558, 1092 -> 1028 us.
 __device__ inline float gelu(float x) {
-    const float ax = __builtin_fabsf(x);
-    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(ax, 0.3275911f * 0.70710678f, 1.f));
-    float e = __builtin_fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
-    e = __builtin_fmaf(t, e, 0.5f * 1.421413741f);
-    e = __builtin_fmaf(t, e, 0.5f * -0.284496736f);
-    e = __builtin_fmaf(t, e, 0.5f * 0.254829592f);
-    const float ex = __builtin_amdgcn_exp2f(x * x * -0.72134752f);
-    return __builtin_fmaf(-ax * t, e * ex, __builtin_fmaxf(x, 0.f));
+    const float a = __builtin_fabsf(x);
+    float p = __builtin_fmaf(a, -1.2898502745883889e-06f, 5.1304265070939437e-05f);
+    p = __builtin_fmaf(a, p, -0.0008600319852121174f);
+    p = __builtin_fmaf(a, p, 0.008291247300803661f);
+    p = __builtin_fmaf(a, p, -0.05365335941314697f);
+    p = __builtin_fmaf(a, p, -0.4586409628391266f);
+    p = __builtin_fmaf(a, p, -1.151228427886963f);
+    p = __builtin_fmaf(a, p, -0.9999922513961792f);
+    return __builtin_fmaf(-a, __builtin_amdgcn_exp2f(p), __builtin_fmaxf(x, 0.f));
 }
 
 }  // namespace enc
