@@ -19,6 +19,11 @@ constexpr int kFrag = 1024;          // bytes of a weight fragment: 16 outputs x
 // (the rows an operand read touches land in distinct banks, and the swizzle is the same for every tile).
 __device__ inline int tile_addr(int row, int unit) { return row * kRow + ((unit ^ (row & 15)) << 4); }
 
+// A lane's place in such a tile, as the operand of a product (unit g of row n) and for four channels of its results (channels
+// 4g .. 4g+3); the units that a step or a tile of outputs lies further on only turn bits over: one instruction by a constant.
+__device__ inline int operand_lane(int n, int g) { return n * kRow + ((g ^ n) << 4); }
+__device__ inline int result_lane(int n, int g) { return n * kRow + (((g >> 1) ^ n) << 4) + (g & 1) * 8; }
+
 // Copy `rows` (a multiple of 16) token rows of `width` bytes, `pitch` bytes apart, into such a tile with loads that write
 // LDS directly; the resource ends behind the last row there is, and bytes past a row's width arrive as zeros.
 template <int ROWS, int NW, int AUX>
@@ -78,25 +83,60 @@ __device__ inline void multiply(f32x4 (&acc)[NA][MT], int a0, Ring<NTW, PF> &rin
         for (int s = P::kSteps; s < PF; ++s)
             if (s < Q::kSteps) ring.fill(next, s, s, lane16);
     }
-    const int xr = n * kRow, xs = 4 * p.x0 + g;
+    // Rows are read one turn (a step, or a tile of it where tiles differ in their inputs) ahead and no further: left to itself
+    // the scheduler reads a whole product's rows at its start, which takes the registers of the waves that would hide the rest.
+    constexpr int kPerStep = P::kSkip ? P::kTiles : 1, kTurns = P::kSteps * kPerStep;
+    const int x_lane = operand_lane(n, g);
+    u32x4 x[2][MT];
+    auto read = [&](int turn) {
+        LDS_PTR(char) at = tile + (x_lane ^ 64 * (p.x0 + P::skip(turn % kPerStep) + turn / kPerStep));
 #pragma unroll
-    for (int s = 0; s < P::kSteps; ++s) {
-        u32x4 x[MT];
+        for (int i = 0; i < MT; ++i) x[turn & 1][i] = *reinterpret_cast<LDS_PTR(u32x4)>(at + i * 16 * kRow);
+    };
+    read(0);
 #pragma unroll
-        for (int j = 0; j < P::kTiles; ++j) {
-            if (j == 0 || P::kSkip) {
-                LDS_PTR(char) at = tile + xr + (((xs + 4 * (P::skip(j) + s)) ^ n) << 4);
+    for (int turn = 0; turn < kTurns; ++turn) {
+        const int s = turn / kPerStep, j0 = turn % kPerStep;
+        if (turn + 1 < kTurns) read(turn + 1);
+        __builtin_amdgcn_sched_barrier(0x27f);       // anything but reads of LDS
 #pragma unroll
-                for (int i = 0; i < MT; ++i) x[i] = *reinterpret_cast<LDS_PTR(u32x4)>(at + i * 16 * kRow);
-            }
+        for (int j = j0; j < (P::kSkip ? j0 + 1 : P::kTiles); ++j)
 #pragma unroll
-            for (int i = 0; i < MT; ++i) acc[a0 + j][i] = Mma<DT>::k32(ring.w[s % PF][j], x[i], acc[a0 + j][i]);
-        }
+            for (int i = 0; i < MT; ++i) acc[a0 + j][i] = Mma<DT>::k32(ring.w[s % PF][j], x[turn & 1][i], acc[a0 + j][i]);
+        if (j0 + 1 < kPerStep) continue;
         if (s + PF < P::kSteps) {
             ring.fill(p, s % PF, s + PF, lane16);
         } else {
             const int t = P::kSteps < PF ? s : s + PF - P::kSteps;
             if (t < Q::kSteps) ring.fill(next, s % PF, t, lane16);
+        }
+    }
+}
+// The same over a number of steps known at run time, from LDS rows that are still on their way: the first weights set out
+// before the wait for the rows.
+template <class DT, int MT, int NTW, int PF, class P>
+__device__ inline void multiply_all(f32x4 (&acc)[NTW][MT], Ring<NTW, PF> &ring, const P &p, int steps, LDS_PTR(char) tile, int n, int g, int lane16) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u)
+        if (u < steps) ring.fill(p, u, u, lane16);
+    wait_direct();
+    barrier_lds();
+    const int x_lane = operand_lane(n, g);
+#pragma unroll 1
+    for (int s0 = 0; s0 < steps; s0 += PF) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) {
+            const int s = s0 + u;
+            if (s >= steps) break;
+            LDS_PTR(char) at = tile + (x_lane ^ 64 * (p.x0 + s));
+            u32x4 x[MT];
+#pragma unroll
+            for (int i = 0; i < MT; ++i) x[i] = *reinterpret_cast<LDS_PTR(u32x4)>(at + i * 16 * kRow);
+#pragma unroll
+            for (int j = 0; j < NTW; ++j)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) acc[j][i] = Mma<DT>::k32(ring.w[u][j], x[i], acc[j][i]);
+            if (s + PF < steps) ring.fill(p, u, s + PF, lane16);
         }
     }
 }

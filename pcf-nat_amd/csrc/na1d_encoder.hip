@@ -59,7 +59,7 @@ template <int G, int NW> struct Groups {
     static constexpr int kPer = kOutTiles >= NW ? kOutTiles / NW : 1;  // of them to a wave
     static constexpr int kActive = kOutTiles < NW ? kOutTiles : NW;    // waves that have any
     static constexpr int kFc2 = G == 8 ? 4 : 8;
-    static constexpr int kAcc = kSets * kPer;                          // output tiles of a wave over all chunks
+    static constexpr int kEach = 4 / kSets;                            // chunks that reach the same ones
     static constexpr int kQkv = G == 1 ? 8 : G == 4 ? 2 : 4;
     static constexpr int kQkvSkip = G == 4 ? 1 : G == 8 ? 2 : 0;
     using Proj = Product<NTW, kProj>;
@@ -85,23 +85,50 @@ template <int G, int NW> struct Groups {
     }
 };
 
+// Places of the biases in LDS, in floats.
+constexpr int kBiasFc1 = 0, kBiasQkv = 0, kBiasProj = kHidden, kBiasFc2 = kBiasProj + kDim, kBias = kBiasFc2 + kDim;
+template <int MT> constexpr size_t layer_lds() { return (size_t)2 * 16 * MT * kRow + kBias * sizeof(float); }
+
 // The number of groups as the kernels know it: every switch over it and every sum over its parts starts from this.
 inline int known_groups(int groups) { return groups == 2 || groups == 4 || groups == 8 ? groups : 1; }
 
-template <class DT, int MT, int NW, int PF> struct LayerWave {
+template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
     static constexpr int NTW = 16 / NW, CW = 16 * NTW;
     const LayerArgs &a;
     LDS_PTR(char) p_lds;
     LDS_PTR(char) q_lds;
+    LDS_PTR(float) b_lds;             // the projections' biases, kBias floats
     int wave, lane, n, g, lane16;
     Ring<NTW, PF> ring;
 
     // LDS place of channels c + 4g .. + 3 of token n (c: a multiple of 16, wave-uniform)
-    __device__ inline int piece(int c) const { return n * kRow + (((c / 8 + (g >> 1)) ^ n) << 4) + (g & 1) * 8; }
     __device__ inline LDS_PTR(u32x2) at(LDS_PTR(char) tile, int c, int i) const {
-        return reinterpret_cast<LDS_PTR(u32x2)>(tile + piece(c) + i * 16 * kRow);
+        return reinterpret_cast<LDS_PTR(u32x2)>(tile + (result_lane(n, g) ^ 2 * c) + i * 16 * kRow);
     }
     __device__ inline f32x4 bias(const float *b, int c) const { return *reinterpret_cast<const f32x4 *>(b + c + 4 * g); }
+    __device__ inline f32x4 staged_bias(int c) const { return *reinterpret_cast<LDS_PTR(f32x4)>(b_lds + c + 4 * g); }
+
+    // Biases come through LDS, and sums start at them: read from memory behind a product, a bias would have to wait for every
+    // weight of the next product that is on its way (loads return in order).  qkv's take the place of fc1's first 768.
+    __device__ inline void stage_bias(const float *b, int count, int to) const {
+        for (int k = wave; k < count / 256; k += NW) load_to_lds<16, kReadShared>(make_rsrc(b, 4 * count), (LDS_PTR(char))(b_lds + to + 256 * k), 1024 * k + lane16);
+    }
+    __device__ inline void stage_tail_biases() const {
+        stage_bias(a.b_proj, kDim, kBiasProj);
+        stage_bias(a.b_fc1, kHidden, kBiasFc1);
+        stage_bias(a.b_fc2, kDim, kBiasFc2);
+    }
+    __device__ inline void stage_qkv_bias() const {
+        if (a.qkv) stage_bias(a.b_qkv, 3 * kDim, kBiasQkv);
+    }
+    template <int NTILES> __device__ inline void begin_sums(f32x4 (&acc)[NTILES][MT], int c) const {
+#pragma unroll
+        for (int j = 0; j < NTILES; ++j) {
+            const f32x4 b = staged_bias(c + 16 * j);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[j][i] = b;
+        }
+    }
 
     // attention rows in p_lds, x in q_lds (on their way) -> x1 in q_lds; the ring holds the start of fc1's chunk c
     template <int G> __device__ inline void project(Rsrc w1, int first_chunk) {
@@ -109,32 +136,31 @@ template <class DT, int MT, int NW, int PF> struct LayerWave {
         const auto proj = S::proj(weight_rsrc(a.w_proj, kDim, kDim), wave);
         ring.begin(proj, lane16);
         f32x4 hid[NTW][MT];
-        clear(hid);
         wait_direct();
         barrier_lds();
+        begin_sums(hid, kBiasProj + CW * wave);
         multiply<DT, MT>(hid, 0, ring, proj, S::fc1(w1, first_chunk, wave), p_lds, n, g, lane16);
 #pragma unroll
         for (int j = 0; j < NTW; ++j) {
             const int c = CW * wave + 16 * j;
-            const f32x4 b = bias(a.b_proj, c);
 #pragma unroll
-            for (int i = 0; i < MT; ++i) *at(q_lds, c, i) = narrow4<DT>(hid[j][i] + b + widen4<DT>(*at(q_lds, c, i)));
+            for (int i = 0; i < MT; ++i) *at(q_lds, c, i) = narrow4<DT>(hid[j][i] + widen4<DT>(*at(q_lds, c, i)));
         }
     }
-    // 256 hidden channels: x1 in q_lds -> their share of the output in acc[a0 ..] (a0 a constant)
-    template <int G, int NA> __device__ inline void chunk(f32x4 (&acc)[NA][MT], Rsrc w1, Rsrc w2, int c, int a0, bool last) {
+    // 256 hidden channels: x1 in q_lds -> their share of the output in acc
+    template <int G, int NA> __device__ inline void chunk(f32x4 (&acc)[NA][MT], Rsrc w1, Rsrc w2, int c, bool last) {
         using S = Groups<G, NW>;
         f32x4 hid[NTW][MT];
-        clear(hid);
+        begin_sums(hid, kBiasFc1 + 256 * c + CW * wave);
         barrier_lds();                           // x1 is whole (first round); every wave is done with the hidden channels before
+        if (c == 3 && !SPLIT) stage_qkv_bias();  // every wave has taken fc1's
         multiply<DT, MT>(hid, 0, ring, S::fc1(w1, c, wave), S::fc2(w2, c, wave), q_lds, n, g, lane16);
 #pragma unroll
         for (int j = 0; j < NTW; ++j) {
             const int ch = CW * wave + 16 * j;
-            const f32x4 b = bias(a.b_fc1, 256 * c + ch);
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
-                f32x4 h = hid[j][i] + b;
+                f32x4 h = hid[j][i];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) h[r] = gelu(h[r]);
                 *at(p_lds, ch, i) = narrow4<DT>(h);
@@ -142,7 +168,7 @@ template <class DT, int MT, int NW, int PF> struct LayerWave {
         }
         barrier_lds();
         if (wave < S::kActive)
-            multiply<DT, MT>(acc, a0, ring, S::fc2(w2, c, wave), S::fc1(w1, last ? 0 : c + 1, wave), p_lds, n, g, lane16);
+            multiply<DT, MT>(acc, 0, ring, S::fc2(w2, c, wave), S::fc1(w1, last ? 0 : c + 1, wave), p_lds, n, g, lane16);
         else
             ring.begin(S::fc1(w1, last ? 0 : c + 1, wave), lane16);
     }
@@ -151,24 +177,28 @@ template <class DT, int MT, int NW, int PF> struct LayerWave {
         using S = Groups<G, NW>;
         const Rsrc w1 = weight_rsrc(a.w_fc1, kHidden, kDim), w2 = weight_rsrc(a.w_fc2, kDim, kHidden);
         project<G>(w1, 0);
-        f32x4 acc[S::kAcc][MT];
-        clear(acc);
-        if constexpr (S::kSets == 1) {
+        // Outputs that a later chunk adds nothing to are written at once, over x1: the chunks behind read other channels.
 #pragma unroll 1
-            for (int c = 0; c < 4; ++c) chunk<G>(acc, w1, w2, c, 0, c == 3);
-        } else {
+        for (int set = 0; set < S::kSets; ++set) {
+            const int first = 16 * (set * S::kOutTiles + wave * S::kPer);
+            f32x4 acc[S::kPer][MT];
+            if (wave < S::kActive) begin_sums(acc, kBiasFc2 + first);
+#pragma unroll 1
+            for (int k = 0; k < S::kEach; ++k) {
+                const int c = set * S::kEach + k;
+                chunk<G>(acc, w1, w2, c, c == 3);
+            }
+            if (wave < S::kActive) {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) chunk<G>(acc, w1, w2, c, c * S::kSets / 4 * S::kPer, c == 3);
-        }
-        if (wave < S::kActive) {
+                for (int t = 0; t < S::kPer; ++t)
 #pragma unroll
-            for (int t = 0; t < S::kAcc; ++t) {
-                const int c = 16 * (t / S::kPer * S::kOutTiles + wave * S::kPer + t % S::kPer);
-                const f32x4 b = bias(a.b_fc2, c);
-#pragma unroll
-                for (int i = 0; i < MT; ++i) *at(q_lds, c, i) = narrow4<DT>(acc[t][i] + b + widen4<DT>(*at(q_lds, c, i)));
+                    for (int i = 0; i < MT; ++i) {
+                        LDS_PTR(u32x2) x = at(q_lds, first + 16 * t, i);
+                        *x = narrow4<DT>(acc[t][i] + widen4<DT>(*x));
+                    }
             }
         }
+        wait_direct();                           // qkv's biases
     }
 
     // a quarter of it: x1 to memory (the first quarter's), the hidden channels' share of the output to `parts`
@@ -178,7 +208,7 @@ template <class DT, int MT, int NW, int PF> struct LayerWave {
         project<G>(w1, c);
         f32x4 acc[S::kPer][MT];
         clear(acc);
-        chunk<G>(acc, w1, w2, c, 0, true);
+        chunk<G>(acc, w1, w2, c, true);
         const Rsrc d = make_rsrc(a.parts + ((int64_t)c * a.M + m0) * kDim, rows * kDim * 4);
         if (wave < S::kActive) {
 #pragma unroll
@@ -226,15 +256,13 @@ template <class DT, int MT, int NW, int PF> struct LayerWave {
 #pragma unroll 1
         for (int which = from; which < to; ++which) {
             f32x4 acc[NTW][MT];
-            clear(acc);
+            begin_sums(acc, kBiasQkv + which * kDim + CW * wave);
             multiply<DT, MT>(acc, 0, ring, S::qkv(w, which, wave), S::qkv(w, min(which + 1, 2), wave), q_lds, n, g, lane16);
             u32x2 o[MT][NTW];
 #pragma unroll
-            for (int j = 0; j < NTW; ++j) {
-                const f32x4 b = bias(a.b_qkv, which * kDim + CW * wave + 16 * j);
+            for (int j = 0; j < NTW; ++j)
 #pragma unroll
-                for (int i = 0; i < MT; ++i) o[i][j] = narrow4<DT>(acc[j][i] + b);
-            }
+                for (int i = 0; i < MT; ++i) o[i][j] = narrow4<DT>(acc[j][i]);
 #pragma unroll
             for (int i = 0; i < MT; ++i)
                 store_tile<CW, 0>(qs, (16 * i + n) * (3 * kRow) + which * kRow + 2 * CW * wave, o[i], g, 2 * CW);
@@ -259,16 +287,17 @@ template <class DT, int MT, int NW, int PF> struct LayerWave {
 template <class DT, int NW, int PF>
 __global__ void __launch_bounds__(64 * NW, 2)
 part_kernel(LayerArgs a) {
-    using W = LayerWave<DT, 1, NW, PF>;
+    using W = LayerWave<DT, 1, NW, PF, true>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    W w{a, (LDS_PTR(char))smem, (LDS_PTR(char))smem + 16 * kRow, wave, lane, lane & 15, lane >> 4, lane * 16};
+    W w{a, (LDS_PTR(char))smem, (LDS_PTR(char))smem + 16 * kRow, (LDS_PTR(float))(smem + 32 * kRow), wave, lane, lane & 15, lane >> 4, lane * 16};
     const int c = (int)(blockIdx.x & 3);
     const int64_t m0 = (int64_t)(blockIdx.x >> 2) * 16;
     const int rows = (int)min((int64_t)16, a.M - m0);
     const Rsrc as = make_rsrc(a.attn + m0 * kRow, rows * kRow), xs = make_rsrc(a.x_in + m0 * a.x_in_pitch, rows * a.x_in_pitch);
     stage_tokens<16, NW, kReadShared>(as, w.p_lds, kRow, kRow, wave, lane);
     stage_tokens<16, NW, kReadShared>(xs, w.q_lds, a.x_in_pitch, kRow, wave, lane);
+    w.stage_tail_biases();
     switch (a.tail_groups) {
         case 8: w.template tail_part<8>(c, m0, rows); break;
         case 4: w.template tail_part<4>(c, m0, rows); break;
@@ -277,22 +306,30 @@ part_kernel(LayerArgs a) {
     }
 }
 
+// Waves on a SIMD.  SPARSE (blocks of 4 or 8 groups before the tile) and dense layers are kernels of their own, so that the
+// former, whose sums never span chunks, run 64 tokens with eight waves of 128 registers: a layer of 64000 tokens 75 -> 70 us,
+// its qkv projection 9 -> 4.5 of a workgroup's 35 us.  Dense layers need the registers for weights that set out four steps
+// ahead (145 -> 134 us); with eight waves of 128 registers they spill 55 and a whole pass takes 3.72 instead of 3.37 ms.
+constexpr int layer_waves(int MT, int NW) { return MT == 2 || (MT == 4 && NW == 8) ? 4 : 2; }
+
 // SPLIT: one workgroup to each of q, k and v of a tile (or one where there is no projection behind); the layer before
 // comes in quarters
-template <class DT, int MT, int NW, int PF, bool SPLIT>
-__global__ void __launch_bounds__(64 * NW, MT == 2 ? 3 : 2)
+template <class DT, int MT, int NW, int PF, bool SPLIT, bool SPARSE>
+__global__ void __launch_bounds__(64 * NW, layer_waves(MT, NW))
 layer_kernel(LayerArgs a) {
-    using W = LayerWave<DT, MT, NW, PF>;
+    using W = LayerWave<DT, MT, NW, PF, SPLIT>;
     constexpr int NTW = W::NTW, CW = W::CW;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // p_lds: attention rows, then 256 hidden channels at a time, then patches; q_lds: x, then x1, then x2
-    W w{a, (LDS_PTR(char))smem, (LDS_PTR(char))smem + 16 * MT * kRow, wave, lane, lane & 15, lane >> 4, lane * 16};
+    W w{a, (LDS_PTR(char))smem, (LDS_PTR(char))smem + 16 * MT * kRow, (LDS_PTR(float))(smem + 32 * MT * kRow), wave, lane, lane & 15, lane >> 4, lane * 16};
     const int each = SPLIT && a.qkv ? 3 : 1, mine = each == 3 ? (int)(blockIdx.x % 3u) : 0;
     const int64_t m0 = (int64_t)(blockIdx.x / (uint32_t)each) * (16 * MT);
     const int rows = (int)min((int64_t)(16 * MT), a.M - m0);
+    if (SPLIT || !a.attn) w.stage_qkv_bias();
     if (SPLIT && a.attn) {
         w.join(m0, rows);
+        wait_direct();                               // qkv's biases
         if (a.block_out && mine == 0) {
             barrier_lds();
             w.write_rows(a.block_out, m0, rows, a.block_pitch);
@@ -301,11 +338,17 @@ layer_kernel(LayerArgs a) {
         const Rsrc as = make_rsrc(a.attn + m0 * kRow, rows * kRow), xs = make_rsrc(a.x_in + m0 * a.x_in_pitch, rows * a.x_in_pitch);
         stage_tokens<16 * MT, NW, kReadOnce>(as, w.p_lds, kRow, kRow, wave, lane);
         stage_tokens<16 * MT, NW, kReadOnce>(xs, w.q_lds, a.x_in_pitch, kRow, wave, lane);
-        switch (a.tail_groups) {
-            case 8: w.template tail<8>(); break;
-            case 4: w.template tail<4>(); break;
-            case 2: w.template tail<2>(); break;
-            default: w.template tail<1>();
+        w.stage_tail_biases();
+        if constexpr (SPARSE) {
+            if (a.tail_groups == 8)
+                w.template tail<8>();
+            else
+                w.template tail<4>();
+        } else {
+            if (a.tail_groups == 2)
+                w.template tail<2>();
+            else
+                w.template tail<1>();
         }
         if (a.block_out) {
             barrier_lds();
@@ -327,14 +370,7 @@ layer_kernel(LayerArgs a) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) acc[j][i] = a.attn ? widen4<DT>(*w.at(w.q_lds, c, i)) + b : b;
         }
-        wait_direct();
-        barrier_lds();
-#pragma unroll 1
-        for (int s = 0; s < ks_all; ++s) {
-            const Product<NTW, 1> p{we, wave * NTW * ks_all + s, ks_all, s};
-            w.ring.fill(p, 0, 0, w.lane16);
-            multiply<DT, MT>(acc, 0, w.ring, p, Nothing{}, w.p_lds, w.n, w.g, w.lane16);
-        }
+        multiply_all<DT, MT>(acc, w.ring, Product<NTW, 1>{we, wave * NTW * ks_all, ks_all, 0}, ks_all, w.p_lds, w.n, w.g, w.lane16);
 #pragma unroll
         for (int j = 0; j < NTW; ++j)
 #pragma unroll
@@ -774,10 +810,10 @@ pool_kernel(PoolArgs a) {
 }
 
 // ----------------------------------------------------------------------------- launchers
-template <class DT, int MT, int NW, int PF>
+template <class DT, int MT, int NW, int PF, bool SPARSE>
 int launch_layer_mt(const LayerArgs &a, hipStream_t s) {
-    auto kern = layer_kernel<DT, MT, NW, PF, false>;
-    const size_t lds = (size_t)2 * 16 * MT * kRow;
+    auto kern = layer_kernel<DT, MT, NW, PF, false, SPARSE>;
+    const size_t lds = layer_lds<MT>();
     if (!allow_lds(kern, lds)) return NA1D_ERR_LAUNCH;
     const int64_t wgs = (a.M + 16 * MT - 1) / (16 * MT);
     kern<<<(unsigned)wgs, 64 * NW, lds, s>>>(a);
@@ -788,23 +824,26 @@ int launch_layer_mt(const LayerArgs &a, hipStream_t s) {
 // 125 tokens 273 and 336 us, 500: 295 and 344, 1000: 335 and 352; 1500: 426 and 370, 4000: 634 and 454.
 constexpr int64_t kSplitTokens = 16 * 64;
 template <class DT> int launch_layer_split(const LayerArgs &a, hipStream_t s) {
-    const size_t lds = (size_t)2 * 16 * kRow;
+    const size_t lds = layer_lds<1>();
     const unsigned tiles = (unsigned)((a.M + 15) / 16);
     if (a.attn) {
         part_kernel<DT, 8, 8><<<4 * tiles, 512, lds, s>>>(a);
         const int st = launch_status();
         if (st != NA1D_OK) return st;
     }
-    layer_kernel<DT, 1, 8, 8, true><<<(a.qkv ? 3 : 1) * tiles, 512, lds, s>>>(a);
+    layer_kernel<DT, 1, 8, 8, true, false><<<(a.qkv ? 3 : 1) * tiles, 512, lds, s>>>(a);
     return launch_status();
 }
 
 template <class DT> int launch_layer(const LayerArgs &a, hipStream_t s) {
     if (a.M <= kSplitTokens) return launch_layer_split<DT>(a, s);
-    // Fewer, larger tiles read the layer's weights fewer times; smaller ones spread few tokens over more CUs.
-    if (a.M <= 16 * 256) return launch_layer_mt<DT, 1, 8, 8>(a, s);
-    if (a.M <= 32 * 512) return launch_layer_mt<DT, 2, 8, 4>(a, s);
-    return launch_layer_mt<DT, 4, 4, 2>(a, s);
+    // Fewer, larger tiles read the layer's weights fewer times; smaller ones spread few tokens over more CUs.  PCF 4x4 passes
+    // with tiles of 16, 32 and 64 tokens: 4000 tokens 454, 496 and 657 us; 6000: 627, 543, 698; 16000: 1124, 900, 909;
+    // 20000: 1350, 1122, 1109; 25600: 1737, 1344, 1222.
+    const bool sparse = a.tail_groups >= 4;
+    if (a.M <= 16 * 256) return sparse ? launch_layer_mt<DT, 1, 8, 8, true>(a, s) : launch_layer_mt<DT, 1, 8, 8, false>(a, s);
+    if (a.M <= 32 * 512) return sparse ? launch_layer_mt<DT, 2, 8, 4, true>(a, s) : launch_layer_mt<DT, 2, 8, 4, false>(a, s);
+    return sparse ? launch_layer_mt<DT, 4, 8, 4, true>(a, s) : launch_layer_mt<DT, 4, 4, 4, false>(a, s);
 }
 
 template <class DT, LinearEnd END> int launch_linear(const LinearArgs &a, hipStream_t s) {

@@ -57,6 +57,15 @@ def test_group_counts_without_kernels_of_their_own(groups, batch, frames):
     assert native is not None and _near(native, modules)
 
 
+@pytest.mark.parametrize("groups", [(8, 4), (2, 1)])
+@pytest.mark.parametrize("batch,frames", [(53, 32), (81, 100), (86, 96), (293, 112), (331, 100)])
+def test_tiles_of_every_size(groups, batch, frames):
+    """Each side of the token counts at which the tiles grow (1024 is the split's; 4096, 16384), the last tile not full."""
+    model = _model(groups=groups)
+    native, modules = _both(model, _input(batch, frames))
+    assert native is not None and _near(native, modules)
+
+
 @pytest.mark.parametrize("groups", [0, 3, 16])
 @pytest.mark.parametrize("batch,frames", [(3, 111), (80, 128)])
 def test_layers_of_the_c_interface_are_dense_unless_2_4_or_8(groups, batch, frames):
