@@ -431,9 +431,9 @@ struct LinearArgs {
     na1d_encoder_norm norm;                             // kShift
 };
 template <class DT, LinearEnd END>
-__device__ inline void finish(const LinearArgs &a, Rsrc out, int64_t m0, int row, int c, f32x4 v) {
+__device__ inline f32x4 ended(const LinearArgs &a, int64_t m, int c, f32x4 v) {
     if constexpr (END == kTanhNorm) {
-        const uint32_t u = (uint32_t)(m0 + row) / (uint32_t)a.T;
+        const uint32_t u = (uint32_t)m / (uint32_t)a.T;
         v += *reinterpret_cast<const f32x4 *>(a.bias + (int64_t)u * a.outputs + c);
     } else if constexpr (END == kShift) {
         v += *reinterpret_cast<const f32x4 *>(a.norm.bias + c) - *reinterpret_cast<const f32x4 *>(a.norm.mean + c) * norm_gain(a.norm, c);
@@ -448,6 +448,11 @@ __device__ inline void finish(const LinearArgs &a, Rsrc out, int64_t m0, int row
             if constexpr (END == kTanhNorm) v[r] = tanh_of(v[r]);
         }
     }
+    return v;
+}
+template <class DT, LinearEnd END>
+__device__ inline void finish(const LinearArgs &a, Rsrc out, int64_t m0, int row, int c, f32x4 v) {
+    v = ended<DT, END>(a, m0 + row, c, v);
     if constexpr (END == kAffine || END == kShift)
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), out, row * a.out_pitch + 4 * c, 0, 0);
     else
@@ -498,6 +503,78 @@ linear_kernel(LinearArgs a, int col_blocks) {
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NTW; ++j) finish<DT, END>(a, os, m0, 16 * i + n, 16 * (tile0 + j) + 4 * g, acc[j][i]);
+}
+
+// Very many rows, outputs in hundreds: 128 rows x 256 outputs to a workgroup of four waves.  A wave's 128 x 64 outputs use each
+// weight eight times and each row's operand four times, which halves what the CU's path to L2 carries per product (64 rows ask
+// for its 64 bytes a clock at the matrix cores' full rate); rows come 128 inputs at a time, so two workgroups share a CU.
+// 1024 inputs, 1536 outputs: 25600 rows 124 -> 72 us, 64000 301 -> 184 us (1.1 PFLOP/s), from what whole passes lose.
+template <class DT, LinearEnd END>
+__global__ void __launch_bounds__(kThreads, 2)
+linear_wide_kernel(LinearArgs a, int col_blocks) {
+    constexpr int MT = 8, NTW = 4, PF = 4, NW = kWaves, kSteps = 4, kPiece = 64 * kSteps;     // bytes of a row's piece
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    LDS_PTR(char) lds = (LDS_PTR(char))smem;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
+    const uint32_t item = xcd_item(blockIdx.x, gridDim.x);           // neighbours share their rows' lines
+    const uint32_t row_block = item / (uint32_t)col_blocks;
+    const int64_t m0 = (int64_t)row_block * (16 * MT);
+    const int rows = (int)min((int64_t)(16 * MT), a.M - m0);
+    const int tile0 = ((int)(item - row_block * col_blocks) * NW + wave) * NTW;
+    const Rsrc xs = make_rsrc(a.x + m0 * a.x_pitch, rows * a.x_pitch), ws = weight_rsrc(a.w, a.outputs, a.inputs);
+    const int steps = a.inputs / 32, pieces = steps / kSteps, lane16 = lane * 16;
+    auto stage = [&](int piece) {                                    // four rows to a load, their 16-byte units swizzled by the row
+#pragma unroll
+        for (int j = 0; j < 16 * MT * kPiece / kChunk / NW; ++j) {
+            const int c = j * NW + wave, row = 4 * c + (lane >> 4);
+            load_to_lds<16, kReadShared>(xs, lds + (piece & 1) * (16 * MT * kPiece) + c * kChunk, row * a.x_pitch + piece * kPiece + ((lane & 15) ^ (row & 15)) * 16);
+        }
+    };
+    stage(0);
+    f32x4 acc[NTW][MT];
+    clear(acc);
+    u32x4 w[PF][NTW];
+    auto fill = [&](int slot, int step) {
+#pragma unroll
+        for (int j = 0; j < NTW; ++j)
+            w[slot][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ws, lane16, ((tile0 + j) * steps + step) * kFrag, 0));
+    };
+#pragma unroll
+    for (int s = 0; s < PF; ++s) fill(s, s);
+    const int x_lane = n * kPiece + ((g ^ n) << 4);
+#pragma unroll 1
+    for (int p = 0; p < pieces; ++p) {
+        wait_direct();
+        barrier_lds();
+        if (p + 1 < pieces) stage(p + 1);
+        LDS_PTR(char) from = lds + (p & 1) * (16 * MT * kPiece);
+        u32x4 x[2][4];
+        auto read = [&](int turn) {                                  // four of the row tiles of a step
+            LDS_PTR(char) at = from + (x_lane ^ 64 * (turn >> 1)) + (turn & 1) * (64 * kPiece);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[turn & 1][i] = *reinterpret_cast<LDS_PTR(u32x4)>(at + i * 16 * kPiece);
+        };
+        read(0);
+#pragma unroll
+        for (int turn = 0; turn < 2 * kSteps; ++turn) {
+            const int s = turn >> 1, i0 = 4 * (turn & 1);
+            if (turn + 1 < 2 * kSteps) read(turn + 1);
+            __builtin_amdgcn_sched_barrier(0x27f);                   // see multiply()
+#pragma unroll
+            for (int j = 0; j < NTW; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[j][i0 + i] = Mma<DT>::k32(w[s % PF][j], x[turn & 1][i], acc[j][i0 + i]);
+            if (turn & 1) fill(s % PF, min(kSteps * p + s + PF, steps - 1));
+        }
+    }
+    const Rsrc os = make_rsrc(a.out + m0 * a.out_pitch, rows * a.out_pitch);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        u32x2 o[NTW];
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) o[j] = narrow4<DT>(ended<DT, END>(a, m0 + 16 * i + n, 16 * (tile0 + j) + 4 * g, acc[j][i]));
+        store_tile<16 * NTW, 0>(os, (16 * i + n) * a.out_pitch + 32 * tile0, o, g, 32 * NTW);
+    }
 }
 
 // Few rows: the inputs are split over the eight waves of a workgroup that computes 16 rows x 16 * NT outputs; rows and
@@ -848,13 +925,15 @@ template <class DT> int launch_layer(const LayerArgs &a, hipStream_t s) {
 
 template <class DT, LinearEnd END> int launch_linear(const LinearArgs &a, hipStream_t s) {
     if (a.inputs % 256 == 0 && a.M > 512) {
-        auto go = [&](auto kern, int mt, int ntw) {
-            const size_t lds = (size_t)2 * 16 * mt * kRow;
+        auto go = [&](auto kern, int mt, int ntw, int row = kRow) {
+            const size_t lds = (size_t)2 * 16 * mt * row;
             if (!allow_lds(kern, lds)) return (int)NA1D_ERR_LAUNCH;
             const int cols = a.outputs / (64 * ntw);
             kern<<<(unsigned)((a.M + 16 * mt - 1) / (16 * mt) * cols), kThreads, lds, s>>>(a, cols);
             return launch_status();
         };
+        if constexpr (END == kReluNorm)
+            if (a.outputs % 256 == 0 && a.M > 8192) return go(linear_wide_kernel<DT, END>, 8, 4, 256);
         if (a.outputs % 256 == 0 && a.M > 8192) return go(linear_kernel<DT, 4, 4, END>, 4, 4);
         if (a.outputs % 128 == 0) return a.M > 8192 ? go(linear_kernel<DT, 4, 2, END>, 4, 2) : go(linear_kernel<DT, 2, 2, END>, 2, 2);
     }

@@ -58,9 +58,9 @@ def test_group_counts_without_kernels_of_their_own(groups, batch, frames):
 
 
 @pytest.mark.parametrize("groups", [(8, 4), (2, 1)])
-@pytest.mark.parametrize("batch,frames", [(53, 32), (81, 100), (86, 96), (293, 112), (331, 100)])
+@pytest.mark.parametrize("batch,frames", [(53, 32), (81, 100), (86, 96), (163, 100), (164, 100), (293, 112), (331, 100)])
 def test_tiles_of_every_size(groups, batch, frames):
-    """Each side of the token counts at which the tiles grow (1024 is the split's; 4096, 16384), the last tile not full."""
+    """Each side of the token counts at which the tiles grow (1024 is the split's; 4096, 8192, 16384), the last tile not full."""
     model = _model(groups=groups)
     native, modules = _both(model, _input(batch, frames))
     assert native is not None and _near(native, modules)
