@@ -749,10 +749,14 @@ stats_kernel(float *__restrict__ mean_std, char *__restrict__ rounded, const cha
     reinterpret_cast<uint16_t *>(rounded)[at + wide] = (uint16_t)Mma<DT>::pack(std, 0.f);
 }
 
-// Attentive statistics pooling of 64 channels of an utterance: logits = W . hidden[t] on the matrix core, softmax over the
-// tokens and the weighted mean and deviation in one pass over the rows, the logits never written.  Lane (n, g) sees
-// channels 4g .. 4g+3 of each 16-channel tile for every 16th token, keeps its own running maximum (moved only when
-// outgrown by 2^8) and sums of p, p d, p d^2 (d = difference to the plain mean), and the lanes and waves meet at the end.
+// Attentive statistics pooling: logits = W . hidden[t] on the matrix core, softmax over the tokens and the weighted mean and
+// deviation in one pass over the rows, the logits never written.  Lane (n, g) sees channels 8g .. 8g+7 of each 32 (two tiles
+// of the product, whose rows are taken in that order) for every 16th token, keeps its own running maximum (moved only when outgrown by 2^8) and sums of p, p d, p d^2 (d =
+// difference to the plain mean), and the lanes meet at the end.  A wave takes 64 channels; the TS of four waves that have the
+// same ones share an utterance's tokens.  Bound by the latency of a wave's few turns and, at 100 tokens, by its two ends (16
+// weights to fetch, 256 steps across lanes): 256 utterances of 100 tokens take 77 us with four waves to an utterance and 47
+// with one, 64 of 1000 94 and 102; 20 of 150 a microsecond less with four.  With loads of 8 bytes in the tiles' own order and
+// none ahead of its turn four waves took 82 and 110.  Half the channels and twice the waves to a SIMD: 56 and 121.
 struct PoolArgs {
     const char *h, *hidden, *w;
     const float *count, *mean_std, *a_pool, *c_pool;
@@ -777,72 +781,89 @@ __device__ inline float row16_sum(float x) {
     x += row_step<0x141>(x);
     return x + row_step<0x140>(x);
 }
-template <class DT>
+template <class DT, int TS>
 __global__ void __launch_bounds__(kThreads, 2)
 pool_kernel(PoolArgs a) {
-    constexpr int kSlack = 8;
-    __shared__ float meet[kWaves][64][4];
+    constexpr int CT = 4, kSlack = 8, kChannels = 16 * CT * kWaves / TS;         // tiles of a wave, channels of a workgroup
+    __shared__ float meet[TS][kChannels][4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
-    const int utt = blockIdx.y, c0 = blockIdx.x * 64, pitch = 2 * a.wide;
+    const int part = wave % TS, mine = 16 * CT * (wave / TS);                    // tokens and channels of this wave
+    const int utt = blockIdx.y, c0 = blockIdx.x * kChannels, pitch = 2 * a.wide;
     const Rsrc hs = make_rsrc(a.h + (int64_t)utt * a.T * pitch, a.T * pitch), ds = make_rsrc(a.hidden + (int64_t)utt * a.T * 256, a.T * 256);
     const Rsrc ws = weight_rsrc(a.w, a.wide, 128);
     const int valid = a.count ? max(0, min(a.T, (int)a.count[utt])) : a.T;
-    u32x4 w[4][4];
+    u32x4 w[CT][4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < CT; ++j)
 #pragma unroll
         for (int s = 0; s < 4; ++s)
-            w[j][s] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ws, lane * 16, ((c0 / 16 + j) * 4 + s) * kFrag, 0));
-    f32x4 mu[4], m[4], s0[4], s1[4], s2[4];
+            w[j][s] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                ws, (n >> 3) * (4 * kFrag) + ((8 * (n >> 2) + 4 * (j & 1) + (n & 3)) % 16 + 16 * g) * 16, (((c0 + mine) / 16 + (j & ~1)) * 4 + s) * kFrag, 0));
+    f32x4 mu[CT], m[CT], s0[CT], s1[CT], s2[CT];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        mu[j] = *reinterpret_cast<const f32x4 *>(a.mean_std + (int64_t)utt * 2 * a.wide + c0 + 16 * j + 4 * g);
+    for (int j = 0; j < CT; ++j) {
+        mu[j] = *reinterpret_cast<const f32x4 *>(a.mean_std + (int64_t)utt * 2 * a.wide + c0 + mine + 32 * (j / 2) + 8 * g + 4 * (j & 1));
         m[j] = f32x4{-1e30f, -1e30f, -1e30f, -1e30f};
         s0[j] = s1[j] = s2[j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     const int tiles = (valid + 15) >> 4;
-    for (int t = wave; t < tiles; t += kWaves) {
+    u32x4 d[4], xr[CT / 2], d_next[4], x_next[CT / 2];
+    auto fetch = [&](int t) {                                // rows past the utterance come as zeros
         const int row = 16 * t + n;
-        u32x4 d[4];
-        u32x2 xr[4];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) d[s] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ds, row * 256 + 64 * s + 16 * g, 0, 0));
+        for (int s = 0; s < 4; ++s) d_next[s] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(ds, row * 256 + 64 * s + 16 * g, 0, 0));
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            xr[j] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(hs, row * pitch + 2 * (c0 + 16 * j + 4 * g), 0, 0));
-        f32x4 z[4];
+        for (int j = 0; j < CT / 2; ++j)
+            x_next[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(hs, row * pitch + 2 * (c0 + mine + 32 * j + 8 * g), 0, 0));
+    };
+    fetch(part);
+    for (int t = part; t < tiles; t += TS) {
+        const int row = 16 * t + n;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int s = 0; s < 4; ++s) d[s] = d_next[s];
+#pragma unroll
+        for (int j = 0; j < CT / 2; ++j) xr[j] = x_next[j];
+        if (t + TS < tiles) fetch(t + TS);
+        f32x4 z[CT], e[CT];                                  // logits, and how far they lie above the maximum
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
             z[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int s = 0; s < 4; ++s) z[j] = Mma<DT>::k32(w[j][s], d[s], z[j]);
         }
-        bool outgrown = false;
+        if (16 * t + 16 > valid) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < CT; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) z[j][r] = row < valid ? z[j][r] : kNegInf;
+        }
+        float most = kNegInf;
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                z[j][r] = row < valid ? z[j][r] * kLog2e : kNegInf;
-                outgrown |= z[j][r] > m[j][r] + kSlack;
+                e[j][r] = __builtin_fmaf(z[j][r], kLog2e, -m[j][r]);
+                most = __builtin_fmaxf(most, e[j][r]);
             }
-        if (__builtin_amdgcn_ballot_w64(outgrown)) {
+        if (__builtin_amdgcn_ballot_w64(most > kSlack)) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < CT; ++j)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float up = __builtin_fmaxf(m[j][r], z[j][r]), f = __builtin_amdgcn_exp2f(m[j][r] - up);
+                    const float up = __builtin_fmaxf(m[j][r], z[j][r] * kLog2e), f = __builtin_amdgcn_exp2f(m[j][r] - up);
                     m[j][r] = up;
                     s0[j][r] *= f;
                     s1[j][r] *= f;
                     s2[j][r] *= f;
+                    e[j][r] = __builtin_fmaf(z[j][r], kLog2e, -up);
                 }
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const f32x4 v = widen4<DT>(xr[j]);
+        for (int j = 0; j < CT; ++j) {
+            const f32x4 v = widen4<DT>(j & 1 ? u32x2{xr[j / 2].z, xr[j / 2].w} : u32x2{xr[j / 2].x, xr[j / 2].y});
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float p = __builtin_amdgcn_exp2f(z[j][r] - m[j][r]), dx = v[r] - mu[j][r], pd = p * dx;
+                const float p = __builtin_amdgcn_exp2f(e[j][r]), dx = v[r] - mu[j][r], pd = p * dx;
                 s0[j][r] += p;
                 s1[j][r] += pd;
                 s2[j][r] = __builtin_fmaf(pd, dx, s2[j][r]);
@@ -850,13 +871,13 @@ pool_kernel(PoolArgs a) {
         }
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < CT; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const float top = row16_max(m[j][r]), f = __builtin_amdgcn_exp2f(m[j][r] - top);
             const float a0 = row16_sum(s0[j][r] * f), a1 = row16_sum(s1[j][r] * f), a2 = row16_sum(s2[j][r] * f);
             if (n == 0) {
-                float *at = meet[wave][16 * j + 4 * g + r];
+                float *at = meet[part][mine + 32 * (j / 2) + 8 * g + 4 * (j & 1) + r];
                 at[0] = top;
                 at[1] = a0;
                 at[2] = a1;
@@ -864,13 +885,13 @@ pool_kernel(PoolArgs a) {
             }
         }
     __syncthreads();
-    if (threadIdx.x >= 64) return;
+    if (threadIdx.x >= kChannels) return;
     const int ch = threadIdx.x;
     float top = meet[0][ch][0], a0 = 0.f, a1 = 0.f, a2 = 0.f;
 #pragma unroll
-    for (int k = 1; k < kWaves; ++k) top = __builtin_fmaxf(top, meet[k][ch][0]);
+    for (int k = 1; k < TS; ++k) top = __builtin_fmaxf(top, meet[k][ch][0]);
 #pragma unroll
-    for (int k = 0; k < kWaves; ++k) {
+    for (int k = 0; k < TS; ++k) {
         const float f = __builtin_amdgcn_exp2f(meet[k][ch][0] - top);
         a0 = __builtin_fmaf(f, meet[k][ch][1], a0);
         a1 = __builtin_fmaf(f, meet[k][ch][2], a1);
@@ -1121,7 +1142,10 @@ int encode(const na1d_encoder &e, char *out, const float *x, const float *lens, 
     NA1D_TRY(launch_linear<DT, kTanhNorm>(d, s));
     PoolArgs p{ws + b.h, ws + b.hidden, (const char *)e.w_logit, count, reinterpret_cast<const float *>(ws + b.stats),
                reinterpret_cast<const float *>(ws + b.pool_map), reinterpret_cast<const float *>(ws + b.pool_map) + 2 * e.wide, ws + b.pooled, (int)T, e.wide};
-    pool_kernel<DT><<<dim3((unsigned)(e.wide / 64), (unsigned)N), kThreads, 0, s>>>(p);
+    if (N * (e.wide / 64) >= (T <= 128 ? 768 : 2048))                // a wave to all tokens of 64 channels
+        pool_kernel<DT, 1><<<dim3((unsigned)(e.wide / 256), (unsigned)N), kThreads, 0, s>>>(p);
+    else
+        pool_kernel<DT, 4><<<dim3((unsigned)(e.wide / 64), (unsigned)N), kThreads, 0, s>>>(p);
     NA1D_TRY(launch_status());
     LinearArgs f{};
     f.x = ws + b.pooled, f.x_pitch = 4 * e.wide, f.inputs = 2 * e.wide, f.M = (int)N;

@@ -66,6 +66,20 @@ def test_tiles_of_every_size(groups, batch, frames):
     assert native is not None and _near(native, modules)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("batch,frames", [(31, 100), (32, 256), (33, 258), (85, 260), (86, 260)])
+def test_pooling_with_one_wave_or_four_to_an_utterance(batch, frames, dtype):
+    """Each side of the sizes at which the waves of a pooling workgroup part by channels alone; lengths from one token on."""
+    model = _model(dtype=dtype)
+    lens = torch.rand(batch, generator=torch.Generator().manual_seed(batch))
+    lens[0], lens[1], lens[2] = 1.0, 2.0 / frames, 34.0 / frames
+    lens = lens.clamp(2.0 / frames, 1.0).cuda()
+    x = _input(batch, frames)
+    x *= (torch.arange(frames).cuda() < (lens * frames).round().unsqueeze(1)).unsqueeze(1)
+    native, modules = _both(model, x, lens, dtype)
+    assert native is not None and _near(native, modules, dtype)
+
+
 @pytest.mark.parametrize("groups", [0, 3, 16])
 @pytest.mark.parametrize("batch,frames", [(3, 111), (80, 128)])
 def test_layers_of_the_c_interface_are_dense_unless_2_4_or_8(groups, batch, frames):
