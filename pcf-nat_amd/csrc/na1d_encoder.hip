@@ -221,30 +221,44 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
         }
         if (c == 0) write_rows(a.x1, m0, rows, kRow);
     }
-    // and the quarters put together: -> x2 in q_lds.  A quarter reaches all outputs (one group), half of them (two) or its own quarter.
-    __device__ inline void join(int64_t m0, int rows) {
-        const int sets = a.tail_groups == 8 ? Groups<8, NW>::kSets : a.tail_groups == 4 ? Groups<4, NW>::kSets : a.tail_groups == 2 ? Groups<2, NW>::kSets
-                                                                                                                            : Groups<1, NW>::kSets;
-        const int per = 4 / sets;
-        const Rsrc xs = make_rsrc(a.x1 + m0 * kRow, rows * kRow);
+    // and the quarters put together: -> x2 in q_lds.  A quarter reaches all outputs (one group), half of them (two) or its own
+    // quarter; the PER that reach an output are fetched together.  (One after the other a dense layer's four took 2.8 of a
+    // launch's 5.2 us.)
+    __device__ inline void join(int64_t m0) {
+        static_assert(Groups<8, NW>::kEach == 1 && Groups<4, NW>::kEach == 1 && Groups<2, NW>::kEach == 2 && Groups<1, NW>::kEach == 4, "quarters of an output");
+        if (a.tail_groups >= 4)
+            join_of<1>(m0);
+        else if (a.tail_groups == 2)
+            join_of<2>(m0);
+        else
+            join_of<4>(m0);
+    }
+    template <int PER> __device__ inline void join_of(int64_t m0) {
+        const Rsrc xs = make_rsrc(a.x1, a.M * kRow), ps = make_rsrc(a.parts, 4 * a.M * (4 * kDim));
+        u32x2 x[NTW][MT];
+        f32x4 part[NTW][MT][PER], b[NTW];
 #pragma unroll
         for (int j = 0; j < NTW; ++j) {
-            const int c = CW * wave + 16 * j, first = c / (64 * per) * per;
-            const f32x4 b = bias(a.b_fc2, c);
+            const int c = CW * wave + 16 * j, first = c / (64 * PER) * PER;
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
-                const int row = 16 * i + n;
-                const f32x4 x = widen4<DT>(__builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(xs, row * kRow + 2 * c + 8 * g, 0, 0)));
-                f32x4 v{0.f, 0.f, 0.f, 0.f};
+                const int row = (int)m0 + 16 * i + n;                    // rows behind the last are not stored
+                x[j][i] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(xs, row * kRow + 2 * c + 8 * g, 0, 0));
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (k < per) {
-                        const Rsrc ps = make_rsrc(a.parts + ((int64_t)(first + k) * a.M + m0) * kDim, rows * kDim * 4);
-                        v += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ps, row * kDim * 4 + 4 * c + 16 * g, 0, 0));
-                    }
-                *at(q_lds, c, i) = narrow4<DT>(v + b + x);
+                for (int k = 0; k < PER; ++k)
+                    part[j][i][k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ps, row * (4 * kDim) + 4 * c + 16 * g, (first + k) * a.M * (4 * kDim), 0));
             }
+            b[j] = bias(a.b_fc2, c);
         }
+#pragma unroll
+        for (int j = 0; j < NTW; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                f32x4 v = part[j][i][0];
+#pragma unroll
+                for (int k = 1; k < PER; ++k) v += part[j][i][k];
+                *at(q_lds, CW * wave + 16 * j, i) = narrow4<DT>(v + b[j] + widen4<DT>(x[j][i]));
+            }
     }
 
     template <int G> __device__ inline void head(int64_t m0, int rows, int from, int to) {
@@ -328,7 +342,7 @@ layer_kernel(LayerArgs a) {
     const int rows = (int)min((int64_t)(16 * MT), a.M - m0);
     if (SPLIT || !a.attn) w.stage_qkv_bias();
     if (SPLIT && a.attn) {
-        w.join(m0, rows);
+        w.join(m0);
         wait_direct();                               // qkv's biases
         if (a.block_out && mine == 0) {
             barrier_lds();
