@@ -58,6 +58,30 @@ def test_global_attention_matches_oracle(geom, dtype):
     assert torch.equal(o2, out)
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=["bf16", "fp16"])
+@pytest.mark.parametrize("N,H,T,C,strength", [(2, 2, 300, 32, 1), (2, 2, 300, 32, 40), (1, 1, 193, 64, 40), (2, 256, 200, 16, 40)])
+def test_padded_keys_count_where_they_outweigh_the_mask(N, H, T, C, strength, dtype):
+    """-100 is added, nothing is cut off: padded keys whose scores reach that far draw a valid row's weight, as the oracle's
+    do, and a value that is not a number is not lost behind a weight of zero."""
+    q, k, v, do = make_inputs(N * H, T, C, 0, 78, dtype, n=4)
+    pad = torch.tensor([T - 70, T // 3][:N])
+    for i in range(N):
+        k.view(N, H, T, C)[i, :, T - int(pad[i]):] *= strength
+    t_valid = (T - pad).to(torch.int32).cuda()
+    qd, kd, vd = (t.cuda().requires_grad_(True) for t in (q, k, v))
+    out = global_attention(qd, kd, vd, H, t_valid=t_valid, scale=C ** -0.5)
+    out.backward(do.cuda())
+    want, _, _ = O.global_forward(q.float(), k.float(), v.float(), C ** -0.5, pad, H)
+    grads = O.global_backward(q.float(), k.float(), v.float(), do.float(), C ** -0.5, pad, H)
+    assert O.rel_l2(out.float(), want) < TOL[dtype]
+    for got, exact in zip((qd.grad, kd.grad, vd.grad), grads):
+        assert O.rel_l2(got.float(), exact) < TOL[dtype]
+    broken = v.clone()
+    broken.view(N, H, T, C)[0, 0, T - 1, 3] = float("nan")                              # a padded row
+    out = global_attention(qd.detach(), kd.detach(), broken.cuda(), H, t_valid=t_valid, scale=C ** -0.5)
+    assert torch.isnan(out.view(N, H, T, C)[0, 0, :, 3]).all() and not torch.isnan(out.view(N, H, T, C)[-1, -1, :, 4]).any()
+
+
 def test_global_attention_without_padding_and_without_lse():
     N, H, T, C, dtype = 2, 2, 150, 32, torch.bfloat16
     B = N * H
