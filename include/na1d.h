@@ -362,6 +362,19 @@ int na1d_train_layer_backward(const na1d_train_layer *l, void *dx, const void *d
                               void *stream);
 
 /*
+ * Backward of attentive statistics pooling in training (Pooling.py:16-59), on contiguous [N, C, T] of 16 bit, C a multiple of 8,
+ * T from 2 to 2048 (others: NA1D_ERR_UNSUPPORTED), 16-byte aligned.
+ * pool: of mean = sum over T of w x and std = sqrt(max(sum over T of w (x - mean)^2, eps)), w = softmax over T of the logits;
+ *   pooled, dpooled: [N, 2 C] fp32, the means and then the deviations, as the forward left them, and their gradients.
+ * context: of [x, mean, std] along C ([N, 3 C, T]; mean and std = sqrt(max(var, eps)) of a row over T, var with T - 1 degrees of
+ *   freedom, repeated along T); var, std: [N, C], as the forward rounded them.
+ */
+int na1d_train_pool_backward(void *dlogits, void *dx, const void *logits, const void *x, const float *pooled, const float *dpooled,
+                             int64_t N, int64_t C, int64_t T, float eps, int dtype, void *stream);
+int na1d_train_context_backward(void *dx, const void *dctx, const void *x, const void *var, const void *std, int64_t N, int64_t C,
+                                int64_t T, float eps, int dtype, void *stream);
+
+/*
  * Profiling hook; no counterpart in the reference.  From this call on, the matrix-core fused kernels that the
  * CALLING THREAD launches record `start` just before and `stop` just after the kernel itself (hipEvent_t handles,
  * recorded by hipExtLaunchKernel: the dispatch's own begin and end, i.e. what a profiler's kernel trace reports,

@@ -502,6 +502,28 @@ int na1d_train_to_channels(const na1d_train_layer *l, void *out, const void *x, 
     return na1d::train::to_channels(*l, out, x, N, T, (hipStream_t)stream);
 }
 
+static int pool_check(int64_t N, int64_t C, int64_t T, int dtype) {
+    if (dtype != NA1D_BF16 && dtype != NA1D_FP16) return NA1D_ERR_DTYPE;
+    if (N < 1 || C < 1 || T < 1) return NA1D_ERR_SHAPE;
+    return na1d::train::pool_ok(N, C, T) ? NA1D_OK : NA1D_ERR_UNSUPPORTED;
+}
+int na1d_train_pool_backward(void *dlogits, void *dx, const void *logits, const void *x, const float *pooled, const float *dpooled, int64_t N, int64_t C,
+                             int64_t T, float eps, int dtype, void *stream) {
+    const int st = pool_check(N, C, T, dtype);
+    if (st != NA1D_OK) return st;
+    if (!dlogits || !dx || !logits || !x || !pooled || !dpooled) return NA1D_ERR_NULL;
+    if (misaligned(dlogits) || misaligned(dx) || misaligned(logits) || misaligned(x)) return NA1D_ERR_ALIGN;
+    return na1d::train::run_pool_backward(dlogits, dx, logits, x, pooled, dpooled, N, C, T, eps, dtype, (hipStream_t)stream);
+}
+int na1d_train_context_backward(void *dx, const void *dctx, const void *x, const void *var, const void *std, int64_t N, int64_t C, int64_t T, float eps,
+                                int dtype, void *stream) {
+    const int st = pool_check(N, C, T, dtype);
+    if (st != NA1D_OK) return st;
+    if (!dx || !dctx || !x || !var || !std) return NA1D_ERR_NULL;
+    if (misaligned(dx) || misaligned(dctx) || misaligned(x)) return NA1D_ERR_ALIGN;
+    return na1d::train::run_context_backward(dx, dctx, x, var, std, N, C, T, eps, dtype, (hipStream_t)stream);
+}
+
 int na1d_train_layer_forward(const na1d_train_layer *l, int part, void *out, const void *x, void *saved, int64_t saved_bytes, void *workspace,
                              int64_t workspace_bytes, int64_t N, int64_t T, void *stream) {
     int st = train_check(l, N, T);

@@ -34,7 +34,7 @@ from .dense import global_attention
 from .encoder import embed as embed_natively
 from .fused import na1d_fused, na1d_fused_qkv
 from .nattn import getNA1dFunction
-from .train import layer as train_layer
+from .train import layer as train_layer, pooled, pooled_of, pooling_context
 
 MASK_VALUE = -100.0   # PCF_NATransformer.py:98
 
@@ -161,21 +161,14 @@ class AttentiveStatisticsPooling(nn.Module):
 
     def forward(self, x, lens=None):
         if lens is None:
-            mask = None
-            mean = x.mean(-1, keepdim=True)
-            std = torch.sqrt(x.var(-1, keepdim=True).clamp(self.eps))
-        else:
-            mask, count = _length_mask(x.shape, lens)
-            mean = (x * mask).sum(-1, keepdim=True) / count
-            std = torch.sqrt((((x - mean).pow(2) * mask).sum(-1, keepdim=True) / count).clamp(self.eps))
+            ctx = pooling_context(x, self.eps)
+            return pooled(self.conv(self.tanh(self.tdnn(ctx))), x, self.eps)
+        mask, count = _length_mask(x.shape, lens)
+        mean = (x * mask).sum(-1, keepdim=True) / count
+        std = torch.sqrt((((x - mean).pow(2) * mask).sum(-1, keepdim=True) / count).clamp(self.eps))
         ctx = torch.cat([x, mean.expand_as(x), std.expand_as(x)], dim=1)
         w = self.conv(self.tanh(self.tdnn(ctx)))
-        if mask is not None:
-            w = w.masked_fill(mask == 0, -torch.inf)
-        w = F.softmax(w, dim=-1)
-        mean = (w * x).sum(-1, keepdim=True)
-        std = torch.sqrt((w * (x - mean).pow(2)).sum(-1, keepdim=True).clamp(self.eps))
-        return torch.cat((mean, std), dim=1).squeeze(-1)
+        return pooled_of(w.masked_fill(mask == 0, -torch.inf), x, self.eps)
 
     def forward_tokens(self, x, lens=None):
         """The same pooling in inference on ``[N, T, C]``: reductions over T run down the columns, and the context

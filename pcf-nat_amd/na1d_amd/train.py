@@ -10,6 +10,7 @@ import ctypes
 
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
 from torch.autograd.function import once_differentiable
 from torch.autograd.graph import increment_version
 
@@ -189,3 +190,96 @@ def layer(m, x, pos_emb=None, attn_mask_global=None):
     scales = (_drop_path_scale(m.drop_path, xt), _drop_path_scale(m.drop_path, xt))
     out = _TrainLayer.apply(xt, by_channel, geom, norms, scales, pos, *params)
     return out.transpose(1, 2) if cf else out
+
+
+# ---------------------------------------------------------------------------------------------- attentive pooling
+def context_of(x, eps):
+    """``[x, mean, std]`` over the last axis along the channels (Pooling.py:30-45), and the variance and deviation in it."""
+    mean, var = x.mean(-1, keepdim=True), x.var(-1, keepdim=True)
+    std = torch.sqrt(var.clamp(eps))
+    return torch.cat([x, mean.expand_as(x), std.expand_as(x)], dim=1), var, std
+
+
+def pooled_of(logits, x, eps):
+    """Mean and standard deviation over the last axis, weighted by the logits' softmax (Pooling.py:47-59)."""
+    w = F.softmax(logits, dim=-1)
+    mean = (w * x).sum(-1, keepdim=True)
+    std = torch.sqrt((w * (x - mean).pow(2)).sum(-1, keepdim=True).clamp(eps))
+    return torch.cat((mean, std), dim=1).squeeze(-1)
+
+
+class _Pooling(torch.autograd.Function):
+    """Torch's forward - training amplifies any difference in it - and a backward of one launch instead of some thirty."""
+
+    @staticmethod
+    def again(ctx, grad, f, *inputs):
+        """The same backward by torch, for a caller that differentiates it again."""
+        with torch.enable_grad(), torch.autocast("cuda", dtype=inputs[-1].dtype):
+            leaves = [t for t, need in zip(inputs, ctx.needs_input_grad) if need]
+            grads = iter(torch.autograd.grad(f(*inputs), leaves, grad, create_graph=True))
+        return tuple(next(grads) if need else None for need in ctx.needs_input_grad)
+
+
+class _Context(_Pooling):
+    @staticmethod
+    def forward(ctx, x, eps):
+        out, var, std = context_of(x, eps)
+        ctx.save_for_backward(x, var, std)
+        ctx.eps = eps
+        return out
+
+    @staticmethod
+    def backward(ctx, dctx):
+        x, var, std = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return _Pooling.again(ctx, dctx, lambda x: context_of(x, ctx.eps)[0], x)
+        n, c, t = x.shape
+        dctx, dx = _aligned(dctx), torch.empty_like(x)
+        with torch.cuda.device(x.device):
+            _lib.check(_lib.load().na1d_train_context_backward(
+                dx.data_ptr(), dctx.data_ptr(), x.data_ptr(), var.data_ptr(), std.data_ptr(), n, c, t,
+                torch.tensor(ctx.eps, dtype=x.dtype).item(), _lib.dtype_tag(x.dtype), torch.cuda.current_stream().cuda_stream),
+                "na1d_train_context_backward")
+        return dx, None
+
+
+class _Pooled(_Pooling):
+    @staticmethod
+    def forward(ctx, logits, x, eps):
+        out = pooled_of(logits, x, eps)
+        ctx.save_for_backward(logits, x, out)
+        ctx.eps = eps
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        logits, x, out = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return _Pooling.again(ctx, dout, lambda z, x: pooled_of(z, x, ctx.eps), logits, x)
+        n, c, t = x.shape
+        dout, dz, dx = dout.contiguous(), torch.empty_like(logits), torch.empty_like(x)
+        with torch.cuda.device(x.device):
+            _lib.check(_lib.load().na1d_train_pool_backward(
+                dz.data_ptr(), dx.data_ptr(), logits.data_ptr(), x.data_ptr(), out.data_ptr(), dout.data_ptr(), n, c, t, ctx.eps,
+                _lib.dtype_tag(x.dtype), torch.cuda.current_stream().cuda_stream), "na1d_train_pool_backward")
+        return dz, dx, None
+
+
+def _pooling_fits(*tensors):
+    x = tensors[-1]
+    return (x.is_cuda and x.dim() == 3 and torch.is_grad_enabled() and any(t.requires_grad for t in tensors) and torch.is_autocast_enabled("cuda")
+            and x.dtype in (torch.bfloat16, torch.float16) and x.dtype == torch.get_autocast_dtype("cuda")
+            and all(plain_call(t) and t.device == x.device and t.dtype == x.dtype and t.shape == x.shape and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in tensors)
+            and 0 < x.shape[0] <= 65535 and x.shape[1] % 8 == 0 and 8 <= x.shape[1] <= 1 << 16 and 2 <= x.shape[2] <= 2048
+            and x.shape[0] * x.shape[1] < 1 << 31)
+
+
+def pooling_context(x, eps):
+    """:func:`context_of` as one autograd node where the kernels take ``x``."""
+    return _Context.apply(x, eps) if _pooling_fits(x) else context_of(x, eps)[0]
+
+
+def pooled(logits, x, eps):
+    """:func:`pooled_of` as one autograd node where the kernels take its inputs."""
+    return _Pooled.apply(logits, x, eps) if _pooling_fits(logits, x) else pooled_of(logits, x, eps)

@@ -4,7 +4,7 @@ import copy
 import pytest
 import torch
 
-from na1d_amd import models
+from na1d_amd import models, train
 from oracle import na1d_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -242,3 +242,29 @@ def test_tokens_first_inputs_lose_nothing(heads, window, dtype):
         errors.append([O.rel_l2(out.float(), want.float()), O.rel_l2(xg.grad.float(), xc.grad.float())])
     print(errors)
     assert all(a < 1.02 * b for a, b in zip(*errors))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,c,t", [(2, 8, 2), (3, 16, 100), (2, 24, 131), (1, 8, 2048), (5, 136, 33), (2, 1536, 100)])
+def test_pooling_nodes_against_64_bits(n, c, t, dtype):
+    """Rows of every remainder, blocks that span samples: the forward is torch's to the bit, the gradients are what the type
+    gives (a rounding or two of 2^-9 or 2^-12; the context's deviations are rounded too), and a second derivative is torch's."""
+    gen = torch.Generator().manual_seed(n * c + t)
+    make = lambda *s: torch.randn(s, generator=gen).to("cuda", dtype).requires_grad_(True)
+    tol = 1e-2 if dtype == torch.bfloat16 else 1.5e-3
+    rel = lambda a, b: float((a.double() - b).norm() / b.norm())
+    x, z, d1 = make(n, c, t), make(n, c, t), torch.randn(n, 3 * c, t, generator=gen).to("cuda", dtype)
+    d2 = torch.randn(n, 2 * c, generator=gen).cuda()
+    with torch.autocast("cuda", dtype=dtype):
+        got, want = train.pooling_context(x, 1e-12), train.context_of(x, 1e-12)[0]
+        assert "Context" in type(got.grad_fn).__name__ and torch.equal(got, want)
+        out, same = train.pooled(z, x, 1e-12), train.pooled_of(z, x, 1e-12)
+        assert "Pooled" in type(out.grad_fn).__name__ and torch.equal(out, same)
+    exact = [v.detach().double().requires_grad_(True) for v in (x, z)]
+    (dx,), (ex,) = torch.autograd.grad(got, (x,), d1), torch.autograd.grad(train.context_of(exact[0], 1e-12)[0], exact[:1], d1.double())
+    assert rel(dx, ex) < tol
+    grads = torch.autograd.grad(out, (x, z), d2, retain_graph=True)
+    for g, e in zip(grads, torch.autograd.grad(train.pooled_of(exact[1], exact[0], 1e-12), exact, d2.double())):
+        assert rel(g, e) < tol
+    twice = [torch.autograd.grad(torch.autograd.grad(o, x, d2, create_graph=True)[0].float().square().sum(), x)[0] for o in (out, same)]
+    assert torch.allclose(*[v.float() for v in twice], rtol=5e-2, atol=1e-3 * float(twice[1].float().abs().max()))
