@@ -370,16 +370,30 @@ gemm_kernel(Gemm a, int col_blocks) {
 #pragma unroll
         for (int j = 0; j < NTW; ++j) bias[j] = *reinterpret_cast<const f32x4 *>(a.bias + 16 * (tile0 + j) + 4 * g);
     }
+    // What an end reads of every output, all at once and store_tile backwards: 16 bytes to a lane, 64 of a row together (GELU's
+    // derivative over 12800 x 1024: 29.0 -> 23.6 us, 27.1 with a row tile's behind the other).
+    u32x4 aux16[MT][NTW / 2];
+    if constexpr (END == kResidual || END == kGeluBack) {
+        const Rsrc as = make_rsrc(a.aux + m0 * pitch, rows * pitch);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int p = 0; p < NTW / 2; ++p)
+                aux16[i][p] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(as, (16 * i + n) * pitch + 32 * tile0 + (2 * p + (g & 1)) * 32 + (g >> 1) * 16, 0, 0));
+    }
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         u32x2 o[NTW];
         const int row_byte = (16 * i + n) * pitch + 32 * tile0;
         f32x4 aux[NTW];
         if constexpr (END == kResidual || END == kGeluBack) {
-            const Rsrc as = make_rsrc(a.aux + m0 * pitch, rows * pitch);
 #pragma unroll
-            for (int j = 0; j < NTW; ++j)
-                aux[j] = widen4<DT>(__builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(as, row_byte + 32 * j + 8 * g, 0, 0)));
+            for (int p = 0; p < NTW / 2; ++p) {
+                const u32x4 v = aux16[i][p];
+                const u32x2 lo = __builtin_amdgcn_permlane16_swap(v.x, v.z, false, false), hi = __builtin_amdgcn_permlane16_swap(v.y, v.w, false, false);
+                aux[2 * p] = widen4<DT>(u32x2{lo.x, hi.x});
+                aux[2 * p + 1] = widen4<DT>(u32x2{lo.y, hi.y});
+            }
         }
         float f = 1.f;
         if constexpr (END == kResidual)
