@@ -297,7 +297,7 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
 
 // Few tokens: a layer's weights (up to 1.6 MB) take a CU 21 us to read, so each 16 tokens go to four workgroups, one for
 // every 256 hidden channels (each works out the output projection), and then to three, one each for q, k and v
-// (layer_kernel with SPLIT, which puts the quarters together).  One 3 s utterance through the 4x4 model: 340 -> 276 us.
+// (layer_kernel with SPLIT, which puts the quarters together).  One 3 s utterance through MFA 4x4: 429 -> 313 us.
 template <class DT, int NW, int PF>
 __global__ void __launch_bounds__(64 * NW, 2)
 part_kernel(LayerArgs a) {
@@ -651,8 +651,8 @@ __global__ void lengths_kernel(int32_t *t_valid, float *count, const float *lens
 // writes run along the rows.  Bound by memory; the work is split over the channels too, or a single utterance is a handful
 // of workgroups (3 s: 19.5 us in three workgroups of whole rows that divided twice for every value).
 // The launch's last slices bring the last layer's weight into fragment order and the pooled norm into an affine map, from
-// the module's own tensors at each call.  A single utterance takes 278 us so, 281 with the last product rounding the fp32
-// rows itself, 275 where both were kept from call to call and a write that no version counts went unseen.
+// the module's own tensors at each call: of a single utterance's 269 us that is 3, and as much again with the last product
+// rounding the fp32 rows itself; kept from call to call, a write that no version counts would go unseen.
 constexpr int kPatchTokens = 32;
 struct Head {
     char *w;                        // 16-bit fragments of ...
@@ -933,7 +933,7 @@ int launch_layer_mt(const LayerArgs &a, hipStream_t s) {
 }
 
 // Up to this many tokens the four quarters of every tile find a CU of their own.  A PCF 4x4 pass with and without:
-// 125 tokens 273 and 336 us, 500: 295 and 344, 1000: 335 and 352; 1500: 426 and 370, 4000: 634 and 454.
+// 500 tokens 290 and 335 us, 1000: 325 and 351; 1500: 416 and 363, 3000: 548 and 415.
 constexpr int64_t kSplitTokens = 16 * 64;
 template <class DT> int launch_layer_split(const LayerArgs &a, hipStream_t s) {
     const size_t lds = layer_lds<1>();
@@ -950,8 +950,9 @@ template <class DT> int launch_layer_split(const LayerArgs &a, hipStream_t s) {
 template <class DT> int launch_layer(const LayerArgs &a, hipStream_t s) {
     if (a.M <= kSplitTokens) return launch_layer_split<DT>(a, s);
     // Fewer, larger tiles read the layer's weights fewer times; smaller ones spread few tokens over more CUs.  PCF 4x4 passes
-    // with tiles of 16, 32 and 64 tokens: 4000 tokens 454, 496 and 657 us; 6000: 627, 543, 698; 16000: 1124, 900, 909;
-    // 20000: 1350, 1122, 1109; 25600: 1737, 1344, 1222.
+    // with tiles of 16, 32 and 64 tokens: 4000 tokens 450, 494 and 653 us; 6000: 623, 539, 694; 16000: 1101, 884, 879;
+    // 20000: 1319, 1083, 1055; 25600: 1668, 1291, 1166; MFA 4x4: 6000: 832, 629, 888; 16000: 1494, 1033, 1075; 25600: 2380,
+    // 1614, 1399.
     const bool sparse = a.tail_groups >= 4;
     if (a.M <= 16 * 256) return sparse ? launch_layer_mt<DT, 1, 8, 8, true>(a, s) : launch_layer_mt<DT, 1, 8, 8, false>(a, s);
     if (a.M <= 32 * 512) return sparse ? launch_layer_mt<DT, 2, 8, 4, true>(a, s) : launch_layer_mt<DT, 2, 8, 4, false>(a, s);

@@ -2,9 +2,10 @@
 // 224-261) in training, forward and backward, on token-major activations: batch norms with batch statistics, projections,
 // GELU, residuals and weight gradients around the attention kernels.
 //
-// A layer of 128 x 100 tokens, 256 channels, fp16, forward and backward: 26 launches of 260 us together and 37 us of torch's
-// statistics, where the modules took some 80 launches and 800 us (torch's batch norm with its copies, bias gradients as reductions of their own, weight
-// gradients through 16-bit sums of chunks).  Everything else than the batch statistics is launched from native code, so the
+// A layer of 128 x 100 tokens, 256 channels, fp16, forward and backward: 26 launches of 240 us together and 38 us of torch's
+// statistics, where the modules took some 80 launches and 800 us (torch's batch norm with its copies, bias gradients as
+// reductions of their own, weight gradients through 16-bit sums of chunks).  The pooling behind the layers has its backward
+// here too.  Everything else than the batch statistics is launched from native code, so the
 // host keeps ahead.  The forward rounds where the modules round and is theirs to the bit wherever the library sums a product in
 // the order of its inputs (at 3 x 50 tokens it does not: 1 to 3 of 38400 values differ): training amplifies a difference
 // anywhere in it, by way of the rounding of sixteen layers, to what 16 bits give (1.2e-3 of the embeddings, 3 % of the
