@@ -213,10 +213,13 @@ class _Pooling(torch.autograd.Function):
 
     @staticmethod
     def again(ctx, grad, f, *inputs):
-        """The same backward by torch, for a caller that differentiates it again."""
+        """The same backward by torch, for a caller that differentiates it again.  It is taken by views of the inputs, each a
+        node of its own: an input that was made from another one (the logits from x) would hand that its gradient here too,
+        and so twice."""
         with torch.enable_grad(), torch.autocast("cuda", dtype=inputs[-1].dtype):
-            leaves = [t for t, need in zip(inputs, ctx.needs_input_grad) if need]
-            grads = iter(torch.autograd.grad(f(*inputs), leaves, grad, create_graph=True))
+            views = [t.view_as(t) for t in inputs]
+            leaves = [t for t, need in zip(views, ctx.needs_input_grad) if need]
+            grads = iter(torch.autograd.grad(f(*views), leaves, grad, create_graph=True))
         return tuple(next(grads) if need else None for need in ctx.needs_input_grad)
 
 

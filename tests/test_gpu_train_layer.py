@@ -268,3 +268,25 @@ def test_pooling_nodes_against_64_bits(n, c, t, dtype):
         assert rel(g, e) < tol
     twice = [torch.autograd.grad(torch.autograd.grad(o, x, d2, create_graph=True)[0].float().square().sum(), x)[0] for o in (out, same)]
     assert torch.allclose(*[v.float() for v in twice], rtol=5e-2, atol=1e-3 * float(twice[1].float().abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_pooling_gradients_that_are_differentiated_again(dtype):
+    """The module's gradients with create_graph and without, and a second derivative, against its operations in 64 bits.  Every
+    tensor on the way is rounded to the type some ten times (2^-9 or 2^-12 each: the operations' own gradients are 9.4e-3 and
+    6.6e-4 off, the second ones 3.9e-2 and, in fp16, no numbers); a path counted twice is 40 % and more."""
+    torch.manual_seed(0)
+    tol = 2e-2 if dtype == torch.bfloat16 else 2e-3
+    pool = models.AttentiveStatisticsPooling(64, 32).cuda()
+    exact = copy.deepcopy(pool).double()
+    x, d = torch.randn(3, 64, 50).to("cuda", dtype).requires_grad_(True), torch.randn(3, 128).cuda()
+    xe, de = x.detach().double().requires_grad_(True), d.double()
+    with torch.autocast("cuda", dtype=dtype):
+        out = pool(x)
+    assert "Pooled" in type(out.grad_fn).__name__
+    (want,) = torch.autograd.grad(exact(xe), xe, de, create_graph=True)
+    (plain,) = torch.autograd.grad(out, x, d, retain_graph=True)
+    (dx,) = torch.autograd.grad(out, x, d, create_graph=True)
+    twice, wanted = (torch.autograd.grad(g.to(w.dtype).square().sum(), v)[0] for g, w, v in ((dx, d, x), (want, de, xe)))
+    assert O.rel_l2(plain.float(), want.float()) < tol and O.rel_l2(dx.float(), want.float()) < tol
+    assert dtype == torch.float16 or O.rel_l2(twice.float(), wanted.float()) < 4 * tol

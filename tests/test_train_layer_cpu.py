@@ -30,3 +30,27 @@ def test_a_norm_whose_counters_the_kernels_cannot_write(change, fits):
     bn = models.BatchNorm1d(256)
     change(bn)
     assert train._norm_fits(bn, 256, torch.device("cpu")) == fits
+
+
+def _pooling(context, pooled, seed=0):
+    """Pooling as a model has it, in 64 bits: the logits are made from x by way of the context."""
+    gen = torch.Generator().manual_seed(seed)
+    x, w = torch.randn(2, 8, 9, generator=gen, dtype=torch.float64).requires_grad_(True), torch.randn(8, 24, generator=gen, dtype=torch.float64)
+    rows = x * 1.0
+    return x, pooled(torch.tanh(w @ context(rows)), rows), torch.randn(2, 16, generator=gen, dtype=torch.float64)
+
+
+_NODES = (lambda x: train._Context.apply(x, 1e-12), lambda z, x: train._Pooled.apply(z, x, 1e-12))
+_OPERATIONS = (lambda x: train.context_of(x, 1e-12)[0], lambda z, x: train.pooled_of(z, x, 1e-12))
+
+
+@pytest.mark.filterwarnings("ignore:.*autocast")
+def test_pooling_gradients_that_are_differentiated_again():
+    """Where one input of a node is made from the other, its gradient counts once; the same sums in 64 bits."""
+    results = []
+    for nodes in (_NODES, _OPERATIONS):
+        x, out, d = _pooling(*nodes)
+        (dx,) = torch.autograd.grad(out, x, d, create_graph=True)
+        results.append((dx, torch.autograd.grad(dx.square().sum(), x, create_graph=True)[0]))
+    for got, want in zip(*results):
+        assert torch.allclose(got, want, rtol=1e-10, atol=1e-10 * float(want.abs().max()))
