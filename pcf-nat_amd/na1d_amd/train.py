@@ -112,7 +112,8 @@ def plain_call(x):
     """Whether nothing but autograd looks at the operations on ``x``: no tracer, transform, subclass or dispatch mode."""
     return (type(x) in (torch.Tensor, nn.Parameter) and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and not torch.nn.modules.module._has_any_global_hook() and torch._C._functorch.peek_interpreter_stack() is None
-            and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0)
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
+            and not torch._C._functorch.is_legacy_batchedtensor(x))       # of is_grads_batched
 
 
 def _norm_fits(bn, dim, device):
@@ -213,13 +214,14 @@ class _Pooling(torch.autograd.Function):
 
     @staticmethod
     def again(ctx, grad, f, *inputs):
-        """The same backward by torch, for a caller that differentiates it again.  It is taken by views of the inputs, each a
-        node of its own: an input that was made from another one (the logits from x) would hand that its gradient here too,
-        and so twice."""
+        """The same backward by torch, for a caller that differentiates it again, or whose gradient is no plain tensor.  It is
+        taken by views of the inputs, each a node of its own: an input that was made from another one (the logits from x)
+        would hand that its gradient here too, and so twice."""
+        create_graph = torch.is_grad_enabled()
         with torch.enable_grad(), torch.autocast("cuda", dtype=inputs[-1].dtype):
             views = [t.view_as(t) for t in inputs]
             leaves = [t for t, need in zip(views, ctx.needs_input_grad) if need]
-            grads = iter(torch.autograd.grad(f(*views), leaves, grad, create_graph=True))
+            grads = iter(torch.autograd.grad(f(*views), leaves, grad, create_graph=create_graph))
         return tuple(next(grads) if need else None for need in ctx.needs_input_grad)
 
 
@@ -234,7 +236,7 @@ class _Context(_Pooling):
     @staticmethod
     def backward(ctx, dctx):
         x, var, std = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if torch.is_grad_enabled() or not plain_call(dctx):
             return _Pooling.again(ctx, dctx, lambda x: context_of(x, ctx.eps)[0], x)
         n, c, t = x.shape
         dctx, dx = _aligned(dctx), torch.empty_like(x)
@@ -257,7 +259,7 @@ class _Pooled(_Pooling):
     @staticmethod
     def backward(ctx, dout):
         logits, x, out = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if torch.is_grad_enabled() or not plain_call(dout):
             return _Pooling.again(ctx, dout, lambda z, x: pooled_of(z, x, ctx.eps), logits, x)
         n, c, t = x.shape
         dout, dz, dx = dout.contiguous(), torch.empty_like(logits), torch.empty_like(x)

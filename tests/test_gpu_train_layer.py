@@ -290,3 +290,18 @@ def test_pooling_gradients_that_are_differentiated_again(dtype):
     twice, wanted = (torch.autograd.grad(g.to(w.dtype).square().sum(), v)[0] for g, w, v in ((dx, d, x), (want, de, xe)))
     assert O.rel_l2(plain.float(), want.float()) < tol and O.rel_l2(dx.float(), want.float()) < tol
     assert dtype == torch.float16 or O.rel_l2(twice.float(), wanted.float()) < 4 * tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_pooling_gradients_in_batches(dtype):
+    """Each of several gradients taken at once is what it is by itself; by the kernels there, which round in other places."""
+    torch.manual_seed(1)
+    pool = models.AttentiveStatisticsPooling(64, 32).cuda()
+    x, d = torch.randn(3, 64, 50).to("cuda", dtype).requires_grad_(True), torch.randn(4, 3, 128).cuda()
+    with torch.autocast("cuda", dtype=dtype):
+        out = pool(x)
+    assert "Pooled" in type(out.grad_fn).__name__
+    (batch,) = torch.autograd.grad(out, x, d, retain_graph=True, is_grads_batched=True)
+    for got, one in zip(batch, d):
+        (want,) = torch.autograd.grad(out, x, one, retain_graph=True)
+        assert O.rel_l2(got.float(), want.float()) < (2e-2 if dtype == torch.bfloat16 else 2e-3)

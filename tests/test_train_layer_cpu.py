@@ -54,3 +54,13 @@ def test_pooling_gradients_that_are_differentiated_again():
         results.append((dx, torch.autograd.grad(dx.square().sum(), x, create_graph=True)[0]))
     for got, want in zip(*results):
         assert torch.allclose(got, want, rtol=1e-10, atol=1e-10 * float(want.abs().max()))
+
+
+@pytest.mark.filterwarnings("ignore:.*autocast")
+def test_pooling_gradients_in_batches():
+    """Several gradients at once (is_grads_batched; jacobian with vectorize), as torch's operations take them; 64 bits."""
+    results = []
+    for nodes in (_NODES, _OPERATIONS):
+        x, out, d = _pooling(*nodes)
+        results.append(torch.autograd.grad(out, x, torch.stack([d, d.flip(0), 2 * d]), is_grads_batched=True)[0])
+    assert torch.allclose(*results, rtol=1e-10, atol=1e-10)
