@@ -254,7 +254,7 @@ class _Pooled(_Pooling):
         out = pooled_of(logits, x, eps)
         ctx.save_for_backward(logits, x, out)
         ctx.eps = eps
-        return out
+        return out.clone()                          # the caller may write to its own
 
     @staticmethod
     def backward(ctx, dout):

@@ -305,3 +305,14 @@ def test_pooling_gradients_in_batches(dtype):
     for got, one in zip(batch, d):
         (want,) = torch.autograd.grad(out, x, one, retain_graph=True)
         assert O.rel_l2(got.float(), want.float()) < (2e-2 if dtype == torch.bfloat16 else 2e-3)
+
+
+def test_pooling_output_can_be_written_to():
+    torch.manual_seed(2)
+    pool = models.AttentiveStatisticsPooling(64, 32).cuda()
+    x, d = torch.randn(3, 64, 50).to("cuda", torch.bfloat16).requires_grad_(True), torch.randn(3, 128).cuda()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        out = pool(x)
+        twice = pool(x).mul_(2)                     # a factor of two rounds nothing
+    assert "Pooled" in type(out.grad_fn).__name__ and torch.equal(twice, 2 * out)
+    assert torch.equal(*(torch.autograd.grad(o, x, d)[0] for o in (twice, 2 * out)))

@@ -64,3 +64,13 @@ def test_pooling_gradients_in_batches():
         x, out, d = _pooling(*nodes)
         results.append(torch.autograd.grad(out, x, torch.stack([d, d.flip(0), 2 * d]), is_grads_batched=True)[0])
     assert torch.allclose(*results, rtol=1e-10, atol=1e-10)
+
+
+@pytest.mark.filterwarnings("ignore:.*autocast")
+def test_pooling_outputs_can_be_written_to():
+    """What the nodes return is the caller's, as what torch's operations return is; 64 bits."""
+    results = []
+    for context, pooled in (_NODES, _OPERATIONS):
+        x, out, d = _pooling(lambda rows: context(rows).mul_(0.5), lambda z, rows: pooled(z, rows).mul_(3).add_(1))
+        results.append((out, torch.autograd.grad(out, x, d, create_graph=True)[0]))
+    assert torch.equal(results[0][0], results[1][0]) and torch.allclose(results[0][1], results[1][1], rtol=1e-10, atol=1e-10)
