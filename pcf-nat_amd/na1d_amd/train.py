@@ -214,11 +214,11 @@ class _Pooling(torch.autograd.Function):
 
     @staticmethod
     def again(ctx, grad, f, *inputs):
-        """The same backward by torch, for a caller that differentiates it again, or whose gradient is no plain tensor.  It is
-        taken by views of the inputs, each a node of its own: an input that was made from another one (the logits from x)
-        would hand that its gradient here too, and so twice."""
+        """The same backward by torch, for a caller that differentiates it again, whose gradient is no plain tensor, or whose
+        hooks hand saved tensors back in another form.  It is taken by views of the inputs, each a node of its own: an input
+        that was made from another one (the logits from x) would hand that its gradient here too, and so twice."""
         create_graph = torch.is_grad_enabled()
-        with torch.enable_grad(), torch.autocast("cuda", dtype=inputs[-1].dtype):
+        with torch.enable_grad(), torch.autocast("cuda", dtype=ctx.dtype):
             views = [t.view_as(t) for t in inputs]
             leaves = [t for t, need in zip(views, ctx.needs_input_grad) if need]
             grads = iter(torch.autograd.grad(f(*views), leaves, grad, create_graph=create_graph))
@@ -230,15 +230,16 @@ class _Context(_Pooling):
     def forward(ctx, x, eps):
         out, var, std = context_of(x, eps)
         ctx.save_for_backward(x, var, std)
-        ctx.eps = eps
+        ctx.eps, ctx.dtype = eps, x.dtype
         return out
 
     @staticmethod
     def backward(ctx, dctx):
         x, var, std = ctx.saved_tensors
-        if torch.is_grad_enabled() or not plain_call(dctx):
-            return _Pooling.again(ctx, dctx, lambda x: context_of(x, ctx.eps)[0], x)
         n, c, t = x.shape
+        if torch.is_grad_enabled() or not (plain_call(dctx) and dctx.shape == (n, 3 * c, t) and _rows_fit(ctx.dtype, x)
+                                           and _lie(x, x.dtype, (n, c, 1), var, std)):
+            return _Pooling.again(ctx, dctx, lambda x: context_of(x, ctx.eps)[0], x)
         dctx, dx = _aligned(dctx), torch.empty_like(x)
         with torch.cuda.device(x.device):
             _lib.check(_lib.load().na1d_train_context_backward(
@@ -253,15 +254,16 @@ class _Pooled(_Pooling):
     def forward(ctx, logits, x, eps):
         out = pooled_of(logits, x, eps)
         ctx.save_for_backward(logits, x, out)
-        ctx.eps = eps
+        ctx.eps, ctx.dtype = eps, x.dtype
         return out.clone()                          # the caller may write to its own
 
     @staticmethod
     def backward(ctx, dout):
         logits, x, out = ctx.saved_tensors
-        if torch.is_grad_enabled() or not plain_call(dout):
-            return _Pooling.again(ctx, dout, lambda z, x: pooled_of(z, x, ctx.eps), logits, x)
         n, c, t = x.shape
+        if torch.is_grad_enabled() or not (plain_call(dout) and dout.shape == (n, 2 * c) and _rows_fit(ctx.dtype, logits, x)
+                                           and _lie(x, torch.float32, (n, 2 * c), out)):
+            return _Pooling.again(ctx, dout, lambda z, x: pooled_of(z, x, ctx.eps), logits, x)
         dout, dz, dx = dout.contiguous(), torch.empty_like(logits), torch.empty_like(x)
         with torch.cuda.device(x.device):
             _lib.check(_lib.load().na1d_train_pool_backward(
@@ -270,14 +272,22 @@ class _Pooled(_Pooling):
         return dz, dx, None
 
 
-def _pooling_fits(*tensors):
+def _lie(x, dtype, shape, *tensors):
+    return all(t.device == x.device and t.dtype == dtype and t.shape == shape and t.is_contiguous() for t in tensors)
+
+
+def _rows_fit(dtype, *tensors):
+    """Whether the kernels take these [N, C, T] tensors."""
     x = tensors[-1]
-    return (x.is_cuda and x.dim() == 3 and torch.is_grad_enabled() and any(t.requires_grad for t in tensors) and torch.is_autocast_enabled("cuda")
-            and x.dtype in (torch.bfloat16, torch.float16) and x.dtype == torch.get_autocast_dtype("cuda")
-            and all(plain_call(t) and t.device == x.device and t.dtype == x.dtype and t.shape == x.shape and t.is_contiguous()
-                    and t.data_ptr() % 16 == 0 for t in tensors)
+    return (x.is_cuda and x.dim() == 3 and dtype in (torch.bfloat16, torch.float16)
+            and _lie(x, dtype, x.shape, *tensors) and all(plain_call(t) and t.data_ptr() % 16 == 0 for t in tensors)
             and 0 < x.shape[0] <= 65535 and x.shape[1] % 8 == 0 and 8 <= x.shape[1] <= 1 << 16 and 2 <= x.shape[2] <= 2048
             and x.shape[0] * x.shape[1] < 1 << 31)
+
+
+def _pooling_fits(*tensors):
+    return (torch.is_grad_enabled() and any(t.requires_grad for t in tensors) and torch.is_autocast_enabled("cuda")
+            and _rows_fit(torch.get_autocast_dtype("cuda"), *tensors))
 
 
 def pooling_context(x, eps):

@@ -1,4 +1,5 @@
 """A windowed encoder layer in training as one native node (na1d_train_layer_*) against the fp32 module on the CPU."""
+import contextlib
 import copy
 
 import pytest
@@ -316,3 +317,22 @@ def test_pooling_output_can_be_written_to():
         twice = pool(x).mul_(2)                     # a factor of two rounds nothing
     assert "Pooled" in type(out.grad_fn).__name__ and torch.equal(twice, 2 * out)
     assert torch.equal(*(torch.autograd.grad(o, x, d)[0] for o in (twice, 2 * out)))
+
+
+@pytest.mark.parametrize("pack,unpack", [(lambda t: t.mT.contiguous() if t.dim() > 1 else t, lambda t: t.mT if t.dim() > 1 else t),
+                                         (lambda t: t.double(), lambda t: t)], ids=["other strides", "another type"])
+def test_pooling_under_hooks_on_saved_tensors(pack, unpack):
+    """Hooks may hand saved tensors back in another form; what torch's operations make of it is what counts."""
+    torch.manual_seed(3)
+    pool, d, grads = models.AttentiveStatisticsPooling(64, 32).cuda(), torch.randn(3, 128).cuda(), []
+    x = torch.randn(3, 64, 50).to("cuda", torch.bfloat16).requires_grad_(True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        hidden = pool.tanh(pool.tdnn(train.context_of(x, pool.eps)[0])).detach()       # the nodes alone under the hooks
+        logits = pool.conv(hidden).detach().requires_grad_(True)
+        for hooked in (False, True):
+            with torch.autograd.graph.saved_tensors_hooks(pack, unpack) if hooked else contextlib.nullcontext():
+                out, ctx = train.pooled(logits, x, pool.eps), train.pooling_context(x, pool.eps)
+            assert "Pooled" in type(out.grad_fn).__name__ and "Context" in type(ctx.grad_fn).__name__
+            grads.append(torch.autograd.grad((out, ctx), (logits, x), (d, torch.ones_like(ctx) * d[:, :1, None].bfloat16())))
+    for got, want in zip(*grads):
+        assert got.dtype == want.dtype and O.rel_l2(got.float(), want.float()) < 2e-2        # bfloat16, see above
