@@ -285,16 +285,16 @@ def _rows_fit(dtype, *tensors):
             and x.shape[0] * x.shape[1] < 1 << 31)
 
 
-def _pooling_fits(*tensors):
-    return (torch.is_grad_enabled() and any(t.requires_grad for t in tensors) and torch.is_autocast_enabled("cuda")
+def _pooling_fits(eps, *tensors):
+    return (isinstance(eps, (int, float)) and torch.is_grad_enabled() and any(t.requires_grad for t in tensors) and torch.is_autocast_enabled("cuda")
             and _rows_fit(torch.get_autocast_dtype("cuda"), *tensors))
 
 
 def pooling_context(x, eps):
     """:func:`context_of` as one autograd node where the kernels take ``x``."""
-    return _Context.apply(x, eps) if _pooling_fits(x) else context_of(x, eps)[0]
+    return _Context.apply(x, eps) if _pooling_fits(eps, x) else context_of(x, eps)[0]
 
 
 def pooled(logits, x, eps):
     """:func:`pooled_of` as one autograd node where the kernels take its inputs."""
-    return _Pooled.apply(logits, x, eps) if _pooling_fits(logits, x) else pooled_of(logits, x, eps)
+    return _Pooled.apply(logits, x, eps) if _pooling_fits(eps, logits, x) else pooled_of(logits, x, eps)

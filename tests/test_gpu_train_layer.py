@@ -336,3 +336,17 @@ def test_pooling_under_hooks_on_saved_tensors(pack, unpack):
             grads.append(torch.autograd.grad((out, ctx), (logits, x), (d, torch.ones_like(ctx) * d[:, :1, None].bfloat16())))
     for got, want in zip(*grads):
         assert got.dtype == want.dtype and O.rel_l2(got.float(), want.float()) < 2e-2        # bfloat16, see above
+
+
+def test_pooling_with_a_tensor_for_eps():
+    """clamp() takes a tensor too; such a bound is left to torch."""
+    torch.manual_seed(4)
+    pool = models.AttentiveStatisticsPooling(64, 32).cuda()
+    x, d, results = torch.randn(3, 64, 50).to("cuda", torch.bfloat16).requires_grad_(True), torch.randn(3, 128).cuda(), []
+    for eps in (1e-3, torch.tensor(1e-3, device="cuda")):
+        pool.eps = eps
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            out = pool(x)
+        results.append((out, torch.autograd.grad(out, x, d)[0]))
+    for got, want in zip(*results):
+        assert O.rel_l2(got.float(), want.float()) < 2e-2
