@@ -277,7 +277,8 @@ int64_t na1d_global_backward_workspace_bytes(int64_t B, int64_t H, int64_t T, in
  *
  * Weights are 16-bit (`dtype`) matrices [outputs, inputs] in fragment order: element (o, i) lies at
  *     ((o / 16 * (inputs / 32) + i / 32) * 64 + i % 32 / 8 * 16 + o % 16) * 8 + i % 8
- * so that the 16 x 32 block a matrix instruction reads is one contiguous kilobyte.  Biases and affine maps are fp32.
+ * so that the 16 x 32 block a matrix instruction reads is one contiguous kilobyte.  They are 16-byte aligned; biases, norms and
+ * affine maps are fp32 and may lie on any float.
  * Tokens have 256 channels, the MLP 1024, the attention of the pooling 128; `wide` (channels of the projection) is a
  * multiple of 256, in_chans * patch a multiple of 32 and at most 256, `emb` a multiple of 16.
  */

@@ -5,10 +5,16 @@
 namespace na1d {
 namespace enc {
 
+// Four floats that a caller may have put on any float.
+__device__ inline f32x4 load4(const float *p) {
+    typedef float on_any_float __attribute__((ext_vector_type(4), aligned(4)));
+    return *reinterpret_cast<const on_any_float *>(p);
+}
+
 // What a batch norm with running statistics multiplies channels c .. c+3 by.  The few norms that no weight has been folded
 // with are read as the module holds them, so that the next call sees what a program writes there.
 __device__ inline f32x4 norm_gain(const na1d_encoder_norm &n, int c) {
-    const f32x4 w = *reinterpret_cast<const f32x4 *>(n.weight + c), v = *reinterpret_cast<const f32x4 *>(n.var + c);
+    const f32x4 w = load4(n.weight + c), v = load4(n.var + c);
     f32x4 gain;
 #pragma unroll
     for (int r = 0; r < 4; ++r) gain[r] = w[r] * __builtin_amdgcn_rsqf(v[r] + n.eps);
@@ -105,13 +111,19 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
     __device__ inline LDS_PTR(u32x2) at(LDS_PTR(char) tile, int c, int i) const {
         return reinterpret_cast<LDS_PTR(u32x2)>(tile + (result_lane(n, g) ^ 2 * c) + i * 16 * kRow);
     }
-    __device__ inline f32x4 bias(const float *b, int c) const { return *reinterpret_cast<const f32x4 *>(b + c + 4 * g); }
+    __device__ inline f32x4 bias(const float *b, int c) const { return load4(b + c + 4 * g); }
     __device__ inline f32x4 staged_bias(int c) const { return *reinterpret_cast<LDS_PTR(f32x4)>(b_lds + c + 4 * g); }
 
     // Biases come through LDS, and sums start at them: read from memory behind a product, a bias would have to wait for every
     // weight of the next product that is on its way (loads return in order).  qkv's take the place of fc1's first 768.
+    // The caller's own parameters may lie on any float (views of one flat buffer); those go a float to a lane.
     __device__ inline void stage_bias(const float *b, int count, int to) const {
-        for (int k = wave; k < count / 256; k += NW) load_to_lds<16, kReadShared>(make_rsrc(b, 4 * count), (LDS_PTR(char))(b_lds + to + 256 * k), 1024 * k + lane16);
+        const Rsrc bs = make_rsrc(b, 4 * count);
+        if ((uintptr_t)b & 15u) {
+            for (int k = wave; k < count / 64; k += NW) load_to_lds<4, 0>(bs, (LDS_PTR(char))(b_lds + to + 64 * k), 256 * k + 4 * lane);
+        } else {
+            for (int k = wave; k < count / 256; k += NW) load_to_lds<16, kReadShared>(bs, (LDS_PTR(char))(b_lds + to + 256 * k), 1024 * k + lane16);
+        }
     }
     __device__ inline void stage_tail_biases() const {
         stage_bias(a.b_proj, kDim, kBiasProj);
@@ -448,14 +460,14 @@ template <class DT, LinearEnd END>
 __device__ inline f32x4 ended(const LinearArgs &a, int64_t m, int c, f32x4 v) {
     if constexpr (END == kTanhNorm) {
         const uint32_t u = (uint32_t)m / (uint32_t)a.T;
-        v += *reinterpret_cast<const f32x4 *>(a.bias + (int64_t)u * a.outputs + c);
+        v += load4(a.bias + (int64_t)u * a.outputs + c);
     } else if constexpr (END == kShift) {
-        v += *reinterpret_cast<const f32x4 *>(a.norm.bias + c) - *reinterpret_cast<const f32x4 *>(a.norm.mean + c) * norm_gain(a.norm, c);
+        v += load4(a.norm.bias + c) - load4(a.norm.mean + c) * norm_gain(a.norm, c);
     } else {
-        v += *reinterpret_cast<const f32x4 *>(a.bias + c);
+        v += load4(a.bias + c);
     }
     if constexpr (END == kReluNorm || END == kTanhNorm) {
-        const f32x4 sc = *reinterpret_cast<const f32x4 *>(a.scale + c), of = *reinterpret_cast<const f32x4 *>(a.offset + c);
+        const f32x4 sc = load4(a.scale + c), of = load4(a.offset + c);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             v[r] = __builtin_fmaf(v[r] < 0.f ? 0.f : v[r], sc[r], of[r]);        // NaN stays

@@ -269,3 +269,22 @@ def test_a_plan_outlives_its_use_on_other_streams():
     torch.cuda.synchronize()
     assert all(torch.equal(o, want) for o in outs) and not _near(after, want[:1])
     del filled
+
+
+@pytest.mark.parametrize("batch,frames", [(3, 64), (40, 128), (86, 96), (331, 100)])
+@pytest.mark.parametrize("groups", [(8, 4), (2, 1)])
+def test_parameters_on_any_float(groups, batch, frames):
+    """Biases that are views of a flat buffer, on 4, 8 and 12 bytes: to the bit what they are on their own."""
+    model = _model(groups=groups)
+    x = _input(batch, frames)
+    want, _ = _both(model, x)
+    moved = copy.deepcopy(model)
+    for at, layer in enumerate(l for b in moved.blocks for l in b.blocks):
+        for k, m in enumerate((layer.attn.proj, layer.mlp.fc2)):
+            flat = torch.zeros(264, device="cuda")
+            at_float = 1 + (2 * at + k) % 3
+            flat[at_float:at_float + 256] = m.bias.detach()
+            m.bias = torch.nn.Parameter(flat[at_float:at_float + 256])
+            assert m.bias.data_ptr() % 16
+    got, _ = _both(moved, x)
+    assert got is not None and torch.equal(got, want)
