@@ -2,6 +2,8 @@
 import copy
 import ctypes
 import gc
+import os
+import re
 import types
 import weakref
 
@@ -158,3 +160,43 @@ def test_missing_pointers_are_refused(name):
         setattr(plan.layers[0] if name in _POINTERS else e, name, None)
     st = lib.na1d_encode(ctypes.byref(e), args["out"], args["x"], None, 2, 64, args["workspace"], need, None)
     assert st in (-1, _lib.UNSUPPORTED)                     # a weight's absence already says that nothing covers the call
+
+
+def _gelu_errors(gelu):
+    """Of an fp32 GELU against 64 bits: largest, largest relative one below 0.1, and rms for arguments of some deviations."""
+    exact = lambda x: 0.5 * x.double() * torch.special.erfc(-x.double() * 0.5 ** 0.5)
+    x = torch.linspace(-14, 14, 2000001)
+    x = x[x != 0]
+    error, small = (gelu(x).double() - exact(x)).abs(), x.abs() < 0.1
+    draws = torch.randn(400000, generator=torch.Generator().manual_seed(0))
+    rms = [(gelu(s * draws).double() - exact(s * draws)).square().mean().sqrt().item() for s in (0.02, 0.1, 0.3, 0.58, 1.0, 2.0, 4.0)]
+    return [error.max().item(), (error / exact(x).abs())[small].max().item(), error[x < -3].max().item()] + rms
+
+
+def test_gelu_is_no_worse_than_by_the_handbook():
+    """The polynomial in inference's GELU, with fp32 roundings behind 64-bit multiply-adds, against formula 7.1.26 of Abramowitz
+    and Stegun's handbook in the same arithmetic, by every measure: small arguments above all, where a constant term that is not
+    -1 to the last bit costs all values the same share."""
+    with open(os.path.join(os.path.dirname(_lib.__file__), "..", "csrc", "na1d_encoder.h")) as f:
+        terms = [float(v.rstrip("f")) for v in re.search(r"kGelu\[\] = \{([^}]*)\}", f.read()).group(1).replace(" ", "").split(",")]
+    fp32 = lambda v: v.float().double()
+
+    def polynomial(x):
+        a = x.double().abs()
+        p = torch.full_like(a, terms[-1]).float().double()
+        for t in terms[-2::-1]:
+            p = fp32(p * a + torch.tensor(t).double())
+        return fp32(x.double().clamp(min=0) - a * fp32(torch.exp2(p)))
+
+    def handbook(x):
+        a = x.double().abs()
+        t = fp32(1 / fp32(a * torch.tensor(0.3275911 * 0.5 ** 0.5).double() + 1))
+        e = torch.full_like(a, 0.5 * 1.061405429).float().double()
+        for k in (-1.453152027, 1.421413741, -0.284496736, 0.254829592):
+            e = fp32(e * t + torch.tensor(0.5 * k).double())
+        e = fp32(e * fp32(torch.exp2(fp32(fp32(x.double() ** 2) * torch.tensor(-0.72134752).double()))))
+        return fp32(x.double().clamp(min=0) - fp32(a * t) * e)
+
+    assert terms[-1] < 0                                                       # the tail vanishes
+    assert all(p <= h for p, h in zip(_gelu_errors(polynomial), _gelu_errors(handbook)))
+    assert polynomial(torch.tensor([1e3, -1e3, 3e4, -3e4])).tolist() == [1e3, 0.0, 3e4, 0.0]
