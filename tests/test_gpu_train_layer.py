@@ -350,3 +350,27 @@ def test_pooling_with_a_tensor_for_eps():
         results.append((out, torch.autograd.grad(out, x, d)[0]))
     for got, want in zip(*results):
         assert O.rel_l2(got.float(), want.float()) < 2e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,c,t", [(2, 16, 9), (3, 72, 100)])
+def test_pooling_nodes_where_the_variance_is_bounded(n, c, t, dtype):
+    """Rows that are constant over T, as a dead channel's, and rows whose variance lies on either side of a bound that 16 bits can
+    hold: no gradient comes through a bounded deviation.  Against 64 bits; rows whose variance is within the rounding of the
+    bound are none here."""
+    gen, eps = torch.Generator().manual_seed(n * c), 2.0 ** -6
+    size = torch.tensor([0.0, 0.03, 1.0, 0.5])[torch.arange(c) % 4].view(1, c, 1)             # variances 0, 2^-10, 1, 2^-2
+    x = (torch.randn(n, c, 1, generator=gen) + size * torch.randn(n, c, t, generator=gen)).to("cuda", dtype).requires_grad_(True)
+    z = (0.1 * torch.randn(n, c, t, generator=gen)).to("cuda", dtype).requires_grad_(True)
+    d1, d2 = torch.randn(n, 3 * c, t, generator=gen).to("cuda", dtype), torch.randn(n, 2 * c, generator=gen).cuda()
+    with torch.autocast("cuda", dtype=dtype):
+        got, out = train.pooling_context(x, eps), train.pooled(z, x, eps)
+    assert "Context" in type(got.grad_fn).__name__ and "Pooled" in type(out.grad_fn).__name__
+    xe, ze = (v.detach().double().requires_grad_(True) for v in (x, z))
+    bounded = (train.context_of(xe, eps)[1] < eps).view(n, c)
+    assert torch.equal(bounded, (torch.arange(c, device="cuda") % 4 < 2).expand(n, c))
+    grads = torch.autograd.grad(got, x, d1) + torch.autograd.grad(out, (x, z), d2)
+    exact = torch.autograd.grad(train.context_of(xe, eps)[0], xe, d1.double()) + torch.autograd.grad(train.pooled_of(ze, xe, eps), (xe, ze), d2.double())
+    for g, e in zip(grads, exact):
+        for rows in (bounded, ~bounded):
+            assert O.rel_l2(g[rows].float(), e[rows].float()) < (1e-2 if dtype == torch.bfloat16 else 1.5e-3)
