@@ -777,12 +777,12 @@ stats_kernel(float *__restrict__ mean_std, char *__restrict__ rounded, const cha
 
 // Attentive statistics pooling: logits = W . hidden[t] on the matrix core, softmax over the tokens and the weighted mean and
 // deviation in one pass over the rows, the logits never written.  Lane (n, g) sees channels 8g .. 8g+7 of each 32 (two tiles
-// of the product, whose rows are taken in that order) for every 16th token, keeps its own running maximum (moved only when outgrown by 2^8) and sums of p, p d, p d^2 (d =
-// difference to the plain mean), and the lanes meet at the end.  A wave takes 64 channels; the TS of four waves that have the
-// same ones share an utterance's tokens.  Bound by the latency of a wave's few turns and, at 100 tokens, by its two ends (16
-// weights to fetch, 256 steps across lanes): 256 utterances of 100 tokens take 77 us with four waves to an utterance and 47
-// with one, 64 of 1000 94 and 102; 20 of 150 a microsecond less with four.  With loads of 8 bytes in the tiles' own order and
-// none ahead of its turn four waves took 82 and 110.  Half the channels and twice the waves to a SIMD: 56 and 121.
+// of the product, whose rows are taken in that order) for every 16th token, keeps its own running maximum (moved only when
+// outgrown by 2^8) and sums of p, p d, p d^2 (d = difference to the plain mean), and the lanes meet at the end.  A wave takes
+// 64 channels; the TS of four waves that have the same ones share an utterance's tokens (one_wave below).  Bound by the latency
+// of a wave's few turns and, at 100 tokens, by its two ends (16 weights to fetch, 256 steps across lanes).  256 utterances of
+// 100 tokens: 42 us; 64 of 1000: 76 us.  With loads of 8 bytes in the tiles' own order and none ahead of its turn 82 and 92.
+// Half the channels and twice the waves to a SIMD: 56 and 121.
 struct PoolArgs {
     const char *h, *hidden, *w;
     const float *count, *mean_std, *a_pool, *c_pool;
@@ -934,6 +934,17 @@ pool_kernel(PoolArgs a) {
 }
 
 // ----------------------------------------------------------------------------- launchers
+// Whether a wave takes all of an utterance's tokens.  Such workgroups last as long as the utterance is and two fit a CU, so what
+// counts is how full the last 512 are; four waves to an utterance even that out, at the price of four times the ends.  1536
+// channels, one and four waves, us: 100 tokens: 24 utterances 11.0 13.5, 32: 11.5 13.0, 96: 24.4 29.2; 200 tokens: 16: 16.2 11.3,
+// 32: 16.4 16.8, 64: 24.0 28.8, 96: 37.4 41.6; 300 tokens: 32: 21.9 20.0, 48: 31.6 29.5, 64: 33.8 36.7, 96: 51.3 50.7, 112: 51.5
+// 60.3; 500 tokens: 64: 47.3 45.3, 85: 47.6 59.4, 96: 76.4 67.3, 112: 76.8 80.4; 1000 tokens: 64: 87.0 75.8, 85: 87.9 102,
+// 86: 151 116, 128: 158 159, 170: 176 210; 2000 tokens: 64: 167 143, 85: 170 191, 128: 313 292.
+inline bool one_wave(int64_t N, int64_t T, int wide) {
+    const int64_t blocks = N * (wide / 256), room = (blocks + 511) / 512 * 512;
+    return T <= 200 ? blocks >= 192 : T <= 500 ? 8 * blocks >= 5 * room : 5 * blocks >= 4 * room;
+}
+
 template <class DT, int MT, int NW, int PF, bool SPARSE>
 int launch_layer_mt(const LayerArgs &a, hipStream_t s) {
     auto kern = layer_kernel<DT, MT, NW, PF, false, SPARSE>;
@@ -1169,7 +1180,7 @@ int encode(const na1d_encoder &e, char *out, const float *x, const float *lens, 
     NA1D_TRY(launch_linear<DT, kTanhNorm>(d, s));
     PoolArgs p{ws + b.h, ws + b.hidden, (const char *)e.w_logit, count, reinterpret_cast<const float *>(ws + b.stats),
                reinterpret_cast<const float *>(ws + b.pool_map), reinterpret_cast<const float *>(ws + b.pool_map) + 2 * e.wide, ws + b.pooled, (int)T, e.wide};
-    if (N * (e.wide / 64) >= (T <= 128 ? 768 : 2048))                // a wave to all tokens of 64 channels
+    if (one_wave(N, T, e.wide))
         pool_kernel<DT, 1><<<dim3((unsigned)(e.wide / 256), (unsigned)N), kThreads, 0, s>>>(p);
     else
         pool_kernel<DT, 4><<<dim3((unsigned)(e.wide / 64), (unsigned)N), kThreads, 0, s>>>(p);

@@ -67,7 +67,8 @@ def test_tiles_of_every_size(groups, batch, frames):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("batch,frames", [(31, 100), (32, 256), (33, 258), (85, 260), (86, 260)])
+@pytest.mark.parametrize("batch,frames", [(31, 100), (32, 256), (33, 258), (85, 260), (86, 260), (31, 400), (32, 400), (32, 402),
+                                          (53, 402), (54, 402), (65, 1000), (65, 1002), (68, 1002), (69, 1002), (86, 1002)])
 def test_pooling_with_one_wave_or_four_to_an_utterance(batch, frames, dtype):
     """Each side of the sizes at which the waves of a pooling workgroup part by channels alone; lengths from one token on."""
     model = _model(dtype=dtype)
