@@ -67,15 +67,11 @@ template <int NTW, int PF> struct Ring {
             if (s < P::kSteps) fill(p, s, s, lane16);
     }
 };
-struct Nothing {
-    static constexpr int kTiles = 0, kSteps = 0;
-    __device__ inline u32x4 load(int, int, int) const { return u32x4{}; }
-};
 
 // acc[j][i] += W[tile j of this wave] . X[token tile i]^T; lane (n, g) ends up with outputs 4g .. 4g+3 of each tile for
 // token n of each token tile.  The ring holds this product's first PF steps on entry and `next`'s on exit.
-template <class DT, int MT, int NTW, int PF, int NA, class P, class Q>
-__device__ inline void multiply(f32x4 (&acc)[NA][MT], int a0, Ring<NTW, PF> &ring, const P &p, const Q &next, LDS_PTR(char) tile,
+template <class DT, int MT, int NTW, int PF, class P, class Q>
+__device__ inline void multiply(f32x4 (&acc)[P::kTiles][MT], Ring<NTW, PF> &ring, const P &p, const Q &next, LDS_PTR(char) tile,
                                 int n, int g, int lane16) {
     static_assert(P::kSteps % PF == 0 || P::kSteps < PF, "slots of a product");
     if constexpr (P::kSteps < PF) {
@@ -102,7 +98,7 @@ __device__ inline void multiply(f32x4 (&acc)[NA][MT], int a0, Ring<NTW, PF> &rin
 #pragma unroll
         for (int j = j0; j < (P::kSkip ? j0 + 1 : P::kTiles); ++j)
 #pragma unroll
-            for (int i = 0; i < MT; ++i) acc[a0 + j][i] = Mma<DT>::k32(ring.w[s % PF][j], x[turn & 1][i], acc[a0 + j][i]);
+            for (int i = 0; i < MT; ++i) acc[j][i] = Mma<DT>::k32(ring.w[s % PF][j], x[turn & 1][i], acc[j][i]);
         if (j0 + 1 < kPerStep) continue;
         if (s + PF < P::kSteps) {
             ring.fill(p, s % PF, s + PF, lane16);

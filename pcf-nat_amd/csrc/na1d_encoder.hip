@@ -151,7 +151,7 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
         wait_direct();
         barrier_lds();
         begin_sums(hid, kBiasProj + CW * wave);
-        multiply<DT, MT>(hid, 0, ring, proj, S::fc1(w1, first_chunk, wave), p_lds, n, g, lane16);
+        multiply<DT, MT>(hid, ring, proj, S::fc1(w1, first_chunk, wave), p_lds, n, g, lane16);
 #pragma unroll
         for (int j = 0; j < NTW; ++j) {
             const int c = CW * wave + 16 * j;
@@ -166,7 +166,7 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
         begin_sums(hid, kBiasFc1 + 256 * c + CW * wave);
         barrier_lds();                           // x1 is whole (first round); every wave is done with the hidden channels before
         if (c == 3 && !SPLIT) stage_qkv_bias();  // every wave has taken fc1's
-        multiply<DT, MT>(hid, 0, ring, S::fc1(w1, c, wave), S::fc2(w2, c, wave), q_lds, n, g, lane16);
+        multiply<DT, MT>(hid, ring, S::fc1(w1, c, wave), S::fc2(w2, c, wave), q_lds, n, g, lane16);
 #pragma unroll
         for (int j = 0; j < NTW; ++j) {
             const int ch = CW * wave + 16 * j;
@@ -180,7 +180,7 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
         }
         barrier_lds();
         if (wave < S::kActive)
-            multiply<DT, MT>(acc, 0, ring, S::fc2(w2, c, wave), S::fc1(w1, last ? 0 : c + 1, wave), p_lds, n, g, lane16);
+            multiply<DT, MT>(acc, ring, S::fc2(w2, c, wave), S::fc1(w1, last ? 0 : c + 1, wave), p_lds, n, g, lane16);
         else
             ring.begin(S::fc1(w1, last ? 0 : c + 1, wave), lane16);
     }
@@ -283,7 +283,7 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
         for (int which = from; which < to; ++which) {
             f32x4 acc[NTW][MT];
             begin_sums(acc, kBiasQkv + which * kDim + CW * wave);
-            multiply<DT, MT>(acc, 0, ring, S::qkv(w, which, wave), S::qkv(w, min(which + 1, 2), wave), q_lds, n, g, lane16);
+            multiply<DT, MT>(acc, ring, S::qkv(w, which, wave), S::qkv(w, min(which + 1, 2), wave), q_lds, n, g, lane16);
             u32x2 o[MT][NTW];
 #pragma unroll
             for (int j = 0; j < NTW; ++j)
@@ -323,7 +323,8 @@ part_kernel(LayerArgs a) {
     const Rsrc as = make_rsrc(a.attn + m0 * kRow, rows * kRow), xs = make_rsrc(a.x_in + m0 * a.x_in_pitch, rows * a.x_in_pitch);
     stage_tokens<16, NW, kReadShared>(as, w.p_lds, kRow, kRow, wave, lane);
     stage_tokens<16, NW, kReadShared>(xs, w.q_lds, a.x_in_pitch, kRow, wave, lane);
-    w.stage_tail_biases();
+    w.stage_bias(a.b_proj, kDim, kBiasProj);
+    w.stage_bias(a.b_fc1 + 256 * c, 256, kBiasFc1 + 256 * c);
     switch (a.tail_groups) {
         case 8: w.template tail_part<8>(c, m0, rows); break;
         case 4: w.template tail_part<4>(c, m0, rows); break;
@@ -522,7 +523,7 @@ linear_kernel(LinearArgs a, int col_blocks) {
         barrier_lds();
         if (p + 1 < pieces) stage(p + 1);
         const P now{ws, tile0 * steps + 8 * p, steps, 0}, next{ws, tile0 * steps + 8 * min(p + 1, pieces - 1), steps, 0};
-        multiply<DT, MT>(acc, 0, ring, now, next, lds + (p & 1) * (16 * MT * kRow), n, g, lane16);
+        multiply<DT, MT>(acc, ring, now, next, lds + (p & 1) * (16 * MT * kRow), n, g, lane16);
     }
     const Rsrc os = make_rsrc(a.out + m0 * a.out_pitch, rows * a.out_pitch);
 #pragma unroll
@@ -991,10 +992,15 @@ template <class DT, LinearEnd END> int launch_linear(const LinearArgs &a, hipStr
             kern<<<(unsigned)((a.M + 16 * mt - 1) / (16 * mt) * cols), kThreads, lds, s>>>(a, cols);
             return launch_status();
         };
-        if constexpr (END == kReluNorm)
-            if (a.outputs % 256 == 0 && a.M > 8192) return go(linear_wide_kernel<DT, END>, 8, 4, 256);
-        if (a.outputs % 256 == 0 && a.M > 8192) return go(linear_kernel<DT, 4, 4, END>, 4, 4);
-        if (a.outputs % 128 == 0) return a.M > 8192 ? go(linear_kernel<DT, 4, 2, END>, 4, 2) : go(linear_kernel<DT, 2, 2, END>, 2, 2);
+        if (a.M > 8192) {
+            if constexpr (END == kReluNorm) return go(linear_wide_kernel<DT, END>, 8, 4, 256);      // outputs in 256s: encoder_ok
+            if constexpr (END == kShift || END == kEmbedding)                                       // the pooling's are 128
+                if (a.outputs % 256 == 0) return go(linear_kernel<DT, 4, 4, END>, 4, 4);
+            if constexpr (END != kReluNorm)
+                if (a.outputs % 128 == 0) return go(linear_kernel<DT, 4, 2, END>, 4, 2);
+        } else if (a.outputs % 128 == 0) {
+            return go(linear_kernel<DT, 2, 2, END>, 2, 2);
+        }
     }
     const int nt = a.outputs % 32 == 0 ? 2 : 1, cols = a.outputs / (16 * nt);
     const unsigned wgs = (unsigned)((a.M + 15) / 16 * cols);

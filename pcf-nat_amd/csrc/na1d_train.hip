@@ -363,7 +363,7 @@ gemm_kernel(Gemm a, int col_blocks) {
         barrier_lds();
         if (p + 1 < pieces) stage(p + 1);
         const P now{ws, tile0 * steps + 8 * p, steps, 0}, next{ws, tile0 * steps + 8 * min(p + 1, pieces - 1), steps, 0};
-        multiply<DT, MT>(acc, 0, ring, now, next, lds + (p & 1) * (16 * MT * kRow), n, g, lane16);
+        multiply<DT, MT>(acc, ring, now, next, lds + (p & 1) * (16 * MT * kRow), n, g, lane16);
     }
     const Rsrc os = make_rsrc(a.out + m0 * pitch, rows * pitch);
     f32x4 bias[NTW];
