@@ -336,7 +336,8 @@ part_kernel(LayerArgs a) {
 // Waves on a SIMD.  SPARSE (blocks of 4 or 8 groups before the tile) and dense layers are kernels of their own, so that the
 // former, whose sums never span chunks, run 64 tokens with eight waves of 128 registers: a layer of 64000 tokens 75 -> 70 us,
 // its qkv projection 9 -> 4.5 of a workgroup's 35 us.  Dense layers need the registers for weights that set out four steps
-// ahead (145 -> 134 us); with eight waves of 128 registers they spill 55 and a whole pass takes 3.72 instead of 3.37 ms.
+// ahead (145 -> 134 us); with eight waves of 128 registers they spill 55 and a whole pass takes 3.72 instead of 3.37 ms.  (On
+// four waves 5 to 13 are spilled around the loops; held to two tiles of GELU at a time they are not, and a pass takes 1 % longer.)
 constexpr int layer_waves(int MT, int NW) { return MT == 2 || (MT == 4 && NW == 8) ? 4 : 2; }
 
 // SPLIT: one workgroup to each of q, k and v of a tile (or one where there is no projection behind); the layer before
@@ -535,7 +536,8 @@ linear_kernel(LinearArgs a, int col_blocks) {
 // Very many rows, outputs in hundreds: 128 rows x 256 outputs to a workgroup of four waves.  A wave's 128 x 64 outputs use each
 // weight eight times and each row's operand four times, which halves what the CU's path to L2 carries per product (64 rows ask
 // for its 64 bytes a clock at the matrix cores' full rate); rows come 128 inputs at a time, so two workgroups share a CU.
-// 1024 inputs, 1536 outputs: 25600 rows 124 -> 72 us, 64000 301 -> 184 us (1.1 PFLOP/s), from what whole passes lose.
+// 1024 inputs, 1536 outputs, this and 64 rows, us in a trace: 8200 rows 35 and 54, 10000: 36 and 57, 25600: 85 and 132 (0.95
+// PFLOP/s), 40000: 133 and 209.  Below the limit linear_kernel's 32 rows x 128 outputs: 2048: 24 and 16, 8000: 35 and 48.
 template <class DT, LinearEnd END>
 __global__ void __launch_bounds__(kThreads, 2)
 linear_wide_kernel(LinearArgs a, int col_blocks) {
@@ -664,7 +666,7 @@ __global__ void lengths_kernel(int32_t *t_valid, float *count, const float *lens
 // writes run along the rows.  Bound by memory; the work is split over the channels too, or a single utterance is a handful
 // of workgroups (3 s: 19.5 us in three workgroups of whole rows that divided twice for every value).
 // The launch's last slices bring the last layer's weight into fragment order and the pooled norm into an affine map, from
-// the module's own tensors at each call: of a single utterance's 269 us that is 3, and as much again with the last product
+// the module's own tensors at each call: of a single utterance's 273 us that is 3, and as much again with the last product
 // rounding the fp32 rows itself; kept from call to call, a write that no version counts would go unseen.
 constexpr int kPatchTokens = 32;
 struct Head {

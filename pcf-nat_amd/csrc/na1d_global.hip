@@ -92,11 +92,12 @@ struct GlobalArgs {
 // tiles that all waves share through LDS; the next chunk is on its way while this one is worked on, so one barrier a
 // chunk.  The wave's query tiles go from memory straight into the registers of the matrix operand.
 //
-// The softmax costs more vector instructions than the two products cost matrix instructions, so a chunk whose keys
-// all count takes a short form: the running maximum comes from the raw products (the scale is positive) and scale
-// and maximum fold into one multiply-add in front of the exponential.  Chunks that reach past the valid keys take the long form with its masks.  A padded
-// query row has -100 added to every score: a constant that leaves its probabilities alone and moves its LSE, which
-// is where it is added.
+// The softmax costs more vector instructions than the two products cost matrix instructions, so a chunk whose scores
+// all have the same mask takes a short form: the running maximum comes from the raw products (the scale is positive) and
+// scale and maximum fold into one multiply-add in front of the exponential.  A padded query row has -100 added to every
+// score: a constant that leaves its probabilities alone and moves its LSE, which is where it is added, so a wave whose rows
+// are all padded takes the short form over padded keys too.  Other chunks that reach past the valid keys take the long form
+// with its masks (or the comparison in front of it, see above).
 template <class DT, int C, bool DROP, int QT>
 __global__ void __launch_bounds__(kThreads)
 global_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__restrict__ q,
@@ -481,7 +482,7 @@ global_fwd_short_kernel(char *__restrict__ out, float *__restrict__ lse, const c
 // A workgroup owns 4 * QT query tiles, QT to a wave, whose Q, dO and O rows go from memory straight into registers,
 // and walks the keys in chunks of 4 tiles (K and V through LDS, the next chunk in flight behind the current one).
 // dQ^T += K^T dS^T runs two key tiles at a time on the 32-deep product.  A padded query row's -100 is folded into
-// its LSE once; chunks whose keys all count skip the masks.
+// its LSE once; masks are skipped as in the forward's short form.
 template <class DT, int C, bool DROP, int QT, bool PACKED>
 __global__ void __launch_bounds__(kThreads)
 global_dq_kernel(char *__restrict__ dq, float *__restrict__ delta, const char *__restrict__ q,

@@ -316,8 +316,8 @@ struct Gemm {
     uint32_t T_magic;
     int late;                              // the sum is rounded before the bias is added (a product and an addition in torch)
 };
-// Phi(x) and x's density, the former by formula 7.1.26 of Abramowitz and Stegun as in gelu(); infinities come out as
-// x * Phi(x) gives them.
+// Phi(x) and x's density, the former by formula 7.1.26 of Abramowitz and Stegun's handbook (error below 1.5e-7); infinities
+// come out as x * Phi(x) gives them.
 __device__ inline void normal_of(float x, float &cdf, float &pdf) {
     const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_fabsf(x), 0.3275911f * 0.70710678f, 1.f));
     float e = __builtin_fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
@@ -608,7 +608,8 @@ grad_fold_kernel(Fold a) {
 // =============================================================================
 // Rows of T values lie one behind the other, so R rows (a multiple of eight) are whole 16-byte units in memory whatever T is:
 // they come to LDS and leave it as such, and 16 lanes work on a row.  Bound by memory.  128 x 1536 rows of 100 values, fp16: 48
-// and 47 us (157 and 197 MB), where torch took some thirty kernels of 440 and 330 us.  A training step: 10.6 -> 9.2 ms.
+// and 47 us (157 and 197 MB), where torch took some thirty kernels of 440 and 330 us.  A training step, which its host paces by
+// then: 10.1-10.3 -> 9.5-9.7 ms.
 constexpr int kPoolLanes = 16, kPoolThreads = 256;
 __device__ inline float over_row(float x) {                       // sum over the 16 lanes of a row
     x += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0xb1, 0xf, 0xf, true));
