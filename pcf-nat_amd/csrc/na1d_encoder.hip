@@ -92,7 +92,7 @@ template <int G, int NW> struct Groups {
 };
 
 // Places of the biases in LDS, in floats.
-constexpr int kBiasFc1 = 0, kBiasQkv = 0, kBiasProj = kHidden, kBiasFc2 = kBiasProj + kDim, kBias = kBiasFc2 + kDim;
+constexpr int kBiasFc1 = 0, kBiasProj = kHidden, kBiasFc2 = kBiasProj + kDim, kBiasQkv = kBiasFc2 + kDim, kBias = kBiasQkv + 3 * kDim;
 template <int MT> constexpr size_t layer_lds() { return (size_t)2 * 16 * MT * kRow + kBias * sizeof(float); }
 
 // The number of groups as the kernels know it: every switch over it and every sum over its parts starts from this.
@@ -115,7 +115,7 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
     __device__ inline f32x4 staged_bias(int c) const { return *reinterpret_cast<LDS_PTR(f32x4)>(b_lds + c + 4 * g); }
 
     // Biases come through LDS, and sums start at them: read from memory behind a product, a bias would have to wait for every
-    // weight of the next product that is on its way (loads return in order).  qkv's take the place of fc1's first 768.
+    // weight of the next product that is on its way (loads return in order).
     // The caller's own parameters may lie on any float (views of one flat buffer); those go a float to a lane.
     __device__ inline void stage_bias(const float *b, int count, int to) const {
         const Rsrc bs = make_rsrc(b, 4 * count);
@@ -165,7 +165,6 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
         f32x4 hid[NTW][MT];
         begin_sums(hid, kBiasFc1 + 256 * c + CW * wave);
         barrier_lds();                           // x1 is whole (first round); every wave is done with the hidden channels before
-        if (c == 3 && !SPLIT) stage_qkv_bias();  // every wave has taken fc1's
         multiply<DT, MT>(hid, ring, S::fc1(w1, c, wave), S::fc2(w2, c, wave), q_lds, n, g, lane16);
 #pragma unroll
         for (int j = 0; j < NTW; ++j) {
@@ -179,7 +178,7 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
             }
         }
         barrier_lds();
-        if (wave < S::kActive)
+        if (S::kActive == NW || wave < S::kActive)
             multiply<DT, MT>(acc, ring, S::fc2(w2, c, wave), S::fc1(w1, last ? 0 : c + 1, wave), p_lds, n, g, lane16);
         else
             ring.begin(S::fc1(w1, last ? 0 : c + 1, wave), lane16);
@@ -194,13 +193,13 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
         for (int set = 0; set < S::kSets; ++set) {
             const int first = 16 * (set * S::kOutTiles + wave * S::kPer);
             f32x4 acc[S::kPer][MT];
-            if (wave < S::kActive) begin_sums(acc, kBiasFc2 + first);
+            if (S::kActive == NW || wave < S::kActive) begin_sums(acc, kBiasFc2 + first);
 #pragma unroll 1
             for (int k = 0; k < S::kEach; ++k) {
                 const int c = set * S::kEach + k;
                 chunk<G>(acc, w1, w2, c, c == 3);
             }
-            if (wave < S::kActive) {
+            if (S::kActive == NW || wave < S::kActive) {
 #pragma unroll
                 for (int t = 0; t < S::kPer; ++t)
 #pragma unroll
@@ -210,7 +209,6 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
                     }
             }
         }
-        wait_direct();                           // qkv's biases
     }
 
     // a quarter of it: x1 to memory (the first quarter's), the hidden channels' share of the output to `parts`
@@ -336,8 +334,7 @@ part_kernel(LayerArgs a) {
 // Waves on a SIMD.  SPARSE (blocks of 4 or 8 groups before the tile) and dense layers are kernels of their own, so that the
 // former, whose sums never span chunks, run 64 tokens with eight waves of 128 registers: a layer of 64000 tokens 75 -> 70 us,
 // its qkv projection 9 -> 4.5 of a workgroup's 35 us.  Dense layers need the registers for weights that set out four steps
-// ahead (145 -> 134 us); with eight waves of 128 registers they spill 55 and a whole pass takes 3.72 instead of 3.37 ms.  (On
-// four waves 5 to 13 are spilled around the loops; held to two tiles of GELU at a time they are not, and a pass takes 1 % longer.)
+// ahead (145 -> 134 us); with eight waves of 128 registers they spill 55 and a whole pass takes 3.72 instead of 3.37 ms.
 constexpr int layer_waves(int MT, int NW) { return MT == 2 || (MT == 4 && NW == 8) ? 4 : 2; }
 
 // SPLIT: one workgroup to each of q, k and v of a tile (or one where there is no projection behind); the layer before
@@ -354,7 +351,7 @@ layer_kernel(LayerArgs a) {
     const int each = SPLIT && a.qkv ? 3 : 1, mine = each == 3 ? (int)(blockIdx.x % 3u) : 0;
     const int64_t m0 = (int64_t)(blockIdx.x / (uint32_t)each) * (16 * MT);
     const int rows = (int)min((int64_t)(16 * MT), a.M - m0);
-    if (SPLIT || !a.attn) w.stage_qkv_bias();
+    w.stage_qkv_bias();
     if (SPLIT && a.attn) {
         w.join(m0);
         wait_direct();                               // qkv's biases
