@@ -174,7 +174,9 @@ __device__ inline float gelu(float x) {
     float p = kGelu[kDegree];
 #pragma unroll
     for (int k = kDegree - 1; k >= 0; --k) p = __builtin_fmaf(a, p, kGelu[k]);
-    return __builtin_fmaf(-a, __builtin_amdgcn_exp2f(p), __builtin_fmaxf(x, 0.f));
+    // The larger of x and 0 as a median: a maximum takes a second instruction that quiets signalling NaN (which the product does
+    // here); with the compiler's two a pass over 25600 tokens is 1.5 % longer.
+    return __builtin_fmaf(-a, __builtin_amdgcn_exp2f(p), __builtin_amdgcn_fmed3f(x, 0.f, 3.402823466e38f));
 }
 
 }  // namespace enc
