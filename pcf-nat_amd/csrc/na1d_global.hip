@@ -538,7 +538,7 @@ global_dq_kernel(char *__restrict__ dq, float *__restrict__ delta, const char *_
     TrLane<C> tr_lane;
     row_lane.init(0, lane);
     tr_lane.init(0, lane);
-    f32x4 acc[QT][CT];
+    f32x4 acc[QT][CT], minus_dl[QT];    // the product dO . V^T starts at minus delta (dropout: at zero)
     float dl[QT], ref[QT];              // ref: minus the row's LSE in the log2 domain, a padded row's -100 taken out of it
     bool row_masked[QT];
     uint32_t drop_key[QT];
@@ -551,6 +551,8 @@ global_dq_kernel(char *__restrict__ dq, float *__restrict__ delta, const char *_
         ref[h] = (row_masked[h] ? mask2 : 0.f) - lse_row[h] * kLog2e;
         // With dropout mask D (0 or 1/(1-p)): O = (D*P) V, so dP = D * (dO . V^T) and delta = rowsum(dO * O) as before.
         drop_key[h] = DROP ? dropout_row_key((uint64_t)b * T + qrow, a.drop) : 0u;
+        const float from = DROP ? 0.f : -dl[h];
+        minus_dl[h] = f32x4{from, from, from, from};
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) acc[h][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -572,7 +574,7 @@ global_dq_kernel(char *__restrict__ dq, float *__restrict__ delta, const char *_
 #pragma unroll
                     for (int h = 0; h < QT; ++h) {
                         const f32x4 s = dot_rows_mma<DT, C>(kop, qop[h]);
-                        const f32x4 dp = dot_rows_mma<DT, C>(vop, gop[h]);
+                        const f32x4 dp = dot_rows_mma<DT, C>(vop, gop[h], minus_dl[h]);
                         float dsv[4];
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
@@ -581,8 +583,8 @@ global_dq_kernel(char *__restrict__ dq, float *__restrict__ delta, const char *_
                             if constexpr (!kWhole) z += (key >= tv && !row_masked[h]) ? mask2 : 0.f;
                             const float p = kWhole || key < T ? __builtin_amdgcn_exp2f(z) : 0.f;
                             float dpr = dp[r];
-                            if constexpr (DROP) dpr *= dropout_keeps(drop_key[h], key, a.drop) ? a.drop.inv_keep : 0.f;
-                            dsv[r] = p * (dpr - dl[h]);
+                            if constexpr (DROP) dpr = __builtin_fmaf(dpr, dropout_keeps(drop_key[h], key, a.drop) ? a.drop.inv_keep : 0.f, -dl[h]);
+                            dsv[r] = p * dpr;
                         }
                         db[h][2 * j] = Mma<DT>::pack(dsv[0], dsv[1]);
                         db[h][2 * j + 1] = Mma<DT>::pack(dsv[2], dsv[3]);
@@ -635,9 +637,16 @@ global_dq_kernel(char *__restrict__ dq, float *__restrict__ delta, const char *_
 // Backward, key side: dK and dV
 // =============================================================================
 // A workgroup owns 4 * QT key tiles, QT to a wave, whose K and V rows go from memory straight into registers, and
-// walks the queries in chunks of 4 tiles (Q, dO, LSE and delta through LDS, double-buffered).  The score product is
-// taken with Q and K swapped, so that P and dS come out as B operands; dV^T += dO^T P and dK^T += Q^T dS run two
-// query tiles at a time on the 32-deep product.
+// walks the queries in chunks of 4 tiles (Q and dO through LDS, double-buffered).  The score product is taken with Q and
+// K swapped, so that P and dS come out as B operands; dV^T += dO^T P and dK^T += Q^T dS run two query tiles at a time on
+// the 32-deep product.
+// A lane has one key of a tile, so everything else in an exponent is a constant of the query row, of which there are two:
+// minus its LSE in the log2 domain, with a padded row's -100 taken out of it, and the same less 100 for valid rows, which
+// is what padded keys see.  The lane's key decides once where it reads, and no score is masked; rows past the sequence
+// have minus infinity there.  Minus delta is where the product dO . V^T starts (without dropout).
+// With the masks and both subtractions worked out for each score (a general form of the loop beside a plain one), in a trace: 64 x 4
+// sequences of up to 1000 rows, 64 channels 193..203 -> 158..180 us (all rows valid: 177 -> 162), 20 x 8 of 700, 32 channels
+// 42.4 -> 35.2, 8 x 8 of 1500, 128 channels 203 -> 188.
 template <class DT, int C, bool DROP, int QT, bool PACKED>
 __global__ void __launch_bounds__(kThreads)
 global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__restrict__ q, const char *__restrict__ k,
@@ -646,8 +655,8 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
     using LL = Lds<C>;
     constexpr int CT = C / 16;
     constexpr int kStep = region_bytes<C>(kStripTiles);
-    constexpr int kRows = 16 * kStripTiles;                 // rows of a chunk: one lse / delta value each
-    constexpr int kBuf = 2 * kStep + 2 * kRows * 4;         // Q, dO, lse, delta of one chunk
+    constexpr int kRows = 16 * kStripTiles;                 // rows of a chunk
+    constexpr int kBuf = 2 * kStep + 3 * kRows * 4;         // Q, dO and the rows' constants of one chunk
     fetch_args_now(dk, dv, q, k, v, dout, lse, delta, t_valid, items, a.T, a.H, a.strips, a.strips_magic, a.heads_magic,
                    a.scale, a.in.pitch);
     if constexpr (!PACKED) fetch_args_now(a.in.sample, a.in.head, a.in.width, a.outl.sample, a.outl.head, a.outl.pitch);
@@ -675,10 +684,16 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
     auto stage = [&](int c0, LDS_PTR(char) buf) {           // chunk of queries c0 .. c0 + 3 into one buffer
         stage_direct<C, kStripTiles, kReadShared>(qs, 16 * c0, buf, kStripTiles, wave, lane_off, pitch);
         stage_direct<C, kStripTiles, kReadShared>(gs, 16 * c0, buf + kStep, kStripTiles, wave, out_lane_off, out_pitch);
-        if (wave == 0) load_to_lds<4, 0>(ls, buf + 2 * kStep, (16 * c0 + lane) * 4);            // rows past T: zeros
-        if (wave == 1) load_to_lds<4, 0>(ds, buf + 2 * kStep + kRows * 4, (16 * c0 + lane) * 4);
+    };
+    // The constants of the chunk's rows 16 * wave + n: loaded with the chunk, written in front of the barrier it waits for.
+    float row_lse, row_delta;
+    auto load_constants = [&](int c0) {
+        const int at = (16 * (c0 + wave) + n) * 4;          // rows past T: zeros
+        row_lse = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ls, at, 0, 0));
+        row_delta = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ds, at, 0, 0));
     };
     stage(0, buf_lds);
+    load_constants(0);
     int kt_own[QT];                                         // this wave's key tiles
     RowOperand<C> kop[QT], vop[QT];
 #pragma unroll
@@ -696,60 +711,52 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
     row_lane.init(0, lane);
     tr_lane.init(0, lane);
     f32x4 acck[QT][CT], accv[QT][CT];
-    bool keys_count = true;             // all keys of this wave's tiles are valid ones
+    int ref_lane[QT];                   // where a lane's key has its rows' constants, behind Q and dO
 #pragma unroll
     for (int h = 0; h < QT; ++h) {
-        keys_count = keys_count && 16 * kt_own[h] + 16 <= tv;
+        ref_lane[h] = 16 * g + (16 * kt_own[h] + n >= tv ? kRows * 4 : 0);
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) acck[h][ct] = accv[h][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
-    // one chunk of queries; `whole`: all of its 64 rows exist and count, and so do this wave's keys
+    // one chunk of queries; `whole`: all of its four tiles exist
     auto chunk = [&](auto whole, int c0, LDS_PTR(char) buf) {
-        constexpr bool kWhole = decltype(whole)::value;
         LDS_PTR(char) q_lds = buf;
         LDS_PTR(char) g_lds = buf + kStep;
-        LDS_PTR(float) lse_lds = (LDS_PTR(float))(buf + 2 * kStep);
-        LDS_PTR(float) del_lds = lse_lds + kRows;
-        const int nq = kWhole ? kStripTiles : min(kStripTiles, tiles - c0);      // query tiles in this chunk
+        LDS_PTR(char) ref_lds = buf + 2 * kStep;
+        LDS_PTR(char) del_lds = ref_lds + 2 * kRows * 4 + 16 * g;
 #pragma unroll
         for (int qi = 0; qi < kStripTiles; qi += 2) {
-            if (qi >= nq) continue;
+            if (!decltype(whole)::value && c0 + qi >= tiles) continue;
             u32x4 pb[QT], db[QT];
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                if (qi + j < nq) {
-                    RowOperand<C> qop, gop;
-                    read_rows<C>(qop, q_lds + (qi + j) * LL::kTileBytes, row_lane);
-                    read_rows<C>(gop, g_lds + (qi + j) * LL::kTileBytes, row_lane);
-                    const f32x4 lse4 = *reinterpret_cast<LDS_PTR(f32x4)>(lse_lds + 16 * (qi + j) + 4 * g);
-                    const f32x4 del4 = *reinterpret_cast<LDS_PTR(f32x4)>(del_lds + 16 * (qi + j) + 4 * g);
+            for (int j = 0; j < 2; ++j) {                   // a tile past the last has zeros in Q, dO and P
+                RowOperand<C> qop, gop;
+                read_rows<C>(qop, q_lds + (qi + j) * LL::kTileBytes, row_lane);
+                read_rows<C>(gop, g_lds + (qi + j) * LL::kTileBytes, row_lane);
+                const f32x4 del4 = *reinterpret_cast<LDS_PTR(f32x4)>(del_lds + 64 * (qi + j));     // minus delta
 #pragma unroll
-                    for (int h = 0; h < QT; ++h) {
-                        const int key = 16 * kt_own[h] + n;
-                        const f32x4 s = dot_rows_mma<DT, C>(qop, kop[h]);        // [query 4g+r][key n]
-                        const f32x4 dp = dot_rows_mma<DT, C>(gop, vop[h]);
-                        float p[4], dsv[4];
+                for (int h = 0; h < QT; ++h) {
+                    const f32x4 ref = *reinterpret_cast<LDS_PTR(f32x4)>(ref_lds + ref_lane[h] + 64 * (qi + j));
+                    const f32x4 s = dot_rows_mma<DT, C>(qop, kop[h]);        // [query 4g+r][key n]
+                    const f32x4 dp = DROP ? dot_rows_mma<DT, C>(gop, vop[h]) : dot_rows_mma<DT, C>(gop, vop[h], del4);
+                    float p[4], dsv[4];
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
+                    for (int r = 0; r < 4; ++r) {
+                        p[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], scale2, ref[r]));
+                        if constexpr (DROP) {       // dP is masked, and dV takes the probability as the forward used it
                             const int qrow = 16 * (c0 + qi + j) + 4 * g + r;
-                            float z = __builtin_fmaf(s[r], scale2, -kLog2e * lse4[r]);
-                            if constexpr (!kWhole) z += (key >= tv || qrow >= tv) ? mask2 : 0.f;
-                            p[r] = kWhole || qrow < T ? __builtin_amdgcn_exp2f(z) : 0.f;     // rows past the sequence do not exist
-                            float f = 1.f;     // dropout: dP is masked, and dV takes the probability as the forward used it
-                            if constexpr (DROP)
-                                f = dropout_keeps(dropout_row_key((uint64_t)b * T + qrow, a.drop), key, a.drop) ? a.drop.inv_keep : 0.f;
-                            dsv[r] = p[r] * (dp[r] * f - del4[r]);
+                            const float f = dropout_keeps(dropout_row_key((uint64_t)b * T + qrow, a.drop), 16 * kt_own[h] + n, a.drop) ? a.drop.inv_keep : 0.f;
+                            dsv[r] = p[r] * __builtin_fmaf(dp[r], f, del4[r]);
                             p[r] *= f;
+                        } else {
+                            dsv[r] = p[r] * dp[r];
                         }
-                        pb[h][2 * j] = Mma<DT>::pack(p[0], p[1]);
-                        pb[h][2 * j + 1] = Mma<DT>::pack(p[2], p[3]);
-                        db[h][2 * j] = Mma<DT>::pack(dsv[0], dsv[1]);
-                        db[h][2 * j + 1] = Mma<DT>::pack(dsv[2], dsv[3]);
                     }
-                } else {
-#pragma unroll
-                    for (int h = 0; h < QT; ++h) pb[h][2 * j] = pb[h][2 * j + 1] = db[h][2 * j] = db[h][2 * j + 1] = 0u;
+                    pb[h][2 * j] = Mma<DT>::pack(p[0], p[1]);
+                    pb[h][2 * j + 1] = Mma<DT>::pack(p[2], p[3]);
+                    db[h][2 * j] = Mma<DT>::pack(dsv[0], dsv[1]);
+                    db[h][2 * j + 1] = Mma<DT>::pack(dsv[2], dsv[3]);
                 }
             }
             LDS_PTR(char) qtile = q_lds + qi * LL::kTileBytes;
@@ -767,18 +774,25 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
             }
         }
     };
-    const int whole_rows = keys_count ? min(T, tv) : 0;
-    int at = 0;
+    int at = 0;                                             // byte offset of the chunk's buffer: 0 or kBuf
     auto step = [&](auto whole, int c0) {
         wait_direct();
+        const int qrow = 16 * (c0 + wave) + n;
+        float constant = (qrow >= tv || g == 1 ? mask2 : 0.f) - kLog2e * row_lse;
+        if (qrow >= T) constant = kNegInf;
+        if (g >= 2) constant = -row_delta;                  // g 2 and 3 the same
+        *reinterpret_cast<LDS_PTR(float)>(buf_lds + at + 2 * kStep + (min(g, 2) * kRows + 16 * wave + n) * 4) = constant;
         barrier_lds();      // this chunk has landed, and every wave is done with the one before, whose buffer the next takes
-        if (c0 + kStripTiles < tiles) stage(c0 + kStripTiles, buf_lds + (at ^ kBuf));
+        if (c0 + kStripTiles < tiles) {
+            stage(c0 + kStripTiles, buf_lds + (kBuf - at));
+            load_constants(c0 + kStripTiles);
+        }
         chunk(whole, c0, buf_lds + at);
-        at ^= kBuf;
+        at = kBuf - at;
     };
     int c0 = 0;
-    for (; 16 * (c0 + kStripTiles) <= whole_rows; c0 += kStripTiles) step(std::true_type{}, c0);
-    for (; c0 < tiles; c0 += kStripTiles) step(std::false_type{}, c0);
+    for (; c0 + kStripTiles <= tiles; c0 += kStripTiles) step(std::true_type{}, c0);
+    if (c0 < tiles) step(std::false_type{}, c0);
 
     const bool stream = stores_whole_lines(pitch, C, 0);
 #pragma unroll
@@ -816,13 +830,15 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
     if constexpr (DROP) fetch_args_now(a.drop.threshold, a.drop.seed_lo, a.drop.seed_hi, a.drop.inv_keep);
     const int T = a.T, tiles = (T + 15) >> 4, pitch = a.in.pitch, out_pitch = a.outl.pitch, width = a.in.width;
     const int region = region_bytes<C>(tiles);
-    extern __shared__ __attribute__((aligned(16))) char smem[];          // 4 * region + 2 * kRows * 4 bytes
+    extern __shared__ __attribute__((aligned(16))) char smem[];          // 4 * region + 4 * kRows * 4 bytes
     LDS_PTR(char) q_lds = (LDS_PTR(char))smem;
     LDS_PTR(char) g_lds = q_lds + region;                   // dO
     LDS_PTR(char) k_lds = g_lds + region;
     LDS_PTR(char) v_lds = k_lds + region;
-    LDS_PTR(float) lse_lds = (LDS_PTR(float))(v_lds + region);
-    LDS_PTR(float) del_lds = lse_lds + kRows;
+    // A row's constants in an exponent, as valid and as padded keys see it (see global_dkv_kernel), minus its delta, and its LSE.
+    LDS_PTR(float) ref_lds = (LDS_PTR(float))(v_lds + region);
+    LDS_PTR(float) del_lds = ref_lds + 2 * kRows;
+    LDS_PTR(float) lse_lds = del_lds + kRows;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -863,22 +879,27 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
     // ---- queries: delta and dQ -------------------------------------------------------------------------------
     {
         RowOperand<C> qop[QT], gop[QT];
-        float dl[QT], lse2[QT];
+        float ref[QT];
+        bool row_masked[QT];
         uint32_t drop_key[QT];
-        f32x4 acc[QT][CT];
+        f32x4 acc[QT][CT], minus_dl[QT];
 #pragma unroll
         for (int h = 0; h < QT; ++h) {
             const int qrow = 16 * own[h] + n;
             read_rows<C>(qop[h], q_lds + own[h] * LL::kTileBytes, row_lane);
             read_rows<C>(gop[h], g_lds + own[h] * LL::kTileBytes, row_lane);
-            dl[h] = xor_sum(dot_lane<DT, C>(gop[h], oop[h]));       // lane (n, g) holds a quarter of row n's channels
-            lse2[h] = lse_lds[qrow] * kLog2e;
-            if (g == 0) del_lds[qrow] = dl[h];
+            const float dl = xor_sum(dot_lane<DT, C>(gop[h], oop[h]));       // lane (n, g) holds a quarter of row n's channels
+            minus_dl[h] = f32x4{-dl, -dl, -dl, -dl};
+            row_masked[h] = qrow >= tv;
+            const float lse2 = lse_lds[qrow] * kLog2e;
+            ref[h] = (row_masked[h] ? mask2 : 0.f) - lse2;
             // With dropout mask D (0 or 1/(1-p)): O = (D*P) V, so dP = D * (dO . V^T) and delta = rowsum(dO * O) as before.
             drop_key[h] = DROP ? dropout_row_key((uint64_t)b * T + qrow, a.drop) : 0u;
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) acc[h][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (g < 3) ref_lds[g * kRows + qrow] = g == 2 ? -dl : qrow >= T ? kNegInf : g == 1 ? mask2 - lse2 : ref[h];
         }
+        const int plain_keys = 16 * own[0] >= tv ? T : min(T, tv);       // keys without a mask: this wave's first tile is padded, so are the others
 #pragma unroll
         for (int kt = 0; kt < TILES; ++kt) {
             if (kt >= tiles) continue;
@@ -886,20 +907,26 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
             read_rows<C>(kop, k_lds + kt * LL::kTileBytes, row_lane);
             read_rows<C>(vop, v_lds + kt * LL::kTileBytes, row_lane);
             u32x2 db[QT];
+            const bool plain = 16 * (kt + 1) <= plain_keys;
 #pragma unroll
             for (int h = 0; h < QT; ++h) {
-                const bool row_masked = 16 * own[h] + n >= tv;
                 const f32x4 sc = dot_rows_mma<DT, C>(kop, qop[h]);
-                const f32x4 dp = dot_rows_mma<DT, C>(vop, gop[h]);
-                float dsv[4];
+                const f32x4 dp = DROP ? dot_rows_mma<DT, C>(vop, gop[h]) : dot_rows_mma<DT, C>(vop, gop[h], minus_dl[h]);
+                float z[4], dsv[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) z[r] = __builtin_fmaf(sc[r], scale2, ref[h]);
+                if (!plain) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int key = 16 * kt + 4 * g + r;
+                        z[r] = key < T ? z[r] + (key >= tv && !row_masked[h] ? mask2 : 0.f) : kNegInf;     // rows past the sequence do not exist
+                    }
+                }
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int key = 16 * kt + 4 * g + r;
-                    const float z = sc[r] * scale2 - lse2[h] + ((key >= tv || row_masked) ? mask2 : 0.f);
-                    const float p = key < T ? __builtin_amdgcn_exp2f(z) : 0.f;
                     float dpr = dp[r];
-                    if constexpr (DROP) dpr *= dropout_keeps(drop_key[h], key, a.drop) ? a.drop.inv_keep : 0.f;
-                    dsv[r] = p * (dpr - dl[h]);
+                    if constexpr (DROP) dpr = __builtin_fmaf(dpr, dropout_keeps(drop_key[h], 16 * kt + 4 * g + r, a.drop) ? a.drop.inv_keep : 0.f, minus_dl[h][r]);
+                    dsv[r] = __builtin_amdgcn_exp2f(z[r]) * dpr;
                 }
                 db[h] = u32x2{Mma<DT>::pack(dsv[0], dsv[1]), Mma<DT>::pack(dsv[2], dsv[3])};
             }
@@ -921,13 +948,15 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
             store_tile<C>(dqs, (16 * own[h] + n) * pitch, qw, g, stores_whole_lines(pitch, C, 0), width);   // rows past T are dropped
         }
     }
-    barrier_lds();                                          // every row's delta is in LDS
+    barrier_lds();                                          // every row's constants are in LDS
 
     // ---- keys: dK and dV -------------------------------------------------------------------------------------
     RowOperand<C> kop[QT], vop[QT];
     f32x4 acck[QT][CT], accv[QT][CT];
+    int ref_lane[QT];                   // where a lane's key has its rows' constants
 #pragma unroll
     for (int h = 0; h < QT; ++h) {
+        ref_lane[h] = 4 * g + (16 * own[h] + n >= tv ? kRows : 0);
         read_rows<C>(kop[h], k_lds + own[h] * LL::kTileBytes, row_lane);
         read_rows<C>(vop[h], v_lds + own[h] * LL::kTileBytes, row_lane);
 #pragma unroll
@@ -939,26 +968,24 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
         RowOperand<C> qop, gop;
         read_rows<C>(qop, q_lds + qi * LL::kTileBytes, row_lane);
         read_rows<C>(gop, g_lds + qi * LL::kTileBytes, row_lane);
-        const f32x4 lse4 = *reinterpret_cast<LDS_PTR(f32x4)>(lse_lds + 16 * qi + 4 * g);
-        const f32x4 del4 = *reinterpret_cast<LDS_PTR(f32x4)>(del_lds + 16 * qi + 4 * g);
+        const f32x4 del4 = *reinterpret_cast<LDS_PTR(f32x4)>(del_lds + 16 * qi + 4 * g);         // minus delta
         u32x2 pb[QT], db[QT];
 #pragma unroll
         for (int h = 0; h < QT; ++h) {
-            const int key = 16 * own[h] + n;
-            const bool col_masked = key >= tv;
+            const f32x4 ref = *reinterpret_cast<LDS_PTR(f32x4)>(ref_lds + ref_lane[h] + 16 * qi);
             const f32x4 sc = dot_rows_mma<DT, C>(qop, kop[h]);       // [query 4g+r][key n]
-            const f32x4 dp = dot_rows_mma<DT, C>(gop, vop[h]);
+            const f32x4 dp = DROP ? dot_rows_mma<DT, C>(gop, vop[h]) : dot_rows_mma<DT, C>(gop, vop[h], del4);
             float p[4], dsv[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int qrow = 16 * qi + 4 * g + r;
-                const float z = sc[r] * scale2 - lse4[r] * kLog2e + ((col_masked || qrow >= tv) ? mask2 : 0.f);
-                p[r] = qrow < T ? __builtin_amdgcn_exp2f(z) : 0.f;   // rows past the sequence do not exist
-                float f = 1.f;             // dropout: dP is masked, and dV takes the probability as the forward used it
-                if constexpr (DROP)
-                    f = dropout_keeps(dropout_row_key((uint64_t)b * T + qrow, a.drop), key, a.drop) ? a.drop.inv_keep : 0.f;
-                dsv[r] = p[r] * (dp[r] * f - del4[r]);
-                p[r] *= f;
+                p[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[r], scale2, ref[r]));
+                if constexpr (DROP) {      // dP is masked, and dV takes the probability as the forward used it
+                    const float f = dropout_keeps(dropout_row_key((uint64_t)b * T + 16 * qi + 4 * g + r, a.drop), 16 * own[h] + n, a.drop) ? a.drop.inv_keep : 0.f;
+                    dsv[r] = p[r] * __builtin_fmaf(dp[r], f, del4[r]);
+                    p[r] *= f;
+                } else {
+                    dsv[r] = p[r] * dp[r];
+                }
             }
             pb[h] = u32x2{Mma<DT>::pack(p[0], p[1]), Mma<DT>::pack(p[2], p[3])};
             db[h] = u32x2{Mma<DT>::pack(dsv[0], dsv[1]), Mma<DT>::pack(dsv[2], dsv[3])};
@@ -1065,7 +1092,7 @@ int launch_global_bwd(void *dq, void *dk, void *dv, float *delta, const void *q,
     a.outl = byte_strides(outl, g);
     if (g.T <= 16 * kShortTiles) {
         const int tiles_max = g.T <= 64 ? 4 : 8;            // a wave per tile either way
-        const size_t lds = 4 * (size_t)region_bytes<C>((int)(g.T + 15) / 16) + 2 * 16 * tiles_max * sizeof(float);
+        const size_t lds = 4 * (size_t)region_bytes<C>((int)(g.T + 15) / 16) + 4 * 16 * tiles_max * sizeof(float);
         auto go = [&](auto kern) {
             if (!allow_lds(kern, lds)) return (int)NA1D_ERR_LAUNCH;
             note_kernel_as("global_bwd_short_kernel<%s, %d, %s, %d, 1>", DT::tag == NA1D_BF16 ? "BF16" : "FP16", C,
@@ -1090,7 +1117,7 @@ int launch_global_bwd(void *dq, void *dk, void *dv, float *delta, const void *q,
     auto is_whole = [&](const Layout &l) { return l.sample == whole.sample && l.head == whole.head && l.row == whole.row; };
     const bool packed = is_whole(in) && is_whole(outl);
     constexpr size_t dq_lds = 4 * (size_t)region_bytes<C>(kStripTiles);
-    constexpr size_t dkv_lds = 2 * (2 * (size_t)region_bytes<C>(kStripTiles) + 2 * 16 * kStripTiles * sizeof(float));
+    constexpr size_t dkv_lds = 2 * (2 * (size_t)region_bytes<C>(kStripTiles) + 3 * 16 * kStripTiles * sizeof(float));
     auto go = [&](auto dq_kern, auto dkv_kern) {
         if (!allow_lds(dq_kern, dq_lds) || !allow_lds(dkv_kern, dkv_lds)) return (int)NA1D_ERR_LAUNCH;
         // the pair of profiling events, if set, spans both kernels

@@ -82,6 +82,23 @@ def test_padded_keys_count_where_they_outweigh_the_mask(N, H, T, C, strength, dt
     assert torch.isnan(out.view(N, H, T, C)[0, 0, :, 3]).all() and not torch.isnan(out.view(N, H, T, C)[-1, -1, :, 4]).any()
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=["bf16", "fp16"])
+@pytest.mark.parametrize("T,C", [(113, 64), (64, 16), (193, 32), (256, 64)])
+def test_lengths_off_the_tiles(T, C, dtype):
+    """Lengths on and beside the borders of tiles and chunks, where a tile's keys read both sets of row constants."""
+    lengths = [n for n in (0, 1, 15, 16, 17, 63, 64, 65, 127, 129, T - 1, T) if n <= T]
+    N, H = len(lengths), 2
+    q, k, v, do = make_inputs(N * H, T, C, 0, 79, dtype, n=4)
+    t_valid = torch.tensor(lengths, dtype=torch.int32)
+    qd, kd, vd = (t.cuda().requires_grad_(True) for t in (q, k, v))
+    global_attention(qd, kd, vd, H, t_valid=t_valid.cuda(), scale=C ** -0.5).backward(do.cuda())
+    want = O.global_backward(q.float(), k.float(), v.float(), do.float(), C ** -0.5, T - t_valid, H)
+    for n, i in zip(lengths, range(N)):
+        for got, exact in zip((qd.grad, kd.grad, vd.grad), want):
+            part = slice(i * H, (i + 1) * H)
+            assert O.rel_l2(got[part].float(), exact[part]) < TOL[dtype], n
+
+
 def test_global_attention_without_padding_and_without_lse():
     N, H, T, C, dtype = 2, 2, 150, 32, torch.bfloat16
     B = N * H
