@@ -309,6 +309,89 @@ MaybeTensor av(const Tensor &attn, const Tensor &v, int64_t W, int64_t left) {
     return AV::apply(attn, v, W, left, done);
 }
 
+// ------------------------------------------------------------------------------------------------ an encoder layer in training
+// What train.py's node does between its checks and its bookkeeping.  A layer is some two dozen allocations and a dozen
+// launches each way: through the interpreter they took longer than the kernels of a small batch.
+void refuse(int64_t status, const char *name) {             // called by Python
+    if (status >= 0) return;
+    PyErr_Format(error_class, "%s failed: %s (status %d)", name, na1d_status_string((int)status), (int)status);
+    throw pybind11::error_already_set();
+}
+// (dtype, dim, hidden, heads, window, left, dilation, groups, ordered, scale, late), as the struct has them
+na1d_train_layer layer_of(const pybind11::tuple &geom) {
+    na1d_train_layer l{};
+    int32_t *const numbers[] = {&l.dtype, &l.dim, &l.hidden, &l.heads, &l.window, &l.left, &l.dilation, &l.groups, &l.ordered};
+    for (int i = 0; i < 9; ++i) *numbers[i] = geom[i].cast<int32_t>();
+    l.scale = geom[9].cast<float>();
+    l.late = geom[10].cast<int32_t>();
+    return l;
+}
+const float *floats(const Tensor &t) { return static_cast<const float *>(t.data_ptr()); }
+const float *floats(const MaybeTensor &t) { return t ? floats(*t) : nullptr; }
+
+// params: rpb or linear_pos' weight, weight and bias of the norms, of qkv, proj, fc1, fc2; state: running mean, running
+// variance and batches of the norms; numbers: their momentum and eps.  Returns the output and what a backward reads.
+std::pair<Tensor, Tensor> train_forward(const Tensor &x, const MaybeTensor &by_channel, const pybind11::tuple &geom, const std::vector<Tensor> &state,
+                                        const std::vector<double> &numbers, const MaybeTensor &scale_attn, const MaybeTensor &scale_mlp, const MaybeTensor &pos,
+                                        const std::vector<Tensor> &params) {
+    na1d_train_layer l = layer_of(geom);
+    const int64_t N = x.size(0), T = x.size(1), dim = x.size(2);
+    for (int i = 0; i < 2; ++i) {
+        l.norm[i].weight = floats(params[1 + 2 * i]);
+        l.norm[i].bias = floats(params[2 + 2 * i]);
+        l.norm[i].batches = static_cast<int64_t *>(state[3 * i + 2].data_ptr());
+        l.norm[i].eps = (float)numbers[2 * i + 1];
+    }
+    for (int i = 0; i < 4; ++i) l.w[i] = floats(params[5 + 2 * i]), l.b[i] = floats(params[6 + 2 * i]);
+    (pos ? l.w[4] : l.rpb) = floats(params[0]);
+    l.pos = pos ? pos->data_ptr() : nullptr;
+    l.scale_attn = floats(scale_attn), l.scale_mlp = floats(scale_mlp);
+    const c10::DeviceGuard guard(x.device());
+    void *const stream = stream_of(x);
+    const int64_t saved_bytes = na1d_train_layer_saved_bytes(&l, N, T), ws_bytes = na1d_train_layer_workspace_bytes(&l, N, T, 0);
+    refuse(std::min(saved_bytes, ws_bytes), "na1d_train_layer_saved_bytes");
+    const auto bytes = x.options().dtype(at::kByte);
+    const Tensor out = at::empty_like(x), saved = at::empty({saved_bytes}, bytes), ws = at::empty({ws_bytes}, bytes);
+    Tensor of = by_channel ? *by_channel : at::empty({N, dim, T}, x.options());
+    if (!by_channel) refuse(na1d_train_to_channels(&l, of.data_ptr(), x.data_ptr(), N, T, stream), "na1d_train_to_channels");
+    const Tensor x1 = at::empty({N, dim, T}, x.options());
+    std::tuple<Tensor, Tensor> stats[2];                    // until the kernels that read them are launched
+    for (int part = 0; part < 2; ++part) {
+        stats[part] = at::batch_norm_update_stats(part ? x1 : of, state[3 * part], state[3 * part + 1], numbers[2 * part]);
+        l.norm[part].batch_mean = floats(std::get<0>(stats[part])), l.norm[part].batch_var = floats(std::get<1>(stats[part]));
+        refuse(na1d_train_layer_forward(&l, part, (part ? out : x1).data_ptr(), x.data_ptr(), saved.data_ptr(), saved_bytes, ws.data_ptr(), ws_bytes, N, T, stream),
+               "na1d_train_layer_forward");
+    }
+    for (const Tensor &t : state) t.unsafeGetTensorImpl()->bump_version();
+    return {out, saved};
+}
+// The gradients of x and of the parameters, in train_forward's order.
+std::vector<Tensor> train_backward(const Tensor &given, const Tensor &x, const Tensor &saved, const pybind11::tuple &geom, const MaybeTensor &rpb, const Tensor &n1w,
+                                   const Tensor &n2w, const MaybeTensor &scale_attn, const MaybeTensor &scale_mlp, const MaybeTensor &pos,
+                                   const std::vector<std::vector<int64_t>> &shapes) {
+    na1d_train_layer l = layer_of(geom);
+    const int64_t N = x.size(0), T = x.size(1);
+    const c10::DeviceGuard guard(x.device());
+    Tensor dout = given.contiguous();
+    if ((uintptr_t)dout.data_ptr() % 16) dout = dout.clone();
+    const auto fp32 = x.options().dtype(at::kFloat);
+    std::vector<Tensor> grads{at::empty_like(x), pos ? at::empty(shapes[0], fp32) : at::zeros(shapes[0], fp32)};      // the scores' bias gradient is added to
+    for (size_t i = 1; i < shapes.size(); ++i) grads.push_back(at::empty(shapes[i], fp32));
+    auto grad = [&](int i) { return static_cast<float *>(grads[1 + i].data_ptr()); };
+    for (int i = 0; i < 4; ++i) l.dw[i] = grad(5 + 2 * i), l.db[i] = grad(6 + 2 * i);
+    (pos ? l.dw[4] : l.drpb) = grad(0);
+    l.norm[0].weight = floats(n1w), l.norm[1].weight = floats(n2w);
+    for (int i = 0; i < 2; ++i) l.norm[i].dweight = grad(1 + 2 * i), l.norm[i].dbias = grad(2 + 2 * i);
+    l.rpb = floats(rpb), l.pos = pos ? pos->data_ptr() : nullptr;
+    l.scale_attn = floats(scale_attn), l.scale_mlp = floats(scale_mlp);
+    const int64_t ws_bytes = na1d_train_layer_workspace_bytes(&l, N, T, 1);
+    refuse(ws_bytes, "na1d_train_layer_workspace_bytes");
+    const Tensor ws = at::empty({ws_bytes}, x.options().dtype(at::kByte));
+    refuse(na1d_train_layer_backward(&l, grads[0].data_ptr(), dout.data_ptr(), x.data_ptr(), saved.data_ptr(), saved.numel(), ws.data_ptr(), ws_bytes, N, T, stream_of(x)),
+           "na1d_train_layer_backward");
+    return grads;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -318,4 +401,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("dense", &dense);
     m.def("qk", &qk);
     m.def("av", &av);
+    m.def("train_forward", &train_forward);
+    m.def("train_backward", &train_backward);
 }

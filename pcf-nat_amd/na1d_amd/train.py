@@ -12,7 +12,6 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 from torch.autograd.function import once_differentiable
-from torch.autograd.graph import increment_version
 
 from . import _lib
 
@@ -29,83 +28,37 @@ class _Layer(ctypes.Structure):                    # na1d_train_layer
                 + [(n, _P) for n in "rpb drpb pos scale_attn scale_mlp".split()])
 
 
-def _ptr(t):
-    return None if t is None else t.data_ptr()
-
-
-def _ptrs(ts):
-    return (_P * 5)(*map(_ptr, ts))
-
-
 def _aligned(t):
     t = t.contiguous()
     return t.clone() if t.data_ptr() % 16 else t
 
 
 class _TrainLayer(torch.autograd.Function):
+    """The node's bookkeeping; allocations and launches are ``train_forward`` and ``train_backward`` of ``csrc/na1d_torch.cpp``."""
+
     @staticmethod
-    def forward(ctx, x, by_channel, geom, norms, scales, pos, extra, n1w, n1b, n2w, n2b, wq, bq, wp, bp, w1, b1, w2, b2):
-        lib = _lib.load()
-        n, t, dim = x.shape
-        dense = pos is not None                     # extra: linear_pos' weight, or the bias of a window's scores
-        weights, biases = (wq, wp, w1, w2, extra if dense else None), (bq, bp, b1, b2)
-        c = _Layer(*geom)
-        c.w, c.b = _ptrs(weights), _ptrs(biases)
-        for to, bn, w, b in zip(c.norm, norms, (n1w, n2w), (n1b, n2b)):
-            to.weight, to.bias, to.eps, to.batches = w.data_ptr(), b.data_ptr(), bn.eps, bn.num_batches_tracked.data_ptr()
-        c.rpb, c.pos, c.scale_attn, c.scale_mlp = None if dense else extra.data_ptr(), _ptr(pos), _ptr(scales[0]), _ptr(scales[1])
-        ref = ctypes.byref(c)
-        out = torch.empty_like(x)
-        with torch.cuda.device(x.device):
-            stream = torch.cuda.current_stream().cuda_stream
-            sizes = lib.na1d_train_layer_saved_bytes(ref, n, t), lib.na1d_train_layer_workspace_bytes(ref, n, t, 0)
-            _lib.check(min(*sizes, 0), "na1d_train_layer_saved_bytes")
-            saved, ws = (torch.empty(s, dtype=torch.uint8, device=x.device) for s in sizes)
-            if by_channel is None:
-                by_channel = x.new_empty((n, dim, t))
-                _lib.check(lib.na1d_train_to_channels(ref, by_channel.data_ptr(), x.data_ptr(), n, t, stream), "na1d_train_to_channels")
-            x1 = x.new_empty((n, dim, t))
-            for part, (of, to) in enumerate(((by_channel, x1), (x1, out))):
-                stats = torch.batch_norm_update_stats(of, norms[part].running_mean, norms[part].running_var, norms[part].momentum)
-                c.norm[part].batch_mean, c.norm[part].batch_var = map(_ptr, stats)
-                _lib.check(lib.na1d_train_layer_forward(ref, part, to.data_ptr(), x.data_ptr(), saved.data_ptr(), sizes[0], ws.data_ptr(),
-                                                        sizes[1], n, t, stream), "na1d_train_layer_forward")
-        increment_version([b for bn in norms for b in (bn.running_mean, bn.running_var, bn.num_batches_tracked)])
-        ctx.save_for_backward(x, saved, pos, None if dense else extra, n1w, n2w, *scales)
-        ctx.late = c.late
-        ctx.geom, ctx.shapes = geom, [p.shape for p in (extra, n1w, n1b, n2w, n2b, wq, bq, wp, bp, w1, b1, w2, b2)]
+    def forward(ctx, x, by_channel, geom, nodes, norms, scales, pos, *params):
+        state = [bn._buffers[name] for bn in norms for name in ("running_mean", "running_var", "num_batches_tracked")]
+        out, saved = nodes.train_forward(x, by_channel, geom, state, [v for bn in norms for v in (bn.momentum, bn.eps)], *scales, pos, params)
+        ctx.save_for_backward(x, saved, pos, params[0] if pos is None else None, params[1], params[3], *scales)
+        ctx.late, ctx.geom, ctx.nodes = geom[-1], geom, nodes
+        ctx.shapes = [p.shape for p in params]
         return out
 
     @staticmethod
     @once_differentiable
     def backward(ctx, dout):
-        lib = _lib.load()
         x, saved, pos, rpb, n1w, n2w, *scales = ctx.saved_tensors
-        n, t, dim = x.shape
-        dout = _aligned(dout)
-        dx = torch.empty_like(x)
-        grads = [torch.zeros(ctx.shapes[0], dtype=torch.float32, device=x.device)]       # the bias of the scores is added to
-        grads += [torch.empty(s, dtype=torch.float32, device=x.device) for s in ctx.shapes[1:]]
-        c = _Layer(*ctx.geom)
-        c.dw, c.db = _ptrs(grads[5::2] + ([] if pos is None else grads[:1])), _ptrs(grads[6::2])
-        for to, w, dw, db in zip(c.norm, (n1w, n2w), grads[1:5:2], grads[2:5:2]):
-            to.weight, to.dweight, to.dbias = w.data_ptr(), dw.data_ptr(), db.data_ptr()
-        c.rpb, c.drpb, c.pos, c.scale_attn, c.scale_mlp = _ptr(rpb), grads[0].data_ptr(), _ptr(pos), _ptr(scales[0]), _ptr(scales[1])
-        ref = ctypes.byref(c)
-        with torch.cuda.device(x.device):
-            nbytes = lib.na1d_train_layer_workspace_bytes(ref, n, t, 1)
-            _lib.check(min(nbytes, 0), "na1d_train_layer_workspace_bytes")
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-            _lib.check(lib.na1d_train_layer_backward(ref, dx.data_ptr(), dout.data_ptr(), x.data_ptr(), saved.data_ptr(), saved.numel(),
-                                                     ws.data_ptr(), nbytes, n, t, torch.cuda.current_stream().cuda_stream),
-                       "na1d_train_layer_backward")
-        return (dx, None, None, None, None, None, *(g if need else None for g, need in zip(grads, ctx.needs_input_grad[6:])))
+        dx, *grads = ctx.nodes.train_backward(dout, x, saved, ctx.geom, rpb, n1w, n2w, *scales, pos, ctx.shapes)
+        return (dx, None, None, None, None, None, None, *(g if need else None for g, need in zip(grads, ctx.needs_input_grad[7:])))
 
 
 def plain(m, *classes):
     """Whether calling module ``m`` runs the forward of its class and nothing else."""
-    return (type(m) in classes and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
-            and "forward" not in m.__dict__)
+    if type(m) not in classes:
+        return False
+    d = m.__dict__
+    return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"] or "forward" in d)
 
 
 def plain_call(x):
@@ -117,9 +70,10 @@ def plain_call(x):
 
 
 def _norm_fits(bn, dim, device):
+    mean, var, batches = (bn._buffers.get(name) for name in ("running_mean", "running_var", "num_batches_tracked"))
     return (bn.training and bn.track_running_stats and bn.affine and bn.momentum is not None and bn.num_features == dim
-            and all(s is not None and s.dtype == torch.float32 and s.device == device and s.shape == (dim,) for s in (bn.running_mean, bn.running_var))
-            and bn.num_batches_tracked is not None and bn.num_batches_tracked.dtype == torch.int64 and bn.num_batches_tracked.device == device)
+            and all(s is not None and s.dtype == torch.float32 and s.device == device and s.shape == (dim,) for s in (mean, var))
+            and batches is not None and batches.dtype == torch.int64 and batches.device == device)
 
 
 def _drop_path_scale(m, x):
@@ -138,16 +92,25 @@ def layer(m, x, pos_emb=None, attn_mask_global=None):
     if not (x.is_cuda and m.training and torch.is_grad_enabled() and torch.is_autocast_enabled("cuda")
             and x.dim() == 3 and x.dtype in (torch.bfloat16, torch.float16) and x.dtype == torch.get_autocast_dtype("cuda")):
         return None
-    a, mlp = m.attn, m.mlp
+    nodes = _lib.nodes()
+    if nodes is None:
+        return None
+    # Sixteen layers a step, some forty lookups each: by the modules' own dictionaries, past nn.Module.__getattr__.
+    parts = m._modules
+    a, mlp, norms = parts.get("attn"), parts.get("mlp"), (parts.get("norm1"), parts.get("norm2"))
     cf = getattr(a, "channels_first", False)
     linear, norm = (M.Conv1x1, M.BatchNorm1d) if cf else (M.TokenLinear, M.TokenBatchNorm)
-    if not (plain_call(x) and plain(a, M.NAttention if m.local else M.GlobalAttention) and plain(mlp, M.Mlp) and plain(m.norm1, norm) and plain(m.norm2, norm)
-            and plain(m.drop_path, nn.Identity, M.DropPath) and plain(mlp.act, nn.GELU) and mlp.act.approximate == "none"
-            and plain(mlp.drop, nn.Dropout) and plain(a.proj_drop, nn.Dropout)
-            and all(plain(p, linear) for p in (a.qkv, a.proj, mlp.fc1, mlp.fc2))):
+    if not (plain_call(x) and plain(a, M.NAttention if m.local else M.GlobalAttention) and plain(mlp, M.Mlp) and plain(norms[0], norm) and plain(norms[1], norm)
+            and plain(parts.get("drop_path"), nn.Identity, M.DropPath)):
         return None
-    norms = (m.norm1, m.norm2) if cf else (m.norm1.norm, m.norm2.norm)
-    if (a.na != "fused_qkv" if m.local else a.dense != "native") or a.attn_drop or not a.training or a.proj_drop.p or mlp.drop.p or (not cf and not all(plain(b, M.BatchNorm1d) for b in norms)):
+    in_a, in_mlp = a._modules, mlp._modules
+    act, drops, projections = in_mlp.get("act"), (in_mlp.get("drop"), in_a.get("proj_drop")), [in_a.get("qkv"), in_a.get("proj"), in_mlp.get("fc1"), in_mlp.get("fc2")]
+    if not (plain(act, nn.GELU) and act.approximate == "none" and plain(drops[0], nn.Dropout) and plain(drops[1], nn.Dropout)
+            and all(plain(p, linear) for p in projections)):
+        return None
+    if not cf:
+        norms = [b._modules.get("norm") for b in norms]
+    if (a.na != "fused_qkv" if m.local else a.dense != "native") or a.attn_drop or not a.training or drops[0].p or drops[1].p or (not cf and not all(plain(b, M.BatchNorm1d) for b in norms)):
         return None
     xt = x.transpose(1, 2) if cf else x
     if xt.is_contiguous() and xt.data_ptr() % 16:
@@ -155,22 +118,23 @@ def layer(m, x, pos_emb=None, attn_mask_global=None):
     n, t, dim = xt.shape
     if (t != a.attn_mask.shape[-2] if m.local else attn_mask_global is not None) or not all(_norm_fits(b, dim, x.device) for b in norms):
         return None
-    projections = [a.qkv, a.proj, mlp.fc1, mlp.fc2]
     pos = None
     if not m.local:
+        linear_pos = in_a.get("linear_pos")
         if (pos_emb is None or type(pos_emb) is not torch.Tensor or pos_emb.requires_grad or pos_emb.device != x.device
-                or pos_emb.shape != ((1, dim, t) if cf else (1, t, dim)) or not plain(a.linear_pos, linear) or a.linear_pos.bias is not None):
+                or pos_emb.shape != ((1, dim, t) if cf else (1, t, dim)) or not plain(linear_pos, linear) or linear_pos.bias is not None):
             return None
-        projections.append(a.linear_pos)
+        projections.append(linear_pos)
     groups = {getattr(p, "groups", 1) for p in projections}
-    params = (a.relative_position_bias if m.local else a.linear_pos.weight, norms[0].weight, norms[0].bias, norms[1].weight, norms[1].bias, a.qkv.weight, a.qkv.bias,
-              a.proj.weight, a.proj.bias, mlp.fc1.weight, mlp.fc1.bias, mlp.fc2.weight, mlp.fc2.bias)
-    hidden = mlp.fc1.weight.shape[0]
-    sizes = (3 * dim, dim, dim, dim, hidden, dim, dim, hidden)
-    if len(groups) != 1 or any(p is None or type(p) is not nn.Parameter or p.dtype != torch.float32 or p.device != x.device
+    params = [a.relative_position_bias if m.local else linear_pos.weight]
+    for p in (*norms, *projections[:4]):
+        params += p._parameters.get("weight"), p._parameters.get("bias")
+    device = x.device
+    if len(groups) != 1 or any(p is None or type(p) is not nn.Parameter or p.dtype != torch.float32 or p.device != device
                                or not p.is_contiguous() or p.data_ptr() % 16 for p in params):
         return None
-    groups = groups.pop()
+    hidden, groups = params[9].shape[0], groups.pop()
+    sizes = (3 * dim, dim, dim, dim, hidden, dim, dim, hidden)
     if any(p.numel() != o * i // groups for p, o, i in zip(params[5::2], sizes[::2], sizes[1::2])):
         return None
     if params[0].numel() != (a.num_heads * a.win_size if m.local else dim * dim // groups):
@@ -188,8 +152,8 @@ def layer(m, x, pos_emb=None, attn_mask_global=None):
     xt = xt.contiguous()
     if not m.local:
         pos = _aligned((pos_emb.transpose(1, 2) if cf else pos_emb).to(x.dtype))
-    scales = (_drop_path_scale(m.drop_path, xt), _drop_path_scale(m.drop_path, xt))
-    out = _TrainLayer.apply(xt, by_channel, geom, norms, scales, pos, *params)
+    scales = (_drop_path_scale(parts.get("drop_path"), xt), _drop_path_scale(parts.get("drop_path"), xt))
+    out = _TrainLayer.apply(xt, by_channel, geom, nodes, norms, scales, pos, *params)
     return out.transpose(1, 2) if cf else out
 
 
