@@ -183,9 +183,126 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
         else
             ring.begin(S::fc1(w1, last ? 0 : c + 1, wave), lane16);
     }
+    // The rest of a layer of 8 or 4 groups, whose channels never meet before the next projection: a group is one wave's, or two
+    // waves' that halve the tokens, from the output projection to x2, without a barrier.  Of every 32 hidden channels lane
+    // (n, g) of two tiles' sums gets channels 8g .. 8g+3 and 8g+4 .. 8g+7 of token n (fc1's rows are taken in that order),
+    // which rounded are the next product's operand as they stand.  Four groups' weights are read by two waves each, 0.6 MB
+    // for 64 tokens, in the shadow of GELU, which bounds it (64 tokens alone on a CU: the layer's rest 15.6 -> 9 us).  In chunks of 256
+    // hidden channels through LDS, all waves together: 16400 tokens 32.8 -> 30.7 us with 8 groups, 38.9 -> 35.2 with 4; 64000: 69.6 -> 65.8,
+    // 81.4 -> 76.8.
+    template <int G> __device__ inline void tail_of_groups() {
+        static_assert(NW == 8 && (G == 8 || (G == 4 && MT % 2 == 0)), "a group to a wave, or to two");
+        constexpr int kOut = G == 8 ? 2 : 4, kSteps = kOut / 2, kTok = G == 8 ? MT : MT / 2, kBlocks = 2 * kOut;     // tiles and steps of a group's channels; its hidden channels in blocks of 32
+        constexpr int kAhead = MT == 4 ? 1 : G == 8 ? 4 : 2;               // blocks whose weights are on their way
+        const int group = G == 8 ? wave : wave >> 1, i0 = G == 8 ? 0 : (wave & 1) * kTok;
+        const Rsrc wp = weight_rsrc(a.w_proj, kDim, kDim), w1 = weight_rsrc(a.w_fc1, kHidden, kDim), w2 = weight_rsrc(a.w_fc2, kDim, kHidden);
+        auto load = [](Rsrc w, int at, int frag) { return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w, at, frag * kFrag, 0)); };
+        int hidden_lane[2];                      // a lane's place in the two fragments of 32 rows of fc1
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int row = 8 * (n >> 2) + (n & 3) + 4 * t;
+            hidden_lane[t] = (row >> 4) * (kDim / 32) * kFrag + (g * 16 + (row & 15)) * 16;
+        }
+        u32x4 p_w[kSteps][kOut], fc1_w[kAhead][kSteps][2], fc2_w[kAhead][kOut];
+        auto fill1 = [&](int slot, int b) {
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) fc1_w[slot][s][t] = load(w1, hidden_lane[t], (2 * kBlocks * group + 2 * b) * (kDim / 32) + kSteps * group + s);
+        };
+        auto fill2 = [&](int slot, int b) {
+#pragma unroll
+            for (int j = 0; j < kOut; ++j) fc2_w[slot][j] = load(w2, lane16, (kOut * group + j) * (kHidden / 32) + kBlocks * group + b);
+        };
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+            for (int j = 0; j < kOut; ++j) p_w[s][j] = load(wp, lane16, (kOut * group + j) * (kDim / 32) + kSteps * group + s);
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) fill1(u, u), fill2(u, u);
+        wait_direct();
+        barrier_lds();
+        const int x_lane = operand_lane(n, g);
+        u32x4 x[kSteps][kTok];
+        auto read = [&](LDS_PTR(char) tile) {
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+                for (int i = 0; i < kTok; ++i) x[s][i] = *reinterpret_cast<LDS_PTR(u32x4)>(tile + (x_lane ^ 64 * (kSteps * group + s)) + (i0 + i) * 16 * kRow);
+        };
+        f32x4 acc[kOut][kTok];
+        auto begin = [&](int bias_at) {
+#pragma unroll
+            for (int j = 0; j < kOut; ++j) {
+                const f32x4 b = staged_bias(bias_at + 16 * (kOut * group + j));
+#pragma unroll
+                for (int i = 0; i < kTok; ++i) acc[j][i] = b;
+            }
+        };
+        auto add_to_x = [&] {
+#pragma unroll
+            for (int j = 0; j < kOut; ++j)
+#pragma unroll
+                for (int i = 0; i < kTok; ++i) {
+                    LDS_PTR(u32x2) to = at(q_lds, 16 * (kOut * group + j), i0 + i);
+                    *to = narrow4<DT>(acc[j][i] + widen4<DT>(*to));
+                }
+        };
+        read(p_lds);
+        begin(kBiasProj);
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+            for (int j = 0; j < kOut; ++j)
+#pragma unroll
+                for (int i = 0; i < kTok; ++i) acc[j][i] = Mma<DT>::k32(p_w[s][j], x[s][i], acc[j][i]);
+        add_to_x();
+        read(q_lds);                             // a wave's LDS operations keep their order
+        begin(kBiasFc2);
+#pragma unroll 1
+        for (int b0 = 0; b0 < kBlocks; b0 += kAhead) {
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int b = b0 + u, next = min(b + kAhead, kBlocks - 1);
+                f32x4 hid[2][kTok];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const f32x4 from = *reinterpret_cast<LDS_PTR(f32x4)>(b_lds + kBiasFc1 + 32 * (kBlocks * group + b) + 8 * g + 4 * t);
+#pragma unroll
+                    for (int i = 0; i < kTok; ++i) hid[t][i] = from;
+                }
+#pragma unroll
+                for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+#pragma unroll
+                        for (int i = 0; i < kTok; ++i) hid[t][i] = Mma<DT>::k32(fc1_w[u][s][t], x[s][i], hid[t][i]);
+                fill1(u, next);
+                __builtin_amdgcn_sched_barrier(0x406);       // see multiply()
+                u32x4 h[kTok];
+#pragma unroll
+                for (int i = 0; i < kTok; ++i) {
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) hid[t][i][r] = gelu(hid[t][i][r]);
+                    const u32x2 lo = narrow4<DT>(hid[0][i]), hi = narrow4<DT>(hid[1][i]);
+                    h[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
+                }
+#pragma unroll
+                for (int j = 0; j < kOut; ++j)
+#pragma unroll
+                    for (int i = 0; i < kTok; ++i) acc[j][i] = Mma<DT>::k32(fc2_w[u][j], h[i], acc[j][i]);
+                fill2(u, next);
+                __builtin_amdgcn_sched_barrier(0x406);
+            }
+        }
+        add_to_x();
+    }
     // the rest of the layer: -> x2 in q_lds
     template <int G> __device__ inline void tail() {
         using S = Groups<G, NW>;
+        if constexpr (G == 8 || (G == 4 && MT % 2 == 0)) return tail_of_groups<G>();
         const Rsrc w1 = weight_rsrc(a.w_fc1, kHidden, kDim), w2 = weight_rsrc(a.w_fc2, kDim, kHidden);
         project<G>(w1, 0);
         // Outputs that a later chunk adds nothing to are written at once, over x1: the chunks behind read other channels.
