@@ -388,6 +388,11 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
             }
     }
 
+    // How a head's rows go to memory.  A launch that is one round of workgroups writes them all at its end and then waits for what
+    // the L2s still hold; streamed, they leave at once (five layers and their attentions, us in a trace: 4000 tokens 127 -> 124,
+    // 6400: 141 -> 132, 10000: 198 -> 192, 12800: 205 -> 204, 16300: 233 -> 234).  With more tokens the attention behind loses what
+    // it would find there (25600: 11 -> 12.8 each), and of few nothing is left to wait for.
+    static constexpr int kQkvAux = !SPLIT && MT <= 2 ? kStoreAux : 0;
     template <int G> __device__ inline void head(int64_t m0, int rows, int from, int to) {
         using S = Groups<G, NW>;
         const Rsrc w = weight_rsrc(a.w_qkv, 3 * kDim, kDim);
@@ -406,7 +411,7 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
                 for (int i = 0; i < MT; ++i) o[i][j] = narrow4<DT>(acc[j][i]);
 #pragma unroll
             for (int i = 0; i < MT; ++i)
-                store_tile<CW, 0>(qs, (16 * i + n) * (3 * kRow) + which * kRow + 2 * CW * wave, o[i], g, 2 * CW);
+                store_tile<CW, kQkvAux>(qs, (16 * i + n) * (3 * kRow) + which * kRow + 2 * CW * wave, o[i], g, 2 * CW);
         }
     }
 
