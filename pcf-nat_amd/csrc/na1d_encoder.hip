@@ -46,6 +46,7 @@ struct LayerArgs {
     int x_in_pitch, block_pitch, patch_width, M, T;
     uint32_t T_magic;
     int tail_groups, head_groups;     // block-diagonal weights: 8, 4, 2; otherwise 1
+    int large;                        // layer_kernel with three row tiles: the first so many workgroups have them, the others two
     char *x1;                         // split layers (part_kernel): [M, 256] ...
     float *parts;                     // ... and what each quarter of the hidden channels adds, [4, M, 256]
 };
@@ -98,7 +99,7 @@ template <int MT> constexpr size_t layer_lds() { return (size_t)2 * 16 * MT * kR
 // The number of groups as the kernels know it: every switch over it and every sum over its parts starts from this.
 inline int known_groups(int groups) { return groups == 2 || groups == 4 || groups == 8 ? groups : 1; }
 
-template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
+template <class DT, int MT, int NW, int PF, bool SPLIT, int QKV_AUX> struct LayerWave {
     static constexpr int NTW = 16 / NW, CW = 16 * NTW;
     const LayerArgs &a;
     LDS_PTR(char) p_lds;
@@ -190,11 +191,11 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
     // for 64 tokens, in the shadow of GELU, which bounds it (64 tokens alone on a CU: the layer's rest 15.6 -> 9 us).  In chunks of 256
     // hidden channels through LDS, all waves together: 16400 tokens 32.8 -> 30.7 us with 8 groups, 38.9 -> 35.2 with 4; 64000: 69.6 -> 65.8,
     // 81.4 -> 76.8.
-    template <int G> __device__ inline void tail_of_groups() {
-        static_assert(NW == 8 && (G == 8 || (G == 4 && MT % 2 == 0)), "a group to a wave, or to two");
-        constexpr int kOut = G == 8 ? 2 : 4, kSteps = kOut / 2, kTok = G == 8 ? MT : MT / 2, kBlocks = 2 * kOut;     // tiles and steps of a group's channels; its hidden channels in blocks of 32
-        constexpr int kAhead = MT == 4 ? 1 : G == 8 ? 4 : 2;               // blocks whose weights are on their way
-        const int group = G == 8 ? wave : wave >> 1, i0 = G == 8 ? 0 : (wave & 1) * kTok;
+    template <int G, int kTok> __device__ inline void tail_of_groups(int i0) {
+        static_assert(NW == 8 && (G == 8 || G == 4), "a group to a wave, or to two");
+        constexpr int kOut = G == 8 ? 2 : 4, kSteps = kOut / 2, kBlocks = 2 * kOut;     // tiles and steps of a group's channels; its hidden channels in blocks of 32
+        constexpr int kAhead = MT > 2 ? 1 : G == 8 ? 4 : 2;                // blocks whose weights are on their way
+        const int group = G == 8 ? wave : wave >> 1;
         const Rsrc wp = weight_rsrc(a.w_proj, kDim, kDim), w1 = weight_rsrc(a.w_fc1, kHidden, kDim), w2 = weight_rsrc(a.w_fc2, kDim, kHidden);
         auto load = [](Rsrc w, int at, int frag) { return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w, at, frag * kFrag, 0)); };
         int hidden_lane[2];                      // a lane's place in the two fragments of 32 rows of fc1
@@ -302,7 +303,14 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
     // the rest of the layer: -> x2 in q_lds
     template <int G> __device__ inline void tail() {
         using S = Groups<G, NW>;
-        if constexpr (G == 8 || (G == 4 && MT % 2 == 0)) return tail_of_groups<G>();
+        if constexpr (G == 8) return tail_of_groups<8, MT>(0);
+        if constexpr (G == 4 && MT % 2 == 0) return tail_of_groups<4, MT / 2>((wave & 1) * MT / 2);
+        if constexpr (G == 4 && MT == 3) {       // two and one; waves w and w + 4 share a SIMD
+            if ((wave ^ wave >> 2) & 1)
+                return tail_of_groups<4, 1>(2);
+            else
+                return tail_of_groups<4, 2>(0);
+        }
         const Rsrc w1 = weight_rsrc(a.w_fc1, kHidden, kDim), w2 = weight_rsrc(a.w_fc2, kDim, kHidden);
         project<G>(w1, 0);
         // Outputs that a later chunk adds nothing to are written at once, over x1: the chunks behind read other channels.
@@ -388,11 +396,10 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
             }
     }
 
-    // How a head's rows go to memory.  A launch that is one round of workgroups writes them all at its end and then waits for what
+    // QKV_AUX: how a head's rows go to memory.  A launch that is one round of workgroups writes them all at its end and then waits for what
     // the L2s still hold; streamed, they leave at once (five layers and their attentions, us in a trace: 4000 tokens 127 -> 124,
     // 6400: 141 -> 132, 10000: 198 -> 192, 12800: 205 -> 204, 16300: 233 -> 234).  With more tokens the attention behind loses what
     // it would find there (25600: 11 -> 12.8 each), and of few nothing is left to wait for.
-    static constexpr int kQkvAux = !SPLIT && MT <= 2 ? kStoreAux : 0;
     template <int G> __device__ inline void head(int64_t m0, int rows, int from, int to) {
         using S = Groups<G, NW>;
         const Rsrc w = weight_rsrc(a.w_qkv, 3 * kDim, kDim);
@@ -411,7 +418,7 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
                 for (int i = 0; i < MT; ++i) o[i][j] = narrow4<DT>(acc[j][i]);
 #pragma unroll
             for (int i = 0; i < MT; ++i)
-                store_tile<CW, kQkvAux>(qs, (16 * i + n) * (3 * kRow) + which * kRow + 2 * CW * wave, o[i], g, 2 * CW);
+                store_tile<CW, QKV_AUX>(qs, (16 * i + n) * (3 * kRow) + which * kRow + 2 * CW * wave, o[i], g, 2 * CW);
         }
     }
 
@@ -433,7 +440,7 @@ template <class DT, int MT, int NW, int PF, bool SPLIT> struct LayerWave {
 template <class DT, int NW, int PF>
 __global__ void __launch_bounds__(64 * NW, 2)
 part_kernel(LayerArgs a) {
-    using W = LayerWave<DT, 1, NW, PF, true>;
+    using W = LayerWave<DT, 1, NW, PF, true, 0>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     W w{a, (LDS_PTR(char))smem, (LDS_PTR(char))smem + 16 * kRow, (LDS_PTR(float))(smem + 32 * kRow), wave, lane, lane & 15, lane >> 4, lane * 16};
@@ -457,21 +464,17 @@ part_kernel(LayerArgs a) {
 // former, whose sums never span chunks, run 64 tokens with eight waves of 128 registers: a layer of 64000 tokens 75 -> 70 us,
 // its qkv projection 9 -> 4.5 of a workgroup's 35 us.  Dense layers need the registers for weights that set out four steps
 // ahead (145 -> 134 us); with eight waves of 128 registers they spill 55 and a whole pass takes 3.72 instead of 3.37 ms.
-constexpr int layer_waves(int MT, int NW) { return MT == 2 || (MT == 4 && NW == 8) ? 4 : 2; }
+constexpr int layer_waves(int MT, int NW) { return MT == 2 || (MT > 2 && NW == 8) ? 4 : 2; }
 
 // SPLIT: one workgroup to each of q, k and v of a tile (or one where there is no projection behind); the layer before
 // comes in quarters
-template <class DT, int MT, int NW, int PF, bool SPLIT, bool SPARSE>
-__global__ void __launch_bounds__(64 * NW, layer_waves(MT, NW))
-layer_kernel(LayerArgs a) {
-    using W = LayerWave<DT, MT, NW, PF, SPLIT>;
+template <class DT, int MT, int NW, int PF, bool SPLIT, bool SPARSE, int QKV_AUX>
+__device__ inline void layer_tile(const LayerArgs &a, char *smem, int64_t m0, int mine, int each) {
+    using W = LayerWave<DT, MT, NW, PF, SPLIT, QKV_AUX>;
     constexpr int NTW = W::NTW, CW = W::CW;
-    extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // p_lds: attention rows, then 256 hidden channels at a time, then patches; q_lds: x, then x1, then x2
     W w{a, (LDS_PTR(char))smem, (LDS_PTR(char))smem + 16 * MT * kRow, (LDS_PTR(float))(smem + 32 * MT * kRow), wave, lane, lane & 15, lane >> 4, lane * 16};
-    const int each = SPLIT && a.qkv ? 3 : 1, mine = each == 3 ? (int)(blockIdx.x % 3u) : 0;
-    const int64_t m0 = (int64_t)(blockIdx.x / (uint32_t)each) * (16 * MT);
     const int rows = (int)min((int64_t)(16 * MT), a.M - m0);
     w.stage_qkv_bias();
     if (SPLIT && a.attn) {
@@ -551,6 +554,16 @@ layer_kernel(LayerArgs a) {
         case 2: w.template head<2>(m0, rows, mine, each == 3 ? mine + 1 : 3); break;
         default: w.template head<1>(m0, rows, mine, each == 3 ? mine + 1 : 3);
     }
+}
+template <class DT, int MT, int NW, int PF, bool SPLIT, bool SPARSE>
+__global__ void __launch_bounds__(64 * NW, layer_waves(MT, NW))
+layer_kernel(LayerArgs a) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int each = SPLIT && a.qkv ? 3 : 1, mine = each == 3 ? (int)(blockIdx.x % 3u) : 0;
+    const int tile = (int)(blockIdx.x / (uint32_t)each);
+    if constexpr (MT == 3)
+        if (tile >= a.large) return layer_tile<DT, 2, NW, PF, SPLIT, SPARSE, 0>(a, smem, (int64_t)16 * (2 * tile + a.large), mine, each);
+    layer_tile<DT, MT, NW, PF, SPLIT, SPARSE, !SPLIT && MT <= 2 ? kStoreAux : 0>(a, smem, (int64_t)16 * MT * tile, mine, each);
 }
 
 // tanh(x) = 1 - 2 / (1 + exp(2x)); its series where that would cancel
@@ -1067,13 +1080,21 @@ inline bool one_wave(int64_t N, int64_t T, int wide) {
     return T <= 200 ? blocks >= 192 : T <= 500 ? 8 * blocks >= 5 * room : 5 * blocks >= 4 * room;
 }
 
+// Two workgroups of two and more row tiles share a CU.  Up to 48 tokens to each of these places all of them get a workgroup and the
+// row tiles are dealt out, three and two: in tiles of 64, some CUs have two and others one.  20000 tokens, us in a trace, layers
+// of 8, 4, 2 and 1 groups: 33.1 -> 29.9, 37.6 -> 35.0, 46.5 -> 41.4, 50.1 -> 50.2 (weights bound these, and every workgroup reads
+// them); dealt out in fours and threes, 25600 tokens gain nothing (240 us for five layers either way) and 30000 lose (259 -> 273).
+constexpr int kLayerPlaces = 512;
 template <class DT, int MT, int NW, int PF, bool SPARSE>
 int launch_layer_mt(const LayerArgs &a, hipStream_t s) {
     auto kern = layer_kernel<DT, MT, NW, PF, false, SPARSE>;
     const size_t lds = layer_lds<MT>();
     if (!allow_lds(kern, lds)) return NA1D_ERR_LAUNCH;
-    const int64_t wgs = (a.M + 16 * MT - 1) / (16 * MT);
-    kern<<<(unsigned)wgs, 64 * NW, lds, s>>>(a);
+    const int64_t tiles = (a.M + 15) / 16;
+    int64_t wgs = (tiles + MT - 1) / MT;
+    LayerArgs args = a;
+    if (MT == 3) wgs = kLayerPlaces, args.large = (int)(tiles - 2 * wgs);
+    kern<<<(unsigned)wgs, 64 * NW, lds, s>>>(args);
     return launch_status();
 }
 
@@ -1097,10 +1118,11 @@ template <class DT> int launch_layer(const LayerArgs &a, hipStream_t s) {
     // Fewer, larger tiles read the layer's weights fewer times; smaller ones spread few tokens over more CUs.  PCF 4x4 passes
     // with tiles of 16, 32 and 64 tokens: 4000 tokens 450, 494 and 653 us; 6000: 623, 539, 694; 16000: 1101, 884, 879;
     // 20000: 1319, 1083, 1055; 25600: 1668, 1291, 1166; MFA 4x4: 6000: 832, 629, 888; 16000: 1494, 1033, 1075; 25600: 2380,
-    // 1614, 1399.
+    // 1614, 1399.  (Measured before the present loops; the lines have been the same since, but for 48 tokens, see above.)
     const bool sparse = a.tail_groups >= 4;
     if (a.M <= 16 * 256) return sparse ? launch_layer_mt<DT, 1, 8, 8, true>(a, s) : launch_layer_mt<DT, 1, 8, 8, false>(a, s);
     if (a.M <= 32 * 512) return sparse ? launch_layer_mt<DT, 2, 8, 4, true>(a, s) : launch_layer_mt<DT, 2, 8, 4, false>(a, s);
+    if (a.M <= 48 * kLayerPlaces) return sparse ? launch_layer_mt<DT, 3, 8, 4, true>(a, s) : launch_layer_mt<DT, 3, 4, 4, false>(a, s);
     return sparse ? launch_layer_mt<DT, 4, 8, 4, true>(a, s) : launch_layer_mt<DT, 4, 4, 4, false>(a, s);
 }
 
