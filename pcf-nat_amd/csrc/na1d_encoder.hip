@@ -669,7 +669,8 @@ linear_kernel(LinearArgs a, int col_blocks) {
 // weight eight times and each row's operand four times, which halves what the CU's path to L2 carries per product (64 rows ask
 // for its 64 bytes a clock at the matrix cores' full rate); rows come 128 inputs at a time, so two workgroups share a CU.
 // 1024 inputs, 1536 outputs, this and 64 rows, us in a trace: 8200 rows 35 and 54, 10000: 36 and 57, 25600: 85 and 132 (0.95
-// PFLOP/s), 40000: 133 and 209.  Below the limit linear_kernel's 32 rows x 128 outputs: 2048: 24 and 16, 8000: 35 and 48.
+// PFLOP/s), 40000: 133 and 209.  Below the limit linear_kernel's 32 rows x 128 outputs: 2048: 24 and 16, 4000: 24.6 and 27.4 (one
+// round of its workgroups more from 4096 on: 30.1), 6400: 34.9 and 41.0, 8000: 35.4 and 48.1.
 template <class DT, LinearEnd END>
 __global__ void __launch_bounds__(kThreads, 2)
 linear_wide_kernel(LinearArgs a, int col_blocks) {
@@ -1135,8 +1136,9 @@ template <class DT, LinearEnd END> int launch_linear(const LinearArgs &a, hipStr
             kern<<<(unsigned)((a.M + 16 * mt - 1) / (16 * mt) * cols), kThreads, lds, s>>>(a, cols);
             return launch_status();
         };
+        if constexpr (END == kReluNorm)
+            if (a.M > 4096) return go(linear_wide_kernel<DT, END>, 8, 4, 256);                      // outputs in 256s: encoder_ok
         if (a.M > 8192) {
-            if constexpr (END == kReluNorm) return go(linear_wide_kernel<DT, END>, 8, 4, 256);      // outputs in 256s: encoder_ok
             if constexpr (END == kShift || END == kEmbedding)                                       // the pooling's are 128
                 if (a.outputs % 256 == 0) return go(linear_kernel<DT, 4, 4, END>, 4, 4);
             if constexpr (END != kReluNorm)
