@@ -235,6 +235,11 @@ int na1d_fused_forward_dilated(void *out, float *lse, const void *q, const void 
                                const int32_t *t_valid, int64_t N, int64_t H, int64_t T, int64_t C, int64_t W,
                                int64_t left, int64_t dilation, float scale, int dtype, const int64_t *qkv_strides,
                                const int64_t *out_strides, float p_drop, uint64_t seed, void *stream);
+/* The same, which also sets `clear` (fp32 [H, W], or NULL) to zero where there are rows: the d rpb that a backward adds to. */
+int na1d_fused_forward_clear(void *out, float *lse, float *clear, const void *q, const void *k, const void *v, const float *rpb,
+                             const int32_t *t_valid, int64_t N, int64_t H, int64_t T, int64_t C, int64_t W, int64_t left,
+                             int64_t dilation, float scale, int dtype, const int64_t *qkv_strides,
+                             const int64_t *out_strides, float p_drop, uint64_t seed, void *stream);
 int na1d_fused_backward_dilated(void *dq, void *dk, void *dv, float *drpb, const void *q, const void *k, const void *v,
                                 const void *dout, const float *lse, const float *rpb, const int32_t *t_valid, int64_t N,
                                 int64_t H, int64_t T, int64_t C, int64_t W, int64_t left, int64_t dilation, float scale,

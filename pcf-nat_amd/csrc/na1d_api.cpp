@@ -343,10 +343,10 @@ int na1d_fused_backward_strided_dropout(void *dq, void *dk, void *dv, float *drp
                           (float *)workspace, workspace ? workspace_bytes : 0, (hipStream_t)stream);
 }
 
-int na1d_fused_forward_dilated(void *out, float *lse, const void *q, const void *k, const void *v, const float *rpb,
-                               const int32_t *t_valid, int64_t N, int64_t H, int64_t T, int64_t C, int64_t W,
-                               int64_t left, int64_t dilation, float scale, int dtype, const int64_t *qkv_strides,
-                               const int64_t *out_strides, float p_drop, uint64_t seed, void *stream) {
+int na1d_fused_forward_clear(void *out, float *lse, float *clear, const void *q, const void *k, const void *v, const float *rpb,
+                             const int32_t *t_valid, int64_t N, int64_t H, int64_t T, int64_t C, int64_t W, int64_t left,
+                             int64_t dilation, float scale, int dtype, const int64_t *qkv_strides, const int64_t *out_strides,
+                             float p_drop, uint64_t seed, void *stream) {
     if (N < 0 || H < 1 || N > INT64_MAX / H || dilation < 1) return NA1D_ERR_SHAPE;
     NA1D_CHECK(out, q, k, N * H, T, C, W, left, H, dtype, g);
     if (bad_scale(scale)) return NA1D_ERR_SCALE;
@@ -359,7 +359,16 @@ int na1d_fused_forward_dilated(void *out, float *lse, const void *q, const void 
     if (!mfma_allowed()) return NA1D_ERR_UNSUPPORTED;
     dilate(g, in, outl, dilation);
     g.drop = na1d::make_dropout(p_drop, seed, (uint32_t)g.dilation, 0, (uint32_t)g.seq_rows);
+    g.clear = clear;
     return mfma_fused_fwd(out, lse, q, k, v, rpb, t_valid, g, in, outl, scale, dtype, (hipStream_t)stream);
+}
+
+int na1d_fused_forward_dilated(void *out, float *lse, const void *q, const void *k, const void *v, const float *rpb,
+                               const int32_t *t_valid, int64_t N, int64_t H, int64_t T, int64_t C, int64_t W,
+                               int64_t left, int64_t dilation, float scale, int dtype, const int64_t *qkv_strides,
+                               const int64_t *out_strides, float p_drop, uint64_t seed, void *stream) {
+    return na1d_fused_forward_clear(out, lse, nullptr, q, k, v, rpb, t_valid, N, H, T, C, W, left, dilation, scale, dtype, qkv_strides,
+                                    out_strides, p_drop, seed, stream);
 }
 
 int na1d_fused_backward_dilated(void *dq, void *dk, void *dv, float *drpb, const void *q, const void *k, const void *v,

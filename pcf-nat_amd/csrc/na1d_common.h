@@ -123,6 +123,8 @@ struct Geom {
     // layouts that go with it hold the row stride of a class.
     int dilation = 1, classes = 1, short_from = 1;
     int64_t seq_rows = 0;          // 0: T
+    // Fused forward on the matrix cores: fp32 [H, W] that the kernel sets to zero for the backward's sums, or NULL.
+    float *clear = nullptr;
 };
 inline void set_dilation(Geom &g, int64_t dilation) {
     const int64_t rows = g.T;

@@ -30,7 +30,7 @@ fused_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__
                  const char *__restrict__ k, const char *__restrict__ v, const float *__restrict__ rpb,
                  const int32_t *__restrict__ t_valid, uint32_t items, int T, int W, int L, int H, int tiles, int nt,
                  int strips, float scale, uint32_t strips_magic, uint32_t heads_magic, Strides in, Strides outl,
-                 int shift_arg, Dropout drop, Classes cls) {
+                 int shift_arg, Dropout drop, Classes cls, float *__restrict__ clear) {
     const int shift = NBV == 3 ? 16 : shift_arg;     // three key blocks always start one tile before the query tile
     constexpr int CS = C * HG;                       // channels of a staged row
     constexpr int NW = HG > 1 ? kGroupWaves : kWaves; // waves of the workgroup
@@ -123,6 +123,7 @@ fused_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__
             stage(Shared{}, Shared{});
     }
     __builtin_amdgcn_sched_barrier(0);       // the copies are on their way: everything else is worked out behind them
+    clear_sums<64 * NW>(clear, H * W);
     BiasTable bias_raw;                      // (the wait for the copies covers this load too, wherever it is issued)
     load_bias_table(bias_raw, rpb ? rpb + head * W : nullptr, W, lane);
     const int out_pitch = PK ? 2 * C : outl.pitch, out_width = PK ? 2 * C : outl.width;
@@ -343,7 +344,7 @@ int launch_fwd_hg(void *out, float *lse, const void *q, const void *k, const voi
                   (const char *)q, (const char *)k, (const char *)v,
                   rpb, t_valid, (uint32_t)sp.items, (int)g.T, g.W, g.L, g.H, sp.tiles, sp.nt, sp.strips, scale,
                   div_magic(sp.strips), div_magic(g.H / HG), byte_strides(in, g), byte_strides(outl, g), window_shift(g),
-                  g.drop, classes_of(g, in, outl));
+                  g.drop, classes_of(g, in, outl), g.clear);
     return launch_status();
 }
 

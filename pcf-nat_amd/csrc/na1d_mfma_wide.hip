@@ -45,7 +45,7 @@ wide_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__r
                 const char *__restrict__ k, const char *__restrict__ v, const float *__restrict__ rpb,
                 const int32_t *__restrict__ t_valid, uint32_t items, int T, int W, int L, int H, int tiles, int nt,
                 int strips, float scale, uint32_t strips_magic, uint32_t heads_magic, Strides in, Strides outl,
-                int shift, Dropout drop, Classes cls) {
+                int shift, Dropout drop, Classes cls, float *__restrict__ clear) {
     using LL = Lds<C>;
     constexpr int CT = C / 16;
     constexpr int MT = Strip<C>::kMaxTiles;
@@ -92,6 +92,7 @@ wide_fwd_kernel(char *__restrict__ out, float *__restrict__ lse, const char *__r
         stage_direct<C, MT + NBV, kReadShared>(vs, 16 * (i0 - sb), v_lds, kt, wave, lane_off, in.pitch);
         stage_bias(bias_lds, rpb ? rpb + head * W : nullptr, W, tid);
     }
+    clear_sums<kThreads>(clear, H * W);
 
     int tv = T;
     if (t_valid) tv = max(0, min(T, cls.count > 1 ? class_valid(t_valid[sample], cr, cls) : t_valid[sample]));
@@ -191,7 +192,7 @@ int launch_wide_fwd_n(void *out, float *lse, const void *q, const void *k, const
     launch_kernel(kern, (unsigned)sp.items, lds, s, (char *)out, lse, (const char *)q, (const char *)k, (const char *)v,
                   rpb, t_valid, (uint32_t)sp.items, (int)g.T, g.W, g.L, g.H, sp.tiles, sp.nt, sp.strips, scale,
                   div_magic(sp.strips), div_magic(g.H), byte_strides(in, g), byte_strides(outl, g), shift, g.drop,
-                  classes_of(g, in, outl));
+                  classes_of(g, in, outl), g.clear);
     return launch_status();
 }
 

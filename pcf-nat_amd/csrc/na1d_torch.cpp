@@ -11,6 +11,7 @@
 
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 
 #include "na1d.h"
 
@@ -77,10 +78,31 @@ Strides strides_of(const Geometry &g) {
     if (g.in_place) return Strides{{g.T * 3 * g.H * g.C, g.C, 3 * g.H * g.C}, {g.T * g.H * g.C, g.C, g.H * g.C}};
     return Strides{{g.H * g.T * g.C, g.T * g.C, g.C}, {g.H * g.T * g.C, g.T * g.C, g.C}};
 }
-int forward_kernel(const Geometry &g, const Tensor &out, const Tensor &lse, const void *q, const void *k, const void *v, const Tensor &rpb, const Tensor &t_valid,
+// The gradient of the bias, which the backward's kernel adds to: the forward's sets it to zero on the way, for the first
+// backward of a node (any further one clears its own).  A graph may hold the one and not the other, or replay them unevenly, so
+// under capture every backward clears its own too.
+struct Cleared : torch::CustomClassHolder {
+    explicit Cleared(Tensor t) : sums(std::move(t)) {}
+    Tensor take() {
+        const std::lock_guard<std::mutex> lock(mutex);
+        return std::exchange(sums, Tensor());
+    }
+
+  private:
+    std::mutex mutex;                                 // a retained graph may be walked by several threads
+    Tensor sums;
+};
+bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
+
+int forward_kernel(const Geometry &g, const Tensor &out, const Tensor &lse, const Tensor &clear, const void *q, const void *k, const void *v, const Tensor &rpb, const Tensor &t_valid,
                    int dtype, void *stream) {
     const float *bias = (const float *)ptr(rpb);
     const int32_t *valid = (const int32_t *)ptr(t_valid);
+    if (clear.defined()) {
+        const Strides s = strides_of(g);
+        return na1d_fused_forward_clear(ptr(out), (float *)ptr(lse), (float *)ptr(clear), q, k, v, bias, valid, g.N, g.H, g.T, g.C, g.W, g.left, g.dilation, (float)g.scale,
+                                        dtype, s.in, s.out, (float)g.drop.p, g.drop.seed, stream);
+    }
     if (g.dilation == 1 && !g.in_place) {
         if (g.drop.p > 0)
             return na1d_fused_forward_dropout(ptr(out), (float *)ptr(lse), q, k, v, bias, valid, g.N * g.H, g.H, g.T, g.C, g.W, g.left, (float)g.scale, dtype,
@@ -106,32 +128,47 @@ int backward_kernel(const Geometry &g, void *dq, void *dk, void *dv, const Tenso
     return na1d_fused_backward_dilated(dq, dk, dv, (float *)ptr(drpb), q, k, v, ptr(dout), (const float *)ptr(lse), bias, valid, g.N, g.H, g.T, g.C, g.W, g.left,
                                        g.dilation, (float)g.scale, dtype, s.in, s.out, (float)g.drop.p, g.drop.seed, nullptr, 0, stream);
 }
-void remember(AutogradContext *ctx, const Geometry &g, const MaybeTensor &rpb) {
+void remember(AutogradContext *ctx, const Geometry &g, const MaybeTensor &rpb, const Tensor &cleared) {
     ctx->saved_data["geometry"] = std::vector<int64_t>{g.N, g.H, g.T, g.C, g.W, g.left, g.dilation, (int64_t)g.drop.seed, g.in_place};
     ctx->saved_data["scale"] = g.scale;
     ctx->saved_data["p"] = g.drop.p;
     ctx->saved_data["bias"] = rpb && rpb->requires_grad();
     ctx->saved_data["bias_shape"] = rpb ? rpb->sizes().vec() : std::vector<int64_t>{};
+    if (cleared.defined()) ctx->saved_data["cleared"] = c10::IValue::make_capsule(c10::make_intrusive<Cleared>(cleared));
+}
+// The bias' gradient, all zeros; undefined where none is asked for.
+Tensor begin_bias_gradient(AutogradContext *ctx, const Tensor &like) {
+    if (!ctx->saved_data["bias"].toBool()) return Tensor();
+    const auto held = ctx->saved_data.find("cleared");
+    if (held != ctx->saved_data.end() && !capturing()) {
+        Tensor t = c10::static_intrusive_pointer_cast<Cleared>(held->second.toCapsule())->take();
+        if (t.defined()) return t;
+    }
+    return at::zeros(ctx->saved_data["bias_shape"].toIntVector(), like.options().dtype(at::kFloat));
 }
 Geometry recall(AutogradContext *ctx) {
     const auto v = ctx->saved_data["geometry"].toIntVector();
     return Geometry{v[0], v[1], v[2], v[3], v[4], v[5], v[6], ctx->saved_data["scale"].toDouble(), {ctx->saved_data["p"].toDouble(), (uint64_t)v[7]}, v[8] != 0};
 }
-Tensor bias_of(const MaybeTensor &rpb, const Geometry &g) {
+Tensor bias_of(const MaybeTensor &rpb, const Geometry &g, bool node) {
+    if (rpb && !node && rpb->scalar_type() == at::kFloat && rpb->is_contiguous()) return *rpb;
     return rpb ? rpb->detach().reshape({g.H, g.W}).to(at::kFloat).contiguous() : Tensor();
 }
 Tensor lengths_of(const MaybeTensor &t_valid, const Tensor &like) { return t_valid ? t_valid->to(like.device(), at::kInt).contiguous() : Tensor(); }
 
 // A forward whose kernels are launched: what its node is built around.
 struct Done {
-    Tensor out, lse, bias, valid;
+    Tensor out, lse, bias, valid, cleared;
 };
+Tensor to_be_cleared(const MaybeTensor &rpb, const Tensor &like, bool node) {
+    return node && rpb && rpb->requires_grad() && !capturing() ? at::empty(rpb->sizes(), like.options().dtype(at::kFloat)) : Tensor();
+}
 
 struct Fused : torch::autograd::Function<Fused> {
     static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const MaybeTensor &rpb, const MaybeTensor &,
                           const Geometry &g, const Done &done) {
         ctx->save_for_backward({q, k, v, done.out, done.bias, done.valid, done.lse});
-        remember(ctx, g, rpb);
+        remember(ctx, g, rpb, done.cleared);
         return done.out;
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
@@ -140,8 +177,7 @@ struct Fused : torch::autograd::Function<Fused> {
         const Tensor &q = s[0];
         const c10::DeviceGuard guard(q.device());
         const Tensor dout = grads[0].contiguous(), dq = at::empty_like(q), dk = at::empty_like(q), dv = at::empty_like(q);
-        Tensor drpb;
-        if (ctx->saved_data["bias"].toBool()) drpb = at::zeros(ctx->saved_data["bias_shape"].toIntVector(), q.options().dtype(at::kFloat));
+        const Tensor drpb = begin_bias_gradient(ctx, q);
         check(backward_kernel(g, ptr(dq), ptr(dk), ptr(dv), drpb, ptr(q), ptr(s[1]), ptr(s[2]), s[3], dout, s[6], s[4], s[5], tag(q), stream_of(q)),
               "na1d_fused_backward");
         return {dq, dk, dv, drpb, Tensor(), Tensor(), Tensor()};
@@ -150,7 +186,7 @@ struct Fused : torch::autograd::Function<Fused> {
 struct FusedQKV : torch::autograd::Function<FusedQKV> {
     static Tensor forward(AutogradContext *ctx, const Tensor &qkv, const MaybeTensor &rpb, const MaybeTensor &, const Geometry &g, const Done &done) {
         ctx->save_for_backward({qkv, done.bias, done.valid, done.lse});
-        remember(ctx, g, rpb);
+        remember(ctx, g, rpb, done.cleared);
         return done.out;
     }
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
@@ -159,8 +195,7 @@ struct FusedQKV : torch::autograd::Function<FusedQKV> {
         const Tensor &qkv = s[0];
         const c10::DeviceGuard guard(qkv.device());
         const Tensor dout = grads[0].contiguous(), dqkv = at::empty_like(qkv);
-        Tensor drpb;
-        if (ctx->saved_data["bias"].toBool()) drpb = at::zeros(ctx->saved_data["bias_shape"].toIntVector(), qkv.options().dtype(at::kFloat));
+        const Tensor drpb = begin_bias_gradient(ctx, qkv);
         const int64_t step = 2 * g.H * g.C;
         char *dq = (char *)ptr(dqkv);
         const char *q = (const char *)ptr(qkv);
@@ -192,8 +227,9 @@ MaybeTensor fused(const Tensor &q, const Tensor &k, const Tensor &v, const Maybe
     if (!covered(g, q, rpb, t_valid)) return std::nullopt;
     const c10::DeviceGuard guard(q.device());
     const bool node = needs_grad({q, k, v}, rpb);      // otherwise no log-sum-exp either
-    const Done done{at::empty_like(q), node ? at::empty({g.N * g.H, g.T}, q.options().dtype(at::kFloat)) : Tensor(), bias_of(rpb, g), lengths_of(t_valid, q)};
-    if (forward_kernel(g, done.out, done.lse, ptr(q), ptr(k), ptr(v), done.bias, done.valid, tag(q), stream_of(q)) != NA1D_OK) return std::nullopt;
+    const Done done{at::empty_like(q), node ? at::empty({g.N * g.H, g.T}, q.options().dtype(at::kFloat)) : Tensor(), bias_of(rpb, g, node),
+                    lengths_of(t_valid, q), to_be_cleared(rpb, q, node)};
+    if (forward_kernel(g, done.out, done.lse, done.cleared, ptr(q), ptr(k), ptr(v), done.bias, done.valid, tag(q), stream_of(q)) != NA1D_OK) return std::nullopt;
     return node ? Fused::apply(q, k, v, rpb, t_valid, g, done) : done.out;
 }
 MaybeTensor fused_qkv(const Tensor &qkv, const MaybeTensor &rpb, const MaybeTensor &t_valid, int64_t W, int64_t left, double scale, int64_t dilation, double p,
@@ -204,10 +240,10 @@ MaybeTensor fused_qkv(const Tensor &qkv, const MaybeTensor &rpb, const MaybeTens
     const c10::DeviceGuard guard(qkv.device());
     const bool node = needs_grad({qkv}, rpb);
     const Done done{at::empty({g.N, g.T, g.H * g.C}, qkv.options()), node ? at::empty({g.N * g.H, g.T}, qkv.options().dtype(at::kFloat)) : Tensor(),
-                    bias_of(rpb, g), lengths_of(t_valid, qkv)};
+                    bias_of(rpb, g, node), lengths_of(t_valid, qkv), to_be_cleared(rpb, qkv, node)};
     const char *q = (const char *)ptr(qkv);
     const int64_t step = 2 * g.H * g.C;
-    if (forward_kernel(g, done.out, done.lse, q, q + step, q + 2 * step, done.bias, done.valid, tag(qkv), stream_of(qkv)) != NA1D_OK) return std::nullopt;
+    if (forward_kernel(g, done.out, done.lse, done.cleared, q, q + step, q + 2 * step, done.bias, done.valid, tag(qkv), stream_of(qkv)) != NA1D_OK) return std::nullopt;
     return node ? FusedQKV::apply(qkv, rpb, t_valid, g, done) : done.out;
 }
 

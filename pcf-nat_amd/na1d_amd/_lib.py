@@ -27,7 +27,7 @@ SYMBOLS = _UNFUSED + ("na1d_fused_forward", "na1d_fused_backward", "na1d_fused_b
                       "na1d_fused_forward_dropout", "na1d_fused_backward_dropout",
                       "na1d_fused_backward_noalloc", "na1d_force_generic", "na1d_profile_last_kernel",
                       "na1d_fused_forward_strided_dropout", "na1d_fused_backward_strided_dropout",
-                      "na1d_fused_forward_dilated", "na1d_fused_backward_dilated",
+                      "na1d_fused_forward_dilated", "na1d_fused_forward_clear", "na1d_fused_backward_dilated",
                       "na1d_fused_backward_dilated_workspace_bytes", "na1d_encode", "na1d_encode_workspace_bytes",
                       "na1d_train_layer_saved_bytes", "na1d_train_layer_workspace_bytes", "na1d_train_layer_forward",
                       "na1d_train_to_channels", "na1d_train_pool_backward", "na1d_train_context_backward",
@@ -89,6 +89,8 @@ def load():
                                                                                 _i64, _i64, _i64, _ptr, _i64, _ptr]
     lib.na1d_fused_forward_dilated.restype = _int
     lib.na1d_fused_forward_dilated.argtypes = [_ptr] * 7 + [_i64] * 7 + [_f32, _int, _ptr, _ptr, _f32, _u64, _ptr]
+    lib.na1d_fused_forward_clear.restype = _int
+    lib.na1d_fused_forward_clear.argtypes = [_ptr] * 8 + [_i64] * 7 + [_f32, _int, _ptr, _ptr, _f32, _u64, _ptr]
     lib.na1d_fused_backward_dilated.restype = _int
     lib.na1d_fused_backward_dilated.argtypes = [_ptr] * 11 + [_i64] * 7 + [_f32, _int, _ptr, _ptr, _f32, _u64, _ptr, _i64,
                                                                           _ptr]

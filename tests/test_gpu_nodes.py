@@ -108,3 +108,46 @@ def test_nodes_leave_what_they_do_not_take_to_python():
         assert nodes.fused_qkv(qkv, None, None, 5, 2, 1.0, 1, 0.0, 0) is None and na1d_fused_qkv(qkv, 5, 2).shape == (2, 20, 16)
     finally:
         _lib.load().na1d_force_generic(old)
+
+
+def _dirty(*shape):
+    """Leaves numbers in the memory that the next allocation of this size gets."""
+    for t in [torch.full(shape, 3.0, device="cuda") for _ in range(8)]:
+        del t
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("N,H,T,C,W,left,dilation,p", [(2, 16, 100, 16, 27, 13, 1, 0.0), (1, 1, 1, 8, 3, 1, 1, 0.0), (3, 5, 150, 32, 65, 32, 1, 0.0),
+                                                       (1, 12, 3, 64, 80, 40, 2, 0.1), (2, 7, 33, 24, 15, 7, 3, 0.0)])
+def test_bias_gradient_begins_at_zero(N, H, T, C, W, left, dilation, p, in_place):
+    """The forward's kernel clears the sums of a node's first backward; backwards of a kept graph, and captured ones, clear their own."""
+    rpb = eager = _rand(1, H, 1, W, dtype=torch.float32, seed=5)
+    tensors = [_rand(N, T, 3, H, C, seed=3)] if in_place else [_rand(N * H, T, C, seed=i) for i in range(3)]
+    g = _rand(*((N, T, H * C) if in_place else (N * H, T, C)), seed=9, grad=False)
+
+    def call():
+        _dirty(1, H, 1, W)
+        if in_place:
+            return _lib.nodes().fused_qkv(tensors[0], rpb, None, W, left, 0.3, dilation, p, 11)
+        return _lib.nodes().fused(*tensors, rpb, None, H, W, left, 0.3, dilation, p, 11)
+
+    if in_place:
+        out = fused._FusedNA1DQKV.apply(*tensors, rpb, None, W, left, 0.3, False, dilation, (p, 11) if p else None)
+    else:
+        out = fused._FusedNA1D.apply(*tensors, rpb, None, H, W, left, 0.3, False, dilation, (p, 11) if p else None)
+    want = torch.autograd.grad(out, rpb, g)[0]
+    out, other = call(), call()
+    for n in range(3):                               # the first is kept unchanged while the second runs
+        first, second = (torch.autograd.grad(o, rpb, g, retain_graph=n < 2)[0] for o in (out, other))
+        for got in (first, second):
+            torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-4 * want.abs().max().item())     # float atomics, as in _same
+    kept = call()
+    # Leaves of the graph's own: the engine joins the stream on which a leaf was first used, which must be a captured one.
+    rpb, tensors = rpb.detach().clone().requires_grad_(True), [t.detach() for t in tensors]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = torch.autograd.grad(call(), rpb, g)[0]
+    for _ in range(3):
+        graph.replay()
+        torch.testing.assert_close(captured, want, rtol=1e-4, atol=1e-4 * want.abs().max().item())
+    torch.testing.assert_close(torch.autograd.grad(kept, eager, g)[0], want, rtol=1e-4, atol=1e-4 * want.abs().max().item())
