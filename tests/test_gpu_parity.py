@@ -456,6 +456,33 @@ def test_full_launches_are_deterministic_and_batch_invariant(case):
     assert O.rel_l2(alone[0].float().cpu(), want) < TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=["bf16", "fp16"])
+@pytest.mark.parametrize("H,T,C,W,L", [(8, 1, 16, 65, 32), (8, 15, 32, 33, 16), (8, 64, 16, 80, 79), (5, 65, 32, 80, 0), (4, 129, 32, 70, 40), (2, 130, 64, 49, 48),
+                                       (2, 145, 64, 80, 41), (1, 97, 128, 65, 30), (1, 80, 128, 33, 0), (1, 176, 24, 40, 17)])
+def test_wide_backward_however_sequences_are_cut(H, T, C, W, L, dtype):
+    """Enough sequences for whole ones, and a few, which are cut into segments: the same bits, and the oracle's gradients."""
+    N = 1040 // H
+    q, k, v, do = make_inputs(N * H, T, C, W, 11, dtype, n=4, scale=C ** -0.5)
+    rpb = torch.randn(H, W, generator=torch.Generator().manual_seed(3)) * 0.5
+    t_valid = torch.full((N,), T, dtype=torch.int32)
+    t_valid[:2] = max(1, T - T // 3)
+    few = 3
+
+    def run(n):
+        leaves = [t[:n * H].cuda().requires_grad_(True) for t in (q, k, v)] + [rpb.cuda().requires_grad_(True)]
+        na1d_fused(*leaves[:3], W, L, rpb=leaves[3], t_valid=t_valid[:n].cuda(), num_heads=H).backward(do[:n * H].cuda())
+        return [t.grad for t in leaves]
+
+    many, some = run(N), run(few)
+    want = O.na1d_backward(*(t[:few * H].float() for t in (q, k, v, do)), W, L, rpb, T - t_valid[:few], H)
+    for name, a, b, ref in zip(("dQ", "dK", "dV", "drpb"), many, some, want):
+        if name == "drpb":                           # zero, but for rounding, where rows have one key
+            assert _err(b, ref) < TOL[dtype], name
+        else:
+            assert torch.equal(a[:few * H], b), name
+            assert O.rel_l2(b.float(), ref) < TOL[dtype], name
+
+
 @pytest.mark.parametrize("case", [(256, 16, 100, 16, 27, 13, torch.bfloat16), (128, 8, 300, 32, 15, 7, torch.float16)],
                          ids=lambda c: "x".join(map(str, c[:6])))
 def test_full_launches_in_the_projection_layout_and_through_the_two_call_api(case):
