@@ -2,7 +2,7 @@
 // 224-261) in training, forward and backward, on token-major activations: batch norms with batch statistics, projections,
 // GELU, residuals and weight gradients around the attention kernels.
 //
-// A layer of 128 x 100 tokens, 256 channels, fp16, forward and backward: 26 launches of 240 us together and 38 us of torch's
+// A layer of 128 x 100 tokens, 256 channels, fp16, forward and backward: 24 launches of 225 us together and 38 us of torch's
 // statistics, where the modules took some 80 launches and 800 us (torch's batch norm with its copies, bias gradients as
 // reductions of their own, weight gradients through 16-bit sums of chunks).  The pooling behind the layers has its backward
 // here too.  Everything else than the batch statistics is launched from native code, so the
@@ -25,7 +25,7 @@ using namespace enc;
 // workgroup takes 64 channels (whole 128-byte lines) of one of up to 64 chunks of rows; the kernel that uses the backward's
 // sums adds up the chunks itself (32 KB from L2) instead of waiting for a third launch.  12800 x 256: 7.9 and 8.7 us
 // backward, where torch took 54 us, and 13 us for each change of layout.
-constexpr int kBnCols = 64, kBnThreads = 256, kBnLanes = kBnThreads / 8, kBnChunks = 64;
+constexpr int kBnCols = 64, kBnThreads = 256, kBnLanes = kBnThreads / 8, kBnChunks = 64, kBnParts = 256;
 struct Chunks {
     int rows, count;          // rows of a chunk (the last may have fewer), chunks
 };
@@ -61,15 +61,6 @@ __device__ inline void meet(float (*part)[kBnCols + 1], float (*quarter)[kBnCols
     __syncthreads();
     total = quarter[0][ch] + quarter[1][ch] + (quarter[2][ch] + quarter[3][ch]);
 }
-// The four groups of 64 threads' sums of one value per channel.
-__device__ inline float across_groups(float (*quarter)[kBnCols], float v) {
-    const int ch = threadIdx.x & 63, q = threadIdx.x >> 6;
-    __syncthreads();
-    quarter[q][ch] = v;
-    __syncthreads();
-    return quarter[0][ch] + quarter[1][ch] + (quarter[2][ch] + quarter[3][ch]);
-}
-
 // [N, T, C] -> [N, C, T], 64 x 64 at a time through LDS: the layout in which torch sums the statistics.
 __global__ void __launch_bounds__(256)
 to_channels_kernel(uint16_t *__restrict__ out, const char *__restrict__ x, int T, int C) {
@@ -155,7 +146,8 @@ bn_apply_kernel(BnApply a) {
     }
 }
 
-// Backward: sums of dy and of dy * (x - mean) over a chunk's rows, then
+// Backward: sums of dy and of dy * (x - mean) over a chunk's rows (behind the product that makes dy, where it is few enough
+// blocks of rows: see launch_gemm), then
 // dx = weight * rstd * (dy - sum(dy) / M - (x - mean) * rstd^2 * sum(dy (x - mean)) / M) + `add`.
 template <class DT>
 __global__ void __launch_bounds__(kBnThreads)
@@ -198,16 +190,25 @@ struct BnBackward {
 template <class DT>
 __global__ void __launch_bounds__(kBnThreads)
 bn_bwd_apply_kernel(BnBackward a) {
-    __shared__ float quarter[4][kBnCols], s_k1[kBnCols], s_k2[kBnCols], s_a[kBnCols];
-    const int c0 = blockIdx.x * kBnCols, ch = threadIdx.x & 63, q = threadIdx.x >> 6;
-    float s1 = 0.f, s2 = 0.f;
-#pragma unroll 4
-    for (int k = q; k < a.chunks; k += 4) {
-        s1 += a.part_dy[(int64_t)k * a.C + c0 + ch];
-        s2 += a.part_dyx[(int64_t)k * a.C + c0 + ch];
+    constexpr int kLanes = kBnThreads / (kBnCols / 4);            // chunks side by side, four channels to a thread
+    __shared__ float met[2][kLanes][kBnCols], s_k1[kBnCols], s_k2[kBnCols], s_a[kBnCols];
+    const int c0 = blockIdx.x * kBnCols, ch = threadIdx.x & 63;
+    {
+        const int lane = threadIdx.x / (kBnCols / 4), at = c0 + 4 * (threadIdx.x % (kBnCols / 4));
+        f32x4 s1 = {0.f, 0.f, 0.f, 0.f}, s2 = s1;
+#pragma unroll 8
+        for (int k = lane; k < a.chunks; k += kLanes) {
+            s1 += *reinterpret_cast<const f32x4 *>(a.part_dy + (int64_t)k * a.C + at);
+            s2 += *reinterpret_cast<const f32x4 *>(a.part_dyx + (int64_t)k * a.C + at);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) met[0][lane][at - c0 + r] = s1[r], met[1][lane][at - c0 + r] = s2[r];
+        __syncthreads();
     }
-    s1 = across_groups(quarter, s1);
-    s2 = across_groups(quarter, s2);
+    float s1 = 0.f, s2 = 0.f;
+    if (threadIdx.x < kBnCols)
+#pragma unroll
+        for (int k = 0; k < kLanes; ++k) s1 += met[0][k][ch], s2 += met[1][k][ch];
     if (threadIdx.x < kBnCols) {
         const float rstd = a.rstd[c0 + ch];
         s_a[ch] = a.weight[c0 + ch] * rstd;
@@ -306,16 +307,25 @@ enum GemmEnd {
     kResidual,        // out = aux + sample_scale * (v + bias)
     kGelu,            // out2 = v + bias, out = gelu(out2)
     kGeluBack,        // out = v * gelu'(aux)
+    kNormBack,        // out = v, and for the norm whose input aux is, sums of v and of v * (aux - mean) over the block's rows
 };
 struct Gemm {
     const char *x, *w;
     char *out, *out2;
     const char *aux;
     const float *bias, *sample_scale;      // one factor per sample of T rows, or NULL
+    const float *mean;                     // kNormBack ...
+    float *part_dy, *part_dyx;             // ... [blocks of rows, outputs]
     int inputs, outputs, M, T;
     uint32_t T_magic;
     int late;                              // the sum is rounded before the bias is added (a product and an addition in torch)
 };
+__device__ inline float over_row(float x) {                       // sum over 16 lanes
+    x += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0xb1, 0xf, 0xf, true));
+    x += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x4e, 0xf, 0xf, true));
+    x += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x141, 0xf, 0xf, true));
+    return x + __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x140, 0xf, 0xf, true));
+}
 // Phi(x) and x's density, the former by formula 7.1.26 of Abramowitz and Stegun's handbook (error below 1.5e-7); infinities
 // come out as x * Phi(x) gives them.
 __device__ inline void normal_of(float x, float &cdf, float &pdf) {
@@ -371,10 +381,15 @@ gemm_kernel(Gemm a, int col_blocks) {
 #pragma unroll
         for (int j = 0; j < NTW; ++j) bias[j] = *reinterpret_cast<const f32x4 *>(a.bias + 16 * (tile0 + j) + 4 * g);
     }
+    f32x4 mean[NTW], s1[NTW], s2[NTW];
+    if constexpr (END == kNormBack) {
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) mean[j] = *reinterpret_cast<const f32x4 *>(a.mean + 16 * (tile0 + j) + 4 * g), s1[j] = s2[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     // What an end reads of every output, all at once and store_tile backwards: 16 bytes to a lane, 64 of a row together (GELU's
     // derivative over 12800 x 1024: 29.0 -> 23.6 us, 27.1 with a row tile's behind the other).
     u32x4 aux16[MT][NTW / 2];
-    if constexpr (END == kResidual || END == kGeluBack) {
+    if constexpr (END == kResidual || END == kGeluBack || END == kNormBack) {
         const Rsrc as = make_rsrc(a.aux + m0 * pitch, rows * pitch);
 #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -387,7 +402,7 @@ gemm_kernel(Gemm a, int col_blocks) {
         u32x2 o[NTW];
         const int row_byte = (16 * i + n) * pitch + 32 * tile0;
         f32x4 aux[NTW];
-        if constexpr (END == kResidual || END == kGeluBack) {
+        if constexpr (END == kResidual || END == kGeluBack || END == kNormBack) {
 #pragma unroll
             for (int p = 0; p < NTW / 2; ++p) {
                 const u32x4 v = aux16[i][p];
@@ -429,9 +444,23 @@ gemm_kernel(Gemm a, int col_blocks) {
                     }
                 }
                 o[j] = narrow4<DT>(v);
+                if constexpr (END == kNormBack) {            // of what is stored; rows behind the last are zeros
+                    const f32x4 d = widen4<DT>(o[j]);
+                    s1[j] += d;
+                    s2[j] += d * (aux[j] - mean[j]);
+                }
             }
         }
         store_tile<16 * NTW, 0>(os, row_byte, o, g, 32 * NTW);
+    }
+    if constexpr (END == kNormBack) {
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s1[j][r] = over_row(s1[j][r]), s2[j][r] = over_row(s2[j][r]);
+            const int64_t at = (int64_t)row_block * a.outputs + 16 * (tile0 + j) + 4 * g;
+            if (n == 0) *reinterpret_cast<f32x4 *>(a.part_dy + at) = s1[j], *reinterpret_cast<f32x4 *>(a.part_dyx + at) = s2[j];
+        }
     }
 }
 
@@ -611,12 +640,6 @@ grad_fold_kernel(Fold a) {
 // and 47 us (157 and 197 MB), where torch took some thirty kernels of 440 and 330 us.  A training step, which its host paces by
 // then: 10.1-10.3 -> 9.5-9.7 ms.
 constexpr int kPoolLanes = 16, kPoolThreads = 256;
-__device__ inline float over_row(float x) {                       // sum over the 16 lanes of a row
-    x += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0xb1, 0xf, 0xf, true));
-    x += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x4e, 0xf, 0xf, true));
-    x += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x141, 0xf, 0xf, true));
-    return x + __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x140, 0xf, 0xf, true));
-}
 __device__ inline float max_over_row(float x) {
     x = __builtin_fmaxf(x, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0xb1, 0xf, 0xf, true)));
     x = __builtin_fmaxf(x, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x4e, 0xf, 0xf, true)));
@@ -802,7 +825,7 @@ struct BackwardScratch : Buffers {
         const int64_t M = N * T, row = M * l.dim * 2;
         const GradPlan p(l, M);
         dz = take(l.scale_mlp ? row : 0), dh = take(M * l.hidden * 2), dy = take(row), dx1 = take(row), ds = take(l.scale_attn ? row : 0);
-        dattn = take(row), dqkv = take(3 * row), part = take((int64_t)2 * kBnChunks * l.dim * 4);
+        dattn = take(row), dqkv = take(3 * row), part = take((int64_t)2 * kBnParts * l.dim * 4);
         grads = take(p.splits * p.part[kWeights] * 4);
         delta = take(l.window ? 0 : M * l.heads * 4), dpos = take(l.window ? 0 : T * l.dim * 2);
     }
@@ -814,6 +837,7 @@ struct BackwardScratch : Buffers {
         if (st_ != NA1D_OK) return st_;     \
     } while (0)
 
+inline int gemm_rows(int64_t M, int outputs) { return (M + 63) / 64 * (outputs / 256) >= 128 ? 64 : 32; }
 // 64 rows x 128 outputs (a hundred registers: four workgroups on a CU); fewer rows where that leaves CUs idle.  Twice the
 // outputs halve the rows' reads but two workgroups on a CU do not hide the ends: GELU's 28 instead of 22 us at 12800 rows.
 template <class DT, GemmEnd END> int launch_gemm(const Gemm &a, hipStream_t s) {
@@ -824,8 +848,7 @@ template <class DT, GemmEnd END> int launch_gemm(const Gemm &a, hipStream_t s) {
         kern<<<(unsigned)((a.M + 16 * mt - 1) / (16 * mt) * cols), kThreads, lds, s>>>(a, cols);
         return launch_status();
     };
-    const int64_t wide = ((int64_t)a.M + 63) / 64 * (a.outputs / 256);
-    if (wide >= 128) return go(gemm_kernel<DT, 4, 2, END>, 4, 2);
+    if (gemm_rows(a.M, a.outputs) == 64) return go(gemm_kernel<DT, 4, 2, END>, 4, 2);
     return go(gemm_kernel<DT, 2, 2, END>, 2, 2);
 }
 template <class DT> int scale_rows(char *out, const char *x, const float *f, int64_t N, int64_t T, int dim, hipStream_t s) {
@@ -854,16 +877,29 @@ int to_channels(const na1d_train_layer &l, void *out, const void *x, int64_t N, 
     to_channels_kernel<<<dim3((unsigned)((T + 63) / 64), (unsigned)(l.dim / 64), (unsigned)N), 256, 0, s>>>((uint16_t *)out, (const char *)x, (int)T, l.dim);
     return launch_status();
 }
+// The product a.x . W, which is the gradient dy of a norm's output (in a.out), and the norm's backward.
+// The product's ends sum up what the norm needs, a row of sums for every block of 64 or 32 tokens, which the kernel behind adds up
+// again (up to kBnParts of them: 0.5 MB from L2); with more blocks of rows a kernel of its own does.
+// 12800 tokens, us: products of 12.5 and sums of 7.8 -> products of 14.9; a step of MFA 4x4 at 128 x 2 s 9070 -> 8700.
 template <class DT>
-int norm_backward(const na1d_train_layer &l, int which, char *dx, const char *dy, const char *x, const char *add, const float *mean, const float *rstd, float *part,
-                  int64_t M, hipStream_t s) {
-    const Chunks c = bn_chunks(M);
+int product_and_norm_backward(Gemm a, const na1d_train_layer &l, int which, char *dx, const char *x, const char *add, const float *mean, const float *rstd, float *part,
+                              hipStream_t s) {
+    const Chunks c = bn_chunks(a.M);
     const dim3 grid((unsigned)(l.dim / kBnCols), (unsigned)c.count);
-    float *part_dyx = part + (int64_t)kBnChunks * l.dim;
-    bn_bwd_sums_kernel<DT><<<grid, kBnThreads, 0, s>>>(part, part_dyx, dy, x, mean, (int)M, l.dim, c.rows);
-    NA1D_TRY(launch_status());
+    float *part_dyx = part + (int64_t)kBnParts * l.dim;
+    const int rows = gemm_rows(a.M, a.outputs);
+    int chunks = (a.M + rows - 1) / rows;
+    if (chunks <= kBnParts) {
+        a.aux = x, a.mean = mean, a.part_dy = part, a.part_dyx = part_dyx;
+        NA1D_TRY(launch_gemm<DT, kNormBack>(a, s));
+    } else {
+        NA1D_TRY(launch_gemm<DT, kStore>(a, s));
+        bn_bwd_sums_kernel<DT><<<grid, kBnThreads, 0, s>>>(part, part_dyx, a.out, x, mean, a.M, l.dim, c.rows);
+        NA1D_TRY(launch_status());
+        chunks = c.count;
+    }
     const na1d_train_norm &n = l.norm[which];
-    bn_bwd_apply_kernel<DT><<<grid, kBnThreads, 0, s>>>(BnBackward{dx, dy, x, add, part, part_dyx, n.weight, mean, rstd, n.dweight, n.dbias, (int)M, l.dim, c.rows, c.count});
+    bn_bwd_apply_kernel<DT><<<grid, kBnThreads, 0, s>>>(BnBackward{dx, a.out, x, add, part, part_dyx, n.weight, mean, rstd, n.dweight, n.dbias, a.M, l.dim, c.rows, chunks});
     return launch_status();
 }
 
@@ -941,8 +977,7 @@ int backward(const na1d_train_layer &l, char *dx, const char *dout, const char *
     a.aux = saved + o.h;
     NA1D_TRY(launch_gemm<DT, kGeluBack>(a, s));
     turned(2, ws + b.dh, ws + b.dy);
-    NA1D_TRY(launch_gemm<DT, kStore>(a, s));
-    NA1D_TRY(norm_backward<DT>(l, 1, ws + b.dx1, ws + b.dy, saved + o.x1, dout, stat(2), stat(3), part, M, s));
+    NA1D_TRY(product_and_norm_backward<DT>(a, l, 1, ws + b.dx1, saved + o.x1, dout, stat(2), stat(3), part, s));
     const char *ds = ws + b.dx1;
     if (l.scale_attn) {
         NA1D_TRY(scale_rows<DT>(ws + b.ds, ds, l.scale_attn, N, T, l.dim, s));
@@ -964,8 +999,7 @@ int backward(const na1d_train_layer &l, char *dx, const char *dout, const char *
         st = wide_bwd(dq, dq + step, dq + 2 * step, l.drpb, q, q + step, q + 2 * step, ws + b.dattn, lse, l.rpb, nullptr, g, in, outl, l.scale, DT::tag, nullptr, 0, s);
     NA1D_TRY(st);
     turned(0, ws + b.dqkv, ws + b.dy);
-    NA1D_TRY(launch_gemm<DT, kStore>(a, s));
-    NA1D_TRY(norm_backward<DT>(l, 0, dx, ws + b.dy, x, ws + b.dx1, stat(0), stat(1), part, M, s));
+    NA1D_TRY(product_and_norm_backward<DT>(a, l, 0, dx, x, ws + b.dx1, stat(0), stat(1), part, s));
     if (!l.window) {
         const int64_t units = T * l.dim / 8;
         sum_samples_kernel<DT><<<(unsigned)((units + 31) / 32), 256, 0, s>>>(ws + b.dpos, ws + b.dy, (int)N, units);
