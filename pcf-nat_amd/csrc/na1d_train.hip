@@ -23,14 +23,15 @@ using namespace enc;
 // The sums of the forward are torch's (batch_norm_update_stats on [N, C, T]), to the bit.
 // What uses the statistics, and the backward, is bound by memory: a pass over 12800 x 256 16-bit values is 6.5 MB.  A
 // workgroup takes 64 channels (whole 128-byte lines) of one of up to 64 chunks of rows; the kernel that uses the backward's
-// sums adds up the chunks itself (32 KB from L2) instead of waiting for a third launch.  12800 x 256: 7.9 and 8.7 us
-// backward, where torch took 54 us, and 13 us for each change of layout.
-constexpr int kBnCols = 64, kBnThreads = 256, kBnLanes = kBnThreads / 8, kBnChunks = 64, kBnParts = 256;
+// sums adds them up itself (from L2) instead of waiting for a third launch, with 16 waves, since with few its workgroups are one to a CU
+// (8.9 -> 7.5 us; more workgroups read the sums more often: 9.7).  The forward, which reads none, has up to 256 chunks (6.0 -> 4.8).
+// 12800 x 256 backward, where torch took 54 us, and 13 us for each change of layout: 7.5 us behind the product that sums.
+constexpr int kBnCols = 64, kBnThreads = 256, kBnLanes = kBnThreads / 8, kBnChunks = 64, kBnParts = 256, kBnApplyThreads = 1024;
 struct Chunks {
     int rows, count;          // rows of a chunk (the last may have fewer), chunks
 };
-inline Chunks bn_chunks(int64_t M) {
-    const int64_t rows = std::max<int64_t>((M + kBnChunks - 1) / kBnChunks, kBnLanes);
+inline Chunks bn_chunks(int64_t M, int most) {
+    const int64_t rows = std::max<int64_t>((M + most - 1) / most, kBnLanes);
     return Chunks{(int)rows, (int)((M + rows - 1) / rows)};
 }
 template <class DT> __device__ inline void unpack(u32x4 w, float (&v)[8]) {
@@ -188,9 +189,9 @@ struct BnBackward {
     int M, C, rows, chunks;
 };
 template <class DT>
-__global__ void __launch_bounds__(kBnThreads)
+__global__ void __launch_bounds__(kBnApplyThreads)
 bn_bwd_apply_kernel(BnBackward a) {
-    constexpr int kLanes = kBnThreads / (kBnCols / 4);            // chunks side by side, four channels to a thread
+    constexpr int kLanes = kBnApplyThreads / (kBnCols / 4);            // chunks side by side, four channels to a thread
     __shared__ float met[2][kLanes][kBnCols], s_k1[kBnCols], s_k2[kBnCols], s_a[kBnCols];
     const int c0 = blockIdx.x * kBnCols, ch = threadIdx.x & 63;
     {
@@ -226,7 +227,7 @@ bn_bwd_apply_kernel(BnBackward a) {
     for (int i = 0; i < 8; ++i) m[i] = a.mean[c0 + 8 * c + i], k1[i] = s_k1[8 * c + i], k2[i] = s_k2[8 * c + i], f[i] = s_a[8 * c + i];
     const int64_t pitch = 2 * (int64_t)a.C, at = 2 * (int64_t)(c0 + 8 * c);
 #pragma unroll 4
-    for (int t = r0 + (threadIdx.x >> 3); t < r1; t += kBnLanes) {
+    for (int t = r0 + (threadIdx.x >> 3); t < r1; t += kBnApplyThreads / 8) {
         float v[8], d[8], e[8];
         unpack<DT>(*reinterpret_cast<const u32x4 *>(a.x + t * pitch + at), v);
         unpack<DT>(*reinterpret_cast<const u32x4 *>(a.dy + t * pitch + at), d);
@@ -867,7 +868,7 @@ inline Geom attention_geom(const na1d_train_layer &l, int64_t N, int64_t T, Layo
 }
 
 template <class DT> int norm_apply(const na1d_train_layer &l, int which, char *y, const char *x, float *mean, float *rstd, int64_t M, const char *add, int64_t T, hipStream_t s) {
-    const Chunks c = bn_chunks(M);
+    const Chunks c = bn_chunks(M, 256);
     const na1d_train_norm &n = l.norm[which];
     bn_apply_kernel<DT><<<dim3((unsigned)(l.dim / kBnCols), (unsigned)c.count), kBnThreads, 0, s>>>(
         BnApply{y, x, n.batch_mean, n.batch_var, n.weight, n.bias, mean, rstd, n.batches, n.eps, (int)M, l.dim, c.rows, add, (int)T});
@@ -884,7 +885,7 @@ int to_channels(const na1d_train_layer &l, void *out, const void *x, int64_t N, 
 template <class DT>
 int product_and_norm_backward(Gemm a, const na1d_train_layer &l, int which, char *dx, const char *x, const char *add, const float *mean, const float *rstd, float *part,
                               hipStream_t s) {
-    const Chunks c = bn_chunks(a.M);
+    const Chunks c = bn_chunks(a.M, 64);
     const dim3 grid((unsigned)(l.dim / kBnCols), (unsigned)c.count);
     float *part_dyx = part + (int64_t)kBnParts * l.dim;
     const int rows = gemm_rows(a.M, a.outputs);
@@ -899,7 +900,7 @@ int product_and_norm_backward(Gemm a, const na1d_train_layer &l, int which, char
         chunks = c.count;
     }
     const na1d_train_norm &n = l.norm[which];
-    bn_bwd_apply_kernel<DT><<<grid, kBnThreads, 0, s>>>(BnBackward{dx, a.out, x, add, part, part_dyx, n.weight, mean, rstd, n.dweight, n.dbias, a.M, l.dim, c.rows, chunks});
+    bn_bwd_apply_kernel<DT><<<grid, kBnApplyThreads, 0, s>>>(BnBackward{dx, a.out, x, add, part, part_dyx, n.weight, mean, rstd, n.dweight, n.dbias, a.M, l.dim, c.rows, chunks});
     return launch_status();
 }
 
