@@ -374,7 +374,9 @@ int na1d_train_layer_backward(const na1d_train_layer *l, void *dx, const void *d
  *   pooled, dpooled: [N, 2 C] fp32, the means and then the deviations, as the forward left them, and their gradients.
  * context: of [x, mean, std] along C ([N, 3 C, T]; mean and std = sqrt(max(var, eps)) of a row over T, var with T - 1 degrees of
  *   freedom, repeated along T); var, std: [N, C], as the forward rounded them.
+ * And the context itself of x, mean and std (T from 8 to 2048, C T^2 below 2^32; 16-bit values of either type).
  */
+int na1d_train_context(void *out, const void *x, const void *mean, const void *std, int64_t N, int64_t C, int64_t T, void *stream);
 int na1d_train_pool_backward(void *dlogits, void *dx, const void *logits, const void *x, const float *pooled, const float *dpooled,
                              int64_t N, int64_t C, int64_t T, float eps, int dtype, void *stream);
 int na1d_train_context_backward(void *dx, const void *dctx, const void *x, const void *var, const void *std, int64_t N, int64_t C,

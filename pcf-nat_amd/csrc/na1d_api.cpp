@@ -524,6 +524,13 @@ int na1d_train_pool_backward(void *dlogits, void *dx, const void *logits, const 
     if (misaligned(dlogits) || misaligned(dx) || misaligned(logits) || misaligned(x)) return NA1D_ERR_ALIGN;
     return na1d::train::run_pool_backward(dlogits, dx, logits, x, pooled, dpooled, N, C, T, eps, dtype, (hipStream_t)stream);
 }
+int na1d_train_context(void *out, const void *x, const void *mean, const void *std, int64_t N, int64_t C, int64_t T, void *stream) {
+    const int st = pool_check(N, C, T, NA1D_BF16);
+    if (st != NA1D_OK) return st;
+    if (!out || !x || !mean || !std) return NA1D_ERR_NULL;
+    if (misaligned(out) || misaligned(x)) return NA1D_ERR_ALIGN;
+    return na1d::train::run_context(out, x, mean, std, N, C, T, (hipStream_t)stream);
+}
 int na1d_train_context_backward(void *dx, const void *dctx, const void *x, const void *var, const void *std, int64_t N, int64_t C, int64_t T, float eps,
                                 int dtype, void *stream) {
     const int st = pool_check(N, C, T, dtype);

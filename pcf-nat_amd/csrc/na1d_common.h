@@ -228,6 +228,7 @@ int run_backward(const na1d_train_layer &l, void *dx, const void *dout, const vo
 bool pool_ok(int64_t N, int64_t C, int64_t T);
 int run_pool_backward(void *dlogits, void *dx, const void *logits, const void *x, const float *pooled, const float *dpooled, int64_t N, int64_t C, int64_t T,
                       float eps, int dtype, hipStream_t s);
+int run_context(void *out, const void *x, const void *mean, const void *std, int64_t N, int64_t C, int64_t T, hipStream_t s);
 int run_context_backward(void *dx, const void *dctx, const void *x, const void *var, const void *std, int64_t N, int64_t C, int64_t T, float eps, int dtype,
                          hipStream_t s);
 }  // namespace train

@@ -30,7 +30,7 @@ SYMBOLS = _UNFUSED + ("na1d_fused_forward", "na1d_fused_backward", "na1d_fused_b
                       "na1d_fused_forward_dilated", "na1d_fused_forward_clear", "na1d_fused_backward_dilated",
                       "na1d_fused_backward_dilated_workspace_bytes", "na1d_encode", "na1d_encode_workspace_bytes",
                       "na1d_train_layer_saved_bytes", "na1d_train_layer_workspace_bytes", "na1d_train_layer_forward",
-                      "na1d_train_to_channels", "na1d_train_pool_backward", "na1d_train_context_backward",
+                      "na1d_train_to_channels", "na1d_train_pool_backward", "na1d_train_context_backward", "na1d_train_context",
                       "na1d_train_layer_backward", "na1d_version", "na1d_status_string")
 UNSUPPORTED = -8
 
@@ -107,6 +107,8 @@ def load():
     lib.na1d_train_layer_forward.argtypes = [_ptr, _int] + [_ptr] * 3 + [_i64, _ptr, _i64, _i64, _i64, _ptr]
     lib.na1d_train_to_channels.restype = _int
     lib.na1d_train_to_channels.argtypes = [_ptr] * 3 + [_i64, _i64, _ptr]
+    lib.na1d_train_context.restype = _int
+    lib.na1d_train_context.argtypes = [_ptr] * 4 + [_i64] * 3 + [_ptr]
     lib.na1d_train_pool_backward.restype = lib.na1d_train_context_backward.restype = _int
     lib.na1d_train_pool_backward.argtypes = [_ptr] * 6 + [_i64] * 3 + [_f32, _int, _ptr]
     lib.na1d_train_context_backward.argtypes = [_ptr] * 5 + [_i64] * 3 + [_f32, _int, _ptr]
