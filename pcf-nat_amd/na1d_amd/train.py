@@ -198,7 +198,7 @@ class _Context(_Pooling):
     def forward(ctx, x, eps):
         n, c, t = x.shape
         mean, var, std = _statistics(x, eps)
-        if t >= 8 and c * t * t < 1 << 32 and _lie(x, x.dtype, (n, c, 1), mean, std):
+        if x.is_cuda and t >= 8 and c * t * t < 1 << 32 and _lie(x, x.dtype, (n, c, 1), mean, std):
             out = torch.empty((n, 3 * c, t), dtype=x.dtype, device=x.device)
             with torch.cuda.device(x.device):
                 _lib.check(_lib.load().na1d_train_context(out.data_ptr(), x.data_ptr(), mean.data_ptr(), std.data_ptr(), n, c, t,
