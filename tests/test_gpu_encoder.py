@@ -66,6 +66,16 @@ def test_tiles_of_every_size(groups, batch, frames):
     assert native is not None and _near(native, modules)
 
 
+@pytest.mark.parametrize("groups", [(8, 4), (2, 1)])
+@pytest.mark.parametrize("batch,frames", [(328, 100), (427, 96), (491, 100), (512, 96), (513, 96)])
+def test_row_tiles_dealt_out_evenly(groups, batch, frames):
+    """16385 to 24576 tokens: the first, the middle and the last numbers of workgroups with three row tiles, the last tile full and
+    not, and the first size behind."""
+    model = _model(groups=groups)
+    native, modules = _both(model, _input(batch, frames))
+    assert native is not None and _near(native, modules)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("batch,frames", [(31, 100), (32, 256), (33, 258), (85, 260), (86, 260), (31, 400), (32, 400), (32, 402),
                                           (53, 402), (54, 402), (65, 1000), (65, 1002), (68, 1002), (69, 1002), (86, 1002)])
