@@ -78,20 +78,6 @@ Strides strides_of(const Geometry &g) {
     if (g.in_place) return Strides{{g.T * 3 * g.H * g.C, g.C, 3 * g.H * g.C}, {g.T * g.H * g.C, g.C, g.H * g.C}};
     return Strides{{g.H * g.T * g.C, g.T * g.C, g.C}, {g.H * g.T * g.C, g.T * g.C, g.C}};
 }
-// The gradient of the bias, which the backward's kernel adds to: the forward's sets it to zero on the way, for the first
-// backward of a node (any further one clears its own).  A graph may hold the one and not the other, or replay them unevenly, so
-// under capture every backward clears its own too.
-struct Cleared : torch::CustomClassHolder {
-    explicit Cleared(Tensor t) : sums(std::move(t)) {}
-    Tensor take() {
-        const std::lock_guard<std::mutex> lock(mutex);
-        return std::exchange(sums, Tensor());
-    }
-
-  private:
-    std::mutex mutex;                                 // a retained graph may be walked by several threads
-    Tensor sums;
-};
 bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
 
 int forward_kernel(const Geometry &g, const Tensor &out, const Tensor &lse, const Tensor &clear, const void *q, const void *k, const void *v, const Tensor &rpb, const Tensor &t_valid,
@@ -134,21 +120,32 @@ void remember(AutogradContext *ctx, const Geometry &g, const MaybeTensor &rpb, c
     ctx->saved_data["p"] = g.drop.p;
     ctx->saved_data["bias"] = rpb && rpb->requires_grad();
     ctx->saved_data["bias_shape"] = rpb ? rpb->sizes().vec() : std::vector<int64_t>{};
-    if (cleared.defined()) ctx->saved_data["cleared"] = c10::IValue::make_capsule(c10::make_intrusive<Cleared>(cleared));
-}
-// The bias' gradient, all zeros; undefined where none is asked for.
-Tensor begin_bias_gradient(AutogradContext *ctx, const Tensor &like) {
-    if (!ctx->saved_data["bias"].toBool()) return Tensor();
-    const auto held = ctx->saved_data.find("cleared");
-    if (held != ctx->saved_data.end() && !capturing()) {
-        Tensor t = c10::static_intrusive_pointer_cast<Cleared>(held->second.toCapsule())->take();
-        if (t.defined()) return t;
-    }
-    return at::zeros(ctx->saved_data["bias_shape"].toIntVector(), like.options().dtype(at::kFloat));
+    if (cleared.defined()) ctx->saved_data["cleared"] = cleared;
 }
 Geometry recall(AutogradContext *ctx) {
     const auto v = ctx->saved_data["geometry"].toIntVector();
     return Geometry{v[0], v[1], v[2], v[3], v[4], v[5], v[6], ctx->saved_data["scale"].toDouble(), {ctx->saved_data["p"].toDouble(), (uint64_t)v[7]}, v[8] != 0};
+}
+// The gradient of the bias, all zeros, which the backward's kernel adds to; undefined where none is asked for.  The forward's kernel has
+// cleared it on the way, for the first backward of a node; any further one, on whatever thread, clears its own.  (The tensor's version
+// says that it is taken, also to a copy of the node's data as compiled autograd makes them.)  A graph may hold the forward and not the
+// backward, or replay them unevenly, so under capture every backward clears its own too.
+Tensor begin_bias_gradient(AutogradContext *ctx, const Tensor &like) {
+    if (!ctx->saved_data["bias"].toBool()) return Tensor();
+    const auto held = ctx->saved_data.find("cleared");
+    if (held != ctx->saved_data.end() && !capturing()) {
+        static std::mutex mutex;
+        const std::lock_guard<std::mutex> lock(mutex);
+        if (held->second.isTensor()) {
+            Tensor t = std::move(held->second).toTensor();
+            held->second = c10::IValue();
+            if (t.defined() && t._version() == 0) {
+                t.unsafeGetTensorImpl()->bump_version();
+                return t;
+            }
+        }
+    }
+    return at::zeros(ctx->saved_data["bias_shape"].toIntVector(), like.options().dtype(at::kFloat));
 }
 Tensor bias_of(const MaybeTensor &rpb, const Geometry &g, bool node) {
     if (rpb && !node && rpb->scalar_type() == at::kFloat && rpb->is_contiguous()) return *rpb;

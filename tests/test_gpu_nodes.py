@@ -151,3 +151,26 @@ def test_bias_gradient_begins_at_zero(N, H, T, C, W, left, dilation, p, in_place
         graph.replay()
         torch.testing.assert_close(captured, want, rtol=1e-4, atol=1e-4 * want.abs().max().item())
     torch.testing.assert_close(torch.autograd.grad(kept, eager, g)[0], want, rtol=1e-4, atol=1e-4 * want.abs().max().item())
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+def test_bias_gradient_under_compiled_autograd(in_place):
+    """Which copies a node's data, also for a graph that is walked twice."""
+    from torch._dynamo import compiled_autograd
+    N, H, T, C, W = 2, 4, 50, 32, 15
+    rpb = _rand(H, W, dtype=torch.float32, seed=5)
+    tensors = [_rand(N, T, 3, H, C, seed=3)] if in_place else [_rand(N * H, T, C, seed=i) for i in range(3)]
+    g = _rand(*((N, T, H * C) if in_place else (N * H, T, C)), seed=9, grad=False)
+
+    def call():
+        _dirty(H, W)
+        return na1d_fused_qkv(*tensors, W, 7, rpb=rpb, scale=0.3) if in_place else na1d_fused(*tensors, W, 7, rpb=rpb, num_heads=H, scale=0.3)
+
+    call().backward(g)
+    want = rpb.grad
+    with compiled_autograd._enable(lambda graph: torch.compile(graph, backend="eager")):
+        out, other = call(), call()
+        for o, keep in ((out, True), (other, False), (out, True), (out, False)):
+            rpb.grad = None
+            o.backward(g, retain_graph=keep)
+            torch.testing.assert_close(rpb.grad, want, rtol=1e-4, atol=1e-4 * want.abs().max().item())     # float atomics, as in _same
