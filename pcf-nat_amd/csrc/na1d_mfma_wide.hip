@@ -324,13 +324,13 @@ wide_bwd_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__restrict__
     row_lane.init(0, lane);
     tr_lane.init(0, lane);
 
-    // The scores' sums start at rpb / scale (-inf outside the window).  Every wave has a table of its own, in the place of its scores.
-    f32x4 bias[NBV];
+    // As the forward adds it, behind the product: rpb / scale, at which the sums could start, has no value for every scale.
+    // Every wave has a table of its own, in the place of its scores.
+    float bias[NBV][4];
     {
         LDS_PTR(float) mine = (LDS_PTR(float))(sc_lds + wave * (NBV * 2 * kScoreTile));
-        const float inv_scale = __builtin_amdgcn_rcpf(scale);
         const float *rpb_h = rpb ? rpb + head * W : nullptr;
-        for (int j = lane; j < kBiasSlots; j += 64) mine[j] = rpb_h && j < W ? rpb_h[j] * inv_scale : 0.f;
+        for (int j = lane; j < kBiasSlots; j += 64) mine[j] = rpb_h && j < W ? rpb_h[j] * kLog2e : 0.f;
 #pragma unroll
         for (int vb = 0; vb < NBV; ++vb)
 #pragma unroll
@@ -394,7 +394,7 @@ wide_bwd_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__restrict__
             RowOperand<C> qop, gop;
             read_rows<C>(qop, q_now + wave * LL::kTileBytes, row_lane);
             read_rows<C>(gop, g_now + wave * LL::kTileBytes, row_lane);
-            const float nlse2 = -lse_lds[(step & 1) * 64 + wave * 16 + n] * kLog2e;
+            const float lse2 = lse_lds[(step & 1) * 64 + wave * 16 + n] * kLog2e;
             const int s0 = 16 * qt - shift;
             const int qrow = 16 * qt + n;
             const bool edge = s0 < 0 || s0 + 16 * NBV > tv;
@@ -412,11 +412,11 @@ wide_bwd_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__restrict__
                 const int off = key_tile(vb);
                 read_rows<C>(kop, k_lds + off, row_lane);
                 read_rows<C>(vop, v_lds + off, row_lane);
-                const f32x4 s = dot_rows_mma<DT, C>(kop, qop, bias[vb]);
+                const f32x4 s = dot_rows_mma<DT, C>(kop, qop);
                 const f32x4 d = dot_rows_mma<DT, C>(vop, gop);
                 float z[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) z[r] = __builtin_fmaf(s[r], scale2, nlse2);
+                for (int r = 0; r < 4; ++r) z[r] = __builtin_fmaf(s[r], scale2, bias[vb][r]) - lse2;
                 if (edge) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {

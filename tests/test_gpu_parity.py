@@ -483,6 +483,21 @@ def test_wide_backward_however_sequences_are_cut(H, T, C, W, L, dtype):
             assert O.rel_l2(b.float(), ref) < TOL[dtype], name
 
 
+@pytest.mark.parametrize("scale,size", [(1e-39, 1.0), (2e38, 1e-30)])
+@pytest.mark.parametrize("H,T,C,W,L", [(2, 100, 16, 65, 32), (4, 150, 32, 33, 16), (2, 300, 64, 80, 40), (2, 33, 128, 49, 24)])
+def test_wide_backward_at_the_ends_of_the_scales(H, T, C, W, L, scale, size):
+    """Scales whose reciprocal is no normal number, and products of which nothing is left: the bias keeps its value."""
+    q, k, v, do = make_inputs(2 * H, T, C, W, 13, torch.bfloat16, n=4)
+    q, k = (t * size for t in (q, k))
+    rpb = torch.randn(H, W, generator=torch.Generator().manual_seed(3)) * 2
+    leaves = [t.cuda().requires_grad_(True) for t in (q, k, v, rpb)]
+    na1d_fused(*leaves[:3], W, L, rpb=leaves[3], num_heads=H, scale=scale).backward(do.cuda())
+    _, _, *want = O.na1d_backward(q.float() * 0, k.float() * 0, v.float(), do.float(), W, L, rpb, None, H)
+    for leaf, ref in zip(leaves[2:], want):
+        assert O.rel_l2(leaf.grad.float().cpu(), ref) < TOL[torch.bfloat16]
+    assert all(torch.isfinite(leaf.grad).all() for leaf in leaves)
+
+
 @pytest.mark.parametrize("case", [(256, 16, 100, 16, 27, 13, torch.bfloat16), (128, 8, 300, 32, 15, 7, torch.float16)],
                          ids=lambda c: "x".join(map(str, c[:6])))
 def test_full_launches_in_the_projection_layout_and_through_the_two_call_api(case):
