@@ -483,6 +483,40 @@ def test_wide_backward_however_sequences_are_cut(H, T, C, W, L, dtype):
             assert O.rel_l2(b.float(), ref) < TOL[dtype], name
 
 
+@pytest.mark.parametrize("H,T,C,W,L,counts", [
+    (8, 16, 16, 80, 40, (1, 300)), (8, 33, 32, 65, 32, (1, 16, 300)), (8, 64, 32, 49, 24, (1, 120)), (8, 64, 64, 65, 32, (2, 10, 130)), (8, 48, 64, 33, 16, (1, 4, 30)),
+    (4, 80, 128, 33, 16, (1, 20, 80)), (8, 96, 64, 33, 16, (1, 12, 60)), (8, 97, 16, 33, 32, (1, 16, 130)), (1, 200, 24, 70, 69, (1, 11, 40)),
+    (2, 300, 128, 80, 0, (1, 14, 60)), (8, 300, 48, 56, 27, (1, 3, 30)), (16, 501, 32, 41, 20, (1, 5, 20))])
+@pytest.mark.parametrize("dilation,p", [(1, 0.0), (3, 0.1)])
+def test_wide_backward_in_strips_and_walking(H, T, C, W, L, counts, dilation, p):
+    """Batches on each side of the rules: one strip, few strips and walked sequences give the first sample the same bits, with
+    a workspace as without, and the oracle's gradients."""
+    dtype = torch.bfloat16
+    N = max(counts)
+    q, k, v, do = make_inputs(N * H, T, C, W, 17, dtype, n=4, scale=C ** -0.5)
+    rpb = torch.randn(H, W, generator=torch.Generator().manual_seed(3)) * 0.5
+    t_valid = torch.full((N,), T - T // 4, dtype=torch.int32)
+    t_valid[1::2] = T
+    got = []
+    for n in counts:
+        leaves = [t[:n * H].cuda().requires_grad_(True) for t in (q, k, v)] + [rpb.cuda().requires_grad_(True)]
+        for deterministic in (False, True):
+            out = na1d_fused(*leaves[:3], W, L, rpb=leaves[3], t_valid=t_valid[:n].cuda(), num_heads=H, dilation=dilation, dropout_p=p, seed=5,
+                             deterministic=deterministic)
+            got.append((n, torch.autograd.grad(out, leaves, do[:n * H].cuda())))
+    for i, (n, grads) in enumerate(got):
+        for a, b in zip(grads[:3], got[0][1][:3]):
+            assert torch.equal(a[:H], b[:H]), n
+        if i % 2:
+            assert O.rel_l2(grads[3].cpu(), got[i - 1][1][3].cpu()) < 1e-4, n            # fp32 sums of one set of terms in two orders
+    n = counts[1 if len(counts) > 1 and counts[1] * H * T < 20000 else 0]
+    if p == 0.0:
+        want = O.na1d_backward(*(t[:n * H].float() for t in (q, k, v, do)), W, L, rpb, T - t_valid[:n], H, dilation=dilation)
+        grads = next(g for m, g in got if m == n)
+        for a, ref in zip(grads, want):
+            assert O.rel_l2(a.float().cpu(), ref) < TOL[dtype]
+
+
 @pytest.mark.parametrize("scale,size", [(1e-39, 1.0), (2e38, 1e-30)])
 @pytest.mark.parametrize("H,T,C,W,L", [(2, 100, 16, 65, 32), (4, 150, 32, 33, 16), (2, 300, 64, 80, 40), (2, 33, 128, 49, 24)])
 def test_wide_backward_at_the_ends_of_the_scales(H, T, C, W, L, scale, size):
