@@ -642,8 +642,9 @@ global_dq_kernel(char *__restrict__ dq, float *__restrict__ delta, const char *_
 // the 32-deep product.
 // A lane has one key of a tile, so everything else in an exponent is a constant of the query row, of which there are two:
 // minus its LSE in the log2 domain, with a padded row's -100 taken out of it, and the same less 100 for valid rows, which
-// is what padded keys see.  The lane's key decides once where it reads, and no score is masked; rows past the sequence
-// have minus infinity there.  Minus delta is where the product dO . V^T starts (without dropout).
+// is what padded keys see.  The lane's key decides once where it reads, and no score is masked.  Minus delta is where the product
+// dO . V^T starts (without dropout).  Rows past the sequence, in the last chunk, are taken out by themselves: their products
+// are not zero where a key is infinite.
 // With the masks and both subtractions worked out for each score (a general form of the loop beside a plain one), in a trace: 64 x 4
 // sequences of up to 1000 rows, 64 channels 193..203 -> 158..180 us (all rows valid: 177 -> 162), 20 x 8 of 700, 32 channels
 // 42.4 -> 35.2, 8 x 8 of 1500, 128 channels 203 -> 188.
@@ -719,7 +720,7 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
         for (int ct = 0; ct < CT; ++ct) acck[h][ct] = accv[h][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
-    // one chunk of queries; `whole`: all of its four tiles exist
+    // one chunk of queries; `whole`: all of its rows exist
     auto chunk = [&](auto whole, int c0, LDS_PTR(char) buf) {
         LDS_PTR(char) q_lds = buf;
         LDS_PTR(char) g_lds = buf + kStep;
@@ -730,7 +731,7 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
             if (!decltype(whole)::value && c0 + qi >= tiles) continue;
             u32x4 pb[QT], db[QT];
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {                   // a tile past the last has zeros in Q, dO and P
+            for (int j = 0; j < 2; ++j) {
                 RowOperand<C> qop, gop;
                 read_rows<C>(qop, q_lds + (qi + j) * LL::kTileBytes, row_lane);
                 read_rows<C>(gop, g_lds + (qi + j) * LL::kTileBytes, row_lane);
@@ -752,6 +753,7 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
                         } else {
                             dsv[r] = p[r] * dp[r];
                         }
+                        if (!decltype(whole)::value && 16 * (c0 + qi + j) + 4 * g + r >= T) p[r] = dsv[r] = 0.f;
                     }
                     pb[h][2 * j] = Mma<DT>::pack(p[0], p[1]);
                     pb[h][2 * j + 1] = Mma<DT>::pack(p[2], p[3]);
@@ -779,7 +781,6 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
         wait_direct();
         const int qrow = 16 * (c0 + wave) + n;
         float constant = (qrow >= tv || g == 1 ? mask2 : 0.f) - kLog2e * row_lse;
-        if (qrow >= T) constant = kNegInf;
         if (g >= 2) constant = -row_delta;                  // g 2 and 3 the same
         *reinterpret_cast<LDS_PTR(float)>(buf_lds + at + 2 * kStep + (min(g, 2) * kRows + 16 * wave + n) * 4) = constant;
         barrier_lds();      // this chunk has landed, and every wave is done with the one before, whose buffer the next takes
@@ -791,7 +792,7 @@ global_dkv_kernel(char *__restrict__ dk, char *__restrict__ dv, const char *__re
         at = kBuf - at;
     };
     int c0 = 0;
-    for (; c0 + kStripTiles <= tiles; c0 += kStripTiles) step(std::true_type{}, c0);
+    for (; 16 * (c0 + kStripTiles) <= T; c0 += kStripTiles) step(std::true_type{}, c0);
     if (c0 < tiles) step(std::false_type{}, c0);
 
     const bool stream = stores_whole_lines(pitch, C, 0);
@@ -897,7 +898,7 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
             drop_key[h] = DROP ? dropout_row_key((uint64_t)b * T + qrow, a.drop) : 0u;
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) acc[h][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (g < 3) ref_lds[g * kRows + qrow] = g == 2 ? -dl : qrow >= T ? kNegInf : g == 1 ? mask2 - lse2 : ref[h];
+            if (g < 3) ref_lds[g * kRows + qrow] = g == 2 ? -dl : g == 1 ? mask2 - lse2 : ref[h];
         }
         const int plain_keys = 16 * own[0] >= tv ? T : min(T, tv);       // keys without a mask: this wave's first tile is padded, so are the others
 #pragma unroll
@@ -986,6 +987,11 @@ global_bwd_short_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__re
                 } else {
                     dsv[r] = p[r] * dp[r];
                 }
+            }
+            if (16 * (qi + 1) > T) {           // rows past the sequence do not exist
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (16 * qi + 4 * g + r >= T) p[r] = dsv[r] = 0.f;
             }
             pb[h] = u32x2{Mma<DT>::pack(p[0], p[1]), Mma<DT>::pack(p[2], p[3])};
             db[h] = u32x2{Mma<DT>::pack(dsv[0], dsv[1]), Mma<DT>::pack(dsv[2], dsv[3])};

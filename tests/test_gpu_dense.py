@@ -99,6 +99,28 @@ def test_lengths_off_the_tiles(T, C, dtype):
             assert O.rel_l2(got[part].float(), exact[part]) < TOL[dtype], n
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=["bf16", "fp16"])
+@pytest.mark.parametrize("T,C", [(17, 16), (50, 64), (100, 32), (127, 128), (129, 64), (144, 16), (150, 128), (210, 32), (300, 64), (1000, 64)])
+def test_keys_whose_scores_are_minus_infinity(T, C, dtype):
+    """They take no part, and have zeros for gradients; so do rows past the sequence, whose products with them are no numbers."""
+    N, H = 2, 2
+    q, k, v, do = make_inputs(N * H, T, C, 0, 83, dtype, n=4)
+    q[..., 3] = q[..., 3].abs() + 0.5
+    gone = sorted({0, 5, T // 2, T - 1})
+    k[:, gone, 3] = -float("inf")
+    t_valid = torch.tensor([T, T - T // 5], dtype=torch.int32)
+    for valid, p in ((None, 0.0), (t_valid, 0.0), (t_valid, 0.25)):
+        qd, kd, vd = (t.cuda().requires_grad_(True) for t in (q, k, v))
+        out = global_attention(qd, kd, vd, H, t_valid=None if valid is None else valid.cuda(), scale=C ** -0.5, dropout_p=p, seed=3)
+        _, dk, dv = torch.autograd.grad(out, (qd, kd, vd), do.cuda())
+        assert torch.isfinite(out).all() and torch.isfinite(dv).all() and torch.isfinite(dk).all()
+        assert not dv[:, gone].any() and not dk[:, gone].any()
+        if p == 0.0:
+            pad = 0 if valid is None else T - valid
+            _, wk, wv = O.global_backward(q.float(), k.float(), v.float(), do.float(), C ** -0.5, torch.zeros(N, dtype=torch.int64) + pad, H)
+            assert O.rel_l2(dk.float(), wk) < TOL[dtype] and O.rel_l2(dv.float(), wv) < TOL[dtype]
+
+
 def test_global_attention_without_padding_and_without_lse():
     N, H, T, C, dtype = 2, 2, 150, 32, torch.bfloat16
     B = N * H
