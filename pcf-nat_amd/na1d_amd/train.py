@@ -12,6 +12,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 from torch.autograd.function import once_differentiable
+from torch.autograd.graph import increment_version
 
 from . import _lib
 
@@ -31,6 +32,65 @@ class _Layer(ctypes.Structure):                    # na1d_train_layer
 def _aligned(t):
     t = t.contiguous()
     return t.clone() if t.data_ptr() % 16 else t
+
+
+class _ByCtypes:
+    """``train_forward`` and ``train_backward`` of ``csrc/na1d_torch.cpp``, which belongs to the library beside it, for one that
+    NA1D_LIB names."""
+
+    @staticmethod
+    def _ptr(t):
+        return None if t is None else t.data_ptr()
+
+    @classmethod
+    def _ptrs(cls, ts):
+        return (_P * 5)(*map(cls._ptr, ts))
+
+    @classmethod
+    def train_forward(cls, x, by_channel, geom, state, numbers, scale_attn, scale_mlp, pos, params):
+        lib, c, (n, t, dim) = _lib.load(), _Layer(*geom), x.shape
+        dense, norms = pos is not None, params[1:5]
+        c.w, c.b = cls._ptrs([*params[5::2], params[0] if dense else None]), cls._ptrs(params[6::2])
+        for i, to in enumerate(c.norm):
+            to.weight, to.bias, to.eps, to.batches = norms[2 * i].data_ptr(), norms[2 * i + 1].data_ptr(), numbers[2 * i + 1], state[3 * i + 2].data_ptr()
+        c.rpb, c.pos, c.scale_attn, c.scale_mlp = None if dense else params[0].data_ptr(), cls._ptr(pos), cls._ptr(scale_attn), cls._ptr(scale_mlp)
+        ref, out = ctypes.byref(c), torch.empty_like(x)
+        with torch.cuda.device(x.device):
+            stream = torch.cuda.current_stream().cuda_stream
+            sizes = lib.na1d_train_layer_saved_bytes(ref, n, t), lib.na1d_train_layer_workspace_bytes(ref, n, t, 0)
+            _lib.check(min(*sizes, 0), "na1d_train_layer_saved_bytes")
+            saved, ws = (torch.empty(s, dtype=torch.uint8, device=x.device) for s in sizes)
+            if by_channel is None:
+                by_channel = x.new_empty((n, dim, t))
+                _lib.check(lib.na1d_train_to_channels(ref, by_channel.data_ptr(), x.data_ptr(), n, t, stream), "na1d_train_to_channels")
+            x1 = x.new_empty((n, dim, t))
+            for part, (of, to) in enumerate(((by_channel, x1), (x1, out))):
+                stats = torch.batch_norm_update_stats(of, state[3 * part], state[3 * part + 1], numbers[2 * part])
+                c.norm[part].batch_mean, c.norm[part].batch_var = map(cls._ptr, stats)
+                _lib.check(lib.na1d_train_layer_forward(ref, part, to.data_ptr(), x.data_ptr(), saved.data_ptr(), sizes[0], ws.data_ptr(),
+                                                        sizes[1], n, t, stream), "na1d_train_layer_forward")
+        increment_version(state)
+        return out, saved
+
+    @classmethod
+    def train_backward(cls, dout, x, saved, geom, rpb, n1w, n2w, scale_attn, scale_mlp, pos, shapes):
+        lib, c, (n, t, _) = _lib.load(), _Layer(*geom), x.shape
+        dout, dx = _aligned(dout), torch.empty_like(x)
+        grads = [torch.zeros(shapes[0], dtype=torch.float32, device=x.device)]       # the bias of the scores is added to
+        grads += [torch.empty(s, dtype=torch.float32, device=x.device) for s in shapes[1:]]
+        c.dw, c.db = cls._ptrs(grads[5::2] + ([] if pos is None else grads[:1])), cls._ptrs(grads[6::2])
+        for to, w, dw, db in zip(c.norm, (n1w, n2w), grads[1:5:2], grads[2:5:2]):
+            to.weight, to.dweight, to.dbias = w.data_ptr(), dw.data_ptr(), db.data_ptr()
+        c.rpb, c.drpb, c.pos, c.scale_attn, c.scale_mlp = cls._ptr(rpb), grads[0].data_ptr(), cls._ptr(pos), cls._ptr(scale_attn), cls._ptr(scale_mlp)
+        ref = ctypes.byref(c)
+        with torch.cuda.device(x.device):
+            nbytes = lib.na1d_train_layer_workspace_bytes(ref, n, t, 1)
+            _lib.check(min(nbytes, 0), "na1d_train_layer_workspace_bytes")
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+            _lib.check(lib.na1d_train_layer_backward(ref, dx.data_ptr(), dout.data_ptr(), x.data_ptr(), saved.data_ptr(), saved.numel(),
+                                                     ws.data_ptr(), nbytes, n, t, torch.cuda.current_stream().cuda_stream),
+                       "na1d_train_layer_backward")
+        return [dx, *grads]
 
 
 class _TrainLayer(torch.autograd.Function):
@@ -92,9 +152,6 @@ def layer(m, x, pos_emb=None, attn_mask_global=None):
     if not (x.is_cuda and m.training and torch.is_grad_enabled() and torch.is_autocast_enabled("cuda")
             and x.dim() == 3 and x.dtype in (torch.bfloat16, torch.float16) and x.dtype == torch.get_autocast_dtype("cuda")):
         return None
-    nodes = _lib.nodes()
-    if nodes is None:
-        return None
     # Sixteen layers a step, some forty lookups each: by the modules' own dictionaries, past nn.Module.__getattr__.
     parts = m._modules
     a, mlp, norms = parts.get("attn"), parts.get("mlp"), (parts.get("norm1"), parts.get("norm2"))
@@ -153,7 +210,7 @@ def layer(m, x, pos_emb=None, attn_mask_global=None):
     if not m.local:
         pos = _aligned((pos_emb.transpose(1, 2) if cf else pos_emb).to(x.dtype))
     scales = (_drop_path_scale(parts.get("drop_path"), xt), _drop_path_scale(parts.get("drop_path"), xt))
-    out = _TrainLayer.apply(xt, by_channel, geom, nodes, norms, scales, pos, *params)
+    out = _TrainLayer.apply(xt, by_channel, geom, _lib.nodes() or _ByCtypes, norms, scales, pos, *params)
     return out.transpose(1, 2) if cf else out
 
 

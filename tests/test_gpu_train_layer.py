@@ -5,7 +5,7 @@ import copy
 import pytest
 import torch
 
-from na1d_amd import models, train
+from na1d_amd import _lib, models, train
 from oracle import na1d_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -141,6 +141,31 @@ def test_what_the_node_does_not_cover_stays_with_the_modules():
         layer(x).sum().backward()
         assert layer.mlp.fc1.weight.grad is None and layer.mlp.fc2.weight.grad is not None
         assert layer.norm1.norm.running_mean._version > before
+
+
+@pytest.mark.parametrize("family,groups,heads,window,drop_path", [("mfa", 1, 16, 27, 0.3), ("pcf", 8, 16, 27, 0.0), ("mfa", 1, 4, 0, 0.0), ("pcf", 1, 4, 0, 0.3)])
+def test_a_library_that_is_named_serves_training_layers_too(family, groups, heads, window, drop_path, monkeypatch):
+    """Without the extension beside the package's own library the launches go through ctypes: the same bits and version counts."""
+    _, gpu = _layers(family, groups, heads, window, 1, 40, drop_path, seed=2)
+    gen = torch.Generator().manual_seed(1)
+    shape = (6, 256, 40) if family == "pcf" else (6, 40, 256)
+    x, g = (torch.randn(shape, generator=gen).half().cuda() for _ in range(2))
+    pos = None if window else models.sinusoid_table(256, 40, family == "pcf").cuda()
+    results = []
+    for named in (False, True):
+        monkeypatch.setattr(_lib, "_other_build", named)
+        layer, leaf = copy.deepcopy(gpu), x.clone().requires_grad_(True)
+        torch.manual_seed(4)
+        with torch.autocast("cuda", dtype=torch.float16):
+            out = models.train_layer(layer, leaf, pos)
+        assert out is not None
+        out.backward(g)
+        results.append(([out.detach(), leaf.grad, *(b for b in layer.buffers())], [p.grad for p in layer.parameters()], [b._version for b in layer.buffers()]))
+    for a, b in zip(results[0][0], results[1][0]):
+        assert torch.equal(a, b)
+    for (name, _), a, b in zip(gpu.named_parameters(), results[0][1], results[1][1]):
+        assert torch.equal(a, b) if "relative" not in name else O.rel_l2(a, b) < 1e-5, name       # the scores' bias: float atomics
+    assert results[0][2] == results[1][2]
 
 
 def _off_alignment(t):
