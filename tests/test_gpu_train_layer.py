@@ -93,6 +93,23 @@ def test_native_training_layer(family, groups, heads, window, dilation, dtype, b
         assert e < bound, (name, e)
 
 
+# The product in front of a norm's backward: it sums for the norm in blocks of 32 rows up to 8128 tokens and of 64 rows up to 16384;
+# beyond, a kernel of its own does.  Last blocks of 4, 6, 64, 44 and 16 rows.
+@pytest.mark.parametrize("batch,T", [(81, 100), (83, 98), (128, 100), (163, 100), (164, 100)])
+@pytest.mark.parametrize("family,groups,heads,window,dtype", [("mfa", 1, 16, 27, "fp16"), ("pcf", 8, 16, 27, "bf16"), ("mfa", 1, 4, 0, "fp16")])
+def test_gradients_behind_every_form_of_the_norms_sums(family, groups, heads, window, dtype, batch, T):
+    """Bounds as in test_native_training_layer."""
+    cpu, gpu = _layers(family, groups, heads, window, 1, T, 0.0, seed=T)
+    gen = torch.Generator().manual_seed(batch)
+    shape = (batch, 256, T) if family == "pcf" else (batch, T, 256)
+    x = torch.randn(shape, generator=gen) + 0.5 * torch.randn((1,) + tuple(256 if s == 256 else 1 for s in shape[1:]), generator=gen)
+    err = _errors(cpu, gpu, x, torch.randn(shape, generator=gen), DT[dtype], None if window else models.sinusoid_table(256, T, False))
+    eps = 2.0 ** -9 if dtype == "bf16" else 2.0 ** -12
+    assert {"dx", "d norm1.norm.weight", "d norm2.norm.bias"} <= set(err) or {"dx", "d norm1.weight", "d norm2.bias"} <= set(err)
+    for name, e in err.items():
+        assert e < (1e-5 if "norm1" in name and "running" in name else 4 * eps if "running" in name or name == "out" else 32 * eps), (name, e)
+
+
 def test_stochastic_depth_draws_like_the_modules():
     cpu, gpu = _layers("mfa", 1, 16, 27, 1, 64, 0.4, seed=1)
     gen = torch.Generator().manual_seed(0)
