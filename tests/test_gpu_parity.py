@@ -483,6 +483,23 @@ def test_wide_backward_however_sequences_are_cut(H, T, C, W, L, dtype):
             assert O.rel_l2(b.float(), ref) < TOL[dtype], name
 
 
+@pytest.mark.parametrize("H,T,C,W,L", [(8, 15, 32, 33, 16), (8, 64, 16, 80, 79), (5, 65, 32, 80, 0), (4, 129, 32, 70, 40), (2, 145, 64, 80, 41), (1, 97, 128, 65, 30),
+                                       (4, 400, 24, 40, 17)])
+def test_bias_gradient_of_a_full_launch(H, T, C, W, L):
+    """The sum of those of its samples a few at a time: the terms are the same to the bit, added in fp32 in another order."""
+    N, few = 1040 // H, 5
+    q, k, v, do = make_inputs(N * H, T, C, W, 19, torch.bfloat16, n=4, scale=C ** -0.5)
+    rpb = torch.randn(H, W, generator=torch.Generator().manual_seed(3)) * 0.5
+
+    def run(lo, hi):
+        leaves = [t[lo * H:hi * H].cuda().requires_grad_(True) for t in (q, k, v)] + [rpb.cuda().requires_grad_(True)]
+        na1d_fused(*leaves[:3], W, L, rpb=leaves[3], num_heads=H).backward(do[lo * H:hi * H].cuda())
+        return leaves[3].grad.double()
+
+    want = sum(run(lo, min(lo + few, N)) for lo in range(0, N, few))
+    assert O.rel_l2(run(0, N), want) < 1e-4
+
+
 @pytest.mark.parametrize("H,T,C,W,L,counts", [
     (8, 16, 16, 80, 40, (1, 300)), (8, 33, 32, 65, 32, (1, 16, 300)), (8, 64, 32, 49, 24, (1, 120)), (8, 64, 64, 65, 32, (2, 10, 130)), (8, 48, 64, 33, 16, (1, 4, 30)),
     (4, 80, 128, 33, 16, (1, 20, 80)), (8, 96, 64, 33, 16, (1, 12, 60)), (8, 97, 16, 33, 32, (1, 16, 130)), (1, 200, 24, 70, 69, (1, 11, 40)),
