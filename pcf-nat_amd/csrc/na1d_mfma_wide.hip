@@ -288,12 +288,13 @@ template <int C> constexpr int kQueryBuffers = C <= 32 ? 2 : 1;
 template <int C, int NBV> constexpr size_t wide_bwd_lds() {
     return (size_t)2 * region_bytes<C>(kRing<NBV>) + kStep * NBV * 2 * 512 + 2 * kQueryBuffers<C> * region_bytes<C>(kStep) + 2 * 64 * sizeof(float);
 }
-// Workgroups of a CU: what its LDS holds, and the registers with it (see the launch bounds).
-template <int C, int NBV> constexpr int wide_bwd_places() {
-    const int by_lds = (int)(128 / ((wide_bwd_lds<C, NBV>() + 1279) / 1280));
-    return by_lds < 4 ? by_lds : 4;
+// Workgroups of a CU: what its LDS holds, and the registers with it (see the launch bounds; a fifth workgroup, of 16 channels and
+// three blocks, is worth 2 to 9 % of a long launch; splits are planned with four).
+template <int C, int NBV> constexpr int wide_bwd_fit() { return (int)(128 / ((wide_bwd_lds<C, NBV>() + 1279) / 1280)); }
+template <int C, int NBV> constexpr int wide_bwd_places() { return std::min(wide_bwd_fit<C, NBV>(), 4); }
+template <int C, int NBV, bool DROP> constexpr int wide_bwd_waves() {
+    return DROP ? std::min(wide_bwd_places<C, NBV>(), NBV == 6 ? 2 : 3) : std::min(wide_bwd_fit<C, NBV>(), 5);
 }
-template <int C, int NBV, bool DROP> constexpr int wide_bwd_waves() { return DROP ? std::min(wide_bwd_places<C, NBV>(), NBV == 6 ? 2 : 3) : wide_bwd_places<C, NBV>(); }
 
 template <class DT, int C, int NBV, bool DROP>
 __global__ void __launch_bounds__(kThreads, (wide_bwd_waves<C, NBV, DROP>()))
@@ -537,7 +538,7 @@ wide_bwd_kernel(char *__restrict__ dq, char *__restrict__ dk, char *__restrict__
             }
 #pragma unroll
             for (int i = 0; i < kSets; ++i) {
-                if (vb + 3 < 4 * i || vb < 4 * i - 3 || set != i) continue;
+                if (vb < 4 * i - 3 || vb > 4 * i + 3 || set != i) continue;
 #pragma unroll
                 for (int ct = 0; ct < CT; ++ct) {
                     accv[i][ct] = Mma<DT>::k16(gt[ct], pb, accv[i][ct]);
@@ -819,7 +820,7 @@ inline size_t strip_lds(int nt, int nbv, const StripShape &w, int &kv_bytes) {
 // places ask for.
 template <int C, int NBV, bool DROP>
 inline Split walk_split(const Geom &g, const WideCover &c) {
-    const int64_t B = g.B * g.classes, places = 256 * wide_bwd_waves<C, NBV, DROP>();
+    const int64_t B = g.B * g.classes, places = 256 * std::min(wide_bwd_waves<C, NBV, DROP>(), 4);
     const int halo = c.nbv - 1 + ((c.shift & 15) ? 1 : 0);
     Split best{};
     int64_t least = INT64_MAX;
