@@ -22,11 +22,13 @@ using namespace enc;
 // =============================================================================
 // The sums of the forward are torch's (batch_norm_update_stats on [N, C, T]), to the bit.
 // What uses the statistics, and the backward, is bound by memory: a pass over 12800 x 256 16-bit values is 6.5 MB.  A
-// workgroup takes 64 channels (whole 128-byte lines) of one of up to 64 chunks of rows; the kernel that uses the backward's
+// workgroup takes 64 channels (whole 128-byte lines) of a chunk of rows; in the backward there are up to 64 chunks, and the kernel that uses the
 // sums adds them up itself (from L2) instead of waiting for a third launch, with 16 waves, since with few its workgroups are one to a CU
 // (8.9 -> 7.5 us; more workgroups read the sums more often: 9.7).  The forward, which reads none, has up to 256 chunks (6.0 -> 4.8).
 // 12800 x 256 backward, where torch took 54 us, and 13 us for each change of layout: 7.5 us behind the product that sums.
-constexpr int kBnCols = 64, kBnThreads = 256, kBnLanes = kBnThreads / 8, kBnChunks = 64, kBnParts = 256, kBnApplyThreads = 1024;
+constexpr int kBnCols = 64, kBnThreads = 256, kBnLanes = kBnThreads / 8, kBnApplyThreads = 1024;
+constexpr int kBnChunks = 64, kBnForwardChunks = 256, kBnParts = 256;         // kBnParts: rows of sums that the workspace holds
+static_assert(kBnChunks <= kBnParts, "a row of sums to a chunk");
 struct Chunks {
     int rows, count;          // rows of a chunk (the last may have fewer), chunks
 };
@@ -897,7 +899,7 @@ inline Geom attention_geom(const na1d_train_layer &l, int64_t N, int64_t T, Layo
 }
 
 template <class DT> int norm_apply(const na1d_train_layer &l, int which, char *y, const char *x, float *mean, float *rstd, int64_t M, const char *add, int64_t T, hipStream_t s) {
-    const Chunks c = bn_chunks(M, 256);
+    const Chunks c = bn_chunks(M, kBnForwardChunks);
     const na1d_train_norm &n = l.norm[which];
     bn_apply_kernel<DT><<<dim3((unsigned)(l.dim / kBnCols), (unsigned)c.count), kBnThreads, 0, s>>>(
         BnApply{y, x, n.batch_mean, n.batch_var, n.weight, n.bias, mean, rstd, n.batches, n.eps, (int)M, l.dim, c.rows, add, (int)T});
@@ -914,7 +916,7 @@ int to_channels(const na1d_train_layer &l, void *out, const void *x, int64_t N, 
 template <class DT>
 int product_and_norm_backward(Gemm a, const na1d_train_layer &l, int which, char *dx, const char *x, const char *add, const float *mean, const float *rstd, float *part,
                               hipStream_t s) {
-    const Chunks c = bn_chunks(a.M, 64);
+    const Chunks c = bn_chunks(a.M, kBnChunks);
     const dim3 grid((unsigned)(l.dim / kBnCols), (unsigned)c.count);
     float *part_dyx = part + (int64_t)kBnParts * l.dim;
     const int rows = gemm_rows(a.M, a.outputs);
