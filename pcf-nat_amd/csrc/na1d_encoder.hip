@@ -302,15 +302,22 @@ template <class DT, int MT, int NW, int PF, bool SPLIT, int QKV_AUX> struct Laye
     }
     // the rest of the layer: -> x2 in q_lds
     template <int G> __device__ inline void tail() {
-        using S = Groups<G, NW>;
-        if constexpr (G == 8) return tail_of_groups<8, MT>(0);
-        if constexpr (G == 4 && MT % 2 == 0) return tail_of_groups<4, MT / 2>((wave & 1) * MT / 2);
-        if constexpr (G == 4 && MT == 3) {       // two and one; waves w and w + 4 share a SIMD
+        if constexpr (G == 8)
+            tail_of_groups<8, MT>(0);
+        else if constexpr (G == 4 && MT % 2 == 0)
+            tail_of_groups<4, MT / 2>((wave & 1) * MT / 2);
+        else if constexpr (G == 4 && MT == 3) {  // two and one; waves w and w + 4 share a SIMD
             if ((wave ^ wave >> 2) & 1)
-                return tail_of_groups<4, 1>(2);
+                tail_of_groups<4, 1>(2);
             else
-                return tail_of_groups<4, 2>(0);
+                tail_of_groups<4, 2>(0);
+        } else {
+            tail_in_chunks<G>();
         }
+    }
+    // through LDS, 256 hidden channels at a time
+    template <int G> __device__ inline void tail_in_chunks() {
+        using S = Groups<G, NW>;
         const Rsrc w1 = weight_rsrc(a.w_fc1, kHidden, kDim), w2 = weight_rsrc(a.w_fc2, kDim, kHidden);
         project<G>(w1, 0);
         // Outputs that a later chunk adds nothing to are written at once, over x1: the chunks behind read other channels.
