@@ -574,8 +574,9 @@ __device__ inline uint32_t xcd_item(uint32_t wg, uint32_t items) {
     return (wg & 7) * per + (wg >> 3);
 }
 
-// The sums of the bias gradient that a backward will add to, set to zero by the forward's first workgroup behind its copies: as a
-// launch of its own in the backward this took the host 5 us of a training layer's 60 (and the GPU 1.5; here nothing that shows).
+// The sums of the bias gradient that a backward will add to, set to zero by the forward's first workgroup behind its copies: a
+// launch less in a backward that its host paces (with its allocation a training layer's pass of 128 x 8 x 300 x 32 went from 80..83
+// to 75..78 us on three boxes, about what two runs of one side differ by; of the GPU it took 1.5, here nothing that shows).
 template <int THREADS> __device__ inline void clear_sums(float *sums, int count) {
     if (sums && blockIdx.x == 0)
         for (int i = threadIdx.x; i < count; i += THREADS) sums[i] = 0.f;

@@ -278,10 +278,10 @@ __device__ inline void add_slot_sums(LDS_PTR(float) rsum, float *drpb, float *dr
 //     complete behind each step.
 // K and V lie in rings of LDS, whose next four tiles are fetched behind pass 1, Q and dO in two buffers up to 32 channels
 // (beyond, a second buffer would cost a workgroup of the CU).
-// Bound by vector instructions, LDS reads and memory in turn.  In strips, with HB + HA query
-// tiles worked out by the neighbours too (at 65 slots as many as a strip's own), and walking, us in a trace: 128 x 8 heads of
-// 300 x 32, W = 65: 57.3 -> 35.9 (3.8 TB/s of what is read and written once), W = 33: 31.7 -> 26.7, W = 80: 112 -> 44; 16 x 4 of
-// 2000 x 64, W = 65: 68 -> 32; 16 x 8 of 1000 x 128: 112 -> 66.
+// Bound by vector instructions, LDS reads and memory in turn.  In strips, with HB + HA query tiles worked out by the neighbours
+// too (at 65 slots as many as a strip's own), and walking, us in a trace: 128 x 8 heads of 300 x 32, W = 65: 57.3 and 36.2
+// (3.8 TB/s of what is read and written once), W = 33: 31.7 and 28.0, W = 80: 123 and 46; 16 x 4 of 2000 x 64, W = 65: 66 and
+// 31; 16 x 8 of 1000 x 128: 111 and 67.
 constexpr int kStep = kWaves;            // query tiles of a step
 template <int NBV> constexpr int kRing = NBV <= 5 ? 8 : 12;            // key tiles that a step reads, in whole steps
 template <int C> constexpr int kQueryBuffers = C <= 32 ? 2 : 1;
